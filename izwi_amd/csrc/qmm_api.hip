@@ -1135,6 +1135,54 @@ namespace {
 int batched_group_on_records(const izwi_qmm_weight* const* weights, int32_t n_weights, const float* x, int64_t m,
                              float* const* ys, void* records, hipStream_t stream);
 
+// The members of a group on bf16 activations, one launch per block type (types in the order of their
+// first members); the launches follow each other on the stream and share the workspace.
+template <class F>
+void for_each_type(const izwi_qmm_weight* const* weights, int32_t n_weights, F&& f) {
+    bool done[QMM_MAX_GROUP] = {};
+    for (int i = 0; i < n_weights; i++) {
+        if (done[i]) continue;
+        int index[QMM_MAX_GROUP], n_sub = 0;
+        for (int j = i; j < n_weights; j++)
+            if (!done[j] && weights[j]->layout.dtype == weights[i]->layout.dtype) index[n_sub++] = j, done[j] = true;
+        f(index, n_sub);
+    }
+}
+
+size_t group_bf16_workspace(const izwi_qmm_weight* const* weights, int32_t n_weights, int64_t m) {
+    size_t need = 0;
+    for_each_type(weights, n_weights, [&](const int* index, int n_sub) {
+        const QmmLayout* layouts[QMM_MAX_GROUP];
+        for (int i = 0; i < n_sub; i++) {
+            layouts[i] = &weights[index[i]]->layout;
+            need = std::max(need, qmm_gemm_workspace_bytes(*layouts[i], m, weights[0]->n_cus));
+        }
+        if (n_sub > 1) need = std::max(need, qmm_gemm_group_workspace_bytes(layouts, n_sub, m, weights[0]->n_cus));
+    });
+    return need;
+}
+
+hipError_t group_bf16_launch(const izwi_qmm_weight* const* weights, int32_t n_weights, const uint16_t* x_bf16, int64_t m,
+                             void* const* ys, int out_bf16, void* workspace, hipStream_t stream) {
+    hipError_t e = hipSuccess;
+    for_each_type(weights, n_weights, [&](const int* index, int n_sub) {
+        if (e != hipSuccess) return;
+        const QmmLayout* layouts[QMM_MAX_GROUP];
+        const void* tiled[QMM_MAX_GROUP];
+        void* outs[QMM_MAX_GROUP];
+        for (int i = 0; i < n_sub; i++)
+            layouts[i] = &weights[index[i]]->layout, tiled[i] = weights[index[i]]->tiled, outs[i] = ys[index[i]];
+        e = n_sub > 1 ? qmm_launch_gemm_bf16_multi(layouts, tiled, n_sub, x_bf16, m, outs, out_bf16, workspace, weights[0]->n_cus, stream)
+                      : hipErrorNotSupported;
+        if (e != hipErrorNotSupported) return;
+        (void)hipGetLastError();
+        e = hipSuccess;
+        for (int i = 0; i < n_sub && e == hipSuccess; i++)
+            e = qmm_launch_gemm_bf16(*layouts[i], tiled[i], x_bf16, m, outs[i], out_bf16, workspace, weights[0]->n_cus, stream);
+    });
+    return e;
+}
+
 int forward_group_impl(const izwi_qmm_weight* const* weights, int32_t n_weights, const float* x, int64_t m,
                        float* const* ys, int mem_space, void* stream_, const float* norm_weight, float norm_eps) {
     QmmCallScope call;
@@ -1226,25 +1274,19 @@ int forward_group_impl(const izwi_qmm_weight* const* weights, int32_t n_weights,
     }
     if (by_type) return call_by_type(x, nullptr);
     // prefill sizes on the bf16 matrix cores: the activations are converted once and the members
-    // share one launch (its grid is the members' column tiles one after the other)
-    if (mem_space == IZWI_QMM_DEVICE && uniform && n_weights >= 2 && m > 128 && large_m_mode() == IZWI_QMM_LARGE_M_BF16) {
+    // of a type share one launch (its grid is the members' column tiles one after the other)
+    if (mem_space == IZWI_QMM_DEVICE && splittable && n_weights >= 2 && m > 64 && large_m_mode() == IZWI_QMM_LARGE_M_BF16) {
         hipStream_t stream = (hipStream_t)stream_;
         const izwi_qmm_weight* w0 = weights[0];
-        const QmmLayout* layouts[QMM_MAX_GROUP];
-        const void* tiled[QMM_MAX_GROUP];
-        void* outs[QMM_MAX_GROUP];
-        for (int i = 0; i < n_weights; i++) layouts[i] = &weights[i]->layout, tiled[i] = weights[i]->tiled, outs[i] = ys[i];
         const size_t xb_bytes = (((size_t)m * w0->layout.k * sizeof(uint16_t)) + 255) & ~(size_t)255;
-        const size_t ws_bytes = qmm_gemm_group_workspace_bytes(layouts, n_weights, m, w0->n_cus);
-        void* xb = nullptr;
-        HIP_TRY(get_scratch(w0->device, stream, xb_bytes + ws_bytes, &xb));
+        uint8_t* xb = nullptr;
+        HIP_TRY(get_scratch(w0->device, stream, xb_bytes + group_bf16_workspace(weights, n_weights, m), (void**)&xb));
         ProfileScope prof(w0, stream);
         HIP_TRY(qmm_launch_f32_to_bf16(x, (uint16_t*)xb, m * w0->layout.k, stream));
-        hipError_t e = qmm_launch_gemm_bf16_multi(layouts, tiled, n_weights, (const uint16_t*)xb, m, outs, 0,
-                                                  ws_bytes ? (uint8_t*)xb + xb_bytes : nullptr, w0->n_cus, stream);
-        if (e == hipSuccess) return IZWI_QMM_OK;
-        if (e != hipErrorNotSupported) return fail_hip(e, "grouped prefill kernel");
-        (void)hipGetLastError();
+        void* outs[QMM_MAX_GROUP];
+        for (int i = 0; i < n_weights; i++) outs[i] = ys[i];
+        HIP_TRY(group_bf16_launch(weights, n_weights, (const uint16_t*)xb, m, outs, 0, xb + xb_bytes, stream));
+        return IZWI_QMM_OK;
     }
     // host buffers, mixed types, prefill sizes: one call per projection (same results)
     if (mem_space != IZWI_QMM_DEVICE || !uniform || n_weights == 1 || m > 64) {
@@ -1303,6 +1345,30 @@ int batched_group_on_records(const izwi_qmm_weight* const* weights, int32_t n_we
 
 int gate_up_silu_impl(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, const float* x, int64_t m, float* h,
                       int mem_space, void* stream_, const float* norm_weight, float norm_eps);
+
+// gate | up at prefill sizes (m > 64, bf16 arithmetic) and silu(gate) * up as f32 or bf16, in
+// gate_up_prefill_bytes of scratch at `ws`: the two products | bf16 x | the group's workspace.
+size_t gate_up_prefill_bytes(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, int64_t m) {
+    const QmmLayout& L = gate->layout;
+    const izwi_qmm_weight* ws[2] = {gate, up};
+    const size_t part = ((size_t)m * L.n * sizeof(float) + 255) & ~(size_t)255;
+    return 2 * part + (((size_t)m * L.k * sizeof(uint16_t) + 255) & ~(size_t)255) + group_bf16_workspace(ws, 2, m);
+}
+
+int gate_up_prefill(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, const float* x, int64_t m, void* h, int h_bf16, uint8_t* ws,
+                    hipStream_t stream) {
+    const QmmLayout& L = gate->layout;
+    const izwi_qmm_weight* gu[2] = {gate, up};
+    const size_t part = ((size_t)m * L.n * sizeof(float) + 255) & ~(size_t)255;
+    void* ys[2] = {ws, ws + part};
+    uint16_t* xb = reinterpret_cast<uint16_t*>(ws + 2 * part);
+    uint8_t* group_ws = ws + 2 * part + (((size_t)m * L.k * sizeof(uint16_t) + 255) & ~(size_t)255);
+    ProfileScope prof(gate, stream);
+    HIP_TRY(qmm_launch_f32_to_bf16(x, xb, m * L.k, stream));
+    HIP_TRY(group_bf16_launch(gu, 2, xb, m, ys, 0, group_ws, stream));
+    HIP_TRY(qmm_launch_silu_mul((const float*)ys[0], (const float*)ys[1], h, h_bf16, m * L.n, stream));
+    return IZWI_QMM_OK;
+}
 
 } // namespace
 
@@ -1374,9 +1440,20 @@ int izwi_qmm_mlp_forward_f32(const izwi_qmm_weight* gate, const izwi_qmm_weight*
         HIP_TRY(qmm_launch_quantize_silu_mul_ws(D.dtype, g, u, m, D.k, rec_h, stream));
         float* dy[1] = {(float*)yo.dev};
         if (int rc = batched_group_on_records(&down, 1, nullptr, m, dy, rec_h, stream)) return rc;
+    } else if (m > 64 && large_m_mode() == IZWI_QMM_LARGE_M_BF16 && G.dtype == U.dtype) {
+        // Prefill sizes: the activation is rounded to bf16 where it is computed, down reads it as it is
+        // (scratch: workspace of either product | bf16 intermediate | what gate | up takes)
+        const size_t ws_bytes = align256(qmm_gemm_workspace_bytes(D, m, down->n_cus)), hb_bytes = align256((size_t)m * D.k * sizeof(uint16_t));
+        uint8_t* ws = nullptr;
+        HIP_TRY(get_scratch(gate->device, stream, ws_bytes + hb_bytes + gate_up_prefill_bytes(gate, up, m), (void**)&ws));
+        uint16_t* hb = reinterpret_cast<uint16_t*>(ws + ws_bytes);
+        if (profiling()) g_silu_fused.fetch_add(1, std::memory_order_relaxed);
+        if (int rc = gate_up_prefill(gate, up, (const float*)xi.dev, m, hb, 1, ws + ws_bytes + hb_bytes, stream)) return rc;
+        ProfileScope prof(down, stream);
+        HIP_TRY(qmm_launch_gemm_bf16(D, down->tiled, hb, m, yo.dev, 0, ws_bytes ? ws : nullptr, down->n_cus, stream));
     } else {
-        // One or two rows (the activation is applied inside the gate | up launch), prefill sizes and
-        // a gate / up pair of two block types: the two calls, with the intermediate in the stream's
+        // One or two rows (the activation is applied inside the gate | up launch), the integer arithmetic
+        // beyond 64 rows and a gate / up pair of two block types: the two calls, with the intermediate in the stream's
         // scratch behind everything those calls use of it themselves.
         const size_t gu_need = forward_scratch_need(G, m, gate->n_cus) + align256((size_t)m * G.k * sizeof(float)) + 2 * part + 1024;
         const size_t d_need = forward_scratch_need(D, m, down->n_cus);
@@ -1461,6 +1538,16 @@ int gate_up_silu_impl(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, co
         ProfileScope prof(gate, stream);
         HIP_TRY(qmm_launch_gemv_gated(L, gate->tiled, up->tiled, xin, m, (float*)ho.dev, gate->n_cus, stream,
                                       norm_weight ? &norm : nullptr));
+    } else if (m > 64 && large_m_mode() == IZWI_QMM_LARGE_M_BF16) {
+        uint8_t* ws = nullptr;
+        const size_t need = (gate_up_prefill_bytes(gate, up, m) + 255) & ~(size_t)255;
+        if (norm_weight) { // the normalized activations behind everything else
+            float* normed = nullptr;
+            if (int rc = normed_copy(gate, xin, m, (const float*)wi.dev, norm_eps, need, 0, stream, &normed)) return rc;
+            xin = normed;
+        }
+        HIP_TRY(get_scratch(gate->device, stream, need, (void**)&ws));
+        if (int rc = gate_up_prefill(gate, up, xin, m, ho.dev, 0, ws, stream)) return rc;
     } else {
         size_t behind = 0; // bytes of the scratch buffer's start that hold the normalized activations
         if (norm_weight) {
@@ -1479,9 +1566,7 @@ int gate_up_silu_impl(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, co
         {
             // the group call below uses the start of the same per-stream scratch for the quantized
             // activations: its own need comes first, the two outputs behind it
-            const size_t group_need =
-                m <= 64 ? qmm_gemv_mfma_workspace_bytes(L, m)
-                        : ((((size_t)m * L.k * sizeof(uint16_t)) + 255) & ~(size_t)255) + qmm_gemm_workspace_bytes(L, m, gate->n_cus);
+            const size_t group_need = qmm_gemv_mfma_workspace_bytes(L, m < 64 ? m : 64);
             const size_t base = std::max((group_need + 255) & ~(size_t)255, behind);
             void* scratch = nullptr;
             HIP_TRY(get_scratch(gate->device, stream, base + 2 * part, &scratch));
@@ -1490,7 +1575,7 @@ int gate_up_silu_impl(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, co
         const izwi_qmm_weight* ws[2] = {gate, up};
         float* ys[2] = {static_cast<float*>(gu), reinterpret_cast<float*>(static_cast<uint8_t*>(gu) + part)};
         if (int rc = izwi_qmm_forward_group_f32(ws, 2, xin, m, ys, IZWI_QMM_DEVICE, stream_)) return rc;
-        HIP_TRY(qmm_launch_silu_mul(ys[0], ys[1], (float*)ho.dev, (int64_t)m * L.n, stream));
+        HIP_TRY(qmm_launch_silu_mul(ys[0], ys[1], ho.dev, 0, (int64_t)m * L.n, stream));
     }
     HIP_TRY(ho.finish(stream));
     return IZWI_QMM_OK;
@@ -1540,7 +1625,7 @@ int izwi_qmm_forward_group_bf16(const izwi_qmm_weight* const* weights, int32_t n
     if (int rc = check_space(mem_space)) return rc;
     if (out_dtype != IZWI_QMM_OUT_F32 && out_dtype != IZWI_QMM_OUT_BF16)
         return fail(IZWI_QMM_ERR_INVALID, "bad out_dtype %d", out_dtype);
-    bool uniform = true;
+    bool splittable = true;
     for (int i = 0; i < n_weights; i++) {
         if (!weights[i]) return fail(IZWI_QMM_ERR_INVALID, "NULL weight");
         const QmmLayout& L = weights[i]->layout;
@@ -1548,27 +1633,21 @@ int izwi_qmm_forward_group_bf16(const izwi_qmm_weight* const* weights, int32_t n
         if (L.k != weights[0]->layout.k)
             return fail(IZWI_QMM_ERR_INVALID, "projection group input mismatch: expected %lld, got %lld",
                         (long long)weights[0]->layout.k, (long long)L.k);
-        if (L.dtype != weights[0]->layout.dtype || L.n == 0 || weights[i]->device != weights[0]->device) uniform = false;
+        if (L.n == 0 || weights[i]->device != weights[0]->device) splittable = false;
         if (m > 0 && L.n > 0 && !ys[i]) return fail(IZWI_QMM_ERR_INVALID, "y is NULL");
     }
     if (m < 0) return fail(IZWI_QMM_ERR_INVALID, "negative m");
     if (m == 0) return IZWI_QMM_OK;
     if (!x_bf16) return fail(IZWI_QMM_ERR_INVALID, "x is NULL");
-    if (mem_space == IZWI_QMM_DEVICE && uniform && n_weights >= 2 && m > 128) {
+    if (mem_space == IZWI_QMM_DEVICE && splittable && n_weights >= 2) {
         hipStream_t stream = (hipStream_t)stream_;
         const izwi_qmm_weight* w0 = weights[0];
-        const QmmLayout* layouts[QMM_MAX_GROUP];
-        const void* tiled[QMM_MAX_GROUP];
-        for (int i = 0; i < n_weights; i++) layouts[i] = &weights[i]->layout, tiled[i] = weights[i]->tiled;
         void* workspace = nullptr;
-        if (const size_t ws_bytes = qmm_gemm_group_workspace_bytes(layouts, n_weights, m, w0->n_cus))
+        if (const size_t ws_bytes = group_bf16_workspace(weights, n_weights, m))
             HIP_TRY(get_scratch(w0->device, stream, ws_bytes, &workspace));
         ProfileScope prof(w0, stream);
-        hipError_t e = qmm_launch_gemm_bf16_multi(layouts, tiled, n_weights, x_bf16, m, ys, out_dtype == IZWI_QMM_OUT_BF16,
-                                                  workspace, w0->n_cus, stream);
-        if (e == hipSuccess) return IZWI_QMM_OK;
-        if (e != hipErrorNotSupported) return fail_hip(e, "grouped prefill kernel");
-        (void)hipGetLastError();
+        HIP_TRY(group_bf16_launch(weights, n_weights, x_bf16, m, ys, out_dtype == IZWI_QMM_OUT_BF16, workspace, stream));
+        return IZWI_QMM_OK;
     }
     for (int i = 0; i < n_weights; i++)
         if (int rc = izwi_qmm_forward_bf16(weights[i], x_bf16, m, ys[i], out_dtype, mem_space, stream_)) return rc;

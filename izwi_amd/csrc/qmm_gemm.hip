@@ -1,8 +1,9 @@
 // Prefill kernel: y[m, n] = x[m, k] * dequant(W)[n, k]^T with bf16 MFMA.
 //
-// A workgroup (4 waves, 2 x 2) owns a BM x BN output tile (256 x 256 when the
-// problem fills the chip with such tiles, smaller tiles otherwise); each wave
-// a (BM/2) x (BN/2) sub-tile held in v_mfma_f32_32x32x16_bf16 accumulators.
+// A workgroup (8 waves, 4 x 2) owns a BM x BN output tile (256 x 256 when the
+// problem fills the chip with such tiles, 256 x 128 otherwise; few rows and small
+// products take qmm_gemm_regb.hip); each wave a (BM/4) x (BN/2) sub-tile held in
+// v_mfma_f32_32x32x16_bf16 accumulators.
 // Per 64-wide k step the workgroup
 //   * copies the BM x 64 bf16 activation tile to LDS,
 //   * reads the matching 64 k-elements of BN weight rows straight from the
@@ -32,7 +33,6 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int BK = 64;
-constexpr int kThreads = 256;
 constexpr int kRowStride = 144; // bytes per LDS tile row: 64 bf16 + 16 B pad
 #ifndef QMM_GEMM_VALU_PER_MFMA
 #define QMM_GEMM_VALU_PER_MFMA 4
@@ -81,279 +81,6 @@ __device__ __forceinline__ float ubyte_f32(uint32_t v) {
     return (float)((v >> (8 * N)) & 0xffu);
 }
 
-// Quant chunks a thread holds for its share of one weight row and k step.
-template <int QT, int TPR>
-struct WRegs {
-    static constexpr int NC = (QT == QMM_Q4_K ? 2 : 4) / TPR;
-    u32x4 hdr;
-    u32x4 q[NC];
-    // Q6_K only (two threads per row): the 32 bytes of high bit pairs and the chunk with d
-    u32x4 qh[2];
-    u32x4 dch;
-};
-
-// Weight row `row`, k step kt (64 elements), part `part` of TPR: header + chunks.
-template <int QT, int TPR>
-__device__ __forceinline__ void load_w(WRegs<QT, TPR>& r, const GemmParams& P, int64_t row, int kt,
-                                       int part) {
-    constexpr int NC = WRegs<QT, TPR>::NC;
-    const int unit = kt >> 2, sub = kt & 3;
-    // branch-free: out-of-range rows / units read a valid address and are zeroed by a select
-    // when the tile is written to LDS, so the k loop stays one basic block and loads, LDS
-    // traffic and MFMAs can interleave
-    const bool ok = (row >> 4) < P.row_tiles && unit < P.k_units;
-    const int64_t rt = ok ? (row >> 4) : 0;
-    const int u = ok ? unit : 0;
-    const int kg = u / P.s, us = u - kg * P.s;
-    const int slot = us * 16 + (int)(row & 15);
-    const u32x4* base =
-        reinterpret_cast<const u32x4*>(P.w + (rt * P.k_groups + kg) * P.panel_bytes) + slot;
-    // (the select itself happens in store_w: applying it here would make every load wait)
-    r.hdr = base[0];
-    if (QT == QMM_Q6_K) {
-        // the 64 elements of step `sub` are one nibble (sub & 1) of the 64 ql bytes of half
-        // sub >> 1 and one bit pair of its 32 qh bytes; byte e of the 64 pairs with qh byte e % 32
-        static_assert(QT != QMM_Q6_K || TPR == 2, "Q6_K tiles use two threads per weight row");
-        const int h = sub >> 1;
-#pragma unroll
-        for (int c = 0; c < NC; c++) r.q[c] = base[(size_t)(1 + 4 * h + part * NC + c) * P.slots];
-        r.qh[0] = base[(size_t)(9 + 2 * h) * P.slots];
-        r.qh[1] = base[(size_t)(10 + 2 * h) * P.slots];
-        r.dch = base[(size_t)13 * P.slots];
-        return;
-    }
-#pragma unroll
-    for (int c = 0; c < NC; c++) r.q[c] = base[(size_t)(1 + sub * NC * TPR + part * NC + c) * P.slots];
-}
-
-// Dequantizes the thread's share of the 64 k-elements to bf16 and writes it to the LDS row.
-template <int QT, int TPR>
-__device__ __forceinline__ void store_w(const WRegs<QT, TPR>& r, int kt, int part, bool ok,
-                                        uint8_t* lds_row) {
-    constexpr int NC = WRegs<QT, TPR>::NC;
-    // This kernel's results are compared within a tolerance (bf16 operands), so the
-    // dequantization may use fused multiply-adds and per-byte converts:
-    // 1 convert + 1 fma + half a pack per weight.
-    if (QT == QMM_Q4_K) {
-        const int g = kt & 3;
-        // a row or unit outside the matrix gets zero scales: every weight becomes 0, no branch
-        const float d = ok ? qmm_f16_bits_to_f32((uint16_t)(r.hdr.x & 0xffffu)) : 0.0f;
-        const float dmin = ok ? qmm_f16_bits_to_f32((uint16_t)(r.hdr.x >> 16)) : 0.0f;
-        uint32_t sc_lo, sc_hi, mn_lo, mn_hi;
-        qmm_unpack_q4k_scales(r.hdr.y, r.hdr.z, r.hdr.w, sc_lo, sc_hi, mn_lo, mn_hi);
-        const float d1 = d * (float)qmm_byte_of(sc_lo, sc_hi, 2 * g);
-        const float m1 = -(dmin * (float)qmm_byte_of(mn_lo, mn_hi, 2 * g));
-        const float d2 = d * (float)qmm_byte_of(sc_lo, sc_hi, 2 * g + 1);
-        const float m2 = -(dmin * (float)qmm_byte_of(mn_lo, mn_hi, 2 * g + 1));
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            const int h = part * NC + c; // which 16-byte half of the 32 nibble bytes
-            uint32_t lo[8], hi[8];
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const uint32_t vl = r.q[c][j] & 0x0f0f0f0fu, vh = (r.q[c][j] >> 4) & 0x0f0f0f0fu;
-                lo[2 * j] = pack_bf16(__builtin_fmaf(d1, ubyte_f32<0>(vl), m1),
-                                      __builtin_fmaf(d1, ubyte_f32<1>(vl), m1));
-                lo[2 * j + 1] = pack_bf16(__builtin_fmaf(d1, ubyte_f32<2>(vl), m1),
-                                          __builtin_fmaf(d1, ubyte_f32<3>(vl), m1));
-                hi[2 * j] = pack_bf16(__builtin_fmaf(d2, ubyte_f32<0>(vh), m2),
-                                      __builtin_fmaf(d2, ubyte_f32<1>(vh), m2));
-                hi[2 * j + 1] = pack_bf16(__builtin_fmaf(d2, ubyte_f32<2>(vh), m2),
-                                          __builtin_fmaf(d2, ubyte_f32<3>(vh), m2));
-            }
-            // low nibbles: k 16h .. 16h+15, high nibbles: k 32 + 16h ..
-            uint4* dl = reinterpret_cast<uint4*>(lds_row + 32 * h);
-            uint4* dh = reinterpret_cast<uint4*>(lds_row + 64 + 32 * h);
-            dl[0] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-            dl[1] = make_uint4(lo[4], lo[5], lo[6], lo[7]);
-            dh[0] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-            dh[1] = make_uint4(hi[4], hi[5], hi[6], hi[7]);
-        }
-    } else if (QT == QMM_Q6_K) {
-        // part p holds the elements 32 p .. 32 p + 31 of the step: nibble s1 of its two ql chunks,
-        // bit pair 4 s1 + 2 p of the 32 qh bytes; the 16-element groups 4 sub + 2 p, + 1 carry
-        // the scales.  w = d * scale * (q - 32) as one fma per weight.
-        const int sub = kt & 3, s1 = sub & 1;
-        const float d = ok ? qmm_f16_bits_to_f32((uint16_t)(r.dch.x & 0xffffu)) : 0.0f;
-        const uint32_t hw[4] = {r.hdr.x, r.hdr.y, r.hdr.z, r.hdr.w};
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            const int j = 4 * sub + 2 * part + c;
-            const float ds = d * (float)(int8_t)((hw[j >> 2] >> (8 * (j & 3))) & 0xffu);
-            const float bias = -32.0f * ds;
-            uint32_t o[8];
-#pragma unroll
-            for (int w = 0; w < 4; w++) {
-                const uint32_t nib = (r.q[c][w] >> (4 * s1)) & 0x0f0f0f0fu;
-                const uint32_t two = (r.qh[c][w] >> (4 * s1 + 2 * part)) & 0x03030303u;
-                const uint32_t q6 = nib | (two << 4);
-                o[2 * w] = pack_bf16(__builtin_fmaf(ds, ubyte_f32<0>(q6), bias),
-                                     __builtin_fmaf(ds, ubyte_f32<1>(q6), bias));
-                o[2 * w + 1] = pack_bf16(__builtin_fmaf(ds, ubyte_f32<2>(q6), bias),
-                                         __builtin_fmaf(ds, ubyte_f32<3>(q6), bias));
-            }
-            uint4* dst = reinterpret_cast<uint4*>(lds_row + 64 * part + 32 * c);
-            dst[0] = make_uint4(o[0], o[1], o[2], o[3]);
-            dst[1] = make_uint4(o[4], o[5], o[6], o[7]);
-        }
-    } else {
-        const int b0 = (kt & 3) * 2; // first of the two 32-element blocks of this k step
-        const uint32_t hw[4] = {r.hdr.x, r.hdr.y, r.hdr.z, r.hdr.w};
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            const int cc = part * NC + c; // chunk 0..3 of the step: block cc / 2, half cc % 2
-            const int b = b0 + (cc >> 1);
-            const float d =
-                ok ? qmm_f16_bits_to_f32((uint16_t)((hw[b >> 1] >> (16 * (b & 1))) & 0xffffu)) : 0.0f;
-            const float bias = -128.0f * d; // int8 q as unsigned byte u = q + 128: q * d = u * d - 128 d
-            uint32_t o[8];
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const uint32_t u = r.q[c][j] ^ 0x80808080u;
-                o[2 * j] = pack_bf16(__builtin_fmaf(d, ubyte_f32<0>(u), bias),
-                                     __builtin_fmaf(d, ubyte_f32<1>(u), bias));
-                o[2 * j + 1] = pack_bf16(__builtin_fmaf(d, ubyte_f32<2>(u), bias),
-                                         __builtin_fmaf(d, ubyte_f32<3>(u), bias));
-            }
-            uint4* dst = reinterpret_cast<uint4*>(lds_row + 32 * cc);
-            dst[0] = make_uint4(o[0], o[1], o[2], o[3]);
-            dst[1] = make_uint4(o[4], o[5], o[6], o[7]);
-        }
-    }
-}
-
-template <int QT, int BM, int BN>
-__global__ __launch_bounds__(kThreads) void gemm_kernel(GemmParams P) {
-    constexpr int MT = BM / 64, NT = BN / 64; // 32x32 MFMA tiles per wave in m and n
-    constexpr int XC = BM / 32;               // 16-byte activation chunks per thread and k step
-    constexpr int TPR = kThreads / BN;        // threads sharing one weight row
-    constexpr int kStage = (BM + BN) * kRowStride;
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-
-    // consecutive workgroups walk down m inside one weight column block, so the
-    // weight rows they share stay in L2 while all of m is swept
-    const int tm = blockIdx.x % P.tiles_m;
-    const int tn = blockIdx.x / P.tiles_m;
-    const int64_t m0 = (int64_t)tm * BM, n0 = P.n_begin + (int64_t)tn * BN;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int k_steps = P.k_units * 4;
-    const int w_row = tid % BN, w_part = tid / BN;
-
-    f32x16 acc[MT][NT];
-#pragma unroll
-    for (int i = 0; i < MT; i++)
-#pragma unroll
-        for (int j = 0; j < NT; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
-
-    // activation tile: BM rows x 8 chunks of 16 B; thread t copies chunks t + 256 i
-    u32x4 xr[XC];
-    WRegs<QT, TPR> wr;
-    // rows past m read row m-1 (their results are never stored); k is a multiple of 32, so a
-    // 16-byte chunk is entirely inside or outside [0, k): outside chunks become zeros
-    auto load_x = [&](int kt) {
-#pragma unroll
-        for (int i = 0; i < XC; i++) {
-            const int c = tid + kThreads * i;
-            const int row = c >> 3, kc = c & 7;
-            const int64_t gm = min(m0 + row, P.m - 1);
-            const int64_t gk = (int64_t)kt * BK + kc * 8;
-            xr[i] = *reinterpret_cast<const u32x4*>(P.x + gm * P.k + (gk < P.k ? gk : 0));
-        }
-    };
-    auto store_tile = [&](int kt, uint8_t* stage) {
-#pragma unroll
-        for (int i = 0; i < XC; i++) {
-            const int c = tid + kThreads * i;
-            const int row = c >> 3, kc = c & 7;
-            const bool ok = (int64_t)kt * BK + kc * 8 < P.k;
-            *reinterpret_cast<u32x4*>(stage + row * kRowStride + kc * 16) = ok ? xr[i] : u32x4{0, 0, 0, 0};
-        }
-        const bool w_ok = ((n0 + w_row) >> 4) < P.row_tiles && (kt >> 2) < P.k_units;
-        store_w<QT, TPR>(wr, kt, w_part, w_ok, stage + (BM + w_row) * kRowStride);
-    };
-    auto load_tile = [&](int kt) {
-        load_x(kt);
-        load_w<QT, TPR>(wr, P, n0 + w_row, kt, w_part);
-    };
-
-    load_tile(0);
-    store_tile(0, smem);
-    if (k_steps > 1) load_tile(1);
-    __syncthreads();
-
-    // One k step: MFMAs out of `cur`; with FEED, the next step's tile (in registers since the
-    // previous step) is dequantized into `next` and the loads of the step after are issued.
-    // No branch inside, so the whole step is one basic block and the scheduler is free to
-    // interleave LDS traffic, dequantization and global loads with the MFMAs.
-    auto k_step = [&](int kt, const uint8_t* cur, uint8_t* next, auto feed) {
-        constexpr bool FEED = decltype(feed)::value;
-        const uint8_t* xs = cur;
-        const uint8_t* ws = cur + BM * kRowStride;
-#pragma unroll
-        for (int kk = 0; kk < 4; kk++) {
-            const int koff = kk * 32 + (lane >> 5) * 16; // bytes inside the tile row
-            bf16x8 a[MT], b[NT];
-#pragma unroll
-            for (int i = 0; i < MT; i++)
-                a[i] = *reinterpret_cast<const bf16x8*>(
-                    xs + (wm * (BM / 2) + i * 32 + (lane & 31)) * kRowStride + koff);
-#pragma unroll
-            for (int j = 0; j < NT; j++)
-                b[j] = *reinterpret_cast<const bf16x8*>(
-                    ws + (wn * (BN / 2) + j * 32 + (lane & 31)) * kRowStride + koff);
-#pragma unroll
-            for (int i = 0; i < MT; i++)
-#pragma unroll
-                for (int j = 0; j < NT; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-            if (FEED && kk == 0) {
-                store_tile(kt + 1, next);
-                load_tile(kt + 2); // past the end this reads a valid address and yields zeros
-            }
-        }
-#ifdef QMM_GEMM_SCHED
-        if (FEED) {
-#pragma unroll
-            for (int i = 0; i < MT * NT * 4; i++) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); // one MFMA
-                __builtin_amdgcn_sched_group_barrier(0x002, QMM_GEMM_SCHED, 0); // VALU
-                if (i % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); // DS read
-                if (i % 4 == 1) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0); // DS write
-                if (i % 5 == 3) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0); // VMEM read
-            }
-        }
-#endif
-        __syncthreads();
-    };
-    for (int kt = 0; kt + 1 < k_steps; kt++)
-        k_step(kt, smem + (kt & 1) * kStage, smem + ((kt + 1) & 1) * kStage, std::true_type{});
-    k_step(k_steps - 1, smem + ((k_steps - 1) & 1) * kStage, nullptr, std::false_type{});
-
-    // D[i][j]: lane holds column j = lane % 32 and rows 8*(r/4) + 4*(lane/32) + r%4
-#pragma unroll
-    for (int i = 0; i < MT; i++) {
-#pragma unroll
-        for (int j = 0; j < NT; j++) {
-            const int64_t gn = n0 + wn * (BN / 2) + j * 32 + (lane & 31);
-            if (gn >= P.n_end) continue;
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int64_t gm = m0 + wm * (BM / 2) + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (gm >= P.m) continue;
-                qmm_store(P.y, QmmEpilogue{P.residual, P.out_bf16}, gm * P.n + gn, acc[i][j][r]);
-            }
-        }
-    }
-}
-
-// ---- software-pipelined variant (BN = 256: one weight row per thread) ----------------
-// With one wave per SIMD nothing hides a wave's own non-matrix work, so the next tile's
-// staging (dequantization, LDS writes, global loads) is cut into slices and one slice
-// is placed after every group of four MFMAs; scheduling fences keep the slices there.
-// The MFMA pipe then drains its queue while the VALU / LDS / memory slices issue.
 template <int N, class F, int... I>
 __device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
     (f(std::integral_constant<int, I>{}), ...);
@@ -370,7 +97,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 // stays in scalar registers, the per-lane part of every address is a 32-bit offset
 // computed once.  XTAIL: k is not a multiple of 64 (Q8_0 only), activation chunks at or
 // past k are zeroed on their way to LDS.
-template <int QT, int BM, int BN, bool XTAIL, int NW = 4>
+template <int QT, int BM, int BN, bool XTAIL, int NW>
 __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
     GemmParams P = P_in;
     int tn_local = (int)(blockIdx.x / P_in.tiles_m);
@@ -805,8 +532,9 @@ __global__ void bf16_to_f32_kernel(const uint16_t* __restrict__ x, float* __rest
     if (i < count) out[i] = qmm_bf16_bits_to_f32(x[i]);
 }
 
-template <int QT, int BM, int BN, int NW = 4>
+template <int QT, int BM, int BN>
 hipError_t launch_tile(GemmParams P, int slices, hipStream_t stream) {
+    constexpr int NW = 8;
     P.tiles_m = (int)((P.m + BM - 1) / BM);
     P.tiles_n = (int)((P.n_end - P.n_begin + BN - 1) / BN);
     if (P.n_weights > 1) { // a projection group: the members' column tiles one after the other
@@ -816,39 +544,25 @@ hipError_t launch_tile(GemmParams P, int slices, hipStream_t stream) {
     }
     const int64_t grid = (int64_t)P.tiles_m * P.tiles_n;
     if (grid > 0x7fffffff) return hipErrorInvalidValue;
-    const size_t lds = (size_t)2 * (BM + BN) * kRowStride;
+    constexpr size_t lds = (size_t)2 * (BM + BN) * kRowStride;
     const bool x_tail = QT == QMM_Q8_0 && (P.k & 63) != 0; // the K-quant types have k a multiple of 256
-    // Q6_K is pipelined with eight waves only (two or four threads per weight row)
-    constexpr bool kPipe = (BM == 256 || BN == 256) && (QT != QMM_Q6_K || NW == 8);
-    const void* fn;
-    if constexpr (kPipe)
-        fn = x_tail ? reinterpret_cast<const void*>(&gemm_pipe_kernel<QT, BM, BN, QT == QMM_Q8_0, NW>)
-                    : reinterpret_cast<const void*>(&gemm_pipe_kernel<QT, BM, BN, false, NW>);
-    else fn = reinterpret_cast<const void*>(&gemm_kernel<QT, BM, BN>);
-    if (lds > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-    }
-    if constexpr (kPipe) {
-        float* partial = P.partial;
-        if (slices > 1) P.slice_units = (P.k_units + slices - 1) / slices;
-        else P.partial = nullptr;
-        const dim3 grid2((unsigned)grid, (unsigned)slices);
-        if (x_tail) gemm_pipe_kernel<QT, BM, BN, QT == QMM_Q8_0, NW><<<grid2, dim3(64 * NW), lds, stream>>>(P);
-        else gemm_pipe_kernel<QT, BM, BN, false, NW><<<grid2, dim3(64 * NW), lds, stream>>>(P);
-        if (slices > 1 && P.n_weights > 1) {
-            for (int i = 0; i < P.n_weights; i++) {
-                const int64_t count = P.m * P.nv[i];
-                splitk_reduce_kernel<<<(unsigned)((count + 255) / 256), 256, 0, stream>>>(
-                    P.partial_v[i], slices, P.m, P.nv[i], 0, P.nv[i], P.yv[i], P.out_bf16, nullptr);
-            }
-        } else if (slices > 1) {
-            const int64_t count = P.m * (P.n_end - P.n_begin);
+    auto fn = x_tail ? &gemm_pipe_kernel<QT, BM, BN, QT == QMM_Q8_0, NW> : &gemm_pipe_kernel<QT, BM, BN, false, NW>;
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    float* partial = P.partial;
+    if (slices > 1) P.slice_units = (P.k_units + slices - 1) / slices;
+    else P.partial = nullptr;
+    fn<<<dim3((unsigned)grid, (unsigned)slices), dim3(64 * NW), lds, stream>>>(P);
+    if (slices > 1 && P.n_weights > 1) {
+        for (int i = 0; i < P.n_weights; i++) {
+            const int64_t count = P.m * P.nv[i];
             splitk_reduce_kernel<<<(unsigned)((count + 255) / 256), 256, 0, stream>>>(
-                partial, slices, P.m, P.n, P.n_begin, P.n_end, P.y, P.out_bf16, P.residual);
+                P.partial_v[i], slices, P.m, P.nv[i], 0, P.nv[i], P.yv[i], P.out_bf16, nullptr);
         }
-    } else {
-        gemm_kernel<QT, BM, BN><<<dim3((unsigned)grid), dim3(kThreads), lds, stream>>>(P);
+    } else if (slices > 1) {
+        const int64_t count = P.m * (P.n_end - P.n_begin);
+        splitk_reduce_kernel<<<(unsigned)((count + 255) / 256), 256, 0, stream>>>(
+            partial, slices, P.m, P.n, P.n_begin, P.n_end, P.y, P.out_bf16, P.residual);
     }
     return hipGetLastError();
 }
@@ -859,20 +573,19 @@ hipError_t launch_tile(GemmParams P, int slices, hipStream_t stream) {
 // second kernel adds the slices in order).  Costs are in k steps of a 256 x 256 tile
 // (relative tile efficiencies measured on the 8B shapes).
 struct GemmPlan {
-    int bm, bn;          // tile of the only / the second launch
-    int slices;          // split along k (BN == 256 tiles only)
+    int bm, bn;          // tile of the only / the second launch: 256 x 256 or 256 x 128
+    int slices;          // split along k
     int64_t full_cols;   // > 0: first a launch of 256 x 256 tiles over this many 256-column strips
 };
 
-// IZWI_QMM_GEMM_TILE="bm,bn,slices" (tuning aid) replaces the plan: bm, bn in {128, 256}.
+// IZWI_QMM_GEMM_TILE="bm,bn,slices" (tuning aid) replaces the plan: bm = 256, bn in {128, 256}.
 bool forced_plan(GemmPlan& plan) {
     static const GemmPlan forced = [] {
         GemmPlan p{0, 0, 1, 0};
         const char* e = getenv("IZWI_QMM_GEMM_TILE");
         if (e && sscanf(e, "%d,%d,%d", &p.bm, &p.bn, &p.slices) >= 2) {
-            const bool ok = (p.bm == 128 || p.bm == 256) && (p.bn == 128 || p.bn == 256) && p.slices >= 1 && p.slices <= 8;
-            if (!ok || (p.bm == 128 && p.bn == 128)) p.slices = 1;
-            if (!ok) p.bm = p.bn = 0;
+            const bool ok = p.bm == 256 && (p.bn == 128 || p.bn == 256) && p.slices >= 1 && p.slices <= 8;
+            if (!ok) p.bm = p.bn = 0, p.slices = 1;
         }
         return p;
     }();
@@ -882,10 +595,8 @@ bool forced_plan(GemmPlan& plan) {
 }
 
 GemmPlan plan_gemm(int64_t m, int64_t n, int k_steps, int n_cus, bool group = false) {
-    // relative rate of a half-size tile (256 x 128 dequantizes half as many weights per MFMA
-    // as 128 x 256 and is used whenever there are more than 128 rows) and of a quarter-size one
-    const double kQ128 = m > 128 ? 0.76 : 0.68, kQ64 = 0.4;
-    const int hm = m > 128 ? 256 : 128, hn = m > 128 ? 128 : 256; // the half-size tile
+    const double kQ128 = 0.76; // relative rate of a half-size tile
+    const int hm = 256, hn = 128;
     {
         GemmPlan forced;
         if (forced_plan(forced)) {
@@ -901,8 +612,6 @@ GemmPlan plan_gemm(int64_t m, int64_t n, int k_steps, int n_cus, bool group = fa
         if (cost < 0.97 * best_cost) best = p, best_cost = cost;
     };
     consider({hm, hn, 1, 0}, rounds(tiles(hm, hn, n)) * k_steps * 0.5 / kQ128);
-    // (a projection group runs on the pipelined tiles only, in one launch)
-    if (!group) consider({128, 128, 1, 0}, rounds(tiles(128, 128, n)) * k_steps * 0.25 / kQ64);
     // whole rounds of 256 x 256 tiles first, the remaining columns as half-size tiles
     const int64_t tiles_m256 = (m + 255) / 256, cols256 = (n + 255) / 256;
     const int64_t full_cols = (tiles_m256 * cols256 / n_cus) * n_cus / tiles_m256;
@@ -931,17 +640,12 @@ hipError_t launch_qt(const GemmParams& P0, int n_cus, hipStream_t stream) {
     if (plan.slices > 1 && P0.partial == nullptr) return hipErrorInvalidValue;
     if (plan.full_cols > 0) {
         P.n_end = plan.full_cols * 256;
-        hipError_t e = launch_tile<QT, 256, 256, 8>(P, 1, stream);
+        hipError_t e = launch_tile<QT, 256, 256>(P, 1, stream);
         if (e != hipSuccess) return e;
         P.n_begin = P.n_end;
         P.n_end = P0.n;
     }
-    if (plan.bm == 256 && plan.bn == 256) return launch_tile<QT, 256, 256, 8>(P, plan.slices, stream);
-    if (plan.bm == 256) return launch_tile<QT, 256, 128, 8>(P, plan.slices, stream);
-    if constexpr (QT != QMM_Q6_K) { // the plan picks this tile for m <= 128 only, where Q6_K does not come here
-        if (plan.bn == 256) return launch_tile<QT, 128, 256>(P, plan.slices, stream);
-    }
-    return launch_tile<QT, 128, 128>(P, 1, stream);
+    return plan.bn == 256 ? launch_tile<QT, 256, 256>(P, plan.slices, stream) : launch_tile<QT, 256, 128>(P, plan.slices, stream);
 }
 
 // n of the single matrix a group is planned as: the members' columns, each rounded up to whole
@@ -963,9 +667,7 @@ hipError_t launch_group_qt(GemmParams P, int64_t n_planned, int n_cus, hipStream
             base += (size_t)plan.slices * (size_t)P.m * (size_t)P.nv[i];
         }
     }
-    if (plan.bm == 256 && plan.bn == 256) return launch_tile<QT, 256, 256, 8>(P, plan.slices, stream);
-    if (plan.bm == 256 && plan.bn == 128) return launch_tile<QT, 256, 128, 8>(P, plan.slices, stream);
-    return hipErrorNotSupported;
+    return plan.bn == 256 ? launch_tile<QT, 256, 256>(P, plan.slices, stream) : launch_tile<QT, 256, 128>(P, plan.slices, stream);
 }
 
 } // namespace
@@ -978,13 +680,15 @@ static bool group_plane_applies(const QmmLayout* const* layouts, int n_weights, 
 }
 
 size_t qmm_gemm_group_workspace_bytes(const QmmLayout* const* layouts, int n_weights, int64_t m, int n_cus) {
-    if (m <= 128 || n_weights < 2) return 0;
+    if (n_weights < 2) return 0;
+    if (n_cus <= 0) n_cus = 1;
+    if (qmm_gemm_regb_applies(layouts, n_weights, m, n_cus)) return qmm_gemm_regb_workspace_bytes(layouts, n_weights, m, n_cus);
     if (group_plane_applies(layouts, n_weights, m)) {
         size_t total = 0;
         for (int i = 0; i < n_weights; i++) total += qmm_gemm_plane_bytes(*layouts[i]);
         return total;
     }
-    const GemmPlan plan = plan_gemm(m, group_columns(layouts, n_weights), (int)layouts[0]->k_units * 4, n_cus > 0 ? n_cus : 1, true);
+    const GemmPlan plan = plan_gemm(m, group_columns(layouts, n_weights), (int)layouts[0]->k_units * 4, n_cus, true);
     if (plan.slices <= 1) return 0;
     size_t total = 0;
     for (int i = 0; i < n_weights; i++) total += (size_t)plan.slices * (size_t)m * (size_t)layouts[i]->n * sizeof(float);
@@ -995,8 +699,9 @@ hipError_t qmm_launch_gemm_bf16_multi(const QmmLayout* const* layouts, const voi
                                       const uint16_t* x_bf16, int64_t m, void* const* ys, int out_bf16,
                                       void* workspace, int n_cus, hipStream_t stream) {
     if (n_weights < 2 || n_weights > QMM_MAX_GROUP) return hipErrorInvalidValue;
-    if (m <= 128) return hipErrorNotSupported; // the plain tile kernels: one call per weight
     if (n_cus <= 0) n_cus = 1;
+    if (qmm_gemm_regb_applies(layouts, n_weights, m, n_cus))
+        return qmm_launch_gemm_regb(layouts, tiled, n_weights, x_bf16, m, ys, out_bf16, workspace, n_cus, stream);
     if (group_plane_applies(layouts, n_weights, m)) {
         if (workspace == nullptr) return hipErrorInvalidValue;
         return qmm_launch_gemm_plane(layouts, tiled, n_weights, x_bf16, m, ys, out_bf16, workspace, n_cus, stream);
@@ -1041,9 +746,12 @@ hipError_t qmm_launch_gemm_bf16_multi(const QmmLayout* const* layouts, const voi
 }
 
 size_t qmm_gemm_workspace_bytes(const QmmLayout& L, int64_t m, int n_cus) {
-    if (m <= 0 || L.n == 0 || (L.dtype == QMM_Q6_K && m <= 128)) return 0;
+    if (m <= 0 || L.n == 0) return 0;
+    if (n_cus <= 0) n_cus = 1;
+    const QmmLayout* lp = &L;
+    if (qmm_gemm_regb_applies(&lp, 1, m, n_cus)) return qmm_gemm_regb_workspace_bytes(&lp, 1, m, n_cus);
     if (qmm_gemm_plane_applies(L, m)) return qmm_gemm_plane_bytes(L);
-    const GemmPlan plan = plan_gemm(m, L.n, (int)L.k_units * 4, n_cus > 0 ? n_cus : 1);
+    const GemmPlan plan = plan_gemm(m, L.n, (int)L.k_units * 4, n_cus);
     return plan.slices > 1 ? (size_t)plan.slices * (size_t)m * (size_t)L.n * sizeof(float) : 0;
 }
 
@@ -1052,9 +760,11 @@ hipError_t qmm_launch_gemm_bf16(const QmmLayout& L, const void* tiled, const uin
                                 hipStream_t stream, const void* residual) {
     if (m <= 0 || L.n == 0) return hipSuccess;
     if (n_cus <= 0) n_cus = 1;
+    const QmmLayout* lp = &L;
+    if (qmm_gemm_regb_applies(&lp, 1, m, n_cus))
+        return qmm_launch_gemm_regb(&lp, &tiled, 1, x_bf16, m, &y, out_bf16, workspace, n_cus, stream, residual);
     if (qmm_gemm_plane_applies(L, m)) {
         if (workspace == nullptr) return hipErrorInvalidValue;
-        const QmmLayout* lp = &L;
         return qmm_launch_gemm_plane(&lp, &tiled, 1, x_bf16, m, &y, out_bf16, workspace, n_cus, stream, residual);
     }
     GemmParams P;
@@ -1079,15 +789,7 @@ hipError_t qmm_launch_gemm_bf16(const QmmLayout& L, const void* tiled, const uin
     P.partial = (float*)workspace;
     P.residual = residual;
     P.n_weights = 0;
-    if (L.dtype == QMM_Q6_K) {
-        // more than 128 rows: the pipelined tiles; up to 128 the plain tile kernel, half-height
-        // tiles when full ones would leave CUs idle
-        static const bool plain_only = getenv("IZWI_QMM_Q6K_PLAIN_TILES") != nullptr; // comparison aid
-        if (m > 128 && !plain_only) return launch_qt<QMM_Q6_K>(P, n_cus, stream);
-        const int64_t t128 = ((m + 127) / 128) * ((L.n + 127) / 128);
-        if (t128 < (int64_t)n_cus && m > 64) return launch_tile<QMM_Q6_K, 64, 128>(P, 1, stream);
-        return launch_tile<QMM_Q6_K, 128, 128>(P, 1, stream);
-    }
+    if (L.dtype == QMM_Q6_K) return launch_qt<QMM_Q6_K>(P, n_cus, stream);
     return L.dtype == QMM_Q4_K ? launch_qt<QMM_Q4_K>(P, n_cus, stream)
                                : launch_qt<QMM_Q8_0>(P, n_cus, stream);
 }

@@ -1,0 +1,552 @@
+// Prefill kernel for few activation rows: y[m, n] = x[m, k] * dequant(W)[n, k]^T with bf16 MFMA,
+// weights dequantized straight into the matrix instruction's operand registers.
+//
+// From 65 to a few hundred rows what counts is that every weight byte is requested early, is
+// dequantized once and needs no trip through LDS.  A workgroup of eight waves owns 32 * MT
+// activation rows x 128 weight rows; wave (c, p) owns 32 of the weight rows and, of every unit of
+// 256 k-elements, half p.  A lane's 16-byte quant chunk holds k-elements of one weight row only,
+// which is what a lane supplies to v_mfma_f32_32x32x16_bf16: the chunk is unpacked into B operands
+// in registers, in the k order the chunk has, and the A operand (activations, staged in LDS by
+// LDS-direct loads, two stages of one unit) is picked in the same order.  No weight tile in LDS, no
+// LDS writes, one barrier per unit.  The two halves' sums meet in LDS at the end; k is split over
+// workgroups where the tiles alone leave compute units idle.
+//
+// Bound by the vector instructions that unpack (7.3 per matrix instruction) beside the matrix
+// instructions (half of the time of a full chip): 2.0 us per unit of 128 rows, and 6.5 to 8 us per
+// workgroup that are no unit (start, first loads, exchange of the sums, stores).  Splitting a unit
+// four ways over the waves (64 x 128 wave tiles, fewer LDS reads) cost 14 us per workgroup instead:
+// the exchange of the sums is 512 KB of LDS traffic there, 128 KB here.  Q4_K, us per call in a
+// graph, before (128 x 256 / 64 x 128 tiles with the weights through LDS, one call per weight) and
+// now: 101 rows: q|k|v 73 -> 23, 4096 x 4096 25.4 -> 21.4, gate|up 76 -> 39, down 42 -> 27; Q6_K
+// down 176 -> 28; 512 rows: q|k|v 51 -> 39, 4096 x 4096 35.5 -> 32.6; 0.6B shapes at 512: 25 -> 14.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstdio>
+#include <cstdlib>
+#include <type_traits>
+#include <utility>
+
+#include "qmm_internal.h"
+
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kCols = 4, kSplits = 2; // waves of a workgroup: column groups x halves of a unit
+constexpr int kWaves = kCols * kSplits;
+constexpr int kBN = 32 * kCols;
+constexpr int kUnitBytes = QMM_UNIT_ELEMS * 2; // one activation row of one unit, bf16
+
+template <int N, class F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+    static_for_impl<N>(f, std::make_integer_sequence<int, N>{});
+}
+
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    bf16x2 v = {(__bf16)a, (__bf16)b}; // round to nearest even
+    return __builtin_bit_cast(uint32_t, v);
+}
+template <int N>
+__device__ __forceinline__ float ubyte_f32(uint32_t v) {
+    return (float)((v >> (8 * N)) & 0xffu);
+}
+// fma(scale, byte, bias) of the eight bytes of (lo, hi) as one bf16 operand
+__device__ __forceinline__ bf16x8 scaled_bytes(uint32_t lo, uint32_t hi, float scale, float bias) {
+    u32x4 o;
+    o.x = pack_bf16(__builtin_fmaf(scale, ubyte_f32<0>(lo), bias), __builtin_fmaf(scale, ubyte_f32<1>(lo), bias));
+    o.y = pack_bf16(__builtin_fmaf(scale, ubyte_f32<2>(lo), bias), __builtin_fmaf(scale, ubyte_f32<3>(lo), bias));
+    o.z = pack_bf16(__builtin_fmaf(scale, ubyte_f32<0>(hi), bias), __builtin_fmaf(scale, ubyte_f32<1>(hi), bias));
+    o.w = pack_bf16(__builtin_fmaf(scale, ubyte_f32<2>(hi), bias), __builtin_fmaf(scale, ubyte_f32<3>(hi), bias));
+    return __builtin_bit_cast(bf16x8, o);
+}
+
+struct RegbParams {
+    const uint16_t* x; // bf16 [m, k], k a multiple of 32
+    int64_t m, k;
+    int k_units, slice_units, slices;
+    int s, slots;
+    int64_t panel_bytes, row_bytes; // row_bytes: all panels of a row tile
+    int tiles_m, cols;              // cols: the members' column tiles times slices
+    uint32_t nibble_mask;           // 0x0f0f0f0f as data: one AND per four weights, v_cvt_f32_ubyteN for each
+    int out_bf16;
+    const void* residual; // single weight only
+    int n_weights;
+    int tn_end[QMM_MAX_GROUP];
+    const uint8_t* wv[QMM_MAX_GROUP];
+    void* yv[QMM_MAX_GROUP];
+    float* partial_v[QMM_MAX_GROUP]; // [slice][m][n] where k is split
+    int64_t nv[QMM_MAX_GROUP], row_tiles_v[QMM_MAX_GROUP];
+};
+
+// What a lane holds of its weight row's half unit (two steps of 64 k-elements).
+template <int QT>
+struct HalfRegs {
+    static constexpr int NQ = QT == QMM_Q8_0 ? 4 : 2;
+    using Header = std::conditional_t<QT == QMM_Q4_K, u32x4, u32x2>; // Q8_0, Q6_K: the two steps' scale dwords
+    Header hdr;
+    u32x4 q[NQ];
+    u32x4 qh;   // Q6_K: the high bit pairs
+    uint32_t d; // Q6_K
+};
+
+// Byte offsets of those pieces from the unit's address (a lane's row included).
+struct HalfOffsets {
+    uint32_t hdr, q, qh, d, q_stride;
+};
+
+template <int QT>
+__device__ __forceinline__ void load_half(HalfRegs<QT>& r, const uint8_t* unit, const HalfOffsets& o) {
+    r.hdr = *reinterpret_cast<const typename HalfRegs<QT>::Header*>(unit + o.hdr);
+#pragma unroll
+    for (int c = 0; c < HalfRegs<QT>::NQ; c++) r.q[c] = *reinterpret_cast<const u32x4*>(unit + o.q + c * o.q_stride);
+    if (QT == QMM_Q6_K) {
+        r.qh = *reinterpret_cast<const u32x4*>(unit + o.qh);
+        r.d = *reinterpret_cast<const uint32_t*>(unit + o.d);
+    }
+}
+
+// A use of the loaded registers: the compiler's own wait for them stands here, where the counter is zero
+// anyway, and not behind the next unit's requests (of which it counts only the register loads).
+template <int QT>
+__device__ __forceinline__ void arrived(HalfRegs<QT>& r) {
+    asm volatile("" : "+v"(r.hdr));
+#pragma unroll
+    for (int c = 0; c < HalfRegs<QT>::NQ; c++) asm volatile("" : "+v"(r.q[c]));
+    if (QT == QMM_Q6_K) asm volatile("" : "+v"(r.qh), "+v"(r.d));
+}
+
+// The factors of a step's two 32-element blocks: w = scale * byte + bias.
+struct StepScales {
+    float scale[2], bias[2];
+};
+template <int QT, int ST>
+__device__ __forceinline__ StepScales step_scales(const HalfRegs<QT>& r, int half, int h) {
+    StepScales s;
+    if constexpr (QT == QMM_Q4_K) {
+        const float d = qmm_f16_bits_to_f32((uint16_t)(r.hdr.x & 0xffffu)), dmin = qmm_f16_bits_to_f32((uint16_t)(r.hdr.x >> 16));
+        uint32_t sc_lo, sc_hi, mn_lo, mn_hi;
+        qmm_unpack_q4k_scales(r.hdr.y, r.hdr.z, r.hdr.w, sc_lo, sc_hi, mn_lo, mn_hi);
+        const uint32_t sc = (half ? sc_hi : sc_lo) >> (16 * ST), mn = (half ? mn_hi : mn_lo) >> (16 * ST); // half is uniform
+        s.scale[0] = d * (float)(sc & 0xffu), s.scale[1] = d * (float)((sc >> 8) & 0xffu);
+        s.bias[0] = -(dmin * (float)(mn & 0xffu)), s.bias[1] = -(dmin * (float)((mn >> 8) & 0xffu));
+    } else if constexpr (QT == QMM_Q8_0) {
+        const uint32_t dd = r.hdr[ST];
+        s.scale[0] = qmm_f16_bits_to_f32((uint16_t)(dd & 0xffffu)), s.scale[1] = qmm_f16_bits_to_f32((uint16_t)(dd >> 16));
+        s.bias[0] = -128.0f * s.scale[0], s.bias[1] = -128.0f * s.scale[1]; // int8 q as unsigned byte u = q + 128
+    } else {
+        const float d = qmm_f16_bits_to_f32((uint16_t)(r.d & 0xffffu));
+        const uint32_t sw = r.hdr[ST] >> (8 * h); // a scale per 16 elements: h, 2 + h of the step's four
+        s.scale[0] = d * (float)(int8_t)(sw & 0xffu), s.scale[1] = d * (float)(int8_t)((sw >> 16) & 0xffu);
+        s.bias[0] = -32.0f * s.scale[0], s.bias[1] = -32.0f * s.scale[1];
+    }
+    return s;
+}
+
+// B operand of matrix instruction SS (of eight): k-elements 64 (SS / 4) + 32 (SS / 2 % 2) + 16 h + 8 (SS % 2) .. + 7
+// of the half unit.
+template <int QT, int SS>
+__device__ __forceinline__ bf16x8 half_operand(const HalfRegs<QT>& r, const StepScales& s, uint32_t nibble_mask) {
+    constexpr int st = SS >> 2, q = (SS >> 1) & 1, e = SS & 1;
+    uint32_t lo, hi;
+    if constexpr (QT == QMM_Q4_K) {
+        lo = (q ? r.q[st][2 * e] >> 4 : r.q[st][2 * e]) & nibble_mask;
+        hi = (q ? r.q[st][2 * e + 1] >> 4 : r.q[st][2 * e + 1]) & nibble_mask;
+    } else if constexpr (QT == QMM_Q8_0) {
+        lo = r.q[2 * st + q][2 * e] ^ 0x80808080u;
+        hi = r.q[2 * st + q][2 * e + 1] ^ 0x80808080u;
+    } else {
+        lo = ((r.q[q][2 * e] >> (4 * st)) & nibble_mask) | (((r.qh[2 * e] >> (4 * st + 2 * q)) & 0x03030303u) << 4);
+        hi = ((r.q[q][2 * e + 1] >> (4 * st)) & nibble_mask) | (((r.qh[2 * e + 1] >> (4 * st + 2 * q)) & 0x03030303u) << 4);
+    }
+    return scaled_bytes(lo, hi, s.scale[q], s.bias[q]);
+}
+
+// 16 bytes per lane from global memory straight into LDS: lane l's bytes land at lds + 16 l.
+__device__ __forceinline__ void load_to_lds(const uint8_t* base, uint32_t lane_off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(lane_off), "s"(base) : "memory", "m0");
+}
+
+template <int QT, int MT>
+__global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P) {
+    constexpr int BM = 32 * MT;
+    constexpr int kStage = BM * kUnitBytes;
+    constexpr int XL = BM / 2 / kWaves; // LDS-direct loads per wave and unit (1 KiB = two rows each)
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+
+    // Workgroups go to the eight XCDs round-robin by their index; the row tiles of one (column tile,
+    // slice) follow each other on one XCD, so its weights come from memory once.
+    const int xcd = blockIdx.x & 7, pos = blockIdx.x >> 3;
+    const int tm = pos % P.tiles_m;
+    const int col = (pos / P.tiles_m) * 8 + xcd;
+    if (col >= P.cols) return; // uniform
+    const int slice = col % P.slices;
+    int tn = col / P.slices, member = 0;
+    while (member + 1 < P.n_weights && tn >= P.tn_end[member]) member++;
+    tn -= member ? P.tn_end[member - 1] : 0;
+    const int64_t n = P.nv[member];
+    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * kBN;
+    const int u0 = slice * P.slice_units, u1 = min(P.k_units, u0 + P.slice_units);
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wc = wave >> 1, half = wave & 1;
+    const int h = lane >> 5;
+
+    // ---- activations: instruction q of a unit moves rows 2 q, 2 q + 1; the 16-byte chunk c of a row
+    // sits at chunk position c ^ (row & 15), so that 16 consecutive rows of one chunk touch every bank once
+    const uint8_t* x_tile = reinterpret_cast<const uint8_t*>(P.x) + m0 * P.k * 2;
+    uint32_t x_off[XL];
+    {
+        const int r0 = 2 * wave + h, c = (lane & 31) ^ (r0 & 15); // (row & 15 is the same for every i)
+#pragma unroll
+        for (int i = 0; i < XL; i++)
+            x_off[i] = (uint32_t)((min(m0 + r0 + 2 * kWaves * i, P.m - 1) - m0) * P.k * 2 + c * 16);
+    }
+    const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
+    // k ends inside the last unit (Q8_0 only): chunks at or past its end read the unit's first chunk
+    // and are zeroed when they have landed
+    const int x_tail = QT == QMM_Q8_0 ? (int)(P.k % QMM_UNIT_ELEMS) / 8 : 0;
+    const int x_chunk = (lane & 31) ^ ((2 * wave + h) & 15);
+    auto issue_x = [&](int u, int stage) {
+        const uint8_t* src = x_tile + (size_t)u * kUnitBytes;
+        const uint32_t dst = lds0 + stage * kStage + wave * 1024;
+        const uint32_t back = x_tail && u == P.k_units - 1 && x_chunk >= x_tail ? x_chunk * 16 : 0;
+#pragma unroll
+        for (int i = 0; i < XL; i++) load_to_lds(src, x_off[i] - back, dst + i * kWaves * 1024);
+    };
+    auto zero_tail = [&](int u, int stage) { // behind this wave's loads of unit u, in front of a barrier
+        if (x_tail && u == P.k_units - 1 && x_chunk >= x_tail)
+#pragma unroll
+            for (int i = 0; i < XL; i++)
+                *reinterpret_cast<u32x4*>(smem + stage * kStage + (wave + i * kWaves) * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
+    };
+
+    // ---- weights: uniform unit address + 32-bit offsets
+    const int64_t rt0 = n0 >> 4;
+    const uint8_t* w_tile = P.wv[member] + rt0 * P.row_bytes;
+    HalfOffsets off;
+    {
+        const int row = wc * 32 + (lane & 31);
+        const int64_t rt = min(rt0 + (row >> 4), P.row_tiles_v[member] - 1);
+        const uint32_t base = (uint32_t)((rt - rt0) * P.row_bytes) + (row & 15) * 16, chunk = (uint32_t)P.slots * 16;
+        off.hdr = base + (QT == QMM_Q4_K ? 0 : 8 * half);
+        off.q = base + (1 + (QT == QMM_Q8_0 ? 8 : 4) * half + h) * chunk;
+        off.q_stride = 2 * chunk;
+        off.qh = base + (9 + 2 * half + h) * chunk;
+        off.d = base + 13 * chunk;
+    }
+    auto load_w = [&](HalfRegs<QT>& r, int u) {
+        const int kg = u / P.s, us = u - kg * P.s;
+        load_half<QT>(r, w_tile + (int64_t)kg * P.panel_bytes + us * 256, off);
+    };
+
+    f32x16 acc[MT];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[i][r] = 0.0f;
+
+    // A operand of matrix instruction ss: row l & 31 of each 32-row block, chunk 16 half + 8 (ss / 4) + 4 (ss / 2 % 2)
+    // + 2 h + ss % 2 of the unit
+    const int frag_x = (lane & 31) * kUnitBytes + (((16 * half + 2 * h) ^ (lane & 15)) << 4);
+
+    // Software pipeline: the operands of instruction ss + 1 are read / unpacked behind instruction ss;
+    // the unit's only barrier sits in front of its last one, where every activation of the unit is in
+    // registers and the next unit has landed, and the unit after that is requested behind it.
+    HalfRegs<QT> w[2];
+    StepScales sc[2];
+    bf16x8 a[2][MT], b[2];
+    auto read_a = [&](int stage, auto SS) {
+        constexpr int ss = decltype(SS)::value;
+        const uint8_t* src = smem + stage * kStage + (frag_x ^ ((8 * (ss >> 2) + 4 * ((ss >> 1) & 1) + (ss & 1)) << 4));
+#pragma unroll
+        for (int i = 0; i < MT; i++) a[ss & 1][i] = *reinterpret_cast<const bf16x8*>(src + i * 32 * kUnitBytes);
+    };
+    const int last = u1 - 1; // past the end: the last unit again, into stages nobody reads
+    issue_x(u0, 0);
+    load_w(w[0], u0);
+    issue_x(min(u0 + 1, last), 1);
+    load_w(w[1], min(u0 + 1, last));
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    zero_tail(u0, 0);
+    zero_tail(min(u0 + 1, last), 1);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    arrived<QT>(w[0]);
+    arrived<QT>(w[1]);
+    read_a(0, std::integral_constant<int, 0>{});
+    sc[0] = step_scales<QT, 0>(w[0], half, h);
+    b[0] = half_operand<QT, 0>(w[0], sc[0], P.nibble_mask);
+    auto unit_step = [&](int u, auto PAR) {
+        constexpr int par = decltype(PAR)::value;
+        static_for<8>([&](auto SS) {
+            constexpr int ss = decltype(SS)::value;
+            if constexpr (ss < 7) {
+                if constexpr (ss == 3) sc[1] = step_scales<QT, 1>(w[par], half, h);
+                read_a(par, std::integral_constant<int, ss + 1>{});
+                b[(ss + 1) & 1] = half_operand<QT, ss + 1>(w[par], sc[(ss + 1) >> 2], P.nibble_mask);
+            } else {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                zero_tail(min(u + 1, last), par ^ 1);
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                arrived<QT>(w[par ^ 1]);
+                const int next = min(u + 2, last);
+                issue_x(next, par);
+                load_w(w[par], next);
+                asm volatile("" ::: "memory"); // the requests stay here
+                read_a(par ^ 1, std::integral_constant<int, 0>{});
+                sc[0] = step_scales<QT, 0>(w[par ^ 1], half, h);
+                b[0] = half_operand<QT, 0>(w[par ^ 1], sc[0], P.nibble_mask);
+            }
+#pragma unroll
+            for (int i = 0; i < MT; i++) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[ss & 1][i], b[ss & 1], acc[i], 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < MT; q++) { // one matrix instruction, then a share of the next one's operands
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 32 / MT, 0);
+            }
+        });
+    };
+    int u = u0;
+    do {
+        unit_step(u, std::integral_constant<int, 0>{});
+        if (++u == u1) break;
+        unit_step(u, std::integral_constant<int, 1>{});
+    } while (++u < u1);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); // the requests past the end
+
+    // ---- the two halves' sums: the wave of half p finishes the 32-row blocks i with i % 2 = p
+    constexpr int kOwn = (MT + 1) / 2;
+    f32x16 sum[kOwn];
+    {
+        uint8_t* dst = smem + wc * (MT * 4096) + lane * 16;
+        auto send = [&](auto PAIR) { // the blocks of the other half
+            static_for<MT>([&](auto I) {
+                constexpr int i = decltype(I)::value;
+                if constexpr (i % 2 == decltype(PAIR)::value)
+                    for (int r = 0; r < 4; r++)
+                        *reinterpret_cast<f32x4*>(dst + i * 4096 + r * 1024) =
+                            f32x4{acc[i][4 * r], acc[i][4 * r + 1], acc[i][4 * r + 2], acc[i][4 * r + 3]};
+            });
+        };
+        if (half) send(std::integral_constant<int, 0>{}); // uniform
+        else send(std::integral_constant<int, 1>{});
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        auto take = [&](auto PAIR) {
+            static_for<MT>([&](auto I) {
+                constexpr int i = decltype(I)::value;
+                if constexpr (i % 2 == decltype(PAIR)::value)
+                    for (int r = 0; r < 4; r++) {
+                        const f32x4 v = *reinterpret_cast<const f32x4*>(dst + i * 4096 + r * 1024);
+                        for (int e = 0; e < 4; e++) sum[i / 2][4 * r + e] = acc[i][4 * r + e] + v[e];
+                    }
+            });
+        };
+        if (half) take(std::integral_constant<int, 1>{});
+        else take(std::integral_constant<int, 0>{});
+    }
+    const bool split = P.slices > 1;
+    const int64_t gn = n0 + wc * 32 + (lane & 31);
+    const int64_t gm0 = m0 + half * 32 + 4 * h;
+    const int rows = gn < n ? (int)min((int64_t)BM, P.m - gm0) : 0; // of this lane's column, from gm0 on
+    auto emit = [&](auto MODE) { // 0: f32, 1: f32 + residual, 2: bf16, 3: bf16 + residual
+        constexpr int mode = decltype(MODE)::value;
+        float* yf = (split ? P.partial_v[member] + (int64_t)slice * P.m * n : static_cast<float*>(P.yv[member])) + gm0 * n + gn;
+        uint16_t* yb = static_cast<uint16_t*>(P.yv[member]) + gm0 * n + gn;
+        const float* rf = static_cast<const float*>(P.residual) + gm0 * n + gn;
+        const uint16_t* rb = static_cast<const uint16_t*>(P.residual) + gm0 * n + gn;
+        static_for<kOwn>([&](auto I) {
+            static_for<16>([&](auto R) {
+                constexpr int i = decltype(I)::value, r = decltype(R)::value, row = 64 * i + 8 * (r >> 2) + (r & 3);
+                if (row < rows && (2 * i + half < MT)) {
+                    const int64_t at = row * n;
+                    float v = sum[i][r];
+                    if (mode == 1) v += rf[at];
+                    if (mode == 3) v += qmm_bf16_bits_to_f32(rb[at]);
+                    if (mode < 2) yf[at] = v;
+                    else yb[at] = (uint16_t)pack_bf16(v, v);
+                }
+            });
+        });
+    };
+    if (split || !(P.out_bf16 || P.residual)) emit(std::integral_constant<int, 0>{});
+    else if (!P.out_bf16) emit(std::integral_constant<int, 1>{});
+    else if (!P.residual) emit(std::integral_constant<int, 2>{});
+    else emit(std::integral_constant<int, 3>{});
+}
+
+// y = sum over slices (in order) of partial[slice] (+ residual), four consecutive values per thread, all
+// members of a group in one launch (blocks of member i: block_end[i - 1] .. block_end[i])
+struct RegbReduceParams {
+    const float* partial[QMM_MAX_GROUP];
+    void* y[QMM_MAX_GROUP];
+    int64_t count[QMM_MAX_GROUP];
+    int block_end[QMM_MAX_GROUP];
+    int n_weights, slices, out_bf16;
+    const void* residual;
+};
+__global__ __launch_bounds__(256) void regb_reduce_kernel(RegbReduceParams P) {
+    int member = 0;
+    while (member + 1 < P.n_weights && (int)blockIdx.x >= P.block_end[member]) member++;
+    const int64_t count = P.count[member];
+    const int64_t i = ((int64_t)(blockIdx.x - (member ? P.block_end[member - 1] : 0)) * 256 + threadIdx.x) * 4;
+    const float* partial = P.partial[member] + i;
+    const QmmEpilogue ep{P.residual, P.out_bf16};
+    if (i + 4 <= count && (count & 3) == 0) {
+        f32x4 sum = *reinterpret_cast<const f32x4*>(partial);
+        for (int s = 1; s < P.slices; s++) sum += *reinterpret_cast<const f32x4*>(partial + s * count);
+#pragma unroll
+        for (int e = 0; e < 4; e++) qmm_store(P.y[member], ep, i + e, sum[e]);
+    } else {
+        for (int e = 0; e < 4 && i + e < count; e++) {
+            float sum = partial[e];
+            for (int s = 1; s < P.slices; s++) sum += partial[s * count + e];
+            qmm_store(P.y[member], ep, i + e, sum);
+        }
+    }
+}
+
+struct RegbPlan {
+    int mt, slices, slice_units;
+    double cost;
+};
+
+RegbPlan plan_regb(const QmmLayout* const* layouts, int n_weights, int64_t m, int n_cus) {
+    RegbPlan p;
+    const int64_t tiles_m = (m + 127) / 128;
+    p.mt = (int)((m + 32 * tiles_m - 1) / (32 * tiles_m));
+    const int k_units = (int)layouts[0]->k_units;
+    int64_t tiles = 0, n_total = 0;
+    for (int i = 0; i < n_weights; i++) n_total += layouts[i]->n, tiles += (layouts[i]->n + kBN - 1) / (kBN);
+    tiles *= tiles_m;
+    // microseconds, fitted to the 8B and 0.6B shapes at 65 to 512 rows: a round of workgroups costs 6.5 plus
+    // its units, the more the fuller the chip; the slices' sums cost a launch and their bytes twice
+    const double row_cost = (0.45 + 0.55 * p.mt / 4.0);
+    double best = 1e30;
+    p.slices = 1;
+    for (int s = 1; s <= 8 && s <= k_units; s++) {
+        const int su = (k_units + s - 1) / s;
+        if ((k_units + su - 1) / su != s) continue;
+        const double rounds = (double)((tiles * s + n_cus - 1) / n_cus);
+        const double unit = (1.6 + 0.5 * std::min(1.0, (double)(tiles * s) / n_cus)) * row_cost;
+        const double cost = rounds * (6.5 + su * unit) + (s > 1 ? 4.0 + s * (double)m * (double)n_total * 4.0 / 2.5e6 : 0.0);
+        if (cost < 0.98 * best) best = cost, p.slices = s;
+    }
+    p.cost = best;
+    p.slice_units = (k_units + p.slices - 1) / p.slices;
+    p.slices = (k_units + p.slice_units - 1) / p.slice_units;
+    return p;
+}
+
+template <int QT, int MT>
+hipError_t launch_regb(const RegbParams& P, int64_t grid, hipStream_t stream) {
+    constexpr size_t stages = (size_t)2 * 32 * MT * kUnitBytes; // the halves' sums reuse it
+    static_assert(stages <= 160 * 1024 && stages >= (size_t)kCols * MT * 4096, "LDS of a CU");
+    auto fn = &gemm_regb_kernel<QT, MT>;
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)stages);
+    if (e != hipSuccess) return e;
+    fn<<<dim3((unsigned)grid), dim3(64 * kWaves), stages, stream>>>(P);
+    return hipGetLastError();
+}
+
+template <int QT>
+hipError_t launch_regb_qt(const RegbParams& P, const RegbPlan& p, int64_t grid, hipStream_t stream) {
+    switch (p.mt) {
+        case 1: return launch_regb<QT, 1>(P, grid, stream);
+        case 2: return launch_regb<QT, 2>(P, grid, stream);
+        case 3: return launch_regb<QT, 3>(P, grid, stream);
+        default: return launch_regb<QT, 4>(P, grid, stream);
+    }
+}
+
+} // namespace
+
+// Up to 128 rows always (it is the only form there), beyond where the 128 x 128 tiles are at most one
+// per compute unit, or at most 96 rows high in two tiles: measured against the 256-row tiles of
+// qmm_gemm.hip (Q4_K, us per call in a graph, here / there): q|k|v 4096 -> 6144 39.0 / 50.9 at 512
+// rows (192 tiles), 71.9 / 64.9 at 768 (288); 4096 x 4096 42.1 / 54.8 at 1024 (256), 93.1 / 80.6 at
+// 2048 (512); gate|up of 2 x 12288 65.9 / 74.8 at 192 (384 tiles of 96 rows), 73.5 / 70.9 at 256
+// (384); gate|up of 2 x 3072 at k = 1024 14.7 / 25.6 at 512 (192), 26.9 / 26.4 at 768 (288).
+bool qmm_gemm_regb_applies(const QmmLayout* const* layouts, int n_weights, int64_t m, int n_cus) {
+    if (m <= 0 || n_weights < 1) return false;
+    int64_t tiles = 0;
+    const int64_t tiles_m = (m + 127) / 128;
+    for (int i = 0; i < n_weights; i++) {
+        const QmmLayout& L = *layouts[i];
+        if (L.n_stacked != 1 || L.n == 0 || L.dtype != layouts[0]->dtype || L.k != layouts[0]->k) return false;
+        tiles += tiles_m * ((L.n + kBN - 1) / kBN);
+    }
+    if (m <= 128) return true;
+    if (qmm_get_prefill_form() >= 0) return false; // one of the other forms was asked for
+    return tiles <= n_cus || m <= 192;
+}
+
+size_t qmm_gemm_regb_workspace_bytes(const QmmLayout* const* layouts, int n_weights, int64_t m, int n_cus) {
+    const RegbPlan p = plan_regb(layouts, n_weights, m, n_cus);
+    if (p.slices <= 1) return 0;
+    size_t total = 0;
+    for (int i = 0; i < n_weights; i++) total += (((size_t)p.slices * (size_t)m * (size_t)layouts[i]->n * sizeof(float)) + 255) & ~(size_t)255;
+    return total;
+}
+
+hipError_t qmm_launch_gemm_regb(const QmmLayout* const* layouts, const void* const* tiled, int n_weights, const uint16_t* x_bf16,
+                                int64_t m, void* const* ys, int out_bf16, void* workspace, int n_cus, hipStream_t stream,
+                                const void* residual) {
+    if (n_weights < 1 || n_weights > QMM_MAX_GROUP || (residual && n_weights != 1)) return hipErrorInvalidValue;
+    const QmmLayout& L0 = *layouts[0];
+    const RegbPlan plan = plan_regb(layouts, n_weights, m, n_cus);
+    if (plan.slices > 1 && workspace == nullptr) return hipErrorInvalidValue;
+    RegbParams P;
+    P.x = x_bf16;
+    P.m = m, P.k = L0.k;
+    P.k_units = (int)L0.k_units, P.slice_units = plan.slice_units, P.slices = plan.slices;
+    P.s = L0.s, P.slots = L0.slots;
+    P.panel_bytes = L0.panel_bytes, P.row_bytes = L0.k_groups * L0.panel_bytes;
+    P.nibble_mask = 0x0f0f0f0fu;
+    P.out_bf16 = out_bf16;
+    P.residual = plan.slices > 1 ? nullptr : residual;
+    P.n_weights = n_weights;
+    P.tiles_m = (int)((m + 32 * plan.mt - 1) / (32 * plan.mt));
+    uint8_t* next = static_cast<uint8_t*>(workspace);
+    int64_t tn = 0;
+    for (int i = 0; i < QMM_MAX_GROUP; i++) {
+        P.tn_end[i] = 0, P.wv[i] = nullptr, P.yv[i] = nullptr, P.partial_v[i] = nullptr, P.nv[i] = 0, P.row_tiles_v[i] = 0;
+        if (i >= n_weights) continue;
+        const QmmLayout& L = *layouts[i];
+        if (L.dtype != L0.dtype || L.k != L0.k || L.n_stacked != 1 || L.n == 0) return hipErrorInvalidValue;
+        tn += (L.n + kBN - 1) / (kBN);
+        P.tn_end[i] = (int)tn;
+        P.wv[i] = static_cast<const uint8_t*>(tiled[i]), P.yv[i] = ys[i];
+        P.nv[i] = L.n, P.row_tiles_v[i] = L.row_tiles;
+        P.partial_v[i] = reinterpret_cast<float*>(next);
+        if (plan.slices > 1) next += (((size_t)plan.slices * (size_t)m * (size_t)L.n * sizeof(float)) + 255) & ~(size_t)255;
+    }
+    const int64_t cols = tn * plan.slices, grid = (cols + 7) / 8 * 8 * P.tiles_m;
+    if (grid > 0x7fffffff) return hipErrorInvalidValue;
+    P.cols = (int)cols;
+    hipError_t e = L0.dtype == QMM_Q6_K   ? launch_regb_qt<QMM_Q6_K>(P, plan, grid, stream)
+                   : L0.dtype == QMM_Q4_K ? launch_regb_qt<QMM_Q4_K>(P, plan, grid, stream)
+                                          : launch_regb_qt<QMM_Q8_0>(P, plan, grid, stream);
+    if (e != hipSuccess || plan.slices <= 1) return e;
+    RegbReduceParams R;
+    int64_t blocks = 0;
+    for (int i = 0; i < QMM_MAX_GROUP; i++) {
+        R.count[i] = i < n_weights ? m * layouts[i]->n : 0;
+        blocks += (R.count[i] + 1023) / 1024;
+        R.partial[i] = P.partial_v[i], R.y[i] = P.yv[i], R.block_end[i] = (int)blocks;
+    }
+    if (blocks > 0x7fffffff) return hipErrorInvalidValue;
+    R.n_weights = n_weights, R.slices = plan.slices, R.out_bf16 = out_bf16, R.residual = residual;
+    regb_reduce_kernel<<<(unsigned)blocks, 256, 0, stream>>>(R);
+    return hipGetLastError();
+}

@@ -194,8 +194,8 @@ hipError_t qmm_launch_gemv_rows(const QmmLayout& L, const void* tiled, const flo
 hipError_t qmm_launch_gemv_gated(const QmmLayout& L, const void* tiled_gate, const void* tiled_up,
                                  const float* x, int64_t m, float* y, int n_cus, hipStream_t stream,
                                  const QmmNorm* norm = nullptr);
-// out[i] = silu(gate[i]) * up[i]
-hipError_t qmm_launch_silu_mul(const float* gate, const float* up, float* out, int64_t count,
+// out[i] = silu(gate[i]) * up[i], f32 or bf16
+hipError_t qmm_launch_silu_mul(const float* gate, const float* up, void* out, int out_bf16, int64_t count,
                                hipStream_t stream);
 
 // Batched decode kernel (int8 MFMA) for 3 <= m <= 64.  `workspace` must hold
@@ -221,11 +221,10 @@ size_t qmm_gemm_workspace_bytes(const QmmLayout& L, int64_t m, int n_cus);
 hipError_t qmm_launch_gemm_bf16(const QmmLayout& L, const void* tiled, const uint16_t* x_bf16,
                                 int64_t m, void* y, int out_bf16, void* workspace, int n_cus,
                                 hipStream_t stream, const void* residual = nullptr);
-// Several weights of equal k and type on the same bf16 activations in ONE launch of the pipelined
-// tiles (m > 128): the grid is the members' column tiles one after the other, planned as one
-// matrix with all the columns.  Per-member results are those of qmm_launch_gemm_bf16 up to the
-// tile plan (which may split k differently).  hipErrorNotSupported: no single-launch form
-// (m <= 128), call the members one by one.
+// Several weights of equal k and type on the same bf16 activations in ONE launch: the grid is the
+// members' column tiles one after the other, planned as one matrix with all the columns.
+// Per-member results are those of qmm_launch_gemm_bf16 up to the tile plan (which may split k
+// differently).
 size_t qmm_gemm_group_workspace_bytes(const QmmLayout* const* layouts, int n_weights, int64_t m, int n_cus);
 hipError_t qmm_launch_gemm_bf16_multi(const QmmLayout* const* layouts, const void* const* tiled, int n_weights,
                                       const uint16_t* x_bf16, int64_t m, void* const* ys, int out_bf16,
@@ -242,6 +241,13 @@ int qmm_get_prefill_form();
 hipError_t qmm_launch_gemm_plane(const QmmLayout* const* layouts, const void* const* tiled, int n_weights,
                                  const uint16_t* x_bf16, int64_t m, void* const* ys, int out_bf16, void* planes,
                                  int n_cus, hipStream_t stream, const void* residual = nullptr);
+// Register form of the prefill product, for few activation rows: one launch for 1..QMM_MAX_GROUP
+// weights of one type and k, behind it one reduce launch where k is split.
+bool qmm_gemm_regb_applies(const QmmLayout* const* layouts, int n_weights, int64_t m, int n_cus);
+size_t qmm_gemm_regb_workspace_bytes(const QmmLayout* const* layouts, int n_weights, int64_t m, int n_cus);
+hipError_t qmm_launch_gemm_regb(const QmmLayout* const* layouts, const void* const* tiled, int n_weights,
+                                const uint16_t* x_bf16, int64_t m, void* const* ys, int out_bf16, void* workspace,
+                                int n_cus, hipStream_t stream, const void* residual = nullptr);
 // y[i] = t[i] (+ residual[i]) as f32 or bf16: the epilogue as a kernel of its own, for the forms
 // that cannot fold it
 hipError_t qmm_launch_epilogue(const float* t, const void* residual, void* y, int y_bf16, int64_t count,

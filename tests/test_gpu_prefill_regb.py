@@ -1,0 +1,96 @@
+"""GPU tests (pytest -m gpu) of the register form of the prefill product (few rows, small products):
+weights unpacked straight into matrix operands, k split over two wave groups and over workgroups.
+
+Reference: float64 products of the bf16 activations with the dequantized weights rounded to bf16.
+The kernel's fused multiply-add rounds once where the codec rounds twice, which moves the bf16
+rounding of about one weight in 2^14 by one step (2^-8): 2^-8 * 2^-7 = 3e-5 of the result's norm;
+f32 sums add about 1e-6.  Bound: 2e-4 (f32 results); a bf16 result is off by at most half of its last
+place, 2^-8 of each value and so of the norm."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+Q8_0, Q4_K, Q6_K = 8, 12, 14
+F32_TOL = 2e-4
+BF16_TOL = 2.0 ** -8 + F32_TOL
+
+
+@pytest.fixture(scope="module")
+def qa():
+    if not torch.cuda.is_available():
+        pytest.fail("no GPU visible: the HIP path cannot run (there is no fallback)")
+    import izwi_amd
+    izwi_amd.lib()
+    torch.cuda.set_device(0)
+    return izwi_amd
+
+
+def weight(qa, oracle, dtype, n, k, seed):
+    if dtype == Q6_K:
+        rng = np.random.default_rng(seed)
+        blocks = rng.integers(0, 256, size=(n * k // 256, 210), dtype=np.uint8)
+        blocks[:, 208:] = (1e-3 * rng.uniform(0.5, 2.0, size=blocks.shape[0])).astype(np.float16).view(np.uint8).reshape(-1, 2)
+        blocks = blocks.reshape(-1)
+    else:
+        blocks = oracle.quantize(dtype, oracle.randn(seed, (n, k), std=0.02))
+    return qa.QMatMul.from_qtensor(qa.QTensor.from_blocks(qa.GgmlDType(dtype), blocks, (n, k)))
+
+
+def dense(mm):
+    return mm.qtensor.dequantize().to(torch.bfloat16).double()
+
+
+def off(y, want):
+    return float((y.double() - want).norm() / want.norm())
+
+
+@pytest.mark.parametrize("dtype,m,n,k", [
+    (Q4_K, 1, 16, 256), (Q4_K, 33, 100, 768), (Q4_K, 65, 128, 256), (Q4_K, 96, 129, 1280), (Q4_K, 97, 300, 512),
+    (Q4_K, 128, 1024, 4096), (Q4_K, 129, 272, 3072), (Q4_K, 192, 1000, 2048), (Q4_K, 500, 384, 1024),
+    (Q8_0, 65, 130, 288), (Q8_0, 100, 64, 32), (Q8_0, 128, 1024, 1056), (Q8_0, 70, 96, 3072), (Q8_0, 193, 200, 800),
+    (Q6_K, 65, 128, 256), (Q6_K, 96, 130, 768), (Q6_K, 127, 257, 2560), (Q6_K, 300, 1024, 4096)])
+def test_product_and_its_epilogues(qa, oracle, dtype, m, n, k):
+    print(f"regb dtype={dtype} m={m} n={n} k={k}", flush=True)
+    mm = weight(qa, oracle, dtype, n, k, 300 + n)
+    x = torch.from_numpy(oracle.randn(301 + m, (m, k))).cuda().to(torch.bfloat16)
+    want = x.double() @ dense(mm).t()
+    assert off(mm.forward_bf16_to_f32(x), want) < F32_TOL
+    assert off(mm.forward(x), want) < BF16_TOL
+    if m > 64:  # (fewer rows run the integer arithmetic in these calls)
+        res = torch.from_numpy(oracle.randn(302 + m, (m, n))).cuda()
+        assert off(mm.forward(x.float()), want) < F32_TOL
+        assert off(mm.forward_fused(x, residual=res, out_dtype=torch.float32), want + res.double()) < F32_TOL
+        resb = res.to(torch.bfloat16)
+        y = resb.clone()
+        mm.forward_fused(x, residual=y, out=y)  # in place
+        assert off(y, want + resb.double()) < BF16_TOL
+
+
+@pytest.mark.parametrize("types,m,ns,k", [
+    ((Q4_K, Q4_K, Q4_K), 65, (256, 128, 100), 512), ((Q4_K, Q4_K, Q6_K), 101, (512, 130, 130), 2048),
+    ((Q8_0, Q8_0), 128, (384, 640), 1056), ((Q6_K, Q4_K, Q6_K, Q4_K), 300, (16, 257, 128, 48), 768)])
+def test_groups_equal_their_members(qa, oracle, types, m, ns, k):
+    parts = [weight(qa, oracle, t, n, k, 400 + 7 * i) for i, (t, n) in enumerate(zip(types, ns))]
+    x = torch.from_numpy(oracle.randn(401, (m, k))).cuda().to(torch.bfloat16)
+    for got_f, got_b, mm in zip(qa.forward_group(parts, x.float()), qa.forward_group(parts, x), parts):
+        want = x.double() @ dense(mm).t()
+        assert off(got_f, want) < F32_TOL
+        assert off(got_b, want) < BF16_TOL
+
+
+@pytest.mark.parametrize("dtype", [Q8_0, Q4_K])
+@pytest.mark.parametrize("m", [65, 129, 150, 179, 192])
+def test_mlp_of_a_small_model_at_prefill_rows(qa, oracle, dtype, m):
+    """gate | up split along k leave their partial sums in scratch memory beside their results."""
+    gate, up, down = (weight(qa, oracle, dtype, n, k, 500 + i) for i, (n, k) in enumerate([(3072, 1024), (3072, 1024), (1024, 3072)]))
+    x = torch.from_numpy(oracle.randn(501 + m, (m, 1024))).cuda()
+    xd = x.to(torch.bfloat16).double()
+    h = torch.nn.functional.silu(xd @ dense(gate).t()) * (xd @ dense(up).t())
+    gate_up = qa.Qwen3GateUpProjection.new_separate(gate, up)
+    got = gate_up.forward_silu_mul(x)
+    assert off(got, h) < 2 * F32_TOL  # two products
+    y = qa.Qwen3Mlp(gate_up, down).forward(x)
+    assert torch.equal(y, down.forward(got))
+    assert off(y, got.to(torch.bfloat16).double() @ dense(down).t()) < F32_TOL
