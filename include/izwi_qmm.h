@@ -399,6 +399,23 @@ int izwi_qmm_forward_gate_up_silu_f32(const izwi_qmm_weight* gate, const izwi_qm
 int izwi_qmm_mlp_forward_f32(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, const izwi_qmm_weight* down,
                              const float* x, int64_t m, float* y, int mem_space, void* stream);
 
+/* One decoder layer at one token, `Qwen3Layer::forward` (qwen3/core.rs:1863-1881), as one call for the
+ * host: the six launches of izwi_qmm_forward_group_normed_f32 (q | k | v behind the input norm),
+ * izwi_decode_attention_step_f32 (scale head_dim^-1/2), izwi_qmm_forward_fused (o, + x),
+ * izwi_qmm_forward_gate_up_silu_normed_f32 and izwi_qmm_forward_fused (down, + residual), whose
+ * arguments and results these are, value for value.  q is `[num_heads * head_dim, hidden]`, k and v
+ * `[num_kv_heads * head_dim, hidden]`, o `[hidden, num_heads * head_dim]`, gate and up `[inter, hidden]`,
+ * down `[hidden, inter]`; x and y are `[hidden]` (y may be x).  The intermediate results lie in `workspace`,
+ * device memory of at least workspace_bytes: q, k, v, attention output (num_heads * head_dim), layer input
+ * of the MLP (hidden) and its product (inter), each rounded up to 128 floats.  Device pointers only. */
+int izwi_qmm_decode_layer_f32(const izwi_qmm_weight* q, const izwi_qmm_weight* k, const izwi_qmm_weight* v,
+                              const izwi_qmm_weight* o, const izwi_qmm_weight* gate, const izwi_qmm_weight* up,
+                              const izwi_qmm_weight* down, const float* x, const float* input_norm,
+                              const float* post_norm, const float* qk_norm, const float* cos_sin, int64_t num_heads,
+                              int64_t num_kv_heads, int64_t head_dim, float eps, float* k_cache, float* v_cache,
+                              int64_t kv_capacity, int64_t pos, float* workspace, uint64_t workspace_bytes, float* y,
+                              void* stream);
+
 /* Prefill form: bf16 activations `[m, k]`, weights dequantized to bf16 in LDS,
  * MFMA with f32 accumulation; y is f32 or bf16 per `out_dtype`.  Replaces the
  * to_dtype(F32) -> QMatMul -> to_dtype(activation dtype) sequence of

@@ -83,6 +83,7 @@ PROTOTYPES = {
     "izwi_qmm_forward_group_bf16": (C.c_int, [_vp, _i32, _vp, _i64, _vp, C.c_int, C.c_int, _vp]),
     "izwi_qmm_forward_gate_up_silu_f32": (C.c_int, [_vp, _vp, _vp, _i64, _vp, C.c_int, _vp]),
     "izwi_qmm_mlp_forward_f32": (C.c_int, [_vp, _vp, _vp, _vp, _i64, _vp, C.c_int, _vp]),
+    "izwi_qmm_decode_layer_f32": (C.c_int, [_vp] * 12 + [_i64] * 3 + [C.c_float, _vp, _vp, _i64, _i64, _vp, _u64, _vp, _vp]),
     "izwi_qmm_forward_normed_f32": (C.c_int, [_vp, _vp, _i64, _vp, C.c_float, _vp, C.c_int, _vp]),
     "izwi_qmm_forward_group_normed_f32": (C.c_int, [_vp, _i32, _vp, _i64, _vp, C.c_float, _vp, C.c_int, _vp]),
     "izwi_qmm_forward_gate_up_silu_normed_f32": (C.c_int, [_vp, _vp, _vp, _i64, _vp, C.c_float, _vp, C.c_int, _vp]),

@@ -4,6 +4,7 @@
 
 #include <atomic>
 #include <chrono>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -1466,6 +1467,47 @@ int izwi_qmm_mlp_forward_f32(const izwi_qmm_weight* gate, const izwi_qmm_weight*
     }
     HIP_TRY(yo.finish(stream));
     return IZWI_QMM_OK;
+    });
+}
+
+int izwi_qmm_decode_layer_f32(const izwi_qmm_weight* q, const izwi_qmm_weight* k, const izwi_qmm_weight* v,
+                              const izwi_qmm_weight* o, const izwi_qmm_weight* gate, const izwi_qmm_weight* up,
+                              const izwi_qmm_weight* down, const float* x, const float* input_norm,
+                              const float* post_norm, const float* qk_norm, const float* cos_sin, int64_t num_heads,
+                              int64_t num_kv_heads, int64_t head_dim, float eps, float* k_cache, float* v_cache,
+                              int64_t kv_capacity, int64_t pos, float* workspace, uint64_t workspace_bytes, float* y,
+                              void* stream) {
+    return qmm_guarded("izwi_qmm_decode_layer_f32", [&]() -> int {
+    if (!q || !k || !v || !o || !gate || !up || !down) return fail(IZWI_QMM_ERR_INVALID, "NULL weight");
+    if (!x || !input_norm || !post_norm || !qk_norm || !cos_sin || !k_cache || !v_cache || !workspace || !y)
+        return fail(IZWI_QMM_ERR_INVALID, "decode_layer: NULL buffer");
+    if (num_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0 || num_heads > (1 << 24) || num_kv_heads > (1 << 24) || head_dim > 8192)
+        return fail(IZWI_QMM_ERR_INVALID, "decode_layer: %lld heads, %lld kv heads, head_dim %lld", (long long)num_heads,
+                    (long long)num_kv_heads, (long long)head_dim);
+    const int64_t hidden = q->layout.k, n_q = num_heads * head_dim, n_kv = num_kv_heads * head_dim, inter = gate->layout.n;
+    auto is = [](const izwi_qmm_weight* w, int64_t rows, int64_t cols) {
+        return w->layout.n_stacked == 1 && w->layout.n == rows && w->layout.k == cols;
+    };
+    if (!is(q, n_q, hidden) || !is(k, n_kv, hidden) || !is(v, n_kv, hidden) || !is(o, hidden, n_q) || !is(gate, inter, hidden) ||
+        !is(up, inter, hidden) || !is(down, hidden, inter))
+        return fail(IZWI_QMM_ERR_INVALID, "decode_layer: the weights' shapes do not fit together");
+    auto padded = [](int64_t count) { return (count + 127) & ~(int64_t)127; };
+    const int64_t pieces[6] = {n_q, n_kv, n_kv, n_q, hidden, inter};
+    float* at[6];
+    uint64_t used = 0;
+    for (int i = 0; i < 6; i++) at[i] = workspace + used, used += (uint64_t)padded(pieces[i]);
+    if (workspace_bytes < used * sizeof(float))
+        return fail(IZWI_QMM_ERR_INVALID, "decode_layer: workspace of %llu bytes, %llu needed", (unsigned long long)workspace_bytes,
+                    (unsigned long long)(used * sizeof(float)));
+    const izwi_qmm_weight* qkv[3] = {q, k, v};
+    if (int rc = izwi_qmm_forward_group_normed_f32(qkv, 3, x, 1, input_norm, eps, at, IZWI_QMM_DEVICE, stream)) return rc;
+    const float scale = (float)(1.0 / std::sqrt((double)head_dim));
+    if (int rc = izwi_decode_attention_step_f32(at[0], at[1], at[2], qk_norm, cos_sin, num_heads, num_kv_heads, head_dim, eps, k_cache,
+                                                v_cache, kv_capacity, pos, scale, at[3], stream))
+        return rc;
+    if (int rc = izwi_qmm_forward_fused(o, at[3], IZWI_QMM_OUT_F32, 1, x, at[4], IZWI_QMM_OUT_F32, IZWI_QMM_DEVICE, stream)) return rc;
+    if (int rc = izwi_qmm_forward_gate_up_silu_normed_f32(gate, up, at[4], 1, post_norm, eps, at[5], IZWI_QMM_DEVICE, stream)) return rc;
+    return izwi_qmm_forward_fused(down, at[5], IZWI_QMM_OUT_F32, 1, at[4], y, IZWI_QMM_OUT_F32, IZWI_QMM_DEVICE, stream);
     });
 }
 

@@ -17,8 +17,12 @@ from .qmatmul import _stream_ptr
 def _ok(*tensors: torch.Tensor) -> bool:
     """All on one GPU, contiguous, one dtype, f32 or f16 (the hooks' `matches!(dtype, F32 | F16)`)."""
     dev, dt = tensors[0].device, tensors[0].dtype
-    return dt in (torch.float32, torch.float16) and all(
-        t.is_cuda and t.device == dev and t.dtype == dt and t.is_contiguous() for t in tensors)
+    if dt is not torch.float32 and dt is not torch.float16:
+        return False
+    for t in tensors:
+        if not (t.is_cuda and t.dtype is dt and t.is_contiguous() and t.device == dev):
+            return False
+    return True
 
 
 def _fn(name: str, t: torch.Tensor):
@@ -30,7 +34,7 @@ def try_fused_rms_norm(input: torch.Tensor, weight: torch.Tensor, eps: float):  
     if input.dim() < 1 or not _ok(input, weight):
         return None
     hidden = input.shape[-1]
-    if hidden == 0 or tuple(weight.shape) != (hidden,) or input.numel() == 0:
+    if hidden == 0 or weight.shape != (hidden,) or input.numel() == 0:
         return None
     out = torch.empty_like(input)
     check(_fn('rms_norm', input)(input.data_ptr(), weight.data_ptr(), input.numel() // hidden, hidden, eps,

@@ -170,6 +170,11 @@ extern "C" {
         m: i64, h: *mut f32, mem_space: c_int, stream: *mut c_void) -> c_int;
     pub fn izwi_qmm_mlp_forward_f32(gate: *const IzwiQmmWeight, up: *const IzwiQmmWeight,
         down: *const IzwiQmmWeight, x: *const f32, m: i64, y: *mut f32, mem_space: c_int, stream: *mut c_void) -> c_int;
+    pub fn izwi_qmm_decode_layer_f32(q: *const IzwiQmmWeight, k: *const IzwiQmmWeight, v: *const IzwiQmmWeight,
+        o: *const IzwiQmmWeight, gate: *const IzwiQmmWeight, up: *const IzwiQmmWeight, down: *const IzwiQmmWeight,
+        x: *const f32, input_norm: *const f32, post_norm: *const f32, qk_norm: *const f32, cos_sin: *const f32,
+        num_heads: i64, num_kv_heads: i64, head_dim: i64, eps: f32, k_cache: *mut f32, v_cache: *mut f32,
+        kv_capacity: i64, pos: i64, workspace: *mut f32, workspace_bytes: u64, y: *mut f32, stream: *mut c_void) -> c_int;
     pub fn izwi_qmm_forward_bf16(w: *const IzwiQmmWeight, x_bf16: *const u16, m: i64, y: *mut c_void,
         out_dtype: c_int, mem_space: c_int, stream: *mut c_void) -> c_int;
     pub fn izwi_qmm_forward_fused(w: *const IzwiQmmWeight, x: *const c_void, x_dtype: c_int, m: i64,

@@ -62,3 +62,44 @@ def test_decode_layer_matches_the_oracle_composition(qa, oracle, hidden, heads, 
         want = x1 + qm("down", hid)
         assert np.abs(got - want).max() <= 2e-3 * np.abs(want).max(), pos
         assert np.abs(kc_d.cpu().numpy() - kc).max() <= 1e-4 * np.abs(kc).max()
+
+
+@pytest.mark.parametrize("hidden,heads,kv_heads,d,inter", [(1024, 8, 2, 128, 3072), (512, 8, 8, 64, 1024), (768, 6, 2, 64, 1280)])
+@pytest.mark.parametrize("types", [(12, 12), (8, 8), (12, 14)])  # of all projections, of v and down
+def test_one_call_layer_equals_its_calls(qa, oracle, hidden, heads, kv_heads, d, inter, types):
+    """The layer as one library call gives the bits of the calls it stands for, output and caches."""
+    from izwi_amd.decode_ops import decode_attention_step
+    from izwi_amd.qmatmul import forward_group
+    from izwi_amd.qwen3_layer import Qwen3DecodeLayer
+    shapes = {"q": (heads * d, hidden), "k": (kv_heads * d, hidden), "v": (kv_heads * d, hidden),
+              "o": (hidden, heads * d), "gate": (inter, hidden), "up": (inter, hidden), "down": (hidden, inter)}
+    if any(k % 256 for _, k in shapes.values()) and types[0] != 8:
+        pytest.skip("k is no whole number of blocks")
+    rng = np.random.default_rng(3)
+    mm = {}
+    for i, (n, s) in enumerate(shapes.items()):
+        t = types[1] if n in ("v", "down") else types[0]
+        if t == 14:  # Q6_K block bytes: any quants and scales, a small block scale
+            b = rng.integers(0, 256, (s[0] * s[1] // 256, 210), dtype=np.uint8)
+            b[:, 208:] = np.array([1e-4], np.float16).view(np.uint8)
+        else:
+            b = oracle.quantize(t, oracle.randn(50 + i, s, std=0.03))
+        mm[n] = qa.QMatMul.from_qtensor(qa.QTensor.from_blocks(qa.GgmlDType(t), b.reshape(-1), s))
+    dev = lambda seed, shape, **kw: torch.from_numpy(oracle.randn(seed, shape, **kw)).cuda()  # noqa: E731
+    w_in, w_post, qk_w = dev(60, (hidden,), mean=1.0, std=0.1), dev(61, (hidden,), mean=1.0, std=0.1), dev(62, (2 * d,), mean=1.0, std=0.1)
+    layer = Qwen3DecodeLayer(w_in, w_post, mm["q"], mm["k"], mm["v"], qk_w, mm["o"], mm["gate"], mm["up"], mm["down"], heads,
+                             kv_heads, d, 1e-6)
+    cap = 40
+    caches = [dev(63 + i, (1, kv_heads, cap, d)) for i in range(2)]
+    ref = [c.clone() for c in caches]
+    for pos in (0, 17, cap - 1):
+        x, cos_sin = dev(70 + pos, (1, hidden)), dev(71 + pos, (1, d))
+        assert layer._forward_one_call(x, cos_sin, caches[0].transpose(1, 2), caches[1].transpose(1, 2), pos) is None
+        got = layer.forward(x, cos_sin, caches[0], caches[1], pos)
+        q, k, v = forward_group(layer.qkv, x, norm_weight=w_in, eps=1e-6)
+        attn = decode_attention_step(q, k, v, qk_w, cos_sin, ref[0], ref[1], pos, 1e-6, d ** -0.5)
+        mid = mm["o"].forward_fused(attn.view(1, heads * d), residual=x)
+        want = mm["down"].forward_fused(layer.gate_up.forward_silu_mul(mid, norm_weight=w_post, eps=1e-6), residual=mid)
+        assert torch.equal(got, want) and torch.equal(caches[0], ref[0]) and torch.equal(caches[1], ref[1])
+    with pytest.raises(qa.QmmError):
+        layer.forward(x, cos_sin, caches[0], caches[1], cap)
