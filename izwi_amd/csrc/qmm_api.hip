@@ -1856,6 +1856,65 @@ int moe_check_stacks(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, con
     return IZWI_QMM_OK;
 }
 
+// Whether the Q4_K expert MLP runs as matrix products over 64-pair chunks: from nine sorted pairs per expert
+// on average.  Measured at 128 experts, top-8, hidden 2048, inter 768, per layer, chunks / expert form on
+// 16-row tiles: 106 / 91 us at 56 tokens, 106 / 103 at 128, 111 / 109 at 136, 109 / 111 at 144 (9 pairs),
+// 111 / 118 at 256, 115 / 138 at 320, 149 / 156 at 512, 224 / 253 at 1024, 318 / 426 at 2048, 592 / 823 at
+// 4096: below, the prefix of a workgroup (its 32 rows at least, over all of k) is not paid back.
+bool moe_on_gemm(const QmmLayout& G, const QmmLayout& D, int64_t t, int top_k) {
+    return qmm_moe_expert_form() < 0 && t * top_k >= 9 * G.n_stacked && qmm_moe_gemm_supported(G, D, t, top_k);
+}
+
+// moe_core on the kernels of qmm_moe_gemm.hip; workspace: y [pairs, hidden] | the token rows' records | the
+// records of silu(gate) * up | chunk tables | routing computed here: ids, weights, perm, offsets, sort scratch
+int moe_gemm(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, const izwi_qmm_weight* down, const float* x,
+             int64_t t, int32_t top_k, const float* logits, const int32_t* ids, const float* weights,
+             const int32_t* perm, const int32_t* offsets, int32_t* ids_out, float* weights_out, float* out, hipStream_t stream) {
+    const QmmLayout& G = gate->layout;
+    const QmmLayout& D = down->layout;
+    const int64_t pairs = t * top_k, hidden = G.k, inter = G.n;
+    const int n_experts = (int)G.n_stacked;
+    const int64_t max_chunks = pairs / QMM_MOE_CHUNK_ROWS + (pairs < n_experts ? pairs : n_experts);
+    size_t total = 0;
+    auto take = [&total](size_t bytes) { const size_t at = total; total += (bytes + 255) & ~(size_t)255; return at; };
+    const size_t y_at = take((size_t)pairs * hidden * 4);
+    const size_t x_at = take(qmm_wide_records_bytes(t, hidden));
+    const size_t h_at = take(qmm_wide_records_bytes(pairs, inter));
+    const size_t chunks_at = take((size_t)(n_experts + 1) * 4), owner_at = take((size_t)max_chunks * 4);
+    const size_t ids_at = take(logits ? (size_t)pairs * 4 : 0), w_at = take(logits ? (size_t)pairs * 4 : 0);
+    const size_t perm_at = take(logits ? (size_t)pairs * 4 : 0), off_at = take(logits ? (size_t)(n_experts + 1) * 4 : 0);
+    const size_t sort_at = take(logits ? (size_t)qmm_moe_sort_scratch_ints(pairs, n_experts) * 4 : 0);
+    uint8_t* ws = nullptr;
+    HIP_TRY(get_scratch(gate->device, stream, total, (void**)&ws));
+    float* y = (float*)(ws + y_at);
+    int32_t *chunks = (int32_t*)(ws + chunks_at), *owner = (int32_t*)(ws + owner_at);
+    hipError_t e = hipSuccess;
+    if (logits) {
+        int32_t *r_ids = (int32_t*)(ws + ids_at), *r_perm = (int32_t*)(ws + perm_at), *r_off = (int32_t*)(ws + off_at);
+        float* r_w = (float*)(ws + w_at);
+        e = qmm_launch_moe_route_wide_rows(logits, t, n_experts, top_k, r_ids, r_w, x, hidden, ws + x_at, stream);
+        if (e == hipSuccess)
+            e = qmm_launch_moe_sort(r_ids, pairs, n_experts, r_perm, r_off, chunks, (int32_t*)(ws + sort_at), stream,
+                                    QMM_MOE_CHUNK_ROWS, owner, max_chunks, nullptr);
+        if (e != hipSuccess) return fail_hip(e, "routing kernels");
+        if (ids_out) HIP_TRY(hipMemcpyAsync(ids_out, r_ids, (size_t)pairs * 4, hipMemcpyDeviceToDevice, stream));
+        if (weights_out) HIP_TRY(hipMemcpyAsync(weights_out, r_w, (size_t)pairs * 4, hipMemcpyDeviceToDevice, stream));
+        weights = r_w, perm = r_perm, offsets = r_off;
+    } else {
+        e = qmm_launch_moe_segments(offsets, n_experts, QMM_MOE_CHUNK_ROWS, chunks, owner, max_chunks, stream, nullptr);
+        if (e == hipSuccess) e = qmm_launch_wide_rows(x, t, hidden, ws + x_at, stream);
+    }
+    if (e == hipSuccess)
+        e = qmm_launch_moe_gemm_gate_up(G, gate->tiled, up->tiled, ws + x_at, top_k, perm, offsets, chunks, owner, n_experts,
+                                        max_chunks, ws + h_at, stream);
+    if (e == hipSuccess)
+        e = qmm_launch_moe_gemm_down(D, down->tiled, ws + h_at, perm, offsets, chunks, owner, n_experts, max_chunks, y, stream);
+    if (e == hipSuccess) e = qmm_launch_moe_combine(y, weights, t, top_k, hidden, out, stream);
+    if (e != hipSuccess) return fail_hip(e, "expert products");
+    if (profiling()) g_silu_fused.fetch_add(1, std::memory_order_relaxed);
+    return IZWI_QMM_OK;
+}
+
 // The expert MLP on device buffers.  With `logits` the routing is computed here too (ids,
 // weights, perm, offsets are then ignored; ids_out / weights_out, if not NULL, receive it): for
 // small batches routing, sort and segment tables are ONE launch.
@@ -1881,6 +1940,10 @@ int moe_core(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, const izwi_
     // workspace: h [pairs, inter] | y [pairs, hidden] | seg_offsets [E + 1]
     //            | tiles: u [pairs, inter], activation records; else: seg_expert [max_segments]
     //            | routing computed here: ids, weights, perm [pairs], offsets [E + 1], sort scratch
+    // Q4_K stacks, many pairs per expert: matrix products over 64-pair chunks, silu(gate) * up quantized where it is
+    // computed (moe_gemm below)
+    if (moe_on_gemm(G, D, t, top_k))
+        return moe_gemm(gate, up, down, x, t, top_k, logits, ids, weights, perm, offsets, ids_out, weights_out, out, stream);
     auto align256 = [](size_t v) { return (v + 255) & ~(size_t)255; };
     const size_t h_bytes = align256((size_t)pairs * inter * sizeof(float));
     const size_t y_bytes = align256((size_t)pairs * hidden * sizeof(float));

@@ -215,7 +215,7 @@ __global__ void quantize_rows_kernel(const float* __restrict__ x, const float* _
 #pragma unroll
         for (int i = 0; i < 16; i++) v[i] = silu_f(v[i]) * u[i];
     }
-    quantize_into_record<QT, true>(v, j, 0, out + group * kRowUnitBytes);
+    quantize_into_record<QT, kRowRecord>(v, j, 0, out + group * kRowUnitBytes);
 }
 
 // Routing of the tokens with the row records of their activation rows: the routing kernel of
@@ -246,7 +246,7 @@ __global__ void route_rows_kernel(const float* __restrict__ logits, int64_t t, i
         const int k0 = unit * 256 + 16 * j;
         float v[16];
         load_run16(x + tok * k + k0, x, k0 + 16 <= k, v);
-        quantize_into_record<QT, true>(v, j, 0, rec + unit * kRowUnitBytes);
+        quantize_into_record<QT, kRowRecord>(v, j, 0, rec + unit * kRowUnitBytes);
     }
 }
 

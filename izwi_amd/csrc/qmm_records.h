@@ -53,13 +53,20 @@ struct Unit {
 // and the scale at 272; Q8_0: the eight block scales at 256.
 constexpr int kRowUnitBytes = 288;
 
+// The wide row record (Q4_K / Q6_K quantization): the same sixteen chunks, then the eight sub-block sums
+// as f16 halves of sum = 32 hi + lo (lo[8] at 256, hi[8] at 272; exact), the scale at 288.
+constexpr int kWideRowUnitBytes = 304;
+enum RecordForm { kTileRecord, kRowRecord, kWideRowRecord };
+
 // ---- launch 1: activation quantizer into the unit records -------------------
 // One 16-lane group per (row, unit); lane j holds elements 16j..16j+15 of the
 // unit in v, i.e. sub-block j / 2, octets 2 (j % 2) and 2 (j % 2) + 1.  `mr` is
-// the row inside the 16-row tile whose record starts at `rec`; with ROW, `rec` is
-// the row's own record of the unit (see kRowUnitBytes) and `mr` is unused.
-template <int QT, bool ROW = false>
+// the row inside the 16-row tile whose record starts at `rec`; in the row forms `rec` is
+// the row's own record of the unit (see kRowUnitBytes, kWideRowUnitBytes) and `mr` is unused.
+template <int QT, RecordForm FORM = kTileRecord>
 __device__ __forceinline__ void quantize_into_record(const float (&v)[16], int j, int mr, uint8_t* rec) {
+    constexpr bool ROW = FORM != kTileRecord;
+    static_assert(FORM != kWideRowRecord || QT == QMM_Q4_K);
     // the lane's first value of largest magnitude (strictly greater: an equal later one does not
     // replace it; a NaN never wins, as with fmaxf), with its sign
     float best = 0.0f;
@@ -80,7 +87,7 @@ __device__ __forceinline__ void quantize_into_record(const float (&v)[16], int j
             scale_mul = __fdiv_rn(-128.0f, (key & 1) ? -amax : amax);
             d = __fdiv_rn(1.0f, scale_mul);
         }
-        if (j == 0) side[ROW ? 4 : mr] = d;
+        if (j == 0) side[FORM == kWideRowRecord ? 8 : ROW ? 4 : mr] = d;
     } else {
         // BlockQ8_0::from_float on the lane pair's 32 values
         amax = fmaxf(amax, __int_as_float(dpp<kDppXor1>(__float_as_int(amax))));
@@ -104,7 +111,13 @@ __device__ __forceinline__ void quantize_into_record(const float (&v)[16], int j
         s16 = __builtin_amdgcn_sdot4((int)q[2], 0x01010101, s16, false);
         s16 = __builtin_amdgcn_sdot4((int)q[3], 0x01010101, s16, false);
         const int bsum = s16 + dpp<kDppXor1>(s16); // the sub-block's 32 quants
-        if ((j & 1) == 0) {
+        if (FORM == kWideRowRecord) {
+            if ((j & 1) == 0) {
+                _Float16* sums = reinterpret_cast<_Float16*>(side);
+                sums[s] = (_Float16)(short)(bsum & 31);
+                sums[8 + s] = (_Float16)(short)(bsum >> 5);
+            }
+        } else if ((j & 1) == 0) {
             uint8_t* planes = ROW ? reinterpret_cast<uint8_t*>(side) : reinterpret_cast<uint8_t*>(side + 16) + mr * 16;
             planes[s] = (uint8_t)(bsum & 127);
             planes[8 + s] = (uint8_t)(bsum >> 7);

@@ -1,0 +1,76 @@
+"""The expert products over 64-pair chunks (Q4_K stacks, many pairs per expert): the same integers and the
+same f32 operations as the 16-row-tile kernels, so the same bits; and the oracle."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def qa():
+    import izwi_amd
+    return izwi_amd
+
+
+def _stacks(qa, oracle, E, hidden, inter, seed):
+    dt = qa.GgmlDType.Q4K
+    raw = [oracle.quantize(int(dt), oracle.randn(seed + i, (E * n, k), std=0.05))
+           for i, (n, k) in enumerate([(inter, hidden), (inter, hidden), (hidden, inter)])]
+    shapes = [(E, inter, hidden), (E, inter, hidden), (E, hidden, inter)]
+    return raw, qa.MoeExperts(*(qa.QTensor.from_blocks(dt, b, s) for b, s in zip(raw, shapes)))
+
+
+# panels of one to four units and a ragged one (1280 = 5 units in panels of four), one to three parts of the
+# down projection's 512 rows with a half-filled one, experts with no, one, 32, 33, 64 and 65 pairs
+@pytest.mark.parametrize("E,hidden,inter,counts", [
+    (6, 256, 256, [0, 1, 32, 33, 64, 65]),
+    (5, 1280, 512, [3, 31, 130, 0, 96]),
+    (4, 2048, 768, [63, 64, 17, 200]),
+    (3, 768, 1792, [40, 20, 1]),
+    (9, 512, 2048, [0, 0, 70, 0, 0, 128, 0, 0, 5]),
+])
+def test_chunks_equal_the_tile_kernels(qa, oracle, E, hidden, inter, counts):
+    import torch
+    from izwi_amd import capi
+    raw, experts = _stacks(qa, oracle, E, hidden, inter, 4100 + hidden)
+    t = sum(counts)
+    assert t >= 9 * E  # the sizes these kernels are taken for
+    rng = np.random.default_rng(5)
+    ids_np = rng.permutation(np.repeat(np.arange(E, dtype=np.int32), counts)).reshape(t, 1)
+    x_np = oracle.randn(4200, (t, hidden))
+    x_np[t // 2, 256:] = 0.0  # units without a scale
+    x = torch.from_numpy(x_np).cuda()
+    ids = torch.from_numpy(ids_np).cuda()
+    wts_np = rng.uniform(0.1, 1.0, (t, 1)).astype(np.float32)
+    wts = torch.from_numpy(wts_np).cuda()
+    perm, offsets = qa.moe_sort(ids, E)
+    got = experts.forward(x, ids, wts, perm, offsets)
+    try:
+        capi.check(capi.lib().izwi_qmm_set_moe_expert_form(1))
+        tiles = experts.forward(x, ids, wts, perm, offsets)
+    finally:
+        capi.check(capi.lib().izwi_qmm_set_moe_expert_form(-1))
+    assert torch.equal(got.view(torch.int32), tiles.view(torch.int32))
+    want = oracle.moe_forward(12, x_np, ids_np, wts_np, *raw, E, inter)
+    g = got.cpu().numpy()
+    # a last-bit difference of silu(gate) * up may move an 8-bit quant of the second product by one step
+    assert np.linalg.norm(g - want) <= 1e-3 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("t", [144, 500, 2100])  # 2100 * 8 pairs: beyond the one-workgroup sort
+def test_layer_equals_the_tile_kernels(qa, oracle, t):
+    import torch
+    from izwi_amd import capi
+    E, hidden, inter = 128, 512, 256
+    _, experts = _stacks(qa, oracle, E, hidden, inter, 4300)
+    x = torch.from_numpy(oracle.randn(4400 + t, (t, hidden))).cuda()
+    logits = torch.from_numpy(oracle.randn(4401 + t, (t, E))).cuda()
+    got = [experts.layer(logits, x, 8, return_routing=True) for _ in range(2)]
+    try:
+        capi.check(capi.lib().izwi_qmm_set_moe_expert_form(1))
+        tiles = experts.layer(logits, x, 8, return_routing=True)
+    finally:
+        capi.check(capi.lib().izwi_qmm_set_moe_expert_form(-1))
+    for g in got:
+        for a, b in zip(g, tiles):
+            assert torch.equal(a.view(torch.int32), b.view(torch.int32))
