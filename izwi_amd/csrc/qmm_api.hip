@@ -1856,6 +1856,39 @@ int moe_check_stacks(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, con
     return IZWI_QMM_OK;
 }
 
+// Where the routing kernels write: straight into the caller's buffers (two copy launches of 1.5 us each and
+// their gaps otherwise), or into the workspace and copied from there where a caller asked for none,
+// or handed buffers that overlap what the later kernels read or write, or are not aligned for them.
+struct RoutingOut {
+    int32_t* ids;
+    float* weights;
+    int32_t* ids_copy = nullptr;
+    float* weights_copy = nullptr;
+    size_t bytes;
+    RoutingOut(int32_t* ids_out, float* weights_out, void* ids_ws, void* weights_ws, const float* logits, const float* x,
+               const float* out, int64_t t, int top_k, int n_experts, int64_t hidden) {
+        bytes = (size_t)t * top_k * 4;
+        auto apart = [](const void* a, size_t na, const void* b, size_t nb) {
+            return (uintptr_t)a + na <= (uintptr_t)b || (uintptr_t)b + nb <= (uintptr_t)a;
+        };
+        auto direct = [&](const void* p, const void* other) {
+            return p && (uintptr_t)p % 4 == 0 && apart(p, bytes, logits, (size_t)t * n_experts * 4) &&
+                   apart(p, bytes, x, (size_t)t * hidden * 4) && apart(p, bytes, out, (size_t)t * hidden * 4) &&
+                   (!other || apart(p, bytes, other, bytes));
+        };
+        const bool d_ids = direct(ids_out, weights_out), d_w = direct(weights_out, ids_out);
+        ids = d_ids ? ids_out : (int32_t*)ids_ws;
+        weights = d_w ? weights_out : (float*)weights_ws;
+        if (!d_ids) ids_copy = ids_out;
+        if (!d_w) weights_copy = weights_out;
+    }
+    hipError_t copy_out(hipStream_t stream) const {
+        if (ids_copy)
+            if (hipError_t e = hipMemcpyAsync(ids_copy, ids, bytes, hipMemcpyDeviceToDevice, stream)) return e;
+        return weights_copy ? hipMemcpyAsync(weights_copy, weights, bytes, hipMemcpyDeviceToDevice, stream) : hipSuccess;
+    }
+};
+
 // Whether the Q4_K expert MLP runs as matrix products over 64-pair chunks: from nine sorted pairs per expert
 // on average.  Measured at 128 experts, top-8, hidden 2048, inter 768, per layer, chunks / expert form on
 // 16-row tiles: 106 / 91 us at 56 tokens, 106 / 103 at 128, 111 / 109 at 136, 109 / 111 at 144 (9 pairs),
@@ -1890,15 +1923,15 @@ int moe_gemm(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, const izwi_
     int32_t *chunks = (int32_t*)(ws + chunks_at), *owner = (int32_t*)(ws + owner_at);
     hipError_t e = hipSuccess;
     if (logits) {
-        int32_t *r_ids = (int32_t*)(ws + ids_at), *r_perm = (int32_t*)(ws + perm_at), *r_off = (int32_t*)(ws + off_at);
-        float* r_w = (float*)(ws + w_at);
+        const RoutingOut routing(ids_out, weights_out, ws + ids_at, ws + w_at, logits, x, out, t, top_k, n_experts, hidden);
+        int32_t *r_ids = routing.ids, *r_perm = (int32_t*)(ws + perm_at), *r_off = (int32_t*)(ws + off_at);
+        float* r_w = routing.weights;
         e = qmm_launch_moe_route_wide_rows(logits, t, n_experts, top_k, r_ids, r_w, x, hidden, ws + x_at, stream);
         if (e == hipSuccess)
             e = qmm_launch_moe_sort(r_ids, pairs, n_experts, r_perm, r_off, chunks, (int32_t*)(ws + sort_at), stream,
                                     QMM_MOE_CHUNK_ROWS, owner, max_chunks, nullptr);
         if (e != hipSuccess) return fail_hip(e, "routing kernels");
-        if (ids_out) HIP_TRY(hipMemcpyAsync(ids_out, r_ids, (size_t)pairs * 4, hipMemcpyDeviceToDevice, stream));
-        if (weights_out) HIP_TRY(hipMemcpyAsync(weights_out, r_w, (size_t)pairs * 4, hipMemcpyDeviceToDevice, stream));
+        HIP_TRY(routing.copy_out(stream));
         weights = r_w, perm = r_perm, offsets = r_off;
     } else {
         e = qmm_launch_moe_segments(offsets, n_experts, QMM_MOE_CHUNK_ROWS, chunks, owner, max_chunks, stream, nullptr);
@@ -1991,8 +2024,9 @@ int moe_core(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, const izwi_
     hipError_t e = hipSuccess;
     if (logits) {
         uint8_t* r = mid + mid_bytes;
-        int32_t* r_ids = (int32_t*)r;
-        float* r_w = (float*)(r + p_bytes);
+        const RoutingOut routing(ids_out, weights_out, r, r + p_bytes, logits, x, out, t, top_k, n_experts, hidden);
+        int32_t* r_ids = routing.ids;
+        float* r_w = routing.weights;
         int32_t* r_perm = (int32_t*)(r + 2 * p_bytes);
         int32_t* r_off = (int32_t*)(r + 3 * p_bytes);
         int32_t* r_sort = (int32_t*)(r + 3 * p_bytes + s_bytes);
@@ -2000,8 +2034,8 @@ int moe_core(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, const izwi_
         // a handful of pairs: the whole layer in two launches (routing inside gate / up, combine
         // inside down), same results
         if (!tiles && pairs <= moe_small_max_pairs() && qmm_moe_small_supported(G, D, t, n_experts, top_k)) {
-            e = qmm_launch_moe_small(G, gate->tiled, up->tiled, D, down->tiled, logits, x, t, n_experts, top_k, h, r_ids,
-                                     r_w, ids_out, weights_out, out, max_segments, gate->n_cus, stream);
+            e = qmm_launch_moe_small(G, gate->tiled, up->tiled, D, down->tiled, logits, x, t, n_experts, top_k, h, (int32_t*)r,
+                                     (float*)(r + p_bytes), ids_out, weights_out, out, max_segments, gate->n_cus, stream);
             if (e == hipSuccess) {
                 if (profiling()) g_silu_fused.fetch_add(1, std::memory_order_relaxed);
                 return IZWI_QMM_OK;
@@ -2031,8 +2065,7 @@ int moe_core(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, const izwi_
             segments_ready = true;
         }
         if (e != hipSuccess) return fail_hip(e, "routing kernels");
-        if (ids_out) HIP_TRY(hipMemcpyAsync(ids_out, r_ids, (size_t)pairs * 4, hipMemcpyDeviceToDevice, stream));
-        if (weights_out) HIP_TRY(hipMemcpyAsync(weights_out, r_w, (size_t)pairs * 4, hipMemcpyDeviceToDevice, stream));
+        HIP_TRY(routing.copy_out(stream));
         ids = r_ids, weights = r_w, perm = r_perm, offsets = r_off;
     }
     if (tiles) {

@@ -74,3 +74,55 @@ def test_layer_equals_the_tile_kernels(qa, oracle, t):
     for g in got:
         for a, b in zip(g, tiles):
             assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
+@pytest.mark.parametrize("pairs,experts", [
+    (16385, 128),   # one pair more than one workgroup's sort takes
+    (17 * 1024, 1), (40001, 3), (20000, 511), (20000, 512),
+    (20000, 513),   # more experts than a workgroup of the wide sort counts
+    (512 * 1024, 128), (512 * 1024 + 1, 128),  # the most workgroups, and one pair beyond them
+])
+def test_sort_of_many_pairs(qa, pairs, experts):
+    import torch
+    rng = np.random.default_rng(pairs + experts)
+    ids = rng.integers(0, experts, size=pairs).astype(np.int32)
+    ids[rng.integers(0, pairs, size=9)] = [-1, experts, 1 << 30, -(1 << 31), -7, experts + 1, -1, experts, 99999]
+    for _ in range(2):  # the scratch memory of the call before is not clean
+        perm, offsets = qa.moe_sort(torch.from_numpy(ids.reshape(-1, 1)).cuda(), experts)
+    valid = np.flatnonzero((ids >= 0) & (ids < experts))
+    want = valid[np.argsort(ids[valid], kind="stable")]
+    assert np.array_equal(perm.cpu().numpy()[:len(want)], want)
+    assert np.array_equal(offsets.cpu().numpy(), np.concatenate([[0], np.cumsum(np.bincount(ids[valid], minlength=experts))]))
+
+
+@pytest.mark.parametrize("t", [1, 16, 24, 56, 144])
+def test_routing_goes_to_the_callers_buffers(qa, oracle, t):
+    """ids and weights from buffers of the caller: plain ones (written by the routing kernel), one inside the
+    logits and the same one for both (copied afterwards, the weights last)."""
+    import torch
+    from izwi_amd import capi
+    E, hidden, inter = 128, 256, 256
+    _, experts = _stacks(qa, oracle, E, hidden, inter, 4500)
+    x = torch.from_numpy(oracle.randn(4600 + t, (t, hidden))).cuda()
+    logits = torch.from_numpy(oracle.randn(4601 + t, (t, E))).cuda()
+    want, want_ids, want_w = experts.layer(logits, x, 8, return_routing=True)
+
+    def call(lg, ids, w):
+        out = torch.empty_like(x)
+        capi.check(capi.lib().izwi_moe_layer_f32(experts.gate._h, experts.up._h, experts.down._h, lg.data_ptr(),
+                                                 x.data_ptr(), t, 8, out.data_ptr(), ids.data_ptr(), w.data_ptr(), capi.DEVICE,
+                                                 torch.cuda.current_stream().cuda_stream))
+        return out
+
+    ids, w = torch.empty_like(want_ids), torch.empty_like(want_w)
+    cases = [(logits, ids, w)]
+    if t > 8:  # (up to 8 tokens the one-launch kernels write both buffers themselves)
+        both = torch.empty_like(want_ids)
+        inside = logits.clone()
+        cases += [(logits, both, both.view(torch.float32)), (inside, inside.view(torch.int32).view(-1)[:t * 8], w)]
+    for i, (lg, a, b) in enumerate(cases):
+        out = call(lg, a, b)
+        assert torch.equal(out, want)
+        if i != 1:
+            assert torch.equal(a.view(-1), want_ids.view(-1))
+        assert torch.equal(b.view(-1), want_w.view(-1))
