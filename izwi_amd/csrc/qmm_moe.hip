@@ -64,8 +64,8 @@ __global__ void sort_hist_kernel(const int32_t* __restrict__ ids, int64_t pairs,
     extern __shared__ int32_t sh[];
     for (int e = threadIdx.x; e < n_experts; e += blockDim.x) sh[e] = 0;
     __syncthreads();
-    int64_t p = (int64_t)blockIdx.x * kSortChunk + threadIdx.x;
-    if (threadIdx.x < kSortChunk && p < pairs) {
+    int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; // a chunk of pairs per workgroup
+    if (p < pairs) {
         int32_t e = ids[p];
         if ((uint32_t)e < (uint32_t)n_experts) atomicAdd(&sh[e], 1); // integer adds: order-free
     }
@@ -335,6 +335,78 @@ bool block_sort_fits(int64_t pairs, int n_experts) {
     return runs <= (int64_t)kBlockSortMaxRuns * (kBlockSortThreads / 64) && block_sort_lds_ints(pairs, n_experts) * 4 <= kBlockSortMaxLds;
 }
 
+// More pairs than one workgroup holds: a workgroup of sixteen waves per 1024 pairs.  Launch 1 counts them per
+// expert (sort_hist_kernel); in launch 2 every workgroup adds up the counts of all workgroups and of
+// those before its own - 512 bytes of L2 reads per 1024 pairs at 128 experts, all requested at once - where a scan
+// launch of one workgroup walked them in a chain, and ranks its pairs as the one-workgroup sort
+// does.  Workgroup 0 writes the tables.  128 experts, 32768 pairs: 5.0 + 50.0 + 17.0 us (count, scan, scatter with
+// a thread per expert) -> 3.5 + 7.1.  The reads grow with the square of the workgroups: to 512 of them.
+constexpr int kWideSortChunk = kBlockSortThreads, kWideSortMaxChunks = 512, kWideSortMaxExperts = 512;
+__global__ __launch_bounds__(kBlockSortThreads) void sort_wide_kernel(const int32_t* __restrict__ ids, int64_t pairs, int n_experts,
+                                                                      const int32_t* __restrict__ hist, int chunks,
+                                                                      int32_t* __restrict__ perm, int32_t* __restrict__ offsets,
+                                                                      int32_t* __restrict__ seg_offsets, int seg_rows,
+                                                                      int32_t* __restrict__ seg_expert, int max_segments) {
+    // before[n_experts] | total[n_experts] | counts[16][n_experts] | masks[16][2 n_experts]
+    extern __shared__ int32_t sh[];
+    __shared__ int32_t wave_tot[16], wave_seg[16], total_segments;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = kBlockSortThreads / 64;
+    int32_t *before = sh, *total = sh + n_experts, *counts = sh + 2 * n_experts;
+    uint32_t* masks = reinterpret_cast<uint32_t*>(counts + waves * n_experts) + wave * 2 * n_experts;
+    const int chunk = blockIdx.x;
+    const int64_t p = (int64_t)chunk * kWideSortChunk + threadIdx.x;
+    const int e = p < pairs ? ids[p] : -1;
+    const bool ok = e >= 0 && e < n_experts;
+    for (int i = threadIdx.x; i < (2 + waves) * n_experts; i += kBlockSortThreads) sh[i] = 0;
+    __syncthreads();
+    {
+        // thread (expert, slice of the chunks)
+        const int slices = kBlockSortThreads / n_experts, per = (chunks + slices - 1) / slices;
+        const int x = (int)threadIdx.x % n_experts, slice = (int)threadIdx.x / n_experts;
+        if (slice < slices) {
+            int b = 0, t = 0;
+#pragma unroll 8
+            for (int c = slice * per; c < min(chunks, slice * per + per); c++) {
+                const int h = hist[(int64_t)c * n_experts + x];
+                t += h, b += c < chunk ? h : 0;
+            }
+            if (b) atomicAdd(&before[x], b); // integer adds: order-free
+            if (t) atomicAdd(&total[x], t);
+        }
+    }
+    int rank, run;
+    wave_ranks(e, n_experts, lane, masks, rank, run);
+    if (ok && rank == 0) counts[wave * n_experts + e] = run;
+    __syncthreads();
+    const int e0 = threadIdx.x;
+    const int c = e0 < n_experts ? total[e0] : 0, sg = (c + seg_rows - 1) / seg_rows;
+    const int inc_c = wave_inclusive_sum(c, lane), inc_s = wave_inclusive_sum(sg, lane);
+    if (lane == 63) wave_tot[wave] = inc_c, wave_seg[wave] = inc_s;
+    __syncthreads();
+    int base_c = 0, base_s = 0;
+    for (int w = 0; w < wave; w++) base_c += wave_tot[w], base_s += wave_seg[w];
+    if (e0 < n_experts) {
+        int at = base_c + inc_c - c + before[e0]; // where the chunk's first pair of the expert goes
+        for (int w = 0; w < waves; w++) {
+            const int n = counts[w * n_experts + e0];
+            counts[w * n_experts + e0] = at;
+            at += n;
+        }
+    }
+    if (chunk == 0 && e0 <= n_experts) { // (thread n_experts holds the grand totals: its own c is 0)
+        offsets[e0] = base_c + inc_c - c;
+        const int first = base_s + inc_s - sg;
+        if (seg_offsets) seg_offsets[e0] = first;
+        if (seg_expert)
+            for (int i = 0; i < sg && first + i < max_segments; i++) seg_expert[first + i] = e0;
+        if (e0 == n_experts) total_segments = first;
+    }
+    __syncthreads();
+    if (ok) perm[counts[wave * n_experts + e] + rank] = (int32_t)p;
+    if (chunk == 0 && seg_expert) // entries past the last segment say so
+        for (int i = total_segments + (int)threadIdx.x; i < max_segments; i += kBlockSortThreads) seg_expert[i] = -1;
+}
+
 // seg_offsets[e] = sum over e' < e of ceil(count(e') / seg_rows).  One block:
 // every thread sums a contiguous run of experts, the runs are scanned in LDS.
 // With seg_expert: seg_expert[s] = expert of segment s, -1 for s past the last
@@ -510,9 +582,23 @@ hipError_t qmm_launch_moe_sort(const int32_t* ids, int64_t pairs, int n_experts,
         sort_block_kernel<<<1, kBlockSortThreads, lds, stream>>>(ids, (int)pairs, n_experts, perm, offsets, seg_offsets, seg_rows, seg_expert, (int)max_segments, expert_order);
         return hipGetLastError();
     }
+    size_t sh = (size_t)n_experts * sizeof(int32_t);
+    if (pairs >= 1 && pairs <= (int64_t)kWideSortMaxChunks * kWideSortChunk && n_experts <= kWideSortMaxExperts) {
+        const int wide_chunks = (int)((pairs + kWideSortChunk - 1) / kWideSortChunk);
+        const size_t lds = (size_t)(2 + 3 * (kBlockSortThreads / 64)) * sh;
+        if (lds > 48 * 1024) {
+            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&sort_wide_kernel),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, kBlockSortMaxLds);
+            if (e != hipSuccess) return e;
+        }
+        sort_hist_kernel<<<(unsigned)wide_chunks, kWideSortChunk, sh, stream>>>(ids, pairs, n_experts, scratch);
+        sort_wide_kernel<<<(unsigned)wide_chunks, kBlockSortThreads, lds, stream>>>(ids, pairs, n_experts, scratch, wide_chunks, perm,
+                                                                                    offsets, seg_offsets, seg_rows, seg_expert,
+                                                                                    (int)max_segments);
+        return hipGetLastError();
+    }
     int64_t chunks = (pairs + kSortChunk - 1) / kSortChunk;
     if (chunks < 1) chunks = 1;
-    size_t sh = (size_t)n_experts * sizeof(int32_t);
     sort_hist_kernel<<<(unsigned)chunks, kSortChunk, sh, stream>>>(ids, pairs, n_experts, scratch);
     sort_scan_kernel<<<1, 256, sh, stream>>>(scratch, chunks, n_experts, offsets, seg_offsets, seg_rows, seg_expert,
                                              (int)max_segments);
