@@ -1891,9 +1891,8 @@ struct RoutingOut {
 
 // Whether the Q4_K expert MLP runs as matrix products over 64-pair chunks: from nine sorted pairs per expert
 // on average.  Measured at 128 experts, top-8, hidden 2048, inter 768, per layer, chunks / expert form on
-// 16-row tiles: 106 / 91 us at 56 tokens, 106 / 103 at 128, 111 / 109 at 136, 109 / 111 at 144 (9 pairs),
-// 111 / 118 at 256, 115 / 138 at 320, 149 / 156 at 512, 224 / 253 at 1024, 318 / 426 at 2048, 592 / 823 at
-// 4096: below, the prefix of a workgroup (its 32 rows at least, over all of k) is not paid back.
+// 16-row tiles: 106 / 91 us at 56 tokens, 104 / 103 at 128, 108 / 111 at 144 (9 pairs), 108 / 118 at 256,
+// 136 / 156 at 512, 206 / 253 at 1024, 294 / 426 at 2048, 497 / 823 at 4096: below, the prefix of a workgroup (its 32 rows at least, over all of k) is not paid back.
 bool moe_on_gemm(const QmmLayout& G, const QmmLayout& D, int64_t t, int top_k) {
     return qmm_moe_expert_form() < 0 && t * top_k >= 9 * G.n_stacked && qmm_moe_gemm_supported(G, D, t, top_k);
 }

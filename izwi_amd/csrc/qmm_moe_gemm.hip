@@ -24,9 +24,12 @@
 //
 // Bound by vector instructions (160 per block of 32 x 32 outputs and unit, half of them the unpacking that two
 // blocks of pairs share, 640 cycles) beside 17 matrix instructions (544 cycles), which two waves per
-// SIMD overlap in part.  128 experts, top-8, 2048 x 768: gate | up 316 us and down 194 at 4096 tokens (650 and
-// 530 TOP/s), where the 16-row-tile kernels took 480 and 260 and the quantizer between them 40;
-// 85 and 44 at 512 tokens, before 92, 48 and 8.  The layer 823 -> 592 us and 156 -> 149.
+// SIMD overlap in part: at 4096 tokens the vector ALU is busy 58 % of the cycles and the matrix pipe 35 %.
+// 128 experts, top-8, 2048 x 768: gate | up 282 us and down 164 at 4096 tokens (730 and 630 TOP/s), where the
+// 16-row-tile kernels took 480 and 260 and the quantizer between them 40; 80 and 41 at 512 tokens, before 92, 48
+// and 8 (a workgroup's life is 40 us there, 1.5 per compute unit).  The layer 823 -> 497 us and 156 -> 136.  Of that,
+// starting on the first unit's records while the others land, stores at 32-bit offsets and the two waves
+// of a SIMD half a phase apart with the one in its matrix instructions preferred: 556 -> 497 and 150 -> 136.
 #include <hip/hip_runtime.h>
 
 #include "qmm_internal.h"
@@ -95,7 +98,7 @@ __device__ __forceinline__ f16x2 mins_pair(uint32_t m, f16x2 c, f16x2 minus_1024
 
 template <bool GATE_UP, int NRB>
 __device__ __forceinline__ void chunk_body(const MoeGemmParams& P, const uint8_t* wbase0, const uint8_t* wbase1, uint8_t* smem,
-                                           UnitRegs (&raw)[2], const uint32_t (&lane_off)[2], const int* out_rows, int part,
+                                           UnitRegs (&raw)[2], const uint32_t (&lane_off)[2], const uint32_t* out_off, int part,
                                            int pos_begin, int pos_end, int wave, int lane) {
     const int row = lane & 31, h = lane >> 5;
     // byte offsets of the lane's A chunks: [b & 1][i], of its sums, and of its four runs of scales
@@ -122,7 +125,12 @@ __device__ __forceinline__ void chunk_body(const MoeGemmParams& P, const uint8_t
     uint32_t unit_off = 0;                    // of the next unit to request: panel, then unit in the panel
     int in_panel = 0;
     const uint8_t* lds = smem;
+    if (wave >= kWaves / 2) __builtin_amdgcn_s_sleep(10); // the two waves of a SIMD half a phase apart
     for (int u = 0; u < P.k_units; u++, lds += kUnitLds) {
+        if (u == 1) { // the other units' records have landed
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            barrier_lds();
+        }
         // (past the last unit the same one is requested again: no branch around the loads)
         if (u + 1 < P.k_units) {
             if (++in_panel == P.s) in_panel = 0, unit_off += (uint32_t)P.panel_bytes - (uint32_t)(P.s - 1) * 256u;
@@ -130,6 +138,8 @@ __device__ __forceinline__ void chunk_body(const MoeGemmParams& P, const uint8_t
         }
 #pragma unroll
         for (int c = 0; c < 2; c++) {
+            // (a wave in its matrix instructions goes before the other one of its SIMD in its finish)
+            __builtin_amdgcn_s_setprio(1);
             UnitRegs& w = raw[c];
             const u32x4 hdr = w.hdr;
             const uint32_t sc[2] = {hdr.y & 0x3f3f3f3fu, (hdr.w & 0x0f0f0f0fu) | (((hdr.y >> 6) & 0x03030303u) << 4)};
@@ -178,6 +188,7 @@ __device__ __forceinline__ void chunk_body(const MoeGemmParams& P, const uint8_t
             // the unit is consumed: the next one into its registers (the fences keep the scheduler from
             // gathering the loads of both columns at the loop's end, where nothing is left to cover them)
             asm volatile("" : "+v"(d), "+v"(dmin)); // (computed here, so that the header's registers are free)
+            __builtin_amdgcn_s_setprio(0);
             if (NRB > 1) __builtin_amdgcn_sched_barrier(0);
             const uint8_t* wu = (c ? wbase1 : wbase0) + unit_off;
             w.hdr = *reinterpret_cast<const u32x4*>(wu + lane_off[c]);
@@ -229,21 +240,24 @@ __device__ __forceinline__ void chunk_body(const MoeGemmParams& P, const uint8_t
                     v, j, 0, static_cast<uint8_t*>(P.out) + ((int64_t)(pos_begin + m) * P.out_units + part) * kWideRowUnitBytes);
         }
     } else {
-        float* y = static_cast<float*>(P.out);
+        // 32-bit byte offsets from one uniform base; only an expert's last chunk has rows that do not exist
+        uint8_t* y = static_cast<uint8_t*>(P.out);
+        const bool whole = pos_end - pos_begin == NRB * 32;
 #pragma unroll
-        for (int rb = 0; rb < NRB; rb++)
+        for (int c = 0; c < 2; c++) {
+            const int n = part * 512 + c * 256 + col;
+            if (n >= P.n) continue; // (uniform: n is a multiple of 256)
 #pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const i32x4 rows = *reinterpret_cast<const i32x4*>(out_rows + rb * 32 + 8 * g + 4 * h);
+            for (int rb = 0; rb < NRB; rb++)
 #pragma unroll
-                for (int c = 0; c < 2; c++) {
-                    const int n = part * 512 + c * 256 + col;
-                    if (n >= P.n) continue;
+                for (int g = 0; g < 4; g++) {
+                    const u32x4 rows = *reinterpret_cast<const u32x4*>(out_off + rb * 32 + 8 * g + 4 * h);
 #pragma unroll
                     for (int r = 0; r < 4; r++)
-                        if (rows[r] >= 0) y[(int64_t)rows[r] * P.n + n] = acc[c][rb][4 * g + r];
+                        if (whole || rb * 32 + 8 * g + 4 * h + r < pos_end - pos_begin)
+                            *reinterpret_cast<float*>(y + (rows[r] + (uint32_t)n * 4u)) = acc[c][rb][4 * g + r];
                 }
-            }
+        }
     }
 }
 
@@ -255,10 +269,34 @@ __device__ __forceinline__ void load_lds4(uint32_t lds, uint32_t off, const uint
     asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
 }
 
+// The records of units [u0, u1) of the chunk's rows into their LDS images
+__device__ __forceinline__ void issue_records(const MoeGemmParams& P, const uint32_t* src_off, uint8_t* smem, int nrb, int u0, int u1,
+                                              int wave, int lane) {
+    const uint32_t lds_base = (uint32_t)(uintptr_t)smem;
+    const int groups = nrb * 4, per_unit = 2 * groups + nrb + 1; // pieces of quants (two halves), sums, scales
+    for (int piece = u0 * per_unit + wave; piece < u1 * per_unit; piece += kWaves) {
+        const int u = piece / per_unit, sub = piece - u * per_unit;
+        const uint32_t unit_lds = lds_base + (uint32_t)u * kUnitLds;
+        const uint8_t* base = P.records + u * kWideRowUnitBytes;
+        if (sub < 2 * groups) {
+            const int p = sub / groups, g = sub - p * groups;
+            const int r = g * 8 + (lane >> 3);
+            load_lds16(__builtin_amdgcn_readfirstlane(unit_lds + p * (kRows * 128) + g * 1024),
+                       src_off[r] + (uint32_t)p * 128u + (uint32_t)((lane & 7) ^ ((r >> 1) & 7)) * 16u, base);
+        } else if (sub < 2 * groups + nrb) {
+            const int q = sub - 2 * groups, r = q * 32 + (lane >> 1);
+            load_lds16(__builtin_amdgcn_readfirstlane(unit_lds + kSumsAt + q * 1024),
+                       src_off[r] + 256u + (uint32_t)((lane & 1) ^ ((r >> 3) & 1)) * 16u, base);
+        } else {
+            load_lds4(__builtin_amdgcn_readfirstlane(unit_lds + kScalesAt), src_off[lane] + 288u, base);
+        }
+    }
+}
+
 template <bool GATE_UP>
 __global__ __launch_bounds__(64 * kWaves) void moe_gemm_q4k_kernel(MoeGemmParams P) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    __shared__ __attribute__((aligned(16))) int out_rows[kRows];
+    __shared__ __attribute__((aligned(16))) uint32_t out_off[kRows]; // down: byte offsets of the output rows
     __shared__ uint32_t src_off[kRows];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -294,35 +332,15 @@ __global__ __launch_bounds__(64 * kWaves) void moe_gemm_q4k_kernel(MoeGemmParams
     if (threadIdx.x < kRows) {
         // (a row past the end reads the chunk's first row; its sums are never stored)
         const int pos = pos_begin + (int)threadIdx.x;
-        const bool exists = pos < pos_end;
-        const int at = exists ? pos : pos_begin;
+        const int at = pos < pos_end ? pos : pos_begin;
         const uint32_t pair = (uint32_t)P.perm[at];
         const uint32_t src = P.row_div == 0 ? (uint32_t)at : P.row_div == 1 ? pair : __umulhi(pair, P.row_magic);
         src_off[threadIdx.x] = src * P.row_bytes;
-        out_rows[threadIdx.x] = exists ? (int)pair : -1;
+        out_off[threadIdx.x] = pair * (uint32_t)P.n * 4u;
     }
     barrier_lds();
-    {
-        const uint32_t lds_base = (uint32_t)(uintptr_t)smem;
-        const int groups = nrb * 4, per_unit = 2 * groups + nrb + 1; // pieces of quants (two halves), sums, scales
-        for (int piece = wave; piece < P.k_units * per_unit; piece += kWaves) {
-            const int u = piece / per_unit, sub = piece - u * per_unit;
-            const uint32_t unit_lds = lds_base + (uint32_t)u * kUnitLds;
-            const uint8_t* base = P.records + u * kWideRowUnitBytes;
-            if (sub < 2 * groups) {
-                const int p = sub / groups, g = sub - p * groups;
-                const int r = g * 8 + (lane >> 3);
-                load_lds16(__builtin_amdgcn_readfirstlane(unit_lds + p * (kRows * 128) + g * 1024),
-                           src_off[r] + (uint32_t)p * 128u + (uint32_t)((lane & 7) ^ ((r >> 1) & 7)) * 16u, base);
-            } else if (sub < 2 * groups + nrb) {
-                const int q = sub - 2 * groups, r = q * 32 + (lane >> 1);
-                load_lds16(__builtin_amdgcn_readfirstlane(unit_lds + kSumsAt + q * 1024),
-                           src_off[r] + 256u + (uint32_t)((lane & 1) ^ ((r >> 3) & 1)) * 16u, base);
-            } else {
-                load_lds4(__builtin_amdgcn_readfirstlane(unit_lds + kScalesAt), src_off[lane] + 288u, base);
-            }
-        }
-    }
+    // The first unit's records, then, under the arithmetic of the first unit, the others'
+    issue_records(P, src_off, smem, nrb, 0, 1, wave, lane);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     // (a use of the loaded registers: the compiler's own wait for them stands here, not in the loop)
 #pragma unroll
@@ -332,10 +350,11 @@ __global__ __launch_bounds__(64 * kWaves) void moe_gemm_q4k_kernel(MoeGemmParams
         for (int b = 0; b < 4; b++) asm volatile("" : "+v"(raw[c].q[b]));
     }
     barrier_lds();
+    issue_records(P, src_off, smem, nrb, 1, P.k_units, wave, lane);
     if (nrb == 2)
-        chunk_body<GATE_UP, 2>(P, wbase0, wbase1, smem, raw, lane_off, out_rows, part, pos_begin, pos_end, wave, lane);
+        chunk_body<GATE_UP, 2>(P, wbase0, wbase1, smem, raw, lane_off, out_off, part, pos_begin, pos_end, wave, lane);
     else
-        chunk_body<GATE_UP, 1>(P, wbase0, wbase1, smem, raw, lane_off, out_rows, part, pos_begin, pos_end, wave, lane);
+        chunk_body<GATE_UP, 1>(P, wbase0, wbase1, smem, raw, lane_off, out_off, part, pos_begin, pos_end, wave, lane);
 }
 
 // ---- the activation rows' records, 16 lanes per (row, unit) ----------------------------------
@@ -415,6 +434,7 @@ bool qmm_moe_gemm_supported(const QmmLayout& G, const QmmLayout& D, int64_t t, i
     // 32-bit offsets into a matrix and into the records, pair / top_k by multiplication, the grid
     if (G.matrix_bytes >= ((int64_t)1 << 31) || D.matrix_bytes >= ((int64_t)1 << 31)) return false;
     if (t * G.k_units * kWideRowUnitBytes >= ((int64_t)1 << 32) || pairs * D.k_units * kWideRowUnitBytes >= ((int64_t)1 << 32)) return false;
+    if (pairs * D.n * 4 >= ((int64_t)1 << 32)) return false;
     const int64_t parts = G.n / 256 > (D.n + 511) / 512 ? G.n / 256 : (D.n + 511) / 512;
     return pairs * top_k < ((int64_t)1 << 32) && (pairs / kRows + G.n_stacked) * parts < 0x7ffffff0;
 }
