@@ -616,11 +616,17 @@ __device__ __forceinline__ void panel_dot(WPanel<QT>& p, const uint8_t* xu0, int
     // activations as their address and a weight scale multiplied by zero wherever the
     // compiler keeps their arithmetic.  (Their header is zero padding or a copy of unit
     // 0's, so every factor is finite.)
+    // NU = 4: all four units exist, a compile-time fact: straight-line code, in which the LDS reads, matrix
+    // instructions and conversions of different units and blocks overlap.  (A branch per unit and block cut
+    // a wave's panel into blocks of one matrix instruction that each waited for its LDS read and its result.  Per
+    // layer in a graph, with the branches / straight-line: 0.6B shapes Q8_0 44.6 / 39.0 us at 8 rows and 50.6 /
+    // 45.4 at 64, 8B shapes Q8_0 86.0 / 81.5 at 8, with Q6_K for v and down 66.1 / 65.0.)
+    static_assert(QT == QMM_Q4_K || NU == 0 || NU == 4);
     int xo[4];
     float ef[4];
 #pragma unroll
     for (int u = 0; u < 4; u++) {
-        const bool exists = u < n_units; // uniform
+        const bool exists = NU == 4 || u < n_units; // uniform
         xo[u] = exists ? u * UB : 0;
         ef[u] = exists ? 1.0f : 0.0f;
     }
@@ -663,7 +669,7 @@ __device__ __forceinline__ void panel_dot(WPanel<QT>& p, const uint8_t* xu0, int
 #pragma unroll
                     for (int e = 0; e < 2; e++) {
                         const int u = 2 * up + e;
-                        if (u >= n_units) continue; // uniform
+                        if (NU == 0 && u >= n_units) continue; // uniform
                         const uint32_t w0 = e ? ql.z : ql.x, w1 = e ? ql.w : ql.y;
                         const uint32_t h0 = e ? qh.z : qh.x, h1 = e ? qh.w : qh.y;
                         // six-bit quants, then q - 32 as int8 in every byte without a borrow
@@ -680,7 +686,7 @@ __device__ __forceinline__ void panel_dot(WPanel<QT>& p, const uint8_t* xu0, int
 #pragma unroll
                     for (int e = 0; e < 2; e++) {
                         const int u = 2 * up + e;
-                        if (u >= n_units) continue;
+                        if (NU == 0 && u >= n_units) continue;
                         const uint32_t hw = t < 2 ? p.hdr[u].x : t < 4 ? p.hdr[u].y : t < 6 ? p.hdr[u].z : p.hdr[u].w;
                         const int sc_lo = (int)(int8_t)((hw >> (16 * (t & 1))) & 0xffu);
                         const int sc_hi = (int)(int8_t)((hw >> (16 * (t & 1) + 8)) & 0xffu);
@@ -693,7 +699,7 @@ __device__ __forceinline__ void panel_dot(WPanel<QT>& p, const uint8_t* xu0, int
         }
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-            if (u >= n_units) continue;
+            if (NU == 0 && u >= n_units) continue;
             const float d = qmm_f16_bits_to_f32((uint16_t)(p.dch[u].x & 0xffffu)) * ef[u];
             const float4 dx = *reinterpret_cast<const float4*>(xu0 + xo[u] + Unit<QT>::kQuant + grp * 16);
             acc[0] += (d * dx.x) * (float)isum[u][0];
@@ -708,7 +714,7 @@ __device__ __forceinline__ void panel_dot(WPanel<QT>& p, const uint8_t* xu0, int
             i32x4 dd[4];
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                if (u >= n_units) continue; // uniform
+                if (NU == 0 && u >= n_units) continue; // uniform
                 const u32x4 qq = p.q[2 * b + (u >> 1)];
                 const uint32_t w0 = (u & 1) ? qq.z : qq.x, w1 = (u & 1) ? qq.w : qq.y;
                 const long a = *reinterpret_cast<const long*>(xu0 + xo[u] + lane16 + (b >> 1) * 1024 + (b & 1) * 8);
@@ -716,7 +722,7 @@ __device__ __forceinline__ void panel_dot(WPanel<QT>& p, const uint8_t* xu0, int
             }
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                if (u >= n_units) continue;
+                if (NU == 0 && u >= n_units) continue;
                 const uint32_t hw = b < 2 ? p.hdr[u].x : b < 4 ? p.hdr[u].y : b < 6 ? p.hdr[u].z : p.hdr[u].w;
                 const float dw = qmm_f16_bits_to_f32((uint16_t)((hw >> (16 * (b & 1))) & 0xffffu)) * ef[u];
                 const float4 dx = *reinterpret_cast<const float4*>(xu0 + xo[u] + Unit<QT>::kQuant +
@@ -962,7 +968,7 @@ __device__ __forceinline__ void oneshot_body(const MfmaParams& P, const MfmaPara
                     for (int b = 0; b < WPanel<QT>::QC / 2; b++) transpose_pair(p.q[2 * b], p.q[2 * b + 1]);
                 }
                 transposed = true;
-                panel_dot<QT, false>(p, xu0, n_units, j, grp, acc);
+                panel_dot<QT, false, NU>(p, xu0, n_units, j, grp, acc);
             }
         }
         if (win == n_win - 1) {
@@ -1589,17 +1595,18 @@ hipError_t launch_expert_form(const MfmaParams& P, dim3 grid, int waves, size_t 
 
 namespace {
 // form 0: one tile of rows, one activation window; 1: the general one-shot form; 2: streaming
-template <int QT, bool EP>
+// (NU: all panels hold that many units, or 0)
+template <int QT, bool EP, int NU = 0>
 hipError_t launch_dense_form(int form, const MfmaParams& P, unsigned grid, int waves, size_t lds, hipStream_t stream) {
-    const void* fn = form == 0   ? reinterpret_cast<const void*>(&gemv_mfma_oneshot_kernel<QT, true, false, EP>)
-                     : form == 1 ? reinterpret_cast<const void*>(&gemv_mfma_oneshot_kernel<QT, false, false, EP>)
+    const void* fn = form == 0   ? reinterpret_cast<const void*>(&gemv_mfma_oneshot_kernel<QT, true, false, EP, NU>)
+                     : form == 1 ? reinterpret_cast<const void*>(&gemv_mfma_oneshot_kernel<QT, false, false, EP, NU>)
                                  : reinterpret_cast<const void*>(&gemv_mfma_stream_kernel<QT, EP>);
     if (lds > 48 * 1024) {
         hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e != hipSuccess) return e;
     }
-    if (form == 0) launch_mfma(gemv_mfma_oneshot_kernel<QT, true, false, EP>, grid, 64 * waves, lds, stream, P);
-    else if (form == 1) launch_mfma(gemv_mfma_oneshot_kernel<QT, false, false, EP>, grid, 64 * waves, lds, stream, P);
+    if (form == 0) launch_mfma(gemv_mfma_oneshot_kernel<QT, true, false, EP, NU>, grid, 64 * waves, lds, stream, P);
+    else if (form == 1) launch_mfma(gemv_mfma_oneshot_kernel<QT, false, false, EP, NU>, grid, 64 * waves, lds, stream, P);
     else gemv_mfma_stream_kernel<QT, EP><<<grid, 64 * waves, lds, stream>>>(P);
     return hipGetLastError();
 }
@@ -1784,6 +1791,12 @@ hipError_t qmm_launch_gemv_mfma(const QmmLayout& L, const void* tiled, const flo
     if (L.dtype == QMM_Q4_K)
         return epilogue ? launch_dense_form<QMM_Q4_K, true>(form, P, grid, waves, lds, stream)
                         : launch_dense_form<QMM_Q4_K, false>(form, P, grid, waves, lds, stream);
+    if (full_panels(L) && L.dtype == QMM_Q6_K)
+        return epilogue ? launch_dense_form<QMM_Q6_K, true, 4>(form, P, grid, waves, lds, stream)
+                        : launch_dense_form<QMM_Q6_K, false, 4>(form, P, grid, waves, lds, stream);
+    if (full_panels(L))
+        return epilogue ? launch_dense_form<QMM_Q8_0, true, 4>(form, P, grid, waves, lds, stream)
+                        : launch_dense_form<QMM_Q8_0, false, 4>(form, P, grid, waves, lds, stream);
     if (L.dtype == QMM_Q6_K)
         return epilogue ? launch_dense_form<QMM_Q6_K, true>(form, P, grid, waves, lds, stream)
                         : launch_dense_form<QMM_Q6_K, false>(form, P, grid, waves, lds, stream);
@@ -2104,6 +2117,9 @@ hipError_t qmm_launch_gemv_mfma_multi(const QmmLayout* const* layouts, const voi
     }
     const size_t lds = std::max((size_t)P.window_units * unit_bytes(L0.dtype), (size_t)waves * 256 * 4);
     if (lds > 160 * 1024) return hipErrorNotSupported;
+    if (L0.dtype != QMM_Q4_K && full_panels(L0))
+        return L0.dtype == QMM_Q6_K ? launch_dense_form<QMM_Q6_K, false, 4>(0, P, grid, waves, lds, stream)
+                                    : launch_dense_form<QMM_Q8_0, false, 4>(0, P, grid, waves, lds, stream);
     const bool full = L0.dtype == QMM_Q4_K && full_panels(L0) && straight_line_fits(groups * (tile_parallel ? n_tiles : 1), waves, n_cus);
     const void* fn = full                   ? reinterpret_cast<const void*>(&gemv_mfma_oneshot_kernel<QMM_Q4_K, true, false, false, 4>)
                      : L0.dtype == QMM_Q4_K ? reinterpret_cast<const void*>(&gemv_mfma_oneshot_kernel<QMM_Q4_K, true>)
