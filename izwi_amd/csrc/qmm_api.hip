@@ -612,6 +612,9 @@ QmmCallScope::~QmmCallScope() {
 }
 
 namespace {
+constexpr int kNotTaken = 1; // (statuses are zero or negative)
+int group_own_quantizer(const izwi_qmm_weight* const* weights, int32_t n_weights, const float* x, int64_t m, float* const* ys,
+                        hipStream_t stream);
 int batched_group_on_records(const izwi_qmm_weight* const* weights, int32_t n_weights, const float* x, int64_t m,
                              float* const* ys, void* records, hipStream_t stream);
 } // namespace
@@ -1314,12 +1317,30 @@ int forward_group_impl(const izwi_qmm_weight* const* weights, int32_t n_weights,
             if (int rc = izwi_qmm_forward_f32(weights[i], x, m, ys[i], mem_space, stream_)) return rc;
         return IZWI_QMM_OK;
     }
+    if (int rc = group_own_quantizer(weights, n_weights, x, m, ys, stream); rc != kNotTaken) return rc;
     // 3 <= m <= 64: the activations are quantized once, every projection reads the same records
     // (up to 16 rows in one launch for all of them)
     void* scratch = nullptr;
     HIP_TRY(get_scratch(w0->device, stream, qmm_gemv_mfma_workspace_bytes(w0->layout, m), &scratch));
     HIP_TRY(qmm_launch_quantize_ws(w0->layout.dtype, x, m, w0->layout.k, scratch, stream));
     return batched_group_on_records(weights, n_weights, x, m, ys, scratch, stream);
+}
+
+// The batched decode kernel for a group of one block type on f32 activations that its workgroups quantize
+// themselves, where that is the better form; kNotTaken (nothing launched) where it is not.
+int group_own_quantizer(const izwi_qmm_weight* const* weights, int32_t n_weights, const float* x, int64_t m, float* const* ys,
+                        hipStream_t stream) {
+    const QmmLayout* layouts[QMM_MAX_GROUP];
+    const void* tiled[QMM_MAX_GROUP];
+    for (int i = 0; i < n_weights; i++) layouts[i] = &weights[i]->layout, tiled[i] = weights[i]->tiled;
+    ProfileScope prof(weights[0], stream);
+    hipError_t e = qmm_launch_gemv_mfma_multi(layouts, tiled, n_weights, m, ys, nullptr, weights[0]->n_cus, stream, x);
+    if (e == hipErrorNotSupported) {
+        (void)hipGetLastError();
+        prof.on = false;
+        return kNotTaken;
+    }
+    return e == hipSuccess ? IZWI_QMM_OK : fail_hip(e, "grouped batched decode kernel");
 }
 
 // The batched decode kernel for a group of one block type whose quantized activations are in `records`.
@@ -1434,10 +1455,14 @@ int izwi_qmm_mlp_forward_f32(const izwi_qmm_weight* gate, const izwi_qmm_weight*
         float* u = reinterpret_cast<float*>(ws + rx + part);
         uint8_t* rec_h = ws + rx + 2 * part;
         if (profiling()) g_silu_fused.fetch_add(1, std::memory_order_relaxed);
-        HIP_TRY(qmm_launch_quantize_ws(G.dtype, (const float*)xi.dev, m, G.k, ws, stream));
         const izwi_qmm_weight* gu[2] = {gate, up};
         float* gu_y[2] = {g, u};
-        if (int rc = batched_group_on_records(gu, 2, nullptr, m, gu_y, ws, stream)) return rc;
+        int rc = group_own_quantizer(gu, 2, (const float*)xi.dev, m, gu_y, stream);
+        if (rc == kNotTaken) {
+            HIP_TRY(qmm_launch_quantize_ws(G.dtype, (const float*)xi.dev, m, G.k, ws, stream));
+            rc = batched_group_on_records(gu, 2, nullptr, m, gu_y, ws, stream);
+        }
+        if (rc) return rc;
         HIP_TRY(qmm_launch_quantize_silu_mul_ws(D.dtype, g, u, m, D.k, rec_h, stream));
         float* dy[1] = {(float*)yo.dev};
         if (int rc = batched_group_on_records(&down, 1, nullptr, m, dy, rec_h, stream)) return rc;

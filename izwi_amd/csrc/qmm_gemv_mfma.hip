@@ -31,6 +31,7 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 #include "qmm_internal.h"
 #include "qmm_moe_route.h"
@@ -266,6 +267,7 @@ struct MfmaParams {
     const uint8_t* wv[QMM_MAX_GROUP];
     float* yv[QMM_MAX_GROUP];
     int m, n;
+    int k, units_magic; // in-kernel quantization: values per activation row; 65536 / k_units, rounded up
     int k_units, k_groups, slots;
     int row_tiles, panel_bytes;
     int nwk, nwr, wave_magic;
@@ -836,7 +838,11 @@ __device__ __forceinline__ bool tile_parallel_decode(int n_tiles, int rt_groups,
 // EP: the sums go through the epilogue of P.ep (residual add, f32 or bf16 store).
 // (the compact single-stage Q4_K form is held to the 80 registers of six waves per SIMD: two 12-wave
 // workgroups per CU keep every panel of gate | up in flight at once)
-template <int QT, bool SINGLE, bool GROUPED, bool EP, int NU>
+// XQ (single-stage, dense): `ws` is the f32 activations and the workgroup quantizes the rows of its tile
+// into the window itself, own_runs (row, unit) pairs at the most per 16 lanes (the compact form's 80 registers
+// hold three).
+__host__ __device__ constexpr int own_runs(bool compact) { return compact ? 3 : 4; }
+template <int QT, bool SINGLE, bool GROUPED, bool EP, int NU, bool XQ = false>
 __device__ __forceinline__ void oneshot_body(const MfmaParams& P, const MfmaParams& P0) {
     constexpr int UB = Unit<QT>::kBytes;
     constexpr int NL = WPanel<QT>::kLoads; // loads of one panel
@@ -891,19 +897,47 @@ __device__ __forceinline__ void oneshot_body(const MfmaParams& P, const MfmaPara
     }
 
     // the first activation window goes first (loads return in order), then the panel
+    // (in-kernel quantization: first the activations' loads, all of them)
+    static_assert(!XQ || (SINGLE && !GROUPED));
+    // (the compact form's 80 registers hold either the activations or the panel)
+    constexpr bool kPanelUnderQuantizer = !(QT == QMM_Q4_K && NU == 0);
+    const int own_rows = min(16, P.m - tile0 * 16), own_items = own_rows * P.k_units, own_groups = waves * 4;
+    constexpr int kOwnRuns = own_runs(!kPanelUnderQuantizer);
+    float own[XQ ? kOwnRuns : 1][16];
+    if constexpr (XQ) {
+        const float* x = reinterpret_cast<const float*>(P.ws) + (int64_t)tile0 * 16 * P.k;
+#pragma unroll
+        for (int i = 0; i < kOwnRuns; i++) {
+            const int item = (int)(threadIdx.x >> 4) + i * own_groups;
+            const int mr = (item * P.units_magic) >> 16, unit = item - mr * P.k_units, k0 = unit * 256 + 16 * j;
+            load_run16<false>(x + (int64_t)mr * P.k + k0, x, item < own_items && k0 + 16 <= P.k, own[i]);
+        }
+    }
     const int w0_units = min(P.window_units, P.k_units);
-    if (!(QMM_MFMA_ABL & 16)) issue_window_copy<QT>(records, lds_x, w0_units, wave, waves, lane);
+    if (!XQ && !(QMM_MFMA_ABL & 16)) issue_window_copy<QT>(records, lds_x, w0_units, wave, waves, lane);
     // A CU's loads return in the order they were issued, for all its waves together: without this
     // barrier the last wave's window pieces queue behind the other waves' panels, and the barrier
     // below - the start of all arithmetic - waits for nearly the whole workgroup's weights.
-    asm volatile("s_barrier" ::: "memory");
+    if (!XQ) asm volatile("s_barrier" ::: "memory");
     // (a group's tables are read here, behind the window copies: those need nothing from them)
     if (!GROUPED && P.n_weights > 1) pick_group_entry(P0, P.n_weights, group_index, rtg, wbase, yout, n_rows, row_tiles);
     const int rt = rtg * P.nwr + wr;
     const bool rt_ok = rt < row_tiles;
     const int row = rt * 16 + j;
     WPanel<QT> p;
-    load_wpanel<QT>(p, wbase + (int64_t)((rt_ok ? rt : 0) * P.k_groups + wk) * P.panel_bytes, P.slots, lane, j);
+    const uint8_t* panel = wbase + (int64_t)((rt_ok ? rt : 0) * P.k_groups + wk) * P.panel_bytes;
+    if (!XQ || kPanelUnderQuantizer) load_wpanel<QT>(p, panel, P.slots, lane, j);
+    if constexpr (XQ) {
+        // (rows past the last are left as they are in LDS: their sums are never stored)
+#pragma unroll
+        for (int i = 0; i < kOwnRuns; i++) {
+            const int item = (int)(threadIdx.x >> 4) + i * own_groups;
+            const int mr = (item * P.units_magic) >> 16, unit = item - mr * P.k_units;
+            if (item < own_items) // (whole 16-lane groups)
+                quantize_into_record<QT == QMM_Q8_0 ? QMM_Q8_0 : QMM_Q4_K>(own[i], j, mr, lds_x + (size_t)unit * UB);
+        }
+        if (!kPanelUnderQuantizer) load_wpanel<QT>(p, panel, P.slots, lane, j);
+    }
     // The window has landed.  The single-stage form lets the panel fly on: its arithmetic starts on the
     // first chunk pair, and all NL loads of the panel are behind the window.  That count is right only
     // while the compiler keeps every load of the panel: it drops a load whose value no path uses (the
@@ -913,7 +947,8 @@ __device__ __forceinline__ void oneshot_body(const MfmaParams& P, const MfmaPara
     // other instantiation waits for everything, as the multi-stage forms do anyway (they transpose the
     // whole panel before their first stage).
     constexpr bool kEveryPanelLoadUsed = NU == 0 || NU == 4;
-    if (SINGLE && kEveryPanelLoadUsed) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL) : "memory");
+    if (XQ) {} // (the quantizer waited for its own loads)
+    else if (SINGLE && kEveryPanelLoadUsed) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     lds_barrier();
 
@@ -1042,14 +1077,14 @@ __device__ __forceinline__ void oneshot_body(const MfmaParams& P, const MfmaPara
     }
 }
 // The dense launches of the one-shot form: leading scalar arguments (see with_leading_args).
-template <int QT, bool SINGLE, bool GROUPED = false, bool EP = false, int NU = 0>
+template <int QT, bool SINGLE, bool GROUPED = false, bool EP = false, int NU = 0, bool XQ = false>
 __global__ __launch_bounds__(64 * kMaxWaves, (QT == QMM_Q4_K && SINGLE && NU == 0) ? 6 : 3) void gemv_mfma_oneshot_kernel(
         const uint8_t* w_arg, const uint8_t* ws_arg, float* y_arg, int k_units_arg, int k_groups_arg, int row_tiles_arg, int panel_bytes_arg,
         int split_arg, int wave_magic_arg, int n_tiles_arg, int window_arg, MfmaParams P0) {
     static_assert(!GROUPED, "the expert-grouped launches go through gemv_mfma_grouped_kernel");
     const MfmaParams P = with_leading_args(P0, w_arg, ws_arg, y_arg, k_units_arg, k_groups_arg, row_tiles_arg, panel_bytes_arg, split_arg,
                                              wave_magic_arg, n_tiles_arg, window_arg);
-    oneshot_body<QT, SINGLE, false, EP, NU>(P, P0);
+    oneshot_body<QT, SINGLE, false, EP, NU, XQ>(P, P0);
 }
 
 // The expert-grouped launches: thousands of short workgroups, whose waves start faster with
@@ -1626,6 +1661,77 @@ bool straight_line_fits(int64_t groups, int waves, int n_cus) {
 }
 } // namespace
 
+namespace {
+// The launch of a single-stage form whose workgroups quantize their own activations (P.ws: the f32 rows).
+// P is set up for the form on records; a workgroup gets more row tiles where its 16-lane groups would otherwise
+// have more than own_runs units to quantize.  hipErrorNotSupported where the quantizer launch is the cheaper
+// one, by the activation bytes that a compute unit reads for its workgroups one after the other: a launch and the
+// gap behind it are 4 us, the loads, the quantizer's 140 instructions per (row, unit) and 16 lanes and a barrier in every workgroup
+// about 2 at 64 KB.  Layer of projections in a graph, us, with the launch / without at this limit / at 128 KB: 0.6B
+// Q8_0 5 rows 38.7 / 32.9 / 33.3, 8 rows 38.8 / 35.1 / 35.5, 16 rows 39.4 / 38.5 / 41.0, 64 rows 45.3 / 43.4 / 46.5; 8B Q4_K
+// 3 rows 55.6 / 53.3 / 53.6, 8 rows 57.1 / 57.2 / 59.9; 8B Q8_0 4 rows 80.5 / 78.4 / 77.6, 8 rows 81.1 / 81.1 / 82.7.
+constexpr int64_t kOwnQuantizerBytes = 96 * 1024;
+hipError_t launch_own_quantizer(const QmmLayout& L0, MfmaParams P, int64_t x_k, int n_cus, bool epilogue, hipStream_t stream) {
+    // (an output that overlaps the activations: they have to be read whole before a sum is stored)
+    const uintptr_t x0 = (uintptr_t)P.ws, x1 = x0 + (size_t)P.m * x_k * 4;
+    for (int i = 0; i < std::max(P.n_weights, 1); i++) {
+        const uintptr_t y0 = (uintptr_t)(P.n_weights ? P.yv[i] : P.y), y1 = y0 + (size_t)P.m * (P.n_weights ? P.nv[i] : P.n) * 4;
+        if (x0 < y1 && y0 < x1) return hipErrorNotSupported;
+    }
+    const int rows = std::min(P.m, 16), items = rows * P.k_units;
+    const bool q4k = L0.dtype == QMM_Q4_K, full = full_panels(L0);
+    int nwr = P.nwr;
+    bool straight = false;
+    int64_t wgs = 0;
+    auto groups_of = [&](int per) { // workgroups of `per` row tiles
+        if (P.n_weights == 0) return (int64_t)(P.row_tiles + per - 1) / per;
+        int64_t groups = 0;
+        for (int i = 0; i < P.n_weights; i++) groups += (P.row_tiles_v[i] + per - 1) / per;
+        return groups;
+    };
+    for (;; nwr++) {
+        if (P.nwk * nwr > kMaxWaves) return hipErrorNotSupported;
+        wgs = groups_of(nwr) * P.n_tiles;
+        straight = full && (!q4k || straight_line_fits(wgs, P.nwk * nwr, n_cus));
+        if (items <= 4 * P.nwk * nwr * own_runs(q4k && !straight)) break;
+    }
+    const int n_weights = std::max(P.n_weights, 1);
+    if (P.n_weights == 0) P.rt_groups = (P.row_tiles + nwr - 1) / nwr;
+    else {
+        int64_t groups = 0;
+        for (int i = 0; i < n_weights; i++) groups += (P.row_tiles_v[i] + nwr - 1) / nwr, P.rtg_end[i] = (int)groups;
+        P.rt_groups = (int)groups;
+    }
+    P.nwr = nwr;
+    const int64_t rounds = (wgs + n_cus - 1) / n_cus;
+    if (rounds * rows * x_k * 4 > kOwnQuantizerBytes) return hipErrorNotSupported;
+    const int waves = P.nwk * nwr;
+    const size_t lds = std::max((size_t)P.window_units * unit_bytes(L0.dtype), (size_t)waves * 256 * 4);
+    if (lds > 160 * 1024) return hipErrorNotSupported;
+    P.k = (int)x_k;
+    P.units_magic = (65536 + P.k_units - 1) / P.k_units; // exact for the up to 768 items of a workgroup and 32 units
+    const unsigned grid = P.n_tiles > 1 ? (unsigned)((P.rt_groups + 7) / 8 * 8 * P.n_tiles) : (unsigned)P.rt_groups;
+    auto go = [&](auto kernel) -> hipError_t {
+        if (lds > 48 * 1024) {
+            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            if (e != hipSuccess) return e;
+        }
+        launch_mfma(kernel, grid, 64 * waves, lds, stream, P);
+        return hipGetLastError();
+    };
+    auto form = [&](auto qt, auto nu) {
+        return epilogue ? go(gemv_mfma_oneshot_kernel<decltype(qt)::value, true, false, true, decltype(nu)::value, true>)
+                        : go(gemv_mfma_oneshot_kernel<decltype(qt)::value, true, false, false, decltype(nu)::value, true>);
+    };
+    using Four = std::integral_constant<int, 4>;
+    using RunTime = std::integral_constant<int, 0>;
+    auto of_type = [&](auto qt) { return straight ? form(qt, Four{}) : form(qt, RunTime{}); };
+    return q4k                       ? of_type(std::integral_constant<int, QMM_Q4_K>{})
+           : L0.dtype == QMM_Q6_K ? of_type(std::integral_constant<int, QMM_Q6_K>{})
+                                     : of_type(std::integral_constant<int, QMM_Q8_0>{});
+}
+} // namespace
+
 hipError_t qmm_launch_quantize_ws(int dtype, const float* x, int64_t m, int64_t k, void* workspace,
                                   hipStream_t stream, bool x_bf16) {
     if (m <= 0 || k <= 0 || m > 0x3fffffff || k > 0x3fffffff) return hipErrorInvalidValue;
@@ -1683,10 +1789,6 @@ hipError_t qmm_launch_gemv_mfma(const QmmLayout& L, const void* tiled, const flo
     // the streaming form adds up activation windows in y itself: no folded epilogue there
     if (epilogue && !(L.k_groups <= kMaxWaves && L.row_tiles < 8 * (int64_t)n_cus) && L.k_units > P.window_units)
         return hipErrorNotSupported;
-    if (quantize) {
-        hipError_t e = qmm_launch_quantize_ws(L.dtype, x, m, L.k, ws, stream, io && io->x_bf16);
-        if (e != hipSuccess) return e;
-    }
     P.w = (const uint8_t*)tiled;
     P.ws = ws;
     P.y = y;
@@ -1730,6 +1832,18 @@ hipError_t qmm_launch_gemv_mfma(const QmmLayout& L, const void* tiled, const flo
     size_t lds;
     unsigned grid;
     int waves;
+    if (quantize) {
+        if (oneshot && stage_tiles == 1 && L.k_units <= P.window_units && !(io && io->x_bf16) &&
+            !direct_form_applies(L.dtype, stage_tiles, oneshot_nwr, true)) {
+            MfmaParams O = P;
+            O.ws = reinterpret_cast<const uint8_t*>(x);
+            O.nwk = (int)L.k_groups, O.nwr = oneshot_nwr, O.wave_magic = (65536 + O.nwk - 1) / O.nwk;
+            hipError_t e = launch_own_quantizer(L, O, L.k, n_cus, epilogue, stream);
+            if (e != hipErrorNotSupported) return e;
+        }
+        hipError_t e = qmm_launch_quantize_ws(L.dtype, x, m, L.k, ws, stream, io && io->x_bf16);
+        if (e != hipSuccess) return e;
+    }
     if (oneshot) {
         P.nwk = (int)L.k_groups;
         P.nwr = oneshot_nwr;
@@ -2026,7 +2140,7 @@ hipError_t qmm_launch_gemv_mfma_grouped(const QmmLayout& L, const void* tiled, c
 
 hipError_t qmm_launch_gemv_mfma_multi(const QmmLayout* const* layouts, const void* const* tiled, int n_weights,
                                       int64_t m, float* const* ys, const void* workspace, int n_cus,
-                                      hipStream_t stream) {
+                                      hipStream_t stream, const float* x) {
     if (n_weights < 1 || n_weights > QMM_MAX_GROUP || m < 1) return hipErrorInvalidValue;
     if (n_cus <= 0) n_cus = 1;
     const QmmLayout& L0 = *layouts[0];
@@ -2085,6 +2199,11 @@ hipError_t qmm_launch_gemv_mfma_multi(const QmmLayout* const* layouts, const voi
         P.yv[i] = ys[i];
     }
     P.rt_groups = (int)groups;
+    if (x) { // f32 activations: only where the workgroups quantize them themselves
+        if ((n_tiles > 1 && !tile_parallel_applies(n_tiles)) || direct_form_applies(L0.dtype, 1, P.nwr, true)) return hipErrorNotSupported;
+        P.ws = reinterpret_cast<const uint8_t*>(x);
+        return launch_own_quantizer(L0, P, L0.k, n_cus, false, stream);
+    }
     const int waves = P.nwk * P.nwr;
     // (every tile of rows with workgroups of its own: the single-stage forms below, a longer launch)
     const bool tile_parallel = tile_parallel_applies(n_tiles);

@@ -274,9 +274,11 @@ hipError_t qmm_launch_quantize_ws(int dtype, const float* x, int64_t m, int64_t 
 hipError_t qmm_launch_quantize_silu_mul_ws(int dtype, const float* gate, const float* up, int64_t m, int64_t k,
                                            void* workspace, hipStream_t stream);
 size_t qmm_records_bytes(int dtype, int64_t m, int64_t k);
+// With x (f32 [m, k]; `workspace` unused) the workgroups quantize the activations themselves;
+// hipErrorNotSupported, nothing launched, where the two launches are the better form.
 hipError_t qmm_launch_gemv_mfma_multi(const QmmLayout* const* layouts, const void* const* tiled, int n_weights,
                                       int64_t m, float* const* ys, const void* workspace, int n_cus,
-                                      hipStream_t stream);
+                                      hipStream_t stream, const float* x = nullptr);
 
 // ---- MoE ---------------------------------------------------------------------
 // Sorted pairs are processed in segments of this many rows that share one expert.
