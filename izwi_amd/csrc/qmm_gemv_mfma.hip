@@ -618,17 +618,16 @@ __device__ __forceinline__ void panel_dot(WPanel<QT>& p, const uint8_t* xu0, int
     // activations as their address and a weight scale multiplied by zero wherever the
     // compiler keeps their arithmetic.  (Their header is zero padding or a copy of unit
     // 0's, so every factor is finite.)
-    // NU = 4: all four units exist, a compile-time fact: straight-line code, in which the LDS reads, matrix
+    // NU > 0: that many units exist, a compile-time fact: straight-line code, in which the LDS reads, matrix
     // instructions and conversions of different units and blocks overlap.  (A branch per unit and block cut
     // a wave's panel into blocks of one matrix instruction that each waited for its LDS read and its result.  Per
     // layer in a graph, with the branches / straight-line: 0.6B shapes Q8_0 44.6 / 39.0 us at 8 rows and 50.6 /
     // 45.4 at 64, 8B shapes Q8_0 86.0 / 81.5 at 8, with Q6_K for v and down 66.1 / 65.0.)
-    static_assert(QT == QMM_Q4_K || NU == 0 || NU == 4);
     int xo[4];
     float ef[4];
 #pragma unroll
     for (int u = 0; u < 4; u++) {
-        const bool exists = NU == 4 || u < n_units; // uniform
+        const bool exists = u < (NU ? NU : n_units); // uniform
         xo[u] = exists ? u * UB : 0;
         ef[u] = exists ? 1.0f : 0.0f;
     }
@@ -671,7 +670,7 @@ __device__ __forceinline__ void panel_dot(WPanel<QT>& p, const uint8_t* xu0, int
 #pragma unroll
                     for (int e = 0; e < 2; e++) {
                         const int u = 2 * up + e;
-                        if (NU == 0 && u >= n_units) continue; // uniform
+                        if (u >= (NU ? NU : n_units)) continue; // uniform
                         const uint32_t w0 = e ? ql.z : ql.x, w1 = e ? ql.w : ql.y;
                         const uint32_t h0 = e ? qh.z : qh.x, h1 = e ? qh.w : qh.y;
                         // six-bit quants, then q - 32 as int8 in every byte without a borrow
@@ -688,7 +687,7 @@ __device__ __forceinline__ void panel_dot(WPanel<QT>& p, const uint8_t* xu0, int
 #pragma unroll
                     for (int e = 0; e < 2; e++) {
                         const int u = 2 * up + e;
-                        if (NU == 0 && u >= n_units) continue;
+                        if (u >= (NU ? NU : n_units)) continue;
                         const uint32_t hw = t < 2 ? p.hdr[u].x : t < 4 ? p.hdr[u].y : t < 6 ? p.hdr[u].z : p.hdr[u].w;
                         const int sc_lo = (int)(int8_t)((hw >> (16 * (t & 1))) & 0xffu);
                         const int sc_hi = (int)(int8_t)((hw >> (16 * (t & 1) + 8)) & 0xffu);
@@ -701,7 +700,7 @@ __device__ __forceinline__ void panel_dot(WPanel<QT>& p, const uint8_t* xu0, int
         }
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-            if (NU == 0 && u >= n_units) continue;
+            if (u >= (NU ? NU : n_units)) continue;
             const float d = qmm_f16_bits_to_f32((uint16_t)(p.dch[u].x & 0xffffu)) * ef[u];
             const float4 dx = *reinterpret_cast<const float4*>(xu0 + xo[u] + Unit<QT>::kQuant + grp * 16);
             acc[0] += (d * dx.x) * (float)isum[u][0];
@@ -716,7 +715,7 @@ __device__ __forceinline__ void panel_dot(WPanel<QT>& p, const uint8_t* xu0, int
             i32x4 dd[4];
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                if (NU == 0 && u >= n_units) continue; // uniform
+                if (u >= (NU ? NU : n_units)) continue; // uniform
                 const u32x4 qq = p.q[2 * b + (u >> 1)];
                 const uint32_t w0 = (u & 1) ? qq.z : qq.x, w1 = (u & 1) ? qq.w : qq.y;
                 const long a = *reinterpret_cast<const long*>(xu0 + xo[u] + lane16 + (b >> 1) * 1024 + (b & 1) * 8);
@@ -724,7 +723,7 @@ __device__ __forceinline__ void panel_dot(WPanel<QT>& p, const uint8_t* xu0, int
             }
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                if (NU == 0 && u >= n_units) continue;
+                if (u >= (NU ? NU : n_units)) continue;
                 const uint32_t hw = b < 2 ? p.hdr[u].x : b < 4 ? p.hdr[u].y : b < 6 ? p.hdr[u].z : p.hdr[u].w;
                 const float dw = qmm_f16_bits_to_f32((uint16_t)((hw >> (16 * (b & 1))) & 0xffffu)) * ef[u];
                 const float4 dx = *reinterpret_cast<const float4*>(xu0 + xo[u] + Unit<QT>::kQuant +
@@ -1343,7 +1342,7 @@ constexpr int kExpertMaxWindowBytes = 160 * 1024 - kRankedExperts * 4 - 1024; //
 // (this general kernel requests a panel where it multiplies it and needs about 150 registers: twelve
 // waves, three per SIMD, hide a panel's round trip better than eight)
 constexpr int kExpertWavesGeneral = 12;
-template <int QT, int TC>
+template <int QT, int TC, int NU>
 __global__ __launch_bounds__(64 * kExpertWavesGeneral) void gemv_mfma_expert_kernel(MfmaParams P) {
     constexpr int UB = Unit<QT>::kBytes;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -1425,7 +1424,7 @@ __global__ __launch_bounds__(64 * kExpertWavesGeneral) void gemv_mfma_expert_ker
 #pragma unroll
                 for (int t = 0; t < TC; t++) {
                     if (t < nt) // uniform
-                        panel_dot<QT, false>(p, smem + ((size_t)t * P.k_units + unit0) * UB, n_units, j, grp, acc[t]);
+                        panel_dot<QT, false, QT == QMM_Q4_K ? 0 : NU>(p, smem + ((size_t)t * P.k_units + unit0) * UB, n_units, j, grp, acc[t]);
                 }
             }
             const int row = rt * 16 + j;
@@ -1615,14 +1614,14 @@ hipError_t launch_expert_q4k(const MfmaParams& P, dim3 grid, int waves, size_t l
     return hipGetLastError();
 }
 
-template <int QT, int TC>
+template <int QT, int TC, int NU = 0>
 hipError_t launch_expert_form(const MfmaParams& P, dim3 grid, int waves, size_t lds, hipStream_t stream) {
     if (lds > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemv_mfma_expert_kernel<QT, TC>),
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemv_mfma_expert_kernel<QT, TC, NU>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, kExpertMaxWindowBytes);
         if (e != hipSuccess) return e;
     }
-    gemv_mfma_expert_kernel<QT, TC><<<grid, 64 * waves, lds, stream>>>(P);
+    gemv_mfma_expert_kernel<QT, TC, NU><<<grid, 64 * waves, lds, stream>>>(P);
     return hipGetLastError();
 }
 
@@ -2086,9 +2085,18 @@ hipError_t qmm_launch_gemv_mfma_grouped(const QmmLayout& L, const void* tiled, c
             if (L.dtype == QMM_Q4_K)
                 return tc == 4 ? launch_expert_form<QMM_Q4_K, 4>(E, grid, waves, lds, stream)
                                : launch_expert_form<QMM_Q4_K, 2>(E, grid, waves, lds, stream);
-            if (L.dtype == QMM_Q6_K)
+            if (L.dtype == QMM_Q6_K) // (straight-line it needs more than the 168 registers)
                 return tc == 4 ? launch_expert_form<QMM_Q6_K, 4>(E, grid, waves, lds, stream)
                                : launch_expert_form<QMM_Q6_K, 2>(E, grid, waves, lds, stream);
+            // Q8_0, straight-line where the panels allow it (per layer of 128 experts, top-8, 2048 x 768, with a
+            // branch per unit / without: 152 / 151 us at 128 tokens, 224 / 206 at 512, 395 / 337 at 1024, 1180 /
+            // 985 at 4096)
+            if (uniform_panel_units(L) == 4)
+                return tc == 4 ? launch_expert_form<QMM_Q8_0, 4, 4>(E, grid, waves, lds, stream)
+                               : launch_expert_form<QMM_Q8_0, 2, 4>(E, grid, waves, lds, stream);
+            if (uniform_panel_units(L) == 3)
+                return tc == 4 ? launch_expert_form<QMM_Q8_0, 4, 3>(E, grid, waves, lds, stream)
+                               : launch_expert_form<QMM_Q8_0, 2, 3>(E, grid, waves, lds, stream);
             return tc == 4 ? launch_expert_form<QMM_Q8_0, 4>(E, grid, waves, lds, stream)
                            : launch_expert_form<QMM_Q8_0, 2>(E, grid, waves, lds, stream);
         }
