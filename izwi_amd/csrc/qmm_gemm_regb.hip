@@ -405,8 +405,15 @@ __global__ __launch_bounds__(256) void regb_reduce_kernel(RegbReduceParams P) {
     if (i + 4 <= count && (count & 3) == 0) {
         f32x4 sum = *reinterpret_cast<const f32x4*>(partial);
         for (int s = 1; s < P.slices; s++) sum += *reinterpret_cast<const f32x4*>(partial + s * count);
+        if (ep.residual) // (all of it before the stores: it may be the output buffer)
+            sum += ep.y_bf16 ? f32x4{qmm_bf16_bits_to_f32(static_cast<const uint16_t*>(ep.residual)[i]),
+                                     qmm_bf16_bits_to_f32(static_cast<const uint16_t*>(ep.residual)[i + 1]),
+                                     qmm_bf16_bits_to_f32(static_cast<const uint16_t*>(ep.residual)[i + 2]),
+                                     qmm_bf16_bits_to_f32(static_cast<const uint16_t*>(ep.residual)[i + 3])}
+                             : f32x4{static_cast<const float*>(ep.residual)[i], static_cast<const float*>(ep.residual)[i + 1],
+                                     static_cast<const float*>(ep.residual)[i + 2], static_cast<const float*>(ep.residual)[i + 3]};
 #pragma unroll
-        for (int e = 0; e < 4; e++) qmm_store(P.y[member], ep, i + e, sum[e]);
+        for (int e = 0; e < 4; e++) qmm_store(P.y[member], QmmEpilogue{nullptr, ep.y_bf16}, i + e, sum[e]);
     } else {
         for (int e = 0; e < 4 && i + e < count; e++) {
             float sum = partial[e];
@@ -429,17 +436,20 @@ RegbPlan plan_regb(const QmmLayout* const* layouts, int n_weights, int64_t m, in
     int64_t tiles = 0, n_total = 0;
     for (int i = 0; i < n_weights; i++) n_total += layouts[i]->n, tiles += (layouts[i]->n + kBN - 1) / (kBN);
     tiles *= tiles_m;
-    // microseconds, fitted to the 8B and 0.6B shapes at 65 to 512 rows: a round of workgroups costs 6.5 plus
-    // its units, the more the fuller the chip; the slices' sums cost a launch and their bytes twice
-    const double row_cost = (0.45 + 0.55 * p.mt / 4.0);
+    // microseconds, fitted to every split of the 8B and 0.6B shapes at 80 to 2048 rows: a round of workgroups costs
+    // 4.2 plus its units, the more the fuller the chip; the slices' sums cost a launch and their bytes twice; one
+    // product alone, not split, stores its outputs (as bf16, with a residual read in front of each store) 6 later.
+    // (Without that 1024 x 2048 at 1024 to 2048 rows was not split: 31 to 33 us, in two slices 22 to 26, on the
+    // 256-row tiles 26 to 31.  Up to four units neither a group nor a product alone is split, so that their sums are the same.)
+    const double row_cost = (0.28 + 0.72 * p.mt / 4.0), unsplit_cost = n_weights == 1 && k_units > 4 ? 6.0 : 0.0;
     double best = 1e30;
     p.slices = 1;
     for (int s = 1; s <= 8 && s <= k_units; s++) {
         const int su = (k_units + s - 1) / s;
         if ((k_units + su - 1) / su != s) continue;
         const double rounds = (double)((tiles * s + n_cus - 1) / n_cus);
-        const double unit = (1.6 + 0.5 * std::min(1.0, (double)(tiles * s) / n_cus)) * row_cost;
-        const double cost = rounds * (6.5 + su * unit) + (s > 1 ? 4.0 + s * (double)m * (double)n_total * 4.0 / 2.5e6 : 0.0);
+        const double unit = (1.6 + 0.4 * std::min(1.0, (double)(tiles * s) / n_cus)) * row_cost;
+        const double cost = rounds * (4.2 + su * unit) + (s > 1 ? 4.2 + s * (double)m * (double)n_total * 4.0 / 2.2e6 : unsplit_cost);
         if (cost < 0.98 * best) best = cost, p.slices = s;
     }
     p.cost = best;
