@@ -477,21 +477,43 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
 
     // a split-k slice stores f32 into its own [m, n] plane of the workspace
     float* out_f32 = P.partial ? P.partial + (int64_t)blockIdx.y * P.m * P.n : reinterpret_cast<float*>(P.y);
+    auto each = [&](auto B, auto&& f) { // the lane's elements of 32 x 32 block B: register, index
+        constexpr int i = decltype(B)::value / NT, j = decltype(B)::value % NT;
+        const int64_t gn = n0 + wn * (BN / 2) + j * 32 + (lane & 31);
+        if (gn >= P.n_end) return;
 #pragma unroll
-    for (int i = 0; i < MT; i++) {
-#pragma unroll
-        for (int j = 0; j < NT; j++) {
-            const int64_t gn = n0 + wn * (BN / 2) + j * 32 + (lane & 31);
-            if (gn >= P.n_end) continue;
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int64_t gm = m0 + wm * (BM / WM) + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (gm >= P.m) continue;
-                if (P.partial) out_f32[gm * P.n + gn] = acc[i][j][r]; // a slice: the second kernel finishes
-                else qmm_store(P.y, QmmEpilogue{P.residual, P.out_bf16}, gm * P.n + gn, acc[i][j][r]);
-            }
+        for (int r = 0; r < 16; r++) {
+            const int64_t gm = m0 + wm * (BM / WM) + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+            if (gm < P.m) f(r, gm * P.n + gn);
         }
+    };
+    if (P.partial || !P.residual) { // uniform; a slice: the second kernel finishes
+        const bool f32 = P.partial || !P.out_bf16;
+        static_for<MT * NT>([&](auto B) {
+            constexpr int i = decltype(B)::value / NT, j = decltype(B)::value % NT;
+            each(B, [&](int r, int64_t at) {
+                if (f32) out_f32[at] = acc[i][j][r];
+                else qmm_store(P.y, QmmEpilogue{nullptr, 1}, at, acc[i][j][r]);
+            });
+        });
+        return;
     }
+    // The residual a block ahead of the stores: it may be the output buffer, so behind a store the compiler would keep
+    // every load, a chain of 16 MT NT round trips.  (The lane reads the elements that it writes.)
+    float res[2][16];
+    auto fetch = [&](auto B) {
+        constexpr int to = decltype(B)::value & 1;
+        each(B, [&](int r, int64_t at) {
+            res[to][r] = P.out_bf16 ? qmm_bf16_bits_to_f32(static_cast<const uint16_t*>(P.residual)[at])
+                                    : static_cast<const float*>(P.residual)[at];
+        });
+    };
+    fetch(std::integral_constant<int, 0>{});
+    static_for<MT * NT>([&](auto B) {
+        constexpr int b = decltype(B)::value;
+        if constexpr (b + 1 < MT * NT) fetch(std::integral_constant<int, b + 1>{});
+        each(B, [&](int r, int64_t at) { qmm_store(P.y, QmmEpilogue{nullptr, P.out_bf16}, at, acc[b / NT][b % NT][r] + res[b & 1][r]); });
+    });
 }
 
 // out[i] = sum over slices (in order) of partial[s][i], as f32 or bf16; i runs over the
