@@ -1139,6 +1139,19 @@ namespace {
 int batched_group_on_records(const izwi_qmm_weight* const* weights, int32_t n_weights, const float* x, int64_t m,
                              float* const* ys, void* records, hipStream_t stream);
 
+// A caller's bf16 rows need not start on 16 bytes (a view into a larger buffer); the prefill kernels move them
+// into LDS in 16-byte pieces that do.  Bytes of scratch for an aligned copy, 0 where the rows are aligned as they
+// are (k is a multiple of 32, so the first row decides for all).
+size_t aligned_rows_bytes(const void* x, int64_t m, int64_t k) {
+    return (uintptr_t)x % 16 == 0 ? 0 : ((size_t)m * (size_t)k * sizeof(uint16_t) + 255) & ~(size_t)255;
+}
+// x itself, or its copy at `copy` (aligned_rows_bytes of it)
+hipError_t aligned_rows(const void* x, int64_t m, int64_t k, void* copy, const uint16_t** rows, hipStream_t stream) {
+    const bool as_it_is = aligned_rows_bytes(x, m, k) == 0;
+    *rows = static_cast<const uint16_t*>(as_it_is ? x : copy);
+    return as_it_is ? hipSuccess : hipMemcpyAsync(copy, x, (size_t)m * (size_t)k * sizeof(uint16_t), hipMemcpyDefault, stream);
+}
+
 // The members of a group on bf16 activations, one launch per block type (types in the order of their
 // first members); the launches follow each other on the stream and share the workspace.
 template <class F>
@@ -1672,11 +1685,14 @@ int izwi_qmm_forward_bf16(const izwi_qmm_weight* w, const uint16_t* x_bf16, int6
     Staged xi, yo;
     HIP_TRY(xi.in(x_bf16, (size_t)m * L.k * sizeof(uint16_t), mem_space, stream));
     HIP_TRY(yo.out(y, ybytes, mem_space, stream));
-    void* workspace = nullptr; // split-k partial tiles, for products with few output tiles only
-    if (const size_t ws_bytes = qmm_gemm_workspace_bytes(L, m, w->n_cus))
-        HIP_TRY(get_scratch(w->device, stream, ws_bytes, &workspace));
-    HIP_TRY(qmm_launch_gemm_bf16(L, w->tiled, (const uint16_t*)xi.dev, m, yo.dev,
-                                 out_dtype == IZWI_QMM_OUT_BF16, workspace, w->n_cus, stream));
+    // scratch: aligned copy of x | split-k partial tiles, each where there is need of it
+    const size_t xb_bytes = aligned_rows_bytes(xi.dev, m, L.k), ws_bytes = qmm_gemm_workspace_bytes(L, m, w->n_cus);
+    void* scratch = nullptr;
+    if (xb_bytes + ws_bytes) HIP_TRY(get_scratch(w->device, stream, xb_bytes + ws_bytes, &scratch));
+    const uint16_t* xb = nullptr;
+    HIP_TRY(aligned_rows(xi.dev, m, L.k, scratch, &xb, stream));
+    HIP_TRY(qmm_launch_gemm_bf16(L, w->tiled, xb, m, yo.dev, out_dtype == IZWI_QMM_OUT_BF16,
+                                 ws_bytes ? static_cast<uint8_t*>(scratch) + xb_bytes : nullptr, w->n_cus, stream));
     HIP_TRY(yo.finish(stream));
     return IZWI_QMM_OK;
     });
@@ -1709,11 +1725,14 @@ int izwi_qmm_forward_group_bf16(const izwi_qmm_weight* const* weights, int32_t n
     if (mem_space == IZWI_QMM_DEVICE && splittable && n_weights >= 2) {
         hipStream_t stream = (hipStream_t)stream_;
         const izwi_qmm_weight* w0 = weights[0];
-        void* workspace = nullptr;
-        if (const size_t ws_bytes = group_bf16_workspace(weights, n_weights, m))
-            HIP_TRY(get_scratch(w0->device, stream, ws_bytes, &workspace));
+        const size_t xb_bytes = aligned_rows_bytes(x_bf16, m, w0->layout.k), ws_bytes = group_bf16_workspace(weights, n_weights, m);
+        void* scratch = nullptr;
+        if (xb_bytes + ws_bytes) HIP_TRY(get_scratch(w0->device, stream, xb_bytes + ws_bytes, &scratch));
         ProfileScope prof(w0, stream);
-        HIP_TRY(group_bf16_launch(weights, n_weights, x_bf16, m, ys, out_dtype == IZWI_QMM_OUT_BF16, workspace, stream));
+        const uint16_t* xb = nullptr;
+        HIP_TRY(aligned_rows(x_bf16, m, w0->layout.k, scratch, &xb, stream));
+        HIP_TRY(group_bf16_launch(weights, n_weights, xb, m, ys, out_dtype == IZWI_QMM_OUT_BF16,
+                                  ws_bytes ? static_cast<uint8_t*>(scratch) + xb_bytes : nullptr, stream));
         return IZWI_QMM_OK;
     }
     for (int i = 0; i < n_weights; i++)
@@ -1791,15 +1810,13 @@ int izwi_qmm_forward_fused(const izwi_qmm_weight* w, const void* x, int x_dtype,
             if (e != hipSuccess) return fail_hip(e, "batched decode kernel");
         }
     } else {
-        const size_t xb_bytes = x_bf16 ? 0 : ((((size_t)m * L.k * sizeof(uint16_t)) + 255) & ~(size_t)255);
+        const size_t xb_bytes = x_bf16 ? aligned_rows_bytes(xi.dev, m, L.k) : ((((size_t)m * L.k * sizeof(uint16_t)) + 255) & ~(size_t)255);
         const size_t ws_bytes = qmm_gemm_workspace_bytes(L, m, w->n_cus);
         void* scratch = nullptr;
         if (xb_bytes + ws_bytes) HIP_TRY(get_scratch(w->device, stream, xb_bytes + ws_bytes, &scratch));
-        const uint16_t* xb = (const uint16_t*)xi.dev;
-        if (!x_bf16) {
-            HIP_TRY(qmm_launch_f32_to_bf16((const float*)xi.dev, (uint16_t*)scratch, m * L.k, stream));
-            xb = (const uint16_t*)scratch;
-        }
+        const uint16_t* xb = (const uint16_t*)scratch;
+        if (x_bf16) HIP_TRY(aligned_rows(xi.dev, m, L.k, scratch, &xb, stream));
+        else HIP_TRY(qmm_launch_f32_to_bf16((const float*)xi.dev, (uint16_t*)scratch, m * L.k, stream));
         HIP_TRY(qmm_launch_gemm_bf16(L, w->tiled, xb, m, yo.dev, io.y_bf16,
                                      ws_bytes ? static_cast<uint8_t*>(scratch) + xb_bytes : nullptr, w->n_cus, stream,
                                      io.residual));

@@ -94,3 +94,20 @@ def test_mlp_of_a_small_model_at_prefill_rows(qa, oracle, dtype, m):
     y = qa.Qwen3Mlp(gate_up, down).forward(x)
     assert torch.equal(y, down.forward(got))
     assert off(y, got.to(torch.bfloat16).double() @ dense(down).t()) < F32_TOL
+
+
+@pytest.mark.parametrize("dtype,m,n,k", [(Q4_K, 1, 64, 256), (Q4_K, 65, 200, 768), (Q8_0, 100, 130, 288), (Q6_K, 140, 96, 512), (Q4_K, 300, 300, 256)])
+@pytest.mark.parametrize("skip", [1, 2, 5])  # values in front of the rows: they start on 2, 4 and 10 bytes
+def test_rows_that_do_not_start_on_sixteen_bytes(qa, oracle, dtype, m, n, k, skip):
+    parts = [weight(qa, oracle, dtype, n, k, 600 + i) for i in range(2)]
+    x = torch.from_numpy(oracle.randn(601 + m, (m, k))).cuda().to(torch.bfloat16)
+    rows = torch.empty(skip + m * k, dtype=torch.bfloat16, device="cuda")[skip:].view(m, k)
+    rows.copy_(x)
+    assert rows.data_ptr() % 16
+    assert torch.equal(parts[0].forward(rows), parts[0].forward(x))
+    assert torch.equal(parts[0].forward_bf16_to_f32(rows), parts[0].forward_bf16_to_f32(x))
+    if m > 64:
+        res = torch.from_numpy(oracle.randn(602, (m, n))).cuda().to(torch.bfloat16)
+        assert torch.equal(parts[0].forward_fused(rows, residual=res), parts[0].forward_fused(x, residual=res))
+        for a, b in zip(qa.forward_group(parts, rows), qa.forward_group(parts, x)):
+            assert torch.equal(a, b)
