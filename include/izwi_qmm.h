@@ -356,7 +356,7 @@ int izwi_qmm_forward_f32_noalloc(const izwi_qmm_weight* w, const float* x, int64
  * izwi_qmm_forward_f32 up to 128 rows (beyond, in the bf16 matrix-core arithmetic, equal up to the
  * f32 summation order: the shared launch may split k differently).  The weights must share k; with equal block types the decode
  * sizes run as one kernel launch (m <= 2; m <= 4 where k <= 3072) or as one activation quantization and one
- * matmul launch (m <= 64), prefill sizes (m > 128, bf16 matrix-core arithmetic) share one conversion of x
+ * matmul launch (m <= 64), prefill sizes (m > 64, bf16 matrix-core arithmetic) share one conversion of x
  * and one launch; members of several block types (attn_q / attn_k in Q4_K beside attn_v in
  * Q6_K, as Q4_K_M files have them) are grouped by type, one such launch per type.
  * n_weights <= 4. */
@@ -365,11 +365,11 @@ int izwi_qmm_forward_group_f32(const izwi_qmm_weight* const* weights, int32_t n_
                                void* stream);
 
 /* izwi_qmm_forward_group_f32 for bf16 activations (prefill): y_i = izwi_qmm_forward_bf16(weights[i], x)
- * for 1..4 weights of equal k on the same x, `out_dtype` f32 or bf16 for every y_i.  With equal block
- * types, device pointers and m > 128 the members run as ONE launch of the bf16 matrix-core kernel
- * (its grid is the members' column tiles one after the other, planned as one matrix): k / v
- * (n = 1024) no longer run alone on a quarter of the chip.  Results are those of the separate calls
- * up to f32 summation order (the tile plan may split k differently). */
+ * for 1..4 weights of equal k on the same x, `out_dtype` f32 or bf16 for every y_i.  With device
+ * pointers the members of a block type run as ONE launch of the bf16 matrix-core kernel
+ * (its grid is the members' column tiles one after the other): k / v (n = 1024) do not run
+ * alone on a quarter of the chip.  Results are those of the separate calls, bit for bit up to 128 rows and
+ * up to f32 summation order beyond (the launch is planned as one matrix there and may split k differently). */
 int izwi_qmm_forward_group_bf16(const izwi_qmm_weight* const* weights, int32_t n_weights, const uint16_t* x_bf16,
                                 int64_t m, void* const* ys, int out_dtype, int mem_space, void* stream);
 
@@ -377,7 +377,8 @@ int izwi_qmm_forward_group_bf16(const izwi_qmm_weight* const* weights, int32_t n
  *     h[m, n] = silu(gate.forward(x)) * up.forward(x)
  * i.e. `gate_up_proj.forward(x)` followed by `try_fused_silu_mul` (kernels/mod.rs:94-108) or
  * `ops::silu(&gate)?.broadcast_mul(&up)` in one call.  `gate` and `up` are [n, k] weights of the
- * same shape and type.  The two sums are those of izwi_qmm_forward_f32 bit for bit; silu(v) =
+ * same shape and type.  The two sums are those of izwi_qmm_forward_group_f32 on the pair (up to
+ * 128 rows those of izwi_qmm_forward_f32 bit for bit, beyond up to the f32 summation order); silu(v) =
  * v / (1 + exp(-v)) in f32.  For m <= 2 the product is applied inside the decode kernel (one
  * launch, h is the only output written); for larger m the two projections run as a projection
  * group into scratch and one elementwise kernel follows.  Counted in

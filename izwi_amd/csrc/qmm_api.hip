@@ -1305,7 +1305,8 @@ int forward_group_impl(const izwi_qmm_weight* const* weights, int32_t n_weights,
         HIP_TRY(group_bf16_launch(weights, n_weights, (const uint16_t*)xb, m, outs, 0, xb + xb_bytes, stream));
         return IZWI_QMM_OK;
     }
-    // host buffers, mixed types, prefill sizes: one call per projection (same results)
+    // host buffers, weights on several devices, the integer arithmetic beyond 64 rows: one call per projection (the
+    // same results, beyond 128 rows of the bf16 arithmetic up to the order of the f32 sums)
     if (mem_space != IZWI_QMM_DEVICE || !uniform || n_weights == 1 || m > 64) {
         for (int i = 0; i < n_weights; i++)
             if (int rc = izwi_qmm_forward_f32(weights[i], x, m, ys[i], mem_space, stream_)) return rc;

@@ -8,17 +8,17 @@
 // which is what a lane supplies to v_mfma_f32_32x32x16_bf16: the chunk is unpacked into B operands
 // in registers, in the k order the chunk has, and the A operand (activations, staged in LDS by
 // LDS-direct loads, two stages of one unit) is picked in the same order.  No weight tile in LDS, no
-// LDS writes, one barrier per unit.  The two halves' sums meet in LDS at the end; k is split over
-// workgroups where the tiles alone leave compute units idle.
+// LDS writes, one barrier per unit.  The two halves' sums meet in LDS at the end.  Where the tiles
+// alone leave compute units idle, k is split over workgroups and the row tiles get lower.
 //
 // Bound by the vector instructions that unpack (7.3 per matrix instruction) beside the matrix
-// instructions (half of the time of a full chip): 2.0 us per unit of 128 rows, and 6.5 to 8 us per
-// workgroup that are no unit (start, first loads, exchange of the sums, stores).  Splitting a unit
-// four ways over the waves (64 x 128 wave tiles, fewer LDS reads) cost 14 us per workgroup instead:
-// the exchange of the sums is 512 KB of LDS traffic there, 128 KB here.  Q4_K, us per call in a
-// graph, before (128 x 256 / 64 x 128 tiles with the weights through LDS, one call per weight) and
-// now: 101 rows: q|k|v 73 -> 23, 4096 x 4096 25.4 -> 21.4, gate|up 76 -> 39, down 42 -> 27; Q6_K
-// down 176 -> 28; 512 rows: q|k|v 51 -> 39, 4096 x 4096 35.5 -> 32.6; 0.6B shapes at 512: 25 -> 14.
+// instructions (half of the time of a full chip): a unit takes 1.1 us at 32 rows, 1.25 at 64, 1.6 at
+// 96, 1.8 to 2.3 at 128, and 6.5 to 8 us per workgroup are no unit (start, first loads, exchange of the
+// sums, stores).  Splitting a unit four ways over the waves (64 x 128 wave tiles, fewer LDS reads) cost
+// 14 us per workgroup instead: the exchange of the sums is 512 KB of LDS traffic there, 128 KB here.  us per
+// call on f32 rows in a graph, one call per weight on 128 x 256 / 64 x 128 tiles with the weights through
+// LDS / here.  Q4_K, 101 rows: q|k|v 81 / 27, 4096 x 4096 28 / 19, gate|up 82 / 47, down 47 / 32; Q6_K down
+// 201 / 35; 512 rows: q|k|v 54 / 45; 0.6B shapes at 512: q|k|v 27 / 15.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -73,15 +73,15 @@ __device__ __forceinline__ bf16x8 scaled_bytes(uint32_t lo, uint32_t hi, float s
 struct RegbParams {
     const uint16_t* x; // bf16 [m, k], k a multiple of 32
     int64_t m, k;
-    int k_units, slice_units, slices;
+    int k_units;
     int s, slots;
     int64_t panel_bytes, row_bytes; // row_bytes: all panels of a row tile
-    int tiles_m, cols;              // cols: the members' column tiles times slices
+    int tiles_m, cols;              // cols: the members' column tiles times their slices
     uint32_t nibble_mask;           // 0x0f0f0f0f as data: one AND per four weights, v_cvt_f32_ubyteN for each
     int out_bf16;
     const void* residual; // single weight only
-    int n_weights;
-    int tn_end[QMM_MAX_GROUP];
+    int col_end[QMM_MAX_GROUP]; // one past each member's last (unused entries: past every column)
+    int slices_v[QMM_MAX_GROUP], slice_units_v[QMM_MAX_GROUP];
     const uint8_t* wv[QMM_MAX_GROUP];
     void* yv[QMM_MAX_GROUP];
     float* partial_v[QMM_MAX_GROUP]; // [slice][m][n] where k is split
@@ -189,13 +189,22 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
     const int tm = pos % P.tiles_m;
     const int col = (pos / P.tiles_m) * 8 + xcd;
     if (col >= P.cols) return; // uniform
-    const int slice = col % P.slices;
-    int tn = col / P.slices, member = 0;
-    while (member + 1 < P.n_weights && tn >= P.tn_end[member]) member++;
-    tn -= member ? P.tn_end[member - 1] : 0;
-    const int64_t n = P.nv[member];
+    // this workgroup's member, by selects: every table entry is loaded at once, none waits for another
+    int slices = P.slices_v[0], slice_units = P.slice_units_v[0], first_col = 0;
+    int64_t n = P.nv[0], row_tiles = P.row_tiles_v[0];
+    const uint8_t* weights = P.wv[0];
+    void* y = P.yv[0];
+    float* partial = P.partial_v[0];
+#pragma unroll
+    for (int i = 1; i < QMM_MAX_GROUP; i++)
+        if (col >= P.col_end[i - 1]) {
+            slices = P.slices_v[i], slice_units = P.slice_units_v[i], first_col = P.col_end[i - 1];
+            n = P.nv[i], row_tiles = P.row_tiles_v[i];
+            weights = P.wv[i], y = P.yv[i], partial = P.partial_v[i];
+        }
+    const int tn = (col - first_col) / slices, slice = col - first_col - tn * slices;
     const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * kBN;
-    const int u0 = slice * P.slice_units, u1 = min(P.k_units, u0 + P.slice_units);
+    const int u0 = slice * slice_units, u1 = min(P.k_units, u0 + slice_units);
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -233,11 +242,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
 
     // ---- weights: uniform unit address + 32-bit offsets
     const int64_t rt0 = n0 >> 4;
-    const uint8_t* w_tile = P.wv[member] + rt0 * P.row_bytes;
+    const uint8_t* w_tile = weights + rt0 * P.row_bytes;
     HalfOffsets off;
     {
         const int row = wc * 32 + (lane & 31);
-        const int64_t rt = min(rt0 + (row >> 4), P.row_tiles_v[member] - 1);
+        const int64_t rt = min(rt0 + (row >> 4), row_tiles - 1);
         const uint32_t base = (uint32_t)((rt - rt0) * P.row_bytes) + (row & 15) * 16, chunk = (uint32_t)P.slots * 16;
         off.hdr = base + (QT == QMM_Q4_K ? 0 : 8 * half);
         off.q = base + (1 + (QT == QMM_Q8_0 ? 8 : 4) * half + h) * chunk;
@@ -355,14 +364,14 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
         if (half) take(std::integral_constant<int, 1>{});
         else take(std::integral_constant<int, 0>{});
     }
-    const bool split = P.slices > 1;
+    const bool split = slices > 1;
     const int64_t gn = n0 + wc * 32 + (lane & 31);
     const int64_t gm0 = m0 + half * 32 + 4 * h;
     const int rows = gn < n ? (int)min((int64_t)BM, P.m - gm0) : 0; // of this lane's column, from gm0 on
     auto emit = [&](auto MODE) { // 0: f32, 1: f32 + residual, 2: bf16, 3: bf16 + residual
         constexpr int mode = decltype(MODE)::value;
-        float* yf = (split ? P.partial_v[member] + (int64_t)slice * P.m * n : static_cast<float*>(P.yv[member])) + gm0 * n + gn;
-        uint16_t* yb = static_cast<uint16_t*>(P.yv[member]) + gm0 * n + gn;
+        float* yf = (split ? partial + (int64_t)slice * P.m * n : static_cast<float*>(y)) + gm0 * n + gn;
+        uint16_t* yb = static_cast<uint16_t*>(y) + gm0 * n + gn;
         const float* rf = static_cast<const float*>(P.residual) + gm0 * n + gn;
         const uint16_t* rb = static_cast<const uint16_t*>(P.residual) + gm0 * n + gn;
         static_for<kOwn>([&](auto I) {
@@ -386,25 +395,30 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
 }
 
 // y = sum over slices (in order) of partial[slice] (+ residual), four consecutive values per thread, all
-// members of a group in one launch (blocks of member i: block_end[i - 1] .. block_end[i])
+// split members of a group in one launch (blocks of member i: block_end[i - 1] .. block_end[i])
 struct RegbReduceParams {
     const float* partial[QMM_MAX_GROUP];
     void* y[QMM_MAX_GROUP];
     int64_t count[QMM_MAX_GROUP];
-    int block_end[QMM_MAX_GROUP];
-    int n_weights, slices, out_bf16;
+    int block_end[QMM_MAX_GROUP], slices[QMM_MAX_GROUP];
+    int out_bf16;
     const void* residual;
 };
 __global__ __launch_bounds__(256) void regb_reduce_kernel(RegbReduceParams P) {
-    int member = 0;
-    while (member + 1 < P.n_weights && (int)blockIdx.x >= P.block_end[member]) member++;
-    const int64_t count = P.count[member];
-    const int64_t i = ((int64_t)(blockIdx.x - (member ? P.block_end[member - 1] : 0)) * 256 + threadIdx.x) * 4;
-    const float* partial = P.partial[member] + i;
+    int slices = P.slices[0], first_block = 0;
+    int64_t count = P.count[0];
+    const float* partial = P.partial[0];
+    void* y = P.y[0];
+#pragma unroll
+    for (int i = 1; i < QMM_MAX_GROUP; i++)
+        if ((int)blockIdx.x >= P.block_end[i - 1])
+            slices = P.slices[i], first_block = P.block_end[i - 1], count = P.count[i], partial = P.partial[i], y = P.y[i];
+    const int64_t i = ((int64_t)(blockIdx.x - first_block) * 256 + threadIdx.x) * 4;
+    partial += i;
     const QmmEpilogue ep{P.residual, P.out_bf16};
     if (i + 4 <= count && (count & 3) == 0) {
         f32x4 sum = *reinterpret_cast<const f32x4*>(partial);
-        for (int s = 1; s < P.slices; s++) sum += *reinterpret_cast<const f32x4*>(partial + s * count);
+        for (int s = 1; s < slices; s++) sum += *reinterpret_cast<const f32x4*>(partial + s * count);
         if (ep.residual) // (all of it before the stores: it may be the output buffer)
             sum += ep.y_bf16 ? f32x4{qmm_bf16_bits_to_f32(static_cast<const uint16_t*>(ep.residual)[i]),
                                      qmm_bf16_bits_to_f32(static_cast<const uint16_t*>(ep.residual)[i + 1]),
@@ -413,49 +427,75 @@ __global__ __launch_bounds__(256) void regb_reduce_kernel(RegbReduceParams P) {
                              : f32x4{static_cast<const float*>(ep.residual)[i], static_cast<const float*>(ep.residual)[i + 1],
                                      static_cast<const float*>(ep.residual)[i + 2], static_cast<const float*>(ep.residual)[i + 3]};
 #pragma unroll
-        for (int e = 0; e < 4; e++) qmm_store(P.y[member], QmmEpilogue{nullptr, ep.y_bf16}, i + e, sum[e]);
+        for (int e = 0; e < 4; e++) qmm_store(y, QmmEpilogue{nullptr, ep.y_bf16}, i + e, sum[e]);
     } else {
         for (int e = 0; e < 4 && i + e < count; e++) {
             float sum = partial[e];
-            for (int s = 1; s < P.slices; s++) sum += partial[s * count + e];
-            qmm_store(P.y[member], ep, i + e, sum);
+            for (int s = 1; s < slices; s++) sum += partial[s * count + e];
+            qmm_store(y, ep, i + e, sum);
         }
     }
 }
 
 struct RegbPlan {
-    int mt, slices, slice_units;
-    double cost;
+    int mt, slices[QMM_MAX_GROUP], slice_units[QMM_MAX_GROUP];
 };
 
+// Slices of k for n columns in `tiles` full-height tiles, in microseconds: a unit costs 1.2 where the row tiles are as
+// low as the compute units allow; the slices' sums a launch (4.2) and their bytes twice.
+int slices_of(int64_t tiles, int64_t n, int64_t m, int k_units, int64_t limit, int min_units, double unsplit_cost) {
+    double best = 1.2 * k_units + unsplit_cost;
+    int slices = 1;
+    for (int s = 2; s <= 8 && tiles * s <= limit; s++) {
+        const int su = (k_units + s - 1) / s;
+        if (su < min_units || (k_units + su - 1) / su != s) continue;
+        const double cost = 1.2 * su + 4.2 + s * (double)m * (double)n * 4.0 / 2.2e6;
+        if (cost < 0.98 * best) best = cost, slices = s;
+    }
+    return slices;
+}
+
+// Up to 128 rows a matrix is split by its own shape and m, whatever group it is in, so that a group's sums are
+// those of its members' separate calls bit for bit.  The split that is best for a wide matrix alone fills the chip once and
+// is a second round in a group (gate|up of 2 x 12288 at k = 4096, 101 rows: 47 us in one slice, 61 in two; one of the
+// two alone 41 and 34): so a split stops at half of the compute units (two such members fill the chip) and at four units
+// per slice.  What that leaves idle the row tiles take: their height is no matter of the sums, so it is chosen for the
+// launch as a whole, the lowest whose workgroups still run in one round (of each XCD, which holds whole
+// column tiles): the 12288 alone 31 us in 64-row tiles, 2 x 6144 at k = 2048 24.6 -> 19.4, 2 x 3072 at k = 1024
+// 16.1 -> 12.2, 1024 x 2048 15.2 -> 12.1.  (It costs a wide matrix alone at 65 to 96 rows, of which the second
+// 64-row tile is half empty: 12288 x 4096 at 65, Q4_K 29.2 -> 31.4, Q8_0 32.7 -> 36.3.)  Matrices more
+// than twice as long as wide (the MLP's last) and up to 64 rows, where groups run the integer arithmetic, come
+// alone: they are split over the whole chip.
+// Beyond 128 rows a group is planned as one matrix (4096 -> 4096 + 1024 + 1024 at 512 rows: 45 us, member by member 52).
 RegbPlan plan_regb(const QmmLayout* const* layouts, int n_weights, int64_t m, int n_cus) {
     RegbPlan p;
-    const int64_t tiles_m = (m + 127) / 128;
-    p.mt = (int)((m + 32 * tiles_m - 1) / (32 * tiles_m));
-    const int k_units = (int)layouts[0]->k_units;
-    int64_t tiles = 0, n_total = 0;
-    for (int i = 0; i < n_weights; i++) n_total += layouts[i]->n, tiles += (layouts[i]->n + kBN - 1) / (kBN);
-    tiles *= tiles_m;
-    // microseconds, fitted to every split of the 8B and 0.6B shapes at 80 to 2048 rows: a round of workgroups costs
-    // 4.2 plus its units, the more the fuller the chip; the slices' sums cost a launch and their bytes twice; one
-    // product alone, not split, stores its outputs (as bf16, with a residual read in front of each store) 6 later.
-    // (Without that 1024 x 2048 at 1024 to 2048 rows was not split: 31 to 33 us, in two slices 22 to 26, on the
-    // 256-row tiles 26 to 31.  Up to four units neither a group nor a product alone is split, so that their sums are the same.)
-    const double row_cost = (0.28 + 0.72 * p.mt / 4.0), unsplit_cost = n_weights == 1 && k_units > 4 ? 6.0 : 0.0;
-    double best = 1e30;
-    p.slices = 1;
-    for (int s = 1; s <= 8 && s <= k_units; s++) {
-        const int su = (k_units + s - 1) / s;
-        if ((k_units + su - 1) / su != s) continue;
-        const double rounds = (double)((tiles * s + n_cus - 1) / n_cus);
-        const double unit = (1.6 + 0.4 * std::min(1.0, (double)(tiles * s) / n_cus)) * row_cost;
-        const double cost = rounds * (4.2 + su * unit) + (s > 1 ? 4.2 + s * (double)m * (double)n_total * 4.0 / 2.2e6 : unsplit_cost);
-        if (cost < 0.98 * best) best = cost, p.slices = s;
+    const int k_units = (int)layouts[0]->k_units, min_units = m <= 32 ? 2 : std::clamp(k_units / 4, 2, 4);
+    const int64_t full_tiles = (m + 127) / 128;
+    int64_t tiles[QMM_MAX_GROUP] = {}, all_tiles = 0, n_total = 0, cols = 0;
+    for (int i = 0; i < n_weights; i++) {
+        tiles[i] = (layouts[i]->n + kBN - 1) / kBN * full_tiles;
+        all_tiles += tiles[i], n_total += layouts[i]->n;
     }
-    p.cost = best;
-    p.slice_units = (k_units + p.slices - 1) / p.slices;
-    p.slices = (k_units + p.slice_units - 1) / p.slice_units;
+    for (int i = 0; i < QMM_MAX_GROUP; i++) {
+        p.slices[i] = 1, p.slice_units[i] = k_units;
+        if (i >= n_weights) continue;
+        const bool alone = m <= 64 || layouts[i]->k > 2 * layouts[i]->n;
+        // (one product may carry a residual, whose reads in front of the stores cost about 2 us where k is not split)
+        p.slices[i] = m <= 128 ? slices_of(tiles[i], layouts[i]->n, m, k_units, alone ? n_cus : n_cus / 2, min_units, 0.0)
+                               : slices_of(all_tiles, n_total, m, k_units, n_cus, min_units, n_weights == 1 ? 2.0 : 0.0);
+        p.slice_units[i] = (k_units + p.slices[i] - 1) / p.slices[i];
+        cols += tiles[i] / full_tiles * p.slices[i];
+    }
+    const int64_t blocks = (m + 31) / 32, cols_xcd = (cols + 7) / 8;
+    p.mt = (int)((blocks + full_tiles - 1) / full_tiles);
+    for (int mt = p.mt - 1; mt >= 1; mt--)
+        if (cols_xcd * ((blocks + mt - 1) / mt) <= n_cus / 8) p.mt = mt;
     return p;
+}
+
+// bytes of member i's partial sums
+size_t partial_bytes(const RegbPlan& p, const QmmLayout& L, int i, int64_t m) {
+    return p.slices[i] <= 1 ? 0 : (((size_t)p.slices[i] * (size_t)m * (size_t)L.n * sizeof(float)) + 255) & ~(size_t)255;
 }
 
 template <int QT, int MT>
@@ -503,9 +543,8 @@ bool qmm_gemm_regb_applies(const QmmLayout* const* layouts, int n_weights, int64
 
 size_t qmm_gemm_regb_workspace_bytes(const QmmLayout* const* layouts, int n_weights, int64_t m, int n_cus) {
     const RegbPlan p = plan_regb(layouts, n_weights, m, n_cus);
-    if (p.slices <= 1) return 0;
     size_t total = 0;
-    for (int i = 0; i < n_weights; i++) total += (((size_t)p.slices * (size_t)m * (size_t)layouts[i]->n * sizeof(float)) + 255) & ~(size_t)255;
+    for (int i = 0; i < n_weights; i++) total += partial_bytes(p, *layouts[i], i, m);
     return total;
 }
 
@@ -515,48 +554,49 @@ hipError_t qmm_launch_gemm_regb(const QmmLayout* const* layouts, const void* con
     if (n_weights < 1 || n_weights > QMM_MAX_GROUP || (residual && n_weights != 1)) return hipErrorInvalidValue;
     const QmmLayout& L0 = *layouts[0];
     const RegbPlan plan = plan_regb(layouts, n_weights, m, n_cus);
-    if (plan.slices > 1 && workspace == nullptr) return hipErrorInvalidValue;
     RegbParams P;
     P.x = x_bf16;
     P.m = m, P.k = L0.k;
-    P.k_units = (int)L0.k_units, P.slice_units = plan.slice_units, P.slices = plan.slices;
+    P.k_units = (int)L0.k_units;
     P.s = L0.s, P.slots = L0.slots;
     P.panel_bytes = L0.panel_bytes, P.row_bytes = L0.k_groups * L0.panel_bytes;
     P.nibble_mask = 0x0f0f0f0fu;
     P.out_bf16 = out_bf16;
-    P.residual = plan.slices > 1 ? nullptr : residual;
-    P.n_weights = n_weights;
+    P.residual = plan.slices[0] > 1 ? nullptr : residual;
     P.tiles_m = (int)((m + 32 * plan.mt - 1) / (32 * plan.mt));
+    RegbReduceParams R;
     uint8_t* next = static_cast<uint8_t*>(workspace);
-    int64_t tn = 0;
+    int64_t cols = 0, blocks = 0;
     for (int i = 0; i < QMM_MAX_GROUP; i++) {
-        P.tn_end[i] = 0, P.wv[i] = nullptr, P.yv[i] = nullptr, P.partial_v[i] = nullptr, P.nv[i] = 0, P.row_tiles_v[i] = 0;
+        P.col_end[i] = 0x7fffffff, P.slices_v[i] = 1, P.slice_units_v[i] = 0, P.wv[i] = nullptr, P.yv[i] = nullptr, P.partial_v[i] = nullptr;
+        P.nv[i] = 0, P.row_tiles_v[i] = 0;
+        R.partial[i] = nullptr, R.y[i] = nullptr, R.count[i] = 0, R.slices[i] = 1, R.block_end[i] = (int)blocks;
         if (i >= n_weights) continue;
         const QmmLayout& L = *layouts[i];
         if (L.dtype != L0.dtype || L.k != L0.k || L.n_stacked != 1 || L.n == 0) return hipErrorInvalidValue;
-        tn += (L.n + kBN - 1) / (kBN);
-        P.tn_end[i] = (int)tn;
+        cols += (L.n + kBN - 1) / kBN * plan.slices[i];
+        if (cols > 0x7ffffff0) return hipErrorInvalidValue;
+        P.col_end[i] = (int)cols;
+        P.slices_v[i] = plan.slices[i], P.slice_units_v[i] = plan.slice_units[i];
         P.wv[i] = static_cast<const uint8_t*>(tiled[i]), P.yv[i] = ys[i];
         P.nv[i] = L.n, P.row_tiles_v[i] = L.row_tiles;
+        if (plan.slices[i] <= 1) continue;
+        if (workspace == nullptr) return hipErrorInvalidValue;
         P.partial_v[i] = reinterpret_cast<float*>(next);
-        if (plan.slices > 1) next += (((size_t)plan.slices * (size_t)m * (size_t)L.n * sizeof(float)) + 255) & ~(size_t)255;
+        next += partial_bytes(plan, L, i, m);
+        R.partial[i] = P.partial_v[i], R.y[i] = ys[i], R.count[i] = m * L.n, R.slices[i] = plan.slices[i];
+        blocks += (R.count[i] + 1023) / 1024;
+        if (blocks > 0x7fffffff) return hipErrorInvalidValue;
+        R.block_end[i] = (int)blocks;
     }
-    const int64_t cols = tn * plan.slices, grid = (cols + 7) / 8 * 8 * P.tiles_m;
+    const int64_t grid = (cols + 7) / 8 * 8 * P.tiles_m;
     if (grid > 0x7fffffff) return hipErrorInvalidValue;
     P.cols = (int)cols;
     hipError_t e = L0.dtype == QMM_Q6_K   ? launch_regb_qt<QMM_Q6_K>(P, plan, grid, stream)
                    : L0.dtype == QMM_Q4_K ? launch_regb_qt<QMM_Q4_K>(P, plan, grid, stream)
                                           : launch_regb_qt<QMM_Q8_0>(P, plan, grid, stream);
-    if (e != hipSuccess || plan.slices <= 1) return e;
-    RegbReduceParams R;
-    int64_t blocks = 0;
-    for (int i = 0; i < QMM_MAX_GROUP; i++) {
-        R.count[i] = i < n_weights ? m * layouts[i]->n : 0;
-        blocks += (R.count[i] + 1023) / 1024;
-        R.partial[i] = P.partial_v[i], R.y[i] = P.yv[i], R.block_end[i] = (int)blocks;
-    }
-    if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-    R.n_weights = n_weights, R.slices = plan.slices, R.out_bf16 = out_bf16, R.residual = residual;
+    if (e != hipSuccess || blocks == 0) return e;
+    R.out_bf16 = out_bf16, R.residual = residual;
     regb_reduce_kernel<<<(unsigned)blocks, 256, 0, stream>>>(R);
     return hipGetLastError();
 }

@@ -361,7 +361,8 @@ def forward_group(projections: Sequence["QMatMul"], x: torch.Tensor, norm_weight
                   eps: float = 1e-6):
     """Several projections on the same activations in one call (the `Separate` arms of
     Qwen3QkvProjection::forward / Qwen3GateUpProjection::forward, qwen3/core.rs:1119-1127,
-    1274-1282).  Returns one output per projection, identical to separate forwards.
+    1274-1282).  Returns one output per projection, identical to separate forwards up to 128 rows and up to
+    the order of the f32 sums beyond.
     With ``norm_weight`` the projections see rms_norm(x, norm_weight, eps) (the layer norm in front of
     them, core.rs:1872), folded into the same launch for one or two rows."""
     assert x.dtype in (torch.float32, torch.bfloat16) and x.is_contiguous()

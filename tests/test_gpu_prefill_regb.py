@@ -68,16 +68,58 @@ def test_product_and_its_epilogues(qa, oracle, dtype, m, n, k):
         assert off(y, want + resb.double()) < BF16_TOL
 
 
+# one member and several of it would be split along k differently if the group were planned as one matrix
 @pytest.mark.parametrize("types,m,ns,k", [
     ((Q4_K, Q4_K, Q4_K), 65, (256, 128, 100), 512), ((Q4_K, Q4_K, Q6_K), 101, (512, 130, 130), 2048),
+    ((Q4_K, Q4_K, Q4_K), 101, (4096, 1024, 1024), 4096), ((Q4_K, Q4_K, Q6_K), 65, (4096, 1024, 1024), 4096),
+    ((Q4_K, Q4_K), 128, (12288, 12288), 4096), ((Q8_0, Q8_0), 70, (6144, 6144), 2048), ((Q4_K, Q4_K), 128, (128, 1024), 1024),
+    ((Q8_0, Q8_0, Q8_0), 96, (1024, 64, 300), 3072), ((Q6_K, Q6_K), 80, (300, 2048), 6144),
     ((Q8_0, Q8_0), 128, (384, 640), 1056), ((Q6_K, Q4_K, Q6_K, Q4_K), 300, (16, 257, 128, 48), 768)])
 def test_groups_equal_their_members(qa, oracle, types, m, ns, k):
+    """Bit for bit up to 128 rows; beyond, where the group is planned as one matrix, up to the order of the f32
+    sums: k / 16 additions of the matrix instruction, each off by at most half of 2^-23 of a partial sum, which is
+    below 1e-5 of the norm for the k here."""
     parts = [weight(qa, oracle, t, n, k, 400 + 7 * i) for i, (t, n) in enumerate(zip(types, ns))]
     x = torch.from_numpy(oracle.randn(401, (m, k))).cuda().to(torch.bfloat16)
     for got_f, got_b, mm in zip(qa.forward_group(parts, x.float()), qa.forward_group(parts, x), parts):
+        alone = mm.forward(x.float())
+        if m <= 128:
+            assert torch.equal(got_f, alone) and torch.equal(got_b, mm.forward(x))
+        assert off(got_f, alone.double()) < 1e-5
         want = x.double() @ dense(mm).t()
         assert off(got_f, want) < F32_TOL
         assert off(got_b, want) < BF16_TOL
+
+
+def test_group_entry_of_few_rows_equals_its_members(qa, oracle):
+    """izwi_qmm_forward_group_bf16 is the bf16 product at any number of rows, a single one included."""
+    import ctypes as C
+    from izwi_amd import capi
+    parts = [weight(qa, oracle, Q4_K, n, 4096, 450 + n) for n in (1024, 200, 4096)]
+    for m in (1, 33, 64):
+        x = torch.from_numpy(oracle.randn(451 + m, (m, 4096))).cuda().to(torch.bfloat16)
+        ys = [torch.empty(m, p.qtensor.dims2()[0], device="cuda", dtype=torch.bfloat16) for p in parts]
+        pointers = C.c_void_p * len(parts)
+        capi.check(capi.lib().izwi_qmm_forward_group_bf16(pointers(*[p.qtensor._h for p in parts]), len(parts), x.data_ptr(), m,
+                                                          pointers(*[y.data_ptr() for y in ys]), capi.OUT_BF16, capi.DEVICE,
+                                                          torch.cuda.current_stream().cuda_stream))
+        for y, p in zip(ys, parts):
+            assert torch.equal(y, p.forward(x))
+
+
+@pytest.mark.parametrize("m", [65, 101, 128])
+def test_gate_up_sums_equal_the_projections(qa, oracle, m):
+    """The two sums under silu(gate) * up are those of the projections alone: with `up` (or `gate`) replaced the
+    other factor is unchanged, so h is silu(g) * u of the separate results in the same f32 operations."""
+    gate, up = (weight(qa, oracle, Q4_K, 3072, 4096, 460 + i) for i in range(2))
+    x = torch.from_numpy(oracle.randn(461 + m, (m, 4096))).cuda()
+    g, u = gate.forward(x), up.forward(x)
+    pair = qa.forward_group((gate, up), x)
+    assert torch.equal(pair[0], g) and torch.equal(pair[1], u)
+    h = qa.Qwen3GateUpProjection.new_separate(gate, up).forward_silu_mul(x)
+    want = g.double() / (1.0 + torch.exp(-g.double())) * u.double()
+    # silu in f32: expf (1 ulp), one addition, one division and one product of 2^-24 each
+    assert bool(((h.double() - want).abs() <= 6 * 2.0 ** -24 * want.abs() + 1e-30).all())
 
 
 @pytest.mark.parametrize("dtype", [Q8_0, Q4_K])
