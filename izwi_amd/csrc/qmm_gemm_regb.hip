@@ -521,12 +521,12 @@ hipError_t launch_regb_qt(const RegbParams& P, const RegbPlan& p, int64_t grid, 
 
 } // namespace
 
-// Up to 128 rows always (it is the only form there), beyond where the 128 x 128 tiles are at most one
-// per compute unit, or at most 96 rows high in two tiles: measured against the 256-row tiles of
-// qmm_gemm.hip (Q4_K, us per call in a graph, here / there): q|k|v 4096 -> 6144 39.0 / 50.9 at 512
-// rows (192 tiles), 71.9 / 64.9 at 768 (288); 4096 x 4096 42.1 / 54.8 at 1024 (256), 93.1 / 80.6 at
-// 2048 (512); gate|up of 2 x 12288 65.9 / 74.8 at 192 (384 tiles of 96 rows), 73.5 / 70.9 at 256
-// (384); gate|up of 2 x 3072 at k = 1024 14.7 / 25.6 at 512 (192), 26.9 / 26.4 at 768 (288).
+// Up to 128 rows always, beyond where the 128 x 128 tiles are at most one per compute unit: measured against
+// the 256-row tiles of qmm_gemm.hip (Q4_K, us per call in a graph, here / there): q|k|v 4096 -> 6144 39.0 / 50.9
+// at 512 rows (192 tiles), 71.9 / 64.9 at 768 (288); 4096 x 4096 42.1 / 54.8 at 1024 (256), 93.1 / 80.6 at
+// 2048 (512); gate|up of 2 x 3072 at k = 1024 14.7 / 25.6 at 512 (192), 26.9 / 26.4 at 768 (288); gate|up of
+// 2 x 12288 at 129, 150 and 192 rows (384) 78 / 83, 75 / 75 and 75 / 71 (Q8_0 at 192: 80 / 74); 65536 x 1024 at
+// 129 rows (1024) 54 / 44, 151936 x 4096 (2374) 363 / 333 and at 193 rows 422 / 316.
 bool qmm_gemm_regb_applies(const QmmLayout* const* layouts, int n_weights, int64_t m, int n_cus) {
     if (m <= 0 || n_weights < 1) return false;
     int64_t tiles = 0;
@@ -538,7 +538,7 @@ bool qmm_gemm_regb_applies(const QmmLayout* const* layouts, int n_weights, int64
     }
     if (m <= 128) return true;
     if (qmm_get_prefill_form() >= 0) return false; // one of the other forms was asked for
-    return tiles <= n_cus || m <= 192;
+    return tiles <= n_cus;
 }
 
 size_t qmm_gemm_regb_workspace_bytes(const QmmLayout* const* layouts, int n_weights, int64_t m, int n_cus) {
