@@ -1935,9 +1935,18 @@ struct RoutingOut {
 // Whether the Q4_K expert MLP runs as matrix products over 64-pair chunks: from nine sorted pairs per expert
 // on average.  Measured at 128 experts, top-8, hidden 2048, inter 768, per layer, chunks / expert form on
 // 16-row tiles: 106 / 91 us at 56 tokens, 104 / 103 at 128, 108 / 111 at 144 (9 pairs), 108 / 118 at 256,
-// 136 / 156 at 512, 206 / 253 at 1024, 294 / 426 at 2048, 497 / 823 at 4096: below, the prefix of a workgroup (its 32 rows at least, over all of k) is not paid back.
-bool moe_on_gemm(const QmmLayout& G, const QmmLayout& D, int64_t t, int top_k) {
-    return qmm_moe_expert_form() < 0 && t * top_k >= 9 * G.n_stacked && qmm_moe_gemm_supported(G, D, t, top_k);
+// 136 / 156 at 512, 206 / 253 at 1024, 294 / 426 at 2048, 497 / 823 at 4096: below, the prefix of a workgroup (its
+// 32 rows at least, over all of k) is not paid back.
+// A workgroup walks all of k alone, about 2.3 us per unit of both products together, whether its neighbours are idle
+// or not, where the tile form cuts an expert's rows into more parts when experts are few.  So few experts with a
+// long k wait for fourteen: hidden 2048, inter 2048, 4, 8 and 16 experts 57 / 53, 60 / 55 and 64 / 59 us at 9 pairs, 57 / 54,
+// 59 / 62 and 64 / 61 at 12, 57 / 61, 60 / 63 and 63 / 67 at 14; inter 1536 52 / 50, 54 / 51 and 58 / 54 at 9, 52 / 57, 54 / 58
+// and 58 / 60 at 14.  With up to twelve units (inter 1024: 48 / 47, 48 / 48 and 52 / 53 at 9; inter 768: 46 / 46, 46 / 47
+// and 48 / 52) or workgroups for half of the compute units (32 experts, inter 1536: 66 / 66 at 9, 66 / 72 at 10; 64 experts,
+// inter 2048: 127 / 137) nine are enough.
+bool moe_on_gemm(const QmmLayout& G, const QmmLayout& D, int64_t t, int top_k, int n_cus) {
+    const bool few_long = G.k_units + D.k_units > 12 && G.n_stacked * (G.n / 256) * 2 <= n_cus;
+    return qmm_moe_expert_form() < 0 && t * top_k >= (few_long ? 14 : 9) * G.n_stacked && qmm_moe_gemm_supported(G, D, t, top_k);
 }
 
 // moe_core on the kernels of qmm_moe_gemm.hip; workspace: y [pairs, hidden] | the token rows' records | the
@@ -2017,7 +2026,7 @@ int moe_core(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, const izwi_
     //            | routing computed here: ids, weights, perm [pairs], offsets [E + 1], sort scratch
     // Q4_K stacks, many pairs per expert: matrix products over 64-pair chunks, silu(gate) * up quantized where it is
     // computed (moe_gemm below)
-    if (moe_on_gemm(G, D, t, top_k))
+    if (moe_on_gemm(G, D, t, top_k, gate->n_cus))
         return moe_gemm(gate, up, down, x, t, top_k, logits, ids, weights, perm, offsets, ids_out, weights_out, out, stream);
     auto align256 = [](size_t v) { return (v + 255) & ~(size_t)255; };
     const size_t h_bytes = align256((size_t)pairs * inter * sizeof(float));

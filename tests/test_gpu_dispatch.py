@@ -1,0 +1,65 @@
+"""Which kernels a call is made of, where both sides of a rule give the same bits or the same values up to rounding:
+kernel names of a child process under torch's profiler (a child, because the switches are read once per process)."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CHILD = """
+import json, sys
+import numpy as np, torch
+import izwi_amd as qa
+from oracle import oracle
+
+def matrix(n, k):
+    return qa.QMatMul.from_qtensor(qa.QTensor.from_blocks(qa.GgmlDType.Q4K, oracle.quantize(12, oracle.randn(n, (n, k), std=0.02)), (n, k)))
+
+def experts(E, hidden, inter):
+    one = {n * k: oracle.quantize(12, oracle.randn(n, (n, k), std=0.02)).reshape(-1) for n, k in ((inter, hidden), (hidden, inter))}
+    stack = lambda n, k: qa.QTensor.from_blocks(qa.GgmlDType.Q4K, np.tile(one[n * k], E), (E, n, k))
+    return qa.MoeExperts(stack(inter, hidden), stack(inter, hidden), stack(hidden, inter))
+
+def call(kind, *sizes):
+    if kind == "moe":
+        E, hidden, inter, top_k, t = sizes
+        layer, x, logits = experts(E, hidden, inter), torch.randn(t, hidden, device="cuda"), torch.randn(t, E, device="cuda")
+        return lambda: layer.layer(logits, x, top_k)
+    n, k, m = sizes
+    mm, x = matrix(n, k), torch.randn(m, k, device="cuda")
+    return lambda: mm.forward(x)
+
+out = []
+for case in json.loads(sys.argv[1]):
+    run = call(*case)
+    run()
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        run()
+        torch.cuda.synchronize()
+    out.append([e.key for e in prof.key_averages()])
+print("NAMES " + json.dumps(out))
+"""
+
+
+def kernels(cases, **env):
+    """Kernel names of one call of each case, in a process with these environment variables."""
+    run = subprocess.run([sys.executable, "-c", CHILD, json.dumps(cases)], cwd=ROOT, env={**os.environ, "PYTHONPATH": ROOT, **env},
+                         capture_output=True, text=True, timeout=100)
+    assert run.returncode == 0, run.stderr[-2000:]
+    names = json.loads(next(line for line in run.stdout.splitlines() if line.startswith("NAMES "))[6:])
+    if not any("kernel" in name for call in names for name in call):
+        pytest.skip("this torch's profiler reports no kernels")
+    return [" ".join(call) for call in names]
+
+
+def test_expert_layers_of_few_experts():
+    """From nine pairs per expert the expert products, from fourteen where experts are few and k is long."""
+    cases = [["moe", 4, 2048, 2048, 2, 18], ["moe", 4, 2048, 2048, 2, 28], ["moe", 16, 2048, 1536, 4, 52], ["moe", 16, 2048, 1536, 4, 56],
+             ["moe", 4, 2048, 1024, 2, 18], ["moe", 4, 2048, 1024, 2, 17], ["moe", 64, 512, 512, 8, 72]]
+    taken = ["moe_gemm_q4k_kernel" in names for names in kernels(cases)]
+    assert taken == [False, True, False, True, True, False, True]
