@@ -105,7 +105,8 @@ int ensure_device(int device, int* n_cus) {
 }
 
 // Whether the expert MLP runs on 16-row matrix-core tiles instead of 4-row dot4 segments: from 3.5
-// sorted pairs per expert on average (IZWI_QMM_MOE_MFMA_MIN_ROWS = a whole number of pairs instead).
+// sorted pairs per expert on average (IZWI_QMM_MOE_MFMA_MIN_ROWS = a whole number of pairs instead); moe_on_gemm
+// says which of those sizes the expert products take.
 // Measured at 128 experts, top-8, per layer, segments / tiles: 68.6 / 80.4 us at 32 tokens, 78.1 / 83.9
 // at 40, 83.5 / 85.4 at 48 (3 pairs per expert), 91.0 / 86.1 at 56, 99 / 87.1 at 64 (4 pairs): the tile
 // path reads every expert once and costs about the same from 16 to 128 tokens, the segment path
@@ -1946,7 +1947,9 @@ struct RoutingOut {
 // inter 2048: 127 / 137) nine are enough.
 bool moe_on_gemm(const QmmLayout& G, const QmmLayout& D, int64_t t, int top_k, int n_cus) {
     const bool few_long = G.k_units + D.k_units > 12 && G.n_stacked * (G.n / 256) * 2 <= n_cus;
-    return qmm_moe_expert_form() < 0 && t * top_k >= (few_long ? 14 : 9) * G.n_stacked && qmm_moe_gemm_supported(G, D, t, top_k);
+    // (moe_on_tiles: a threshold raised through the environment holds for these kernels too)
+    return qmm_moe_expert_form() < 0 && moe_on_tiles(t * top_k, (int)G.n_stacked) &&
+           t * top_k >= (few_long ? 14 : 9) * G.n_stacked && qmm_moe_gemm_supported(G, D, t, top_k);
 }
 
 // moe_core on the kernels of qmm_moe_gemm.hip; workspace: y [pairs, hidden] | the token rows' records | the

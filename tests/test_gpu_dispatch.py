@@ -63,3 +63,12 @@ def test_expert_layers_of_few_experts():
              ["moe", 4, 2048, 1024, 2, 18], ["moe", 4, 2048, 1024, 2, 17], ["moe", 64, 512, 512, 8, 72]]
     taken = ["moe_gemm_q4k_kernel" in names for names in kernels(cases)]
     assert taken == [False, True, False, True, True, False, True]
+
+
+def test_expert_threshold_of_the_environment():
+    """IZWI_QMM_MOE_MFMA_MIN_ROWS: below that many pairs per expert no matrix-core kernel, the products included."""
+    case = ["moe", 8, 512, 512, 2, 80]  # 20 pairs per expert
+    assert "moe_gemm_q4k_kernel" in kernels([case])[0]
+    raised, = kernels([case], IZWI_QMM_MOE_MFMA_MIN_ROWS="21")
+    assert "moe_gemm" not in raised and "mfma" not in raised
+    assert "moe_gemm_q4k_kernel" in kernels([case], IZWI_QMM_MOE_MFMA_MIN_ROWS="20")[0]
