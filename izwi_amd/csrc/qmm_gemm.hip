@@ -600,7 +600,8 @@ struct GemmPlan {
     int64_t full_cols;   // > 0: first a launch of 256 x 256 tiles over this many 256-column strips
 };
 
-// IZWI_QMM_GEMM_TILE="bm,bn,slices" (tuning aid) replaces the plan: bm = 256, bn in {128, 256}.
+// IZWI_QMM_GEMM_TILE="bm,bn,slices" (tuning aid) replaces the plan, at every number of rows, and the choice of
+// the few-row kernel: bm = 256, bn in {128, 256}.
 bool forced_plan(GemmPlan& plan) {
     static const GemmPlan forced = [] {
         GemmPlan p{0, 0, 1, 0};
@@ -693,6 +694,11 @@ hipError_t launch_group_qt(GemmParams P, int64_t n_planned, int n_cus, hipStream
 }
 
 } // namespace
+
+bool qmm_gemm_tile_forced() {
+    GemmPlan plan;
+    return forced_plan(plan);
+}
 
 // a group takes the plane form when every member can
 static bool group_plane_applies(const QmmLayout* const* layouts, int n_weights, int64_t m) {

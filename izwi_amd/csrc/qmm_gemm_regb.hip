@@ -528,7 +528,7 @@ hipError_t launch_regb_qt(const RegbParams& P, const RegbPlan& p, int64_t grid, 
 // 2 x 12288 at 129, 150 and 192 rows (384) 78 / 83, 75 / 75 and 75 / 71 (Q8_0 at 192: 80 / 74); 65536 x 1024 at
 // 129 rows (1024) 54 / 44, 151936 x 4096 (2374) 363 / 333 and at 193 rows 422 / 316.
 bool qmm_gemm_regb_applies(const QmmLayout* const* layouts, int n_weights, int64_t m, int n_cus) {
-    if (m <= 0 || n_weights < 1) return false;
+    if (m <= 0 || n_weights < 1 || qmm_gemm_tile_forced()) return false;
     int64_t tiles = 0;
     const int64_t tiles_m = (m + 127) / 128;
     for (int i = 0; i < n_weights; i++) {

@@ -243,6 +243,7 @@ hipError_t qmm_launch_gemm_plane(const QmmLayout* const* layouts, const void* co
                                  int n_cus, hipStream_t stream, const void* residual = nullptr);
 // Register form of the prefill product, for few activation rows: one launch for 1..QMM_MAX_GROUP
 // weights of one type and k, behind it one reduce launch where k is split.
+bool qmm_gemm_tile_forced(); // IZWI_QMM_GEMM_TILE: the tiles of qmm_gemm.hip for every product
 bool qmm_gemm_regb_applies(const QmmLayout* const* layouts, int n_weights, int64_t m, int n_cus);
 size_t qmm_gemm_regb_workspace_bytes(const QmmLayout* const* layouts, int n_weights, int64_t m, int n_cus);
 hipError_t qmm_launch_gemm_regb(const QmmLayout* const* layouts, const void* const* tiled, int n_weights,

@@ -72,3 +72,14 @@ def test_expert_threshold_of_the_environment():
     raised, = kernels([case], IZWI_QMM_MOE_MFMA_MIN_ROWS="21")
     assert "moe_gemm" not in raised and "mfma" not in raised
     assert "moe_gemm_q4k_kernel" in kernels([case], IZWI_QMM_MOE_MFMA_MIN_ROWS="20")[0]
+
+
+def test_prefill_kernels_by_size_and_by_the_environment():
+    """The few-row kernel up to 128 rows and one tile per compute unit, the 256-row tiles beyond and wherever
+    IZWI_QMM_GEMM_TILE asks for them."""
+    cases = [["product", 512, 1024, 65], ["product", 512, 256, 300], ["product", 33024, 256, 129]]
+    for names, few_row in zip(kernels(cases), (True, True, False)):
+        assert ("gemm_regb_kernel" in names, "gemm_pipe_kernel" in names) == (few_row, not few_row)
+    forced = kernels(cases, IZWI_QMM_GEMM_TILE="256,128,2")
+    assert all("gemm_regb_kernel" not in names and "gemm_pipe_kernel" in names for names in forced)
+    assert ["splitk_reduce_kernel" in names for names in forced] == [True, False, False]  # (k = 256 is one unit)
