@@ -1,0 +1,64 @@
+"""GPU tests (pytest -m gpu) of the 256-row tiles of the prefill product (gemm_pipe_kernel): ragged rows, columns
+and k, splits along k, strips of 256 columns with a narrower rest, groups, and the residual read in front of the
+stores, in place as well.  Products that would take the few-row kernel come here through the in-LDS form.
+
+Reference: float64 products of the bf16 activations with the dequantized weights rounded to bf16; bounds as in
+test_gpu_prefill_regb.py.  With a residual the result is the plain call's f32 sum plus the residual, rounded once:
+the same bits."""
+import pytest
+import torch
+
+from test_gpu_prefill_regb import BF16_TOL, F32_TOL, Q4_K, Q6_K, Q8_0, dense, off, qa, weight  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def tiles(qa):  # noqa: F811
+    before = qa.get_prefill_form()
+    qa.set_prefill_form(0)
+    yield
+    qa.set_prefill_form(before)
+
+
+def check(qa, oracle, dtype, m, n, k):  # noqa: F811
+    print(f"tiles dtype={dtype} m={m} n={n} k={k}", flush=True)
+    mm = weight(qa, oracle, dtype, n, k, 700 + n)
+    x = torch.from_numpy(oracle.randn(701 + m, (m, k))).cuda().to(torch.bfloat16)
+    want = x.double() @ dense(mm).t()
+    y = mm.forward_bf16_to_f32(x)
+    assert off(y, want) < F32_TOL
+    assert off(mm.forward(x), want) < BF16_TOL
+    assert torch.equal(mm.forward(x.float()), y)
+    res = torch.from_numpy(oracle.randn(702 + m, (m, n))).cuda()
+    for r in (res, res.to(torch.bfloat16)):
+        total = (y + r.float()).to(r.dtype)
+        assert torch.equal(mm.forward_fused(x, residual=r, out_dtype=r.dtype), total)
+        inout = r.clone()
+        mm.forward_fused(x, residual=inout, out=inout, out_dtype=r.dtype)
+        assert torch.equal(inout, total)
+
+
+@pytest.mark.parametrize("dtype,m,n,k", [
+    (Q4_K, 129, 300, 256), (Q4_K, 256, 256, 768), (Q4_K, 300, 1000, 4096), (Q4_K, 513, 130, 2048),
+    (Q8_0, 129, 257, 288), (Q8_0, 260, 384, 1056), (Q8_0, 511, 1025, 3072),
+    (Q6_K, 129, 255, 512), (Q6_K, 300, 513, 4096), (Q6_K, 700, 1000, 12288), (Q6_K, 257, 128, 2560)])
+def test_small_products(qa, oracle, tiles, dtype, m, n, k):  # noqa: F811
+    check(qa, oracle, dtype, m, n, k)
+
+
+# more 128 x 128 tiles than compute units: taken by size.  65900 columns: whole rounds of 256-column strips, then
+# half-size tiles; the others have a rest in both directions
+@pytest.mark.parametrize("dtype,m,n,k", [(Q4_K, 2100, 2100, 256), (Q8_0, 190, 17000, 320), (Q6_K, 1000, 5000, 1024), (Q4_K, 150, 65900, 256)])
+def test_large_products(qa, oracle, dtype, m, n, k):  # noqa: F811
+    check(qa, oracle, dtype, m, n, k)
+
+
+@pytest.mark.parametrize("dtype,m,ns,k", [(Q6_K, 300, (513, 128, 200), 4096), (Q4_K, 129, (1000, 256), 2048), (Q8_0, 400, (257, 257), 1056)])
+def test_groups(qa, oracle, tiles, dtype, m, ns, k):  # noqa: F811
+    parts = [weight(qa, oracle, dtype, n, k, 720 + i) for i, n in enumerate(ns)]
+    x = torch.from_numpy(oracle.randn(721, (m, k))).cuda().to(torch.bfloat16)
+    for got_f, got_b, mm in zip(qa.forward_group(parts, x.float()), qa.forward_group(parts, x), parts):
+        want = x.double() @ dense(mm).t()
+        assert off(got_f, want) < F32_TOL
+        assert off(got_b, want) < BF16_TOL

@@ -108,9 +108,9 @@ def test_q6_k_rows_are_independent(qa, oracle):
         assert rel_err(mm.forward(x[r:r + 1].contiguous()).cpu().numpy(), y[r:r + 1].cpu().numpy().astype(np.float64)) <= 2e-6
 
 
-# beyond 128 rows the pipelined tiles: split along k (512 x 1024 x 4096), ragged half-size tiles, one
-# round of 256 x 256 tiles (2048 x 8192), and whole rounds of them followed by half-size tiles (8704
-# columns); up to 128 rows the plain tile kernel
+# up to 128 rows and up to one 128 x 128 tile per compute unit the few-row kernel, split along k (512 x 1024 x
+# 4096) and ragged; beyond, one round of 256 x 256 tiles (2048 x 8192), and whole rounds of them followed by
+# half-size tiles (8704 columns).  Ragged and split 256-row tiles: test_gpu_prefill_tiles.py
 @pytest.mark.parametrize("m,n,k", [(512, 1024, 4096), (300, 200, 768), (65, 256, 1024), (129, 144, 1280), (70, 16, 256),
                                    (600, 1100, 1024), (2048, 8192, 256), (2048, 8704, 512)])
 def test_q6_k_prefill_against_oracle(qa, oracle, m, n, k):
