@@ -167,8 +167,9 @@ int izwi_qmm_get_large_m_arithmetic(void);
  * kernel, tile by tile, on their way into LDS.  IZWI_QMM_PREFILL_PLANE: one pass per call dequantizes
  * the weight into a bf16 plane in the stream's scratch memory (2 bytes per weight element, see
  * izwi_qmm_scratch_reserve), and the matmul kernel streams both operands into LDS without touching
- * them.  IZWI_QMM_PREFILL_AUTO (the default): chosen by size - today the in-LDS form everywhere, which
- * is the faster one up to 4096 rows on the Qwen3-8B shapes.  IZWI_QMM_PREFILL_FORM=lds / plane at
+ * them.  IZWI_QMM_PREFILL_AUTO (the default): chosen by size - the in-LDS form, which
+ * is the faster one up to 4096 rows on the Qwen3-8B shapes, and where its tiles would leave compute units idle (at most one
+ * 128 x 128 tile per unit) the few-row kernel, which unpacks the weights in registers and is the only form up to 128 rows.  IZWI_QMM_PREFILL_FORM=lds / plane at
  * start-up forces one.  Same bf16 operands and f32 accumulation in both; the sums may
  * differ in their last bits (order of the k steps inside a matrix instruction is the same, the split
  * of k over workgroups is not).  No counterpart in the reference. */
@@ -255,7 +256,8 @@ int izwi_qmm_forward_rows_f32(const izwi_qmm_weight* w, const uint32_t* row_ids,
 /* --- activation records: quantized activations handed over by their producer ---------- */
 
 /* For 3 <= m <= 64 rows (5 <= m <= 64 where k <= 3072: three and four rows of a short k stay on the
- * single-launch kernel, four rows per pass) izwi_qmm_forward_f32 is two launches: the activation quantizer (candle-core's
+ * single-launch kernel, four rows per pass) izwi_qmm_forward_f32 is two launches, or one whose workgroups do both where
+ * few activation bytes are read (at most 96 KB per compute unit): the activation quantizer (candle-core's
  * `BlockQ8_0::from_float` / `BlockQ8K::from_float` per row, qwen3 call site core.rs:812) writes
  * "records" into scratch, the matrix-core kernel multiplies them.  The kernel that PRODUCES the
  * activations can write the records itself and save that launch on the token's critical path:
@@ -395,7 +397,8 @@ int izwi_qmm_forward_gate_up_silu_f32(const izwi_qmm_weight* gate, const izwi_qm
  * adds is the route between the three projections: for 3 <= m <= 64 (5 <= m where hidden or
  * intermediate is at most 3072; gate and up of one block type) x is quantized once, gate | up run as one launch on its records, silu(g) * u is quantized
  * straight into the records that `down` multiplies (four launches; the separate calls take five
- * and write and read the intermediate as an f32 matrix); other sizes run the two calls with the
+ * and write and read the intermediate as an f32 matrix); beyond, in the bf16 arithmetic, the intermediate is
+ * rounded to bf16 where it is computed; other sizes run the two calls with the
  * intermediate in the stream's scratch. */
 int izwi_qmm_mlp_forward_f32(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, const izwi_qmm_weight* down,
                              const float* x, int64_t m, float* y, int mem_space, void* stream);

@@ -2028,7 +2028,7 @@ int moe_core(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, const izwi_
     //            | tiles: u [pairs, inter], activation records; else: seg_expert [max_segments]
     //            | routing computed here: ids, weights, perm [pairs], offsets [E + 1], sort scratch
     // Q4_K stacks, many pairs per expert: matrix products over 64-pair chunks, silu(gate) * up quantized where it is
-    // computed (moe_gemm below)
+    // computed (moe_gemm above, with a workspace of its own)
     if (moe_on_gemm(G, D, t, top_k, gate->n_cus))
         return moe_gemm(gate, up, down, x, t, top_k, logits, ids, weights, perm, offsets, ids_out, weights_out, out, stream);
     auto align256 = [](size_t v) { return (v + 255) & ~(size_t)255; };
@@ -2217,7 +2217,7 @@ int izwi_moe_layer_f32(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, c
     HIP_TRY(li.in(logits, (size_t)t * n_experts * sizeof(float), mem_space, stream));
     HIP_TRY(xi.in(x, (size_t)t * hidden * sizeof(float), mem_space, stream));
     HIP_TRY(oo.out(out, (size_t)t * hidden * sizeof(float), mem_space, stream));
-    // (ids and weights reach their outputs through device-to-device copy calls)
+    // (ids and weights in device memory: the routing kernels write them, the sort and the combine read them back)
     if (ids_out) HIP_TRY(io.out(ids_out, (size_t)pairs * sizeof(int32_t), mem_space, stream, false));
     if (weights_out) HIP_TRY(wo.out(weights_out, (size_t)pairs * sizeof(float), mem_space, stream, false));
     if (int rc = moe_core(gate, up, down, (const float*)xi.dev, t, top_k, (const float*)li.dev, nullptr, nullptr,

@@ -317,7 +317,7 @@ hipError_t launch_plane_tile(PlaneGemmParams P, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// 0: in-LDS form always; 1: plane form wherever it can run (m > 128); -1: by size (today: in-LDS)
+// 0: in-LDS form always; 1: plane form wherever it can run (m > 128); -1: by size (today: never this form)
 int plane_mode() {
     static const int mode = [] {
         const char* e = getenv("IZWI_QMM_PREFILL_FORM");

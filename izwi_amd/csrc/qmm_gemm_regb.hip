@@ -11,10 +11,11 @@
 // LDS writes, one barrier per unit.  The two halves' sums meet in LDS at the end.  Where the tiles
 // alone leave compute units idle, k is split over workgroups and the row tiles get lower.
 //
-// Bound by the vector instructions that unpack (7.3 per matrix instruction) beside the matrix
-// instructions (half of the time of a full chip): a unit takes 1.1 us at 32 rows, 1.25 at 64, 1.6 at
-// 96, 1.8 to 2.3 at 128, and 6.5 to 8 us per workgroup are no unit (start, first loads, exchange of the
-// sums, stores).  Splitting a unit four ways over the waves (64 x 128 wave tiles, fewer LDS reads) cost
+// Bound by the life of a workgroup: a unit takes 1.1 us at 32 rows, 1.25 at 64, 1.6 at 96, 1.8 to 2.3 at
+// 128, between barriers at which two waves per SIMD meet, and 6.5 to 8 us are no unit (start, first
+// loads, exchange of the sums, stores).  The pipes are idle in between: gate|up at 101 rows keeps the
+// matrix pipe and the vector instructions that unpack (7.3 per matrix instruction in the loop, 8.2 in
+// all) busy a third of the time each on the compute units in use, and reads 1.6 TB/s.  Splitting a unit four ways over the waves (64 x 128 wave tiles, fewer LDS reads) cost
 // 14 us per workgroup instead: the exchange of the sums is 512 KB of LDS traffic there, 128 KB here.  us per
 // call on f32 rows in a graph, one call per weight on 128 x 256 / 64 x 128 tiles with the weights through
 // LDS / here.  Q4_K, 101 rows: q|k|v 81 / 27, 4096 x 4096 28 / 19, gate|up 82 / 47, down 47 / 32; Q6_K down

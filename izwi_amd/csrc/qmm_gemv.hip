@@ -704,7 +704,7 @@ hipError_t qmm_launch_gemv_rows(const QmmLayout& L, const void* tiled, const flo
 namespace {
 
 // silu(gate) * up, four consecutive values per thread, as f32 or rounded to bf16 (what a prefill
-// product reads: one launch and 6 of 14 bytes per value less than f32 and a conversion behind it)
+// product reads: one launch and 8 of 18 bytes per value less than f32 and a conversion behind it)
 template <bool BF16>
 __global__ void silu_mul_kernel(const float* __restrict__ gate, const float* __restrict__ up, void* __restrict__ out,
                                 int64_t count, int aligned) {

@@ -1708,7 +1708,7 @@ hipError_t launch_own_quantizer(const QmmLayout& L0, MfmaParams P, int64_t x_k, 
     const size_t lds = std::max((size_t)P.window_units * unit_bytes(L0.dtype), (size_t)waves * 256 * 4);
     if (lds > 160 * 1024) return hipErrorNotSupported;
     P.k = (int)x_k;
-    P.units_magic = (65536 + P.k_units - 1) / P.k_units; // exact for the up to 768 items of a workgroup and 32 units
+    P.units_magic = (65536 + P.k_units - 1) / P.k_units; // exact for the up to 192 items (12 waves, 4 groups, 4 runs) of a workgroup and 32 units
     const unsigned grid = P.n_tiles > 1 ? (unsigned)((P.rt_groups + 7) / 8 * 8 * P.n_tiles) : (unsigned)P.rt_groups;
     auto go = [&](auto kernel) -> hipError_t {
         if (lds > 48 * 1024) {

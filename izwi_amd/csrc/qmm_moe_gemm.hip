@@ -19,12 +19,13 @@
 // waves walk k on their own; a lane's weight chunks are requested one unit ahead.
 //
 // gate | up: the 256 columns of a workgroup are one unit of the down projection's input, so
-// silu(gate) * up is quantized here, in LDS, and leaves as records: 9 bytes instead of 64 per eight
+// silu(gate) * up is quantized here, in LDS, and leaves as records: 9.5 bytes instead of 64 per eight
 // values, no launch in between.
 //
-// Bound by vector instructions (160 per block of 32 x 32 outputs and unit, half of them the unpacking that two
-// blocks of pairs share, 640 cycles) beside 17 matrix instructions (544 cycles), which two waves per
-// SIMD overlap in part: at 4096 tokens the vector ALU is busy 58 % of the cycles and the matrix pipe 35 %.
+// Bound by vector instructions (about 160 per block of 32 x 32 outputs and unit in the loop, half of them the
+// unpacking that two blocks of pairs share, 640 cycles; 209 and 191 with everything around it) beside 17 matrix
+// instructions (544 cycles), which two waves per SIMD overlap in part: at 4096 tokens the vector ALU is busy
+// 56 % of the cycles of gate | up and the matrix pipe 36 %.
 // 128 experts, top-8, 2048 x 768: gate | up 282 us and down 164 at 4096 tokens (730 and 630 TOP/s), where the
 // 16-row-tile kernels took 480 and 260 and the quantizer between them 40; 80 and 41 at 512 tokens, before 92, 48
 // and 8 (a workgroup's life is 40 us there, 1.5 per compute unit).  The layer 823 -> 497 us and 156 -> 136.  Of that,

@@ -69,7 +69,7 @@ class Qwen3DecodeLayer:
     def _forward_one_call(self, x, cos_sin, k_cache, v_cache, pos):
         """The fused form's five calls as one library call (the same kernels, the same results): the calls' own
         preparation, allocations and foreign-function overhead took 40 us of host time per layer, more than the
-        launches of a 0.6B layer run for (28 layers and the head: 1770 us a token as calls, 755 this way).
+        launches of a 0.6B layer run for (28 layers and the head: 1850 us a token as calls, 855 this way).
         None for arguments it does not cover: those go call by call."""
         gate_up = self.gate_up._parts
         if gate_up is None or not _ok(x, self.w_in, self.w_post, self.qk_w, cos_sin, k_cache, v_cache):
