@@ -52,6 +52,18 @@ def off(y, want):
     (Q8_0, 65, 130, 288), (Q8_0, 100, 64, 32), (Q8_0, 128, 1024, 1056), (Q8_0, 70, 96, 3072), (Q8_0, 193, 200, 800),
     (Q6_K, 65, 128, 256), (Q6_K, 96, 130, 768), (Q6_K, 127, 257, 2560), (Q6_K, 300, 1024, 4096)])
 def test_product_and_its_epilogues(qa, oracle, dtype, m, n, k):
+    product_and_its_epilogues(qa, oracle, dtype, m, n, k)
+
+
+# row tiles of 64, 96 and 128 rows (narrow products take the lowest ones): whole and ragged last tiles in both directions,
+# one row tile and two, k that ends inside a unit
+@pytest.mark.parametrize("m,n", [(64, 16500), (101, 9000), (65, 16500), (96, 16512), (97, 16500), (128, 16500), (150, 16000), (250, 15900)])
+@pytest.mark.parametrize("dtype,k", [(Q4_K, 512), (Q8_0, 288), (Q6_K, 256)])
+def test_row_tile_heights(qa, oracle, dtype, m, n, k):
+    product_and_its_epilogues(qa, oracle, dtype, m, n, k)
+
+
+def product_and_its_epilogues(qa, oracle, dtype, m, n, k):
     print(f"regb dtype={dtype} m={m} n={n} k={k}", flush=True)
     mm = weight(qa, oracle, dtype, n, k, 300 + n)
     x = torch.from_numpy(oracle.randn(301 + m, (m, k))).cuda().to(torch.bfloat16)
