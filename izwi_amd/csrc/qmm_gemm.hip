@@ -25,6 +25,7 @@
 #include <utility>
 
 #include "qmm_internal.h"
+#include "qmm_tile.h"
 
 namespace {
 
@@ -68,27 +69,6 @@ struct GemmParams {
     int64_t nv[QMM_MAX_GROUP], row_tiles_v[QMM_MAX_GROUP];
     float* partial_v[QMM_MAX_GROUP];
 };
-
-__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    bf16x2 v = {(__bf16)a, (__bf16)b}; // v_cvt_pk_bf16_f32: round to nearest even
-    return __builtin_bit_cast(uint32_t, v);
-}
-
-// byte N of v as float (v_cvt_f32_ubyteN)
-template <int N>
-__device__ __forceinline__ float ubyte_f32(uint32_t v) {
-    return (float)((v >> (8 * N)) & 0xffu);
-}
-
-template <int N, class F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    static_for_impl<N>(f, std::make_integer_sequence<int, N>{});
-}
 
 // Pipelined 256-column tile.  The k loop runs over units of 256 k-elements with the four
 // 64-wide steps of a unit unrolled, so that the sub-block index, the LDS stage and the

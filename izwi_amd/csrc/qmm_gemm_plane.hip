@@ -25,6 +25,7 @@
 #include <utility>
 
 #include "qmm_internal.h"
+#include "qmm_tile.h"
 
 namespace {
 
@@ -35,16 +36,6 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kRowBytes = 128;                  // 64 bf16: one tile row of one k step
 constexpr int kBlockRows = 256;                 // rows of a plane block
 constexpr int kBlockBytes = kBlockRows * kRowBytes;
-
-__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    bf16x2 v = {(__bf16)a, (__bf16)b}; // round to nearest even
-    return __builtin_bit_cast(uint32_t, v);
-}
-template <int N>
-__device__ __forceinline__ float ubyte_f32(uint32_t v) {
-    return (float)((v >> (8 * N)) & 0xffu);
-}
 
 struct PlaneDequantParams {
     const uint8_t* w;
@@ -129,15 +120,6 @@ __global__ __launch_bounds__(256) void plane_dequant_kernel(PlaneDequantParams P
     }
 }
 
-template <int N, class F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    static_for_impl<N>(f, std::make_integer_sequence<int, N>{});
-}
-
 struct PlaneGemmParams {
     const uint16_t* x; // bf16 [m, k]
     int64_t m, k;
@@ -151,11 +133,6 @@ struct PlaneGemmParams {
     int out_bf16;
     const void* residual; // single weight only
 };
-
-// 16 bytes per lane from global memory straight into LDS: lane l's bytes land at lds + 16 l.
-__device__ __forceinline__ void load_to_lds(const uint8_t* base, uint32_t lane_off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(lane_off), "s"(base) : "memory", "m0");
-}
 
 // BM x BN output tile, NW waves as an (NW / 2) x 2 grid, NS LDS stages of one 64-wide k step.
 // The k loop has one barrier per step, at the three-quarter point: by then every fragment of the

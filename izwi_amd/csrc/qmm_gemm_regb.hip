@@ -29,6 +29,7 @@
 #include <utility>
 
 #include "qmm_internal.h"
+#include "qmm_tile.h"
 
 namespace {
 
@@ -43,24 +44,6 @@ constexpr int kWaves = kCols * kSplits;
 constexpr int kBN = 32 * kCols;
 constexpr int kUnitBytes = QMM_UNIT_ELEMS * 2; // one activation row of one unit, bf16
 
-template <int N, class F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    static_for_impl<N>(f, std::make_integer_sequence<int, N>{});
-}
-
-__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    bf16x2 v = {(__bf16)a, (__bf16)b}; // round to nearest even
-    return __builtin_bit_cast(uint32_t, v);
-}
-template <int N>
-__device__ __forceinline__ float ubyte_f32(uint32_t v) {
-    return (float)((v >> (8 * N)) & 0xffu);
-}
 // fma(scale, byte, bias) of the eight bytes of (lo, hi) as one bf16 operand
 __device__ __forceinline__ bf16x8 scaled_bytes(uint32_t lo, uint32_t hi, float scale, float bias) {
     u32x4 o;
@@ -170,11 +153,6 @@ __device__ __forceinline__ bf16x8 half_operand(const HalfRegs<QT>& r, const Step
         hi = ((r.q[q][2 * e + 1] >> (4 * st)) & nibble_mask) | (((r.qh[2 * e + 1] >> (4 * st + 2 * q)) & 0x03030303u) << 4);
     }
     return scaled_bytes(lo, hi, s.scale[q], s.bias[q]);
-}
-
-// 16 bytes per lane from global memory straight into LDS: lane l's bytes land at lds + 16 l.
-__device__ __forceinline__ void load_to_lds(const uint8_t* base, uint32_t lane_off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(lane_off), "s"(base) : "memory", "m0");
 }
 
 template <int QT, int MT>

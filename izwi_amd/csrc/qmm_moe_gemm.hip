@@ -36,6 +36,7 @@
 #include "qmm_internal.h"
 #include "qmm_moe_route.h"
 #include "qmm_records.h"
+#include "qmm_tile.h"
 
 namespace {
 
@@ -262,14 +263,6 @@ __device__ __forceinline__ void chunk_body(const MoeGemmParams& P, const uint8_t
     }
 }
 
-// LDS-direct load of 16 (4) bytes per lane to lds + 16 (4) * lane
-__device__ __forceinline__ void load_lds16(uint32_t lds, uint32_t off, const uint8_t* base) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
-}
-__device__ __forceinline__ void load_lds4(uint32_t lds, uint32_t off, const uint8_t* base) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
-}
-
 // The records of units [u0, u1) of the chunk's rows into their LDS images
 __device__ __forceinline__ void issue_records(const MoeGemmParams& P, const uint32_t* src_off, uint8_t* smem, int nrb, int u0, int u1,
                                               int wave, int lane) {
@@ -282,14 +275,15 @@ __device__ __forceinline__ void issue_records(const MoeGemmParams& P, const uint
         if (sub < 2 * groups) {
             const int p = sub / groups, g = sub - p * groups;
             const int r = g * 8 + (lane >> 3);
-            load_lds16(__builtin_amdgcn_readfirstlane(unit_lds + p * (kRows * 128) + g * 1024),
-                       src_off[r] + (uint32_t)p * 128u + (uint32_t)((lane & 7) ^ ((r >> 1) & 7)) * 16u, base);
+            const uint32_t to = __builtin_amdgcn_readfirstlane(unit_lds + p * (kRows * 128) + g * 1024);
+            load_to_lds(base, src_off[r] + (uint32_t)p * 128u + (uint32_t)((lane & 7) ^ ((r >> 1) & 7)) * 16u, to);
         } else if (sub < 2 * groups + nrb) {
             const int q = sub - 2 * groups, r = q * 32 + (lane >> 1);
-            load_lds16(__builtin_amdgcn_readfirstlane(unit_lds + kSumsAt + q * 1024),
-                       src_off[r] + 256u + (uint32_t)((lane & 1) ^ ((r >> 3) & 1)) * 16u, base);
+            const uint32_t to = __builtin_amdgcn_readfirstlane(unit_lds + kSumsAt + q * 1024);
+            load_to_lds(base, src_off[r] + 256u + (uint32_t)((lane & 1) ^ ((r >> 3) & 1)) * 16u, to);
         } else {
-            load_lds4(__builtin_amdgcn_readfirstlane(unit_lds + kScalesAt), src_off[lane] + 288u, base);
+            const uint32_t to = __builtin_amdgcn_readfirstlane(unit_lds + kScalesAt);
+            load_to_lds4(base, src_off[lane] + 288u, to);
         }
     }
 }
