@@ -165,3 +165,27 @@ def test_rows_that_do_not_start_on_sixteen_bytes(qa, oracle, dtype, m, n, k, ski
         assert torch.equal(parts[0].forward_fused(rows, residual=res), parts[0].forward_fused(x, residual=res))
         for a, b in zip(qa.forward_group(parts, rows), qa.forward_group(parts, x)):
             assert torch.equal(a, b)
+
+
+def test_copied_rows_in_a_captured_graph(qa, oracle):
+    """The copy of rows that do not start on 16 bytes is part of the graph: every replay reads the rows of its time."""
+    m, n, k = 100, 300, 512
+    mm = weight(qa, oracle, Q4_K, n, k, 650)
+    rows = torch.empty(1 + m * k, dtype=torch.bfloat16, device="cuda")[1:].view(m, k)
+    xs = [torch.from_numpy(oracle.randn(651 + i, (m, k))).cuda().to(torch.bfloat16) for i in range(4)]
+    rows.copy_(xs[0])
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        mm.forward(rows)  # the stream's scratch grows before the capture
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        y = mm.forward(rows)
+    for x in xs:
+        rows.copy_(x)
+        want = mm.forward(x)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
