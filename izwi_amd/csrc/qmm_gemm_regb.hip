@@ -7,19 +7,26 @@
 // 256 k-elements, half p.  A lane's 16-byte quant chunk holds k-elements of one weight row only,
 // which is what a lane supplies to v_mfma_f32_32x32x16_bf16: the chunk is unpacked into B operands
 // in registers, in the k order the chunk has, and the A operand (activations, staged in LDS by
-// LDS-direct loads, two stages of one unit) is picked in the same order.  No weight tile in LDS, no
-// LDS writes, one barrier per unit.  The two halves' sums meet in LDS at the end.  Where the tiles
-// alone leave compute units idle, k is split over workgroups and the row tiles get lower.
+// LDS-direct loads) is picked in the same order.  No weight tile in LDS, no LDS writes, one barrier per
+// unit.  The two halves' sums meet in LDS at the end.  Where the tiles alone leave compute units idle, k is
+// split over workgroups and the row tiles get lower.
 //
-// Bound by the life of a workgroup: a unit takes 1.1 us at 32 rows, 1.25 at 64, 1.6 at 96, 1.8 to 2.3 at
-// 128, between barriers at which two waves per SIMD meet, and 6.5 to 8 us are no unit (start, first
-// loads, exchange of the sums, stores).  The pipes are idle in between: gate|up at 101 rows keeps the
-// matrix pipe and the vector instructions that unpack (7.3 per matrix instruction in the loop, 8.2 in
-// all) busy a third of the time each on the compute units in use, and reads 1.6 TB/s.  Splitting a unit four ways over the waves (64 x 128 wave tiles, fewer LDS reads) cost
+// The loads run ahead of the units: weights four to six units in registers, activations two or three in LDS, and the
+// first unit waits for its own loads alone.  The workgroups of an XCD begin at different units of k: beginning
+// together they read the same 512 bytes of every activation row at once, and rows lie a power of two apart.
+//
+// Bound by the life of a workgroup: at 2 x 12288 x 4096 (Q4_K, cold weights; time stamps) it has its arguments after 1.0 us
+// and its first operands 4.2 later, takes 30 in sixteen units (1.95 a unit at 101 rows, 1.65 at 65; 2.1 and 1.8 with the
+// loads one unit ahead and all workgroups at the same unit) and 2.2 for the exchange of the sums and the stores.  Of a
+// unit's 1.95 us 1.57 remain without its loads and 1.3 without unpacking and activations: matrix instructions (1.0),
+// unpacking (1.0), LDS reads (0.9 to 1.2) and the loads share the compute unit, and two waves per SIMD overlap them in
+// part.  An unpacking of a fifth fewer vector instructions (mixed-precision fma on f16 denormals) gave nothing.
+// Splitting a unit four ways over the waves (64 x 128 wave tiles, fewer LDS reads) cost
 // 14 us per workgroup instead: the exchange of the sums is 512 KB of LDS traffic there, 128 KB here.  us per
 // call on f32 rows in a graph, one call per weight on 128 x 256 / 64 x 128 tiles with the weights through
-// LDS / here.  Q4_K, 101 rows: q|k|v 81 / 27, 4096 x 4096 28 / 19, gate|up 82 / 47, down 47 / 32; Q6_K down
-// 201 / 35; 512 rows: q|k|v 54 / 45; 0.6B shapes at 512: q|k|v 27 / 15.
+// LDS / here with the loads one unit ahead.  Q4_K, 101 rows: q|k|v 81 / 27, 4096 x 4096 28 / 19, gate|up 82 / 47, down 47 / 32; Q6_K down
+// 201 / 35; 512 rows: q|k|v 54 / 45; 0.6B shapes at 512: q|k|v 27 / 15.  The calls of one layer on bf16 rows, loads one unit
+// ahead / now: 8B Q4_K 111 / 107 us at 128 rows, Q8_0 116 / 112, 0.6B Q4_K 39.1 / 38.2 at 65, 55.8 / 53.7 at 400.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -76,6 +83,7 @@ struct RegbParams {
 template <int QT>
 struct HalfRegs {
     static constexpr int NQ = QT == QMM_Q8_0 ? 4 : 2;
+    static constexpr int kLoads = 1 + NQ + (QT == QMM_Q6_K ? 2 : 0); // load instructions of load_half
     using Header = std::conditional_t<QT == QMM_Q4_K, u32x4, u32x2>; // Q8_0, Q6_K: the two steps' scale dwords
     Header hdr;
     u32x4 q[NQ];
@@ -155,11 +163,29 @@ __device__ __forceinline__ bf16x8 half_operand(const HalfRegs<QT>& r, const Step
     return scaled_bytes(lo, hi, s.scale[q], s.bias[q]);
 }
 
+// Stages of activations in LDS (as many units as fit, up to three) and units of weights in registers, for row tiles of 32 * mt
+constexpr int x_stages(int mt) { return mt <= 3 ? 3 : 2; }
+constexpr int weight_buffers(int mt) { return mt <= 3 ? 6 : 4; }
+
+// f(I, false); if there is more, f(I, true) and the same from I + 1 on (nested, not a loop with exits: every
+// step is reached from one place, so the compiler's waits there are for what was requested on that path)
+template <int I, int N, class F, class M>
+__device__ __forceinline__ void chain(F&& f, M&& more) {
+    f(std::integral_constant<int, I>{}, std::false_type{});
+    if constexpr (I + 1 < N)
+        if (more()) {
+            f(std::integral_constant<int, I>{}, std::true_type{});
+            chain<I + 1, N>(f, more);
+        }
+}
+
 template <int QT, int MT>
 __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P) {
     constexpr int BM = 32 * MT;
     constexpr int kStage = BM * kUnitBytes;
     constexpr int XL = BM / 2 / kWaves; // LDS-direct loads per wave and unit (1 KiB = two rows each)
+    constexpr int NS = x_stages(MT), DW = weight_buffers(MT), WL = HalfRegs<QT>::kLoads;
+    static_assert(DW % NS == 0 && (DW - 2) * WL >= WL + (NS - 2) * (XL + WL));
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
 
     // Workgroups go to the eight XCDs round-robin by their index; the row tiles of one (column tile,
@@ -183,7 +209,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
         }
     const int tn = (col - first_col) / slices, slice = col - first_col - tn * slices;
     const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * kBN;
+    // A workgroup's units u0 .. u1 - 1 of k in turn, from `first` on: those that share an XCD begin at different
+    // ones (see above).
     const int u0 = slice * slice_units, u1 = min(P.k_units, u0 + slice_units);
+    const int first = (tn >> 3) % (u1 - u0);
+    auto unit_of = [&](int u) { return u + first < u1 ? u + first : u + first - (u1 - u0); };
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -205,15 +235,16 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
     // and are zeroed when they have landed
     const int x_tail = QT == QMM_Q8_0 ? (int)(P.k % QMM_UNIT_ELEMS) / 8 : 0;
     const int x_chunk = (lane & 31) ^ ((2 * wave + h) & 15);
-    auto issue_x = [&](int u, int stage) {
+    auto issue_x = [&](int at, int stage) {
+        const int u = unit_of(at);
         const uint8_t* src = x_tile + (size_t)u * kUnitBytes;
         const uint32_t dst = lds0 + stage * kStage + wave * 1024;
         const uint32_t back = x_tail && u == P.k_units - 1 && x_chunk >= x_tail ? x_chunk * 16 : 0;
 #pragma unroll
         for (int i = 0; i < XL; i++) load_to_lds(src, x_off[i] - back, dst + i * kWaves * 1024);
     };
-    auto zero_tail = [&](int u, int stage) { // behind this wave's loads of unit u, in front of a barrier
-        if (x_tail && u == P.k_units - 1 && x_chunk >= x_tail)
+    auto zero_tail = [&](int at, int stage) { // behind this wave's loads of the unit, in front of a barrier
+        if (x_tail && unit_of(at) == P.k_units - 1 && x_chunk >= x_tail)
 #pragma unroll
             for (int i = 0; i < XL; i++)
                 *reinterpret_cast<u32x4*>(smem + stage * kStage + (wave + i * kWaves) * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
@@ -233,7 +264,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
         off.qh = base + (9 + 2 * half + h) * chunk;
         off.d = base + 13 * chunk;
     }
-    auto load_w = [&](HalfRegs<QT>& r, int u) {
+    auto load_w = [&](HalfRegs<QT>& r, int at) {
+        const int u = unit_of(at);
         const int kg = u / P.s, us = u - kg * P.s;
         load_half<QT>(r, w_tile + (int64_t)kg * P.panel_bytes + us * 256, off);
     };
@@ -250,8 +282,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
 
     // Software pipeline: the operands of instruction ss + 1 are read / unpacked behind instruction ss;
     // the unit's only barrier sits in front of its last one, where every activation of the unit is in
-    // registers and the next unit has landed, and the unit after that is requested behind it.
-    HalfRegs<QT> w[2];
+    // registers and the next unit has landed; behind it the activations NS units on and the weights DW units
+    // on are requested, in this order.  Loads land in order: what may still be in flight at a barrier is
+    // what was requested behind the next unit's activations.  (The compiler's own waits count the weights
+    // alone; DW is as large as it takes for them to ask for no more.)
+    HalfRegs<QT> w[DW];
     StepScales sc[2];
     bf16x8 a[2][MT], b[2];
     auto read_a = [&](int stage, auto SS) {
@@ -260,58 +295,80 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
 #pragma unroll
         for (int i = 0; i < MT; i++) a[ss & 1][i] = *reinterpret_cast<const bf16x8*>(src + i * 32 * kUnitBytes);
     };
-    const int last = u1 - 1; // past the end: the last unit again, into stages nobody reads
+    const int last = u1 - 1;
+    // (past the end: the last unit's weights again, never used)
+    auto request_w = [&](auto I) {
+        load_w(w[decltype(I)::value], min(u0 + decltype(I)::value, last));
+        asm volatile("" ::: "memory"); // the requests stay here, in this order
+    };
     issue_x(u0, 0);
-    load_w(w[0], u0);
-    issue_x(min(u0 + 1, last), 1);
-    load_w(w[1], min(u0 + 1, last));
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    static_for<DW - NS + 1>(request_w);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((DW - NS) * WL) : "memory");
     zero_tail(u0, 0);
-    zero_tail(min(u0 + 1, last), 1);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     arrived<QT>(w[0]);
-    arrived<QT>(w[1]);
+    static_for<NS - 1>([&](auto I) { // only now: the first unit does not wait for them
+        constexpr int i = decltype(I)::value + 1;
+        if (u0 + i <= last) issue_x(u0 + i, i);
+        request_w(std::integral_constant<int, DW - NS + i>{});
+    });
     read_a(0, std::integral_constant<int, 0>{});
     sc[0] = step_scales<QT, 0>(w[0], half, h);
     b[0] = half_operand<QT, 0>(w[0], sc[0], P.nibble_mask);
-    auto unit_step = [&](int u, auto PAR) {
-        constexpr int par = decltype(PAR)::value;
-        static_for<8>([&](auto SS) {
+    int u = u0;
+    auto multiply = [&](auto SS) {
+        constexpr int ss = decltype(SS)::value;
+#pragma unroll
+        for (int j = 0; j < MT; j++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[ss & 1][j], b[ss & 1], acc[j], 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < MT; q++) { // one matrix instruction, then a share of the next one's operands
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 32 / MT, 0);
+        }
+    };
+    auto front = [&](auto I) { // matrix instructions 0 .. 6 of the unit in stage I % NS, buffer I
+        constexpr int i = decltype(I)::value;
+        static_for<7>([&](auto SS) {
             constexpr int ss = decltype(SS)::value;
-            if constexpr (ss < 7) {
-                if constexpr (ss == 3) sc[1] = step_scales<QT, 1>(w[par], half, h);
-                read_a(par, std::integral_constant<int, ss + 1>{});
-                b[(ss + 1) & 1] = half_operand<QT, ss + 1>(w[par], sc[(ss + 1) >> 2], P.nibble_mask);
-            } else {
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                zero_tail(min(u + 1, last), par ^ 1);
-                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-                arrived<QT>(w[par ^ 1]);
-                const int next = min(u + 2, last);
-                issue_x(next, par);
-                load_w(w[par], next);
-                asm volatile("" ::: "memory"); // the requests stay here
-                read_a(par ^ 1, std::integral_constant<int, 0>{});
-                sc[0] = step_scales<QT, 0>(w[par ^ 1], half, h);
-                b[0] = half_operand<QT, 0>(w[par ^ 1], sc[0], P.nibble_mask);
-            }
-#pragma unroll
-            for (int i = 0; i < MT; i++) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[ss & 1][i], b[ss & 1], acc[i], 0, 0, 0);
-#pragma unroll
-            for (int q = 0; q < MT; q++) { // one matrix instruction, then a share of the next one's operands
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 32 / MT, 0);
-            }
+            if constexpr (ss == 3) sc[1] = step_scales<QT, 1>(w[i], half, h);
+            read_a(i % NS, std::integral_constant<int, ss + 1>{});
+            b[(ss + 1) & 1] = half_operand<QT, ss + 1>(w[i], sc[(ss + 1) >> 2], P.nibble_mask);
+            multiply(SS);
         });
     };
-    int u = u0;
-    do {
-        unit_step(u, std::integral_constant<int, 0>{});
-        if (++u == u1) break;
-        unit_step(u, std::integral_constant<int, 1>{});
-    } while (++u < u1);
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); // the requests past the end
+    // The turn to the next unit around the last matrix instruction.  Behind the next unit's activations may still
+    // fly: the weights requested with them and, per turn since, activations (where there were any left) and weights.
+    auto turn = [&](auto I, auto REQUESTS, auto BEHIND, auto BEHIND_LAST) {
+        constexpr int i = decltype(I)::value, next = (i + 1) % DW;
+        if (NS > 2 && u + 2 <= last) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(BEHIND)::value) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(BEHIND_LAST)::value) : "memory");
+        zero_tail(u + 1, (i + 1) % NS);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        arrived<QT>(w[next]);
+        if (u + NS <= last) issue_x(u + NS, i % NS);
+        asm volatile("" ::: "memory");
+        if constexpr (decltype(REQUESTS)::value) load_w(w[i], min(u + DW, last));
+        asm volatile("" ::: "memory"); // the requests stay here
+        read_a((i + 1) % NS, std::integral_constant<int, 0>{});
+        sc[0] = step_scales<QT, 0>(w[next], half, h);
+        b[0] = half_operand<QT, 0>(w[next], sc[0], P.nibble_mask);
+        multiply(std::integral_constant<int, 7>{});
+        u++;
+    };
+    while (u + DW <= last)
+        static_for<DW>([&](auto I) {
+            front(I);
+            turn(I, std::true_type{}, std::integral_constant<int, WL + (NS - 2) * (XL + WL)>{}, std::integral_constant<int, (NS - 1) * WL>{});
+        });
+    // the last 1 .. DW units, whose weights have all been requested
+    chain<0, DW>([&](auto I, auto MORE) {
+        constexpr int i = decltype(I)::value, w_behind = i < NS - 1 ? (NS - 1 - i) * WL : 0;
+        if constexpr (!decltype(MORE)::value) front(I);
+        else turn(I, std::false_type{}, std::integral_constant<int, w_behind + (NS - 2) * XL>{}, std::integral_constant<int, w_behind>{});
+    }, [&] { return u < last; });
+    multiply(std::integral_constant<int, 7>{});
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); // (every activation request has been waited for)
 
     // ---- the two halves' sums: the wave of half p finishes the 32-row blocks i with i % 2 = p
     constexpr int kOwn = (MT + 1) / 2;
@@ -480,7 +537,7 @@ size_t partial_bytes(const RegbPlan& p, const QmmLayout& L, int i, int64_t m) {
 
 template <int QT, int MT>
 hipError_t launch_regb(const RegbParams& P, int64_t grid, hipStream_t stream) {
-    constexpr size_t stages = (size_t)2 * 32 * MT * kUnitBytes; // the halves' sums reuse it
+    constexpr size_t stages = (size_t)x_stages(MT) * 32 * MT * kUnitBytes; // the halves' sums reuse it
     static_assert(stages <= 160 * 1024 && stages >= (size_t)kCols * MT * 4096, "LDS of a CU");
     auto fn = &gemm_regb_kernel<QT, MT>;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)stages);

@@ -63,6 +63,18 @@ def test_row_tile_heights(qa, oracle, dtype, m, n, k):
     product_and_its_epilogues(qa, oracle, dtype, m, n, k)
 
 
+# units of 256 k per workgroup around the depth of the kernel's loads (four or six units of weights, two or three of
+# activations): one to five without a split, then eight slices of 4 .. 14 units, the last one a unit shorter
+@pytest.mark.parametrize("units", [1, 2, 3, 4, 5] + [8 * j - 1 for j in (4, 5, 6, 7, 8, 9, 10, 12, 13, 14)])
+@pytest.mark.parametrize("dtype,m", [(Q4_K, 33), (Q8_0, 64), (Q6_K, 96), (Q4_K, 101), (Q8_0, 128)])
+def test_units_of_a_workgroup(qa, oracle, dtype, m, units):
+    k = 256 * units - (64 if dtype == Q8_0 else 0)  # k of Q8_0 may end inside a unit
+    print(f"regb dtype={dtype} m={m} units={units}", flush=True)
+    mm = weight(qa, oracle, dtype, 200, k, 310 + units)
+    x = torch.from_numpy(oracle.randn(311 + m, (m, k))).cuda().to(torch.bfloat16)
+    assert off(mm.forward_bf16_to_f32(x), x.double() @ dense(mm).t()) < F32_TOL
+
+
 def product_and_its_epilogues(qa, oracle, dtype, m, n, k):
     print(f"regb dtype={dtype} m={m} n={n} k={k}", flush=True)
     mm = weight(qa, oracle, dtype, n, k, 300 + n)
