@@ -27,8 +27,8 @@
 // instructions (544 cycles), which two waves per SIMD overlap in part: at 4096 tokens the vector ALU is busy
 // 56 % of the cycles of gate | up and the matrix pipe 36 %.
 // 128 experts, top-8, 2048 x 768: gate | up 282 us and down 164 at 4096 tokens (730 and 630 TOP/s), where the
-// 16-row-tile kernels took 480 and 260 and the quantizer between them 40; 80 and 41 at 512 tokens, before 92, 48
-// and 8 (a workgroup's life is 40 us there, 1.5 per compute unit).  The layer 823 -> 497 us and 156 -> 136.  Of that,
+// 16-row-tile kernels took 480 and 260 and the quantizer between them 40; 80 and 41 at 512 tokens (75 and 38 with the long
+// items first), before 92, 48 and 8 (a workgroup's life is 40 us there, 1.5 per compute unit).  The layer 823 -> 497 us and 156 -> 136.  Of that,
 // starting on the first unit's records while the others land, stores at 32-bit offsets and the two waves
 // of a SIMD half a phase apart with the one in its matrix instructions preferred: 556 -> 497 and 150 -> 136.
 #include <hip/hip_runtime.h>
@@ -288,7 +288,22 @@ __device__ __forceinline__ void issue_records(const MoeGemmParams& P, const uint
     }
 }
 
-template <bool GATE_UP>
+struct WorkItem {
+    int e, part, pos_begin, pos_end;
+};
+constexpr int kCusPerXcd = 32;
+constexpr int kOrderedItems = 4 * kCusPerXcd; // the longest run of an XCD's items that is put in order
+constexpr int kOrderedPerLane = (kOrderedItems + 63) / 64;
+
+__device__ __forceinline__ WorkItem work_item(const MoeGemmParams& P, int item) {
+    const int e = P.chunk_expert[item / P.parts]; // (an expert's items begin at parts * its first chunk)
+    const int chunk0 = P.chunks[e], n_chunks = P.chunks[e + 1] - chunk0;
+    const int local = item - chunk0 * P.parts, part = local / n_chunks, chunk = local - part * n_chunks;
+    const int begin = P.offsets[e] + chunk * kRows;
+    return {e, part, begin, min(P.offsets[e + 1], begin + kRows)};
+}
+
+template <bool GATE_UP, bool ORDERED>
 __global__ __launch_bounds__(64 * kWaves) void moe_gemm_q4k_kernel(MoeGemmParams P) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     __shared__ __attribute__((aligned(16))) uint32_t out_off[kRows]; // down: byte offsets of the output rows
@@ -300,12 +315,45 @@ __global__ __launch_bounds__(64 * kWaves) void moe_gemm_q4k_kernel(MoeGemmParams
     // runs: workgroups go to the XCDs round-robin, so a run is one XCD's, and the chunks that read the same weights
     // follow one another there and find them in its L2.
     const int items = P.chunks[P.n_experts] * P.parts, per_xcd = (items + 7) >> 3;
-    const int slot = (int)(blockIdx.x >> 3), item = (int)(blockIdx.x & 7) * per_xcd + slot;
-    if (slot >= per_xcd || item >= items) return; // uniform
-    const int e = P.chunk_expert[item / P.parts]; // (an expert's items begin at parts * its first chunk)
-    const int chunk0 = P.chunks[e], n_chunks = P.chunks[e + 1] - chunk0;
-    const int local = item - chunk0 * P.parts, part = local / n_chunks, chunk = local - part * n_chunks;
-    const int pos_begin = P.offsets[e] + chunk * kRows, pos_end = min(P.offsets[e + 1], pos_begin + kRows);
+    const int slot = (int)(blockIdx.x >> 3), first = (int)(blockIdx.x & 7) * per_xcd;
+    const int run = min(per_xcd, items - first); // items of this XCD
+    if (slot >= run) return; // uniform
+    // Where a run is a few items per compute unit, those of more than 32 pairs go first (every wave looks at the
+    // whole run, a lane per item) and the short ones fill in behind them.
+    WorkItem it;
+    if (ORDERED && run <= kOrderedItems) {
+        WorkItem mine[kOrderedPerLane];
+        uint64_t heavy[kOrderedPerLane], light[kOrderedPerLane];
+        int heavies = 0;
+#pragma unroll
+        for (int j = 0; j < kOrderedPerLane; j++) {
+            heavy[j] = light[j] = 0;
+            if (64 * j >= run) continue; // uniform
+            const bool exists = 64 * j + lane < run;
+            mine[j] = work_item(P, first + (exists ? 64 * j + lane : 0));
+            heavy[j] = __ballot(exists && mine[j].pos_end - mine[j].pos_begin > 32);
+            light[j] = __ballot(exists && mine[j].pos_end - mine[j].pos_begin <= 32);
+            heavies += __popcll(heavy[j]);
+        }
+        int rank = slot < heavies ? slot : slot - heavies;
+        bool found = false;
+#pragma unroll
+        for (int j = 0; j < kOrderedPerLane; j++) {
+            const uint64_t set = slot < heavies ? heavy[j] : light[j];
+            const int in_set = __popcll(set);
+            if (!found && rank < in_set) { // uniform
+                const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(set >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)set, 0));
+                const int at = __ffsll((unsigned long long)__ballot((set >> lane & 1) && below == rank)) - 1;
+                it.e = __builtin_amdgcn_readlane(mine[j].e, at), it.part = __builtin_amdgcn_readlane(mine[j].part, at);
+                it.pos_begin = __builtin_amdgcn_readlane(mine[j].pos_begin, at), it.pos_end = __builtin_amdgcn_readlane(mine[j].pos_end, at);
+                found = true;
+            }
+            rank -= in_set;
+        }
+    } else {
+        it = work_item(P, first + slot);
+    }
+    const int e = it.e, part = it.part, pos_begin = it.pos_begin, pos_end = it.pos_end;
     const int nrb = pos_end - pos_begin > 32 ? 2 : 1;
 
     const uint8_t* wbase0 = P.w0 + (int64_t)e * P.matrix_bytes;
@@ -396,16 +444,31 @@ __global__ void route_wide_rows_kernel(const float* __restrict__ logits, int64_t
     }
 }
 
-template <bool GATE_UP>
-hipError_t launch(const MoeGemmParams& P, int64_t max_chunks, hipStream_t stream) {
+template <bool GATE_UP, bool ORDERED>
+hipError_t launch_form(const MoeGemmParams& P, int64_t max_chunks, hipStream_t stream) {
     const size_t window = (size_t)P.k_units * kUnitLds, hbuf = GATE_UP ? (size_t)kRows * kHStride * 4 : 0;
     const size_t lds = window > hbuf ? window : hbuf;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_gemm_q4k_kernel<GATE_UP>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, kMaxUnits * kUnitLds);
+    auto fn = &moe_gemm_q4k_kernel<GATE_UP, ORDERED>;
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kMaxUnits * kUnitLds);
     if (e != hipSuccess) return e;
     const unsigned grid = (unsigned)((max_chunks * P.parts + 7) / 8 * 8);
-    moe_gemm_q4k_kernel<GATE_UP><<<grid, 64 * kWaves, lds, stream>>>(P);
+    fn<<<grid, 64 * kWaves, lds, stream>>>(P);
     return hipGetLastError();
+}
+
+// An item of up to 32 pairs is done in two thirds of the time of a longer one, and at one to three items per compute
+// unit a launch ends with whoever started a long one last.  The order pays where long items are about one per compute unit
+// and short ones follow: around the 22 to 32 pairs per expert at which a third to half of the experts have more than 32,
+// and around one chunk, where many experts spill a short second one.  us per layer (128 experts, top-8, 2048 x 768) in the
+// order of the experts / long ones first: 128.5 / 121 at 370 to 420 tokens, 145 / 137 at 512, 206 / 202 at 1000, 215 / 205 at
+// 1024.  Elsewhere finding the order costs up to two microseconds (200 tokens 113.5 / 114.5, 560 to 950 2 % more), and
+// from 80 pairs on an expert's chunks, set apart, read its weights again (1500 tokens 250 / 263, 4096 521 / 542).
+template <bool GATE_UP>
+hipError_t launch(const MoeGemmParams& P, int64_t pairs, int64_t max_chunks, hipStream_t stream) {
+    const int64_t per_expert = pairs / P.n_experts;
+    const bool ordered = ((per_expert >= 22 && per_expert <= 32) || (per_expert >= 61 && per_expert <= 68)) &&
+                         P.n_experts * P.parts > 8 * kCusPerXcd;
+    return ordered ? launch_form<GATE_UP, true>(P, max_chunks, stream) : launch_form<GATE_UP, false>(P, max_chunks, stream);
 }
 
 MoeGemmParams base_params(const QmmLayout& L, const int32_t* perm, const int32_t* offsets, const int32_t* chunks,
@@ -454,7 +517,7 @@ hipError_t qmm_launch_moe_route_wide_rows(const float* logits, int64_t t, int n_
 
 hipError_t qmm_launch_moe_gemm_gate_up(const QmmLayout& G, const void* gate, const void* up, const void* records, int top_k,
                                        const int32_t* perm, const int32_t* offsets, const int32_t* chunks,
-                                       const int32_t* chunk_expert, int n_experts, int64_t max_chunks, void* out_records,
+                                       const int32_t* chunk_expert, int n_experts, int64_t pairs, int64_t max_chunks, void* out_records,
                                        hipStream_t stream) {
     MoeGemmParams P = base_params(G, perm, offsets, chunks, chunk_expert, n_experts);
     P.w0 = (const uint8_t*)gate, P.w1 = (const uint8_t*)up;
@@ -462,16 +525,16 @@ hipError_t qmm_launch_moe_gemm_gate_up(const QmmLayout& G, const void* gate, con
     P.row_div = top_k;
     P.row_magic = top_k > 1 ? (uint32_t)((((uint64_t)1 << 32) / (uint32_t)top_k) + 1) : 0;
     P.parts = (int)(G.n / 256), P.out_units = P.parts;
-    return launch<true>(P, max_chunks, stream);
+    return launch<true>(P, pairs, max_chunks, stream);
 }
 
 hipError_t qmm_launch_moe_gemm_down(const QmmLayout& D, const void* down, const void* records, const int32_t* perm,
                                     const int32_t* offsets, const int32_t* chunks, const int32_t* chunk_expert, int n_experts,
-                                    int64_t max_chunks, float* y, hipStream_t stream) {
+                                    int64_t pairs, int64_t max_chunks, float* y, hipStream_t stream) {
     MoeGemmParams P = base_params(D, perm, offsets, chunks, chunk_expert, n_experts);
     P.w0 = P.w1 = (const uint8_t*)down;
     P.records = (const uint8_t*)records, P.out = y;
     P.row_div = 0;
     P.parts = (int)((D.n + 511) / 512);
-    return launch<false>(P, max_chunks, stream);
+    return launch<false>(P, pairs, max_chunks, stream);
 }

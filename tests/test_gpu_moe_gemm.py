@@ -57,6 +57,41 @@ def test_chunks_equal_the_tile_kernels(qa, oracle, E, hidden, inter, counts):
     assert np.linalg.norm(g - want) <= 1e-3 * np.linalg.norm(want)
 
 
+# long work items before short ones (22 to 32 and 61 to 68 pairs per expert, several items per compute unit): even and
+# skewed counts, experts with none, a run of an XCD's items longer than what is put in order
+@pytest.mark.parametrize("per_expert,skew", [(21, 0), (22, 0), (27, 9), (32, 20), (33, 5), (61, 0), (64, 30), (68, 60), (69, 3)])
+def test_long_items_first(qa, per_expert, skew):
+    import torch
+    from izwi_amd import capi
+    E, hidden, inter = 128, 1280, 768  # 384 items in both products where no expert has more than 64 pairs
+    rng = np.random.default_rng(4700 + per_expert)
+
+    def stack(n, k):
+        blocks = rng.integers(0, 256, size=(E * n * k // 256, 144), dtype=np.uint8)
+        blocks[:, :4] = (1e-3 * rng.uniform(0.5, 2.0, size=(blocks.shape[0], 2))).astype(np.float16).view(np.uint8)
+        return qa.QTensor.from_blocks(qa.GgmlDType.Q4K, blocks.reshape(-1), (E, n, k))
+
+    experts = qa.MoeExperts(stack(inter, hidden), stack(inter, hidden), stack(hidden, inter))
+    counts = np.full(E, per_expert)
+    for i in range(skew):  # from one expert to another, some until nothing is left
+        take = min(int(counts[2 * i]), int(rng.integers(1, per_expert + 1)) if i % 3 else per_expert)
+        counts[2 * i] -= take
+        counts[2 * i + 1] += take
+    t = int(counts.sum())
+    ids = torch.from_numpy(rng.permutation(np.repeat(np.arange(E, dtype=np.int32), counts)).reshape(t, 1)).cuda()
+    gen = torch.Generator(device="cuda").manual_seed(4701)
+    x = torch.randn(t, hidden, device="cuda", generator=gen)
+    wts = torch.rand(t, 1, device="cuda", generator=gen)
+    perm, offsets = qa.moe_sort(ids, E)
+    got = experts.forward(x, ids, wts, perm, offsets)
+    try:
+        capi.check(capi.lib().izwi_qmm_set_moe_expert_form(1))
+        tiles = experts.forward(x, ids, wts, perm, offsets)
+    finally:
+        capi.check(capi.lib().izwi_qmm_set_moe_expert_form(-1))
+    assert torch.equal(got.view(torch.int32), tiles.view(torch.int32))
+
+
 @pytest.mark.parametrize("t", [144, 500, 2100])  # 2100 * 8 pairs: beyond the one-workgroup sort
 def test_layer_equals_the_tile_kernels(qa, oracle, t):
     import torch
