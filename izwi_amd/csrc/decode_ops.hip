@@ -10,6 +10,11 @@
 //    each keeps running (max, sum, weighted value sum) per head and the splits are merged by a
 //    second small kernel.  Inside a workgroup 8 lanes share a cache row as 8 x 16 B pieces of
 //    every 128-byte segment (coalesced), 32 rows are in flight per workgroup.
+//
+// At one token what counts is the chain inside a launch: every kernel here requests all it will need before its first
+// reduction (a second trip to memory is 0.7 to 1 us) and reduces over lanes on the vector ALU (six shuffles through LDS
+// are 0.3 us).  A decode step of 28 layers of the 0.6B shapes at 300 positions 665 -> 624 us in a graph, of 8 layers of the
+// 8B shapes at 1501 418 -> 404, against norm weights, the new value and the splits' statistics and sums read where used.
 #include <hip/hip_runtime.h>
 
 #include <chrono>
@@ -111,9 +116,18 @@ __device__ __forceinline__ void st16(T* p, const float (&v)[kEC<T>]) {
     }
 }
 
+// Sum over the wave, in every lane: halves, rows of 16, then the lanes 8, 4, 2 and 1 away, on the vector ALU (six
+// shuffles through LDS were a third of a microsecond of a one-token kernel)
+template <int CTRL>
+__device__ __forceinline__ float dpp_f(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    v = qmm_add_lane16(qmm_add_lane32(v));
+    v += dpp_f<0x128>(v); // row_ror:8
+    v += dpp_f<0x124>(v); // row_ror:4 (lanes 8 apart are equal by now)
+    v += dpp_f<0x4E>(v);  // quad_perm [2,3,0,1]
+    v += dpp_f<0xB1>(v);  // quad_perm [1,0,3,2]
     return v;
 }
 
@@ -159,14 +173,21 @@ __global__ void rms_norm_kernel(NormParams<T> P) {
     T* y = first ? P.out_a + row * P.hidden : P.out_b + (row - P.rows_a) * P.hidden;
     const int tid = threadIdx.x, nt = blockDim.x;
     float sum = 0.0f;
-    float keepv[PER][EC];
+    float keepv[PER][EC], keepw[PER][EC]; // (the weights are requested with the row: one trip to memory, not two)
     float keep1[PER];
     const int nv = P.hidden / EC;
     if (VEC) {
 #pragma unroll
         for (int i = 0; i < PER; i++) {
             const int idx = tid + i * nt;
-            if (idx < nv) ld16<T>(x + (int64_t)idx * EC, keepv[i]);
+            if (idx < nv) {
+                ld16<T>(x + (int64_t)idx * EC, keepv[i]);
+                ld16<T>(w + (int64_t)idx * EC, keepw[i]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            const int idx = tid + i * nt;
 #pragma unroll
             for (int c = 0; c < EC; c++) {
                 if (idx >= nv) keepv[i][c] = 0.0f;
@@ -195,9 +216,8 @@ __global__ void rms_norm_kernel(NormParams<T> P) {
     for (int i = 0; i < (nt + 63) / 64; i++) total += partial[i];
     const float scale = 1.0f / sqrtf(total / (float)P.hidden + P.eps);
     if (VEC) {
-        auto finish = [&](int idx, const float (&v)[EC]) {
-            float ww[EC], o[EC];
-            ld16<T>(w + (int64_t)idx * EC, ww);
+        auto finish = [&](int idx, const float (&v)[EC], const float (&ww)[EC]) {
+            float o[EC];
 #pragma unroll
             for (int c = 0; c < EC; c++) o[c] = v[c] * scale * ww[c];
             if constexpr (REC != 0) {
@@ -210,12 +230,13 @@ __global__ void rms_norm_kernel(NormParams<T> P) {
 #pragma unroll
         for (int i = 0; i < PER; i++) {
             const int idx = tid + i * nt;
-            if (idx < nv) finish(idx, keepv[i]);
+            if (idx < nv) finish(idx, keepv[i], keepw[i]);
         }
         for (int idx = tid + PER * nt; idx < nv; idx += nt) {
-            float v[EC];
+            float v[EC], ww[EC];
             ld16<T>(x + (int64_t)idx * EC, v);
-            finish(idx, v);
+            ld16<T>(w + (int64_t)idx * EC, ww);
+            finish(idx, v, ww);
         }
     } else {
 #pragma unroll
@@ -464,10 +485,6 @@ __device__ __forceinline__ float merge_weight(float m, float mn) { return m == -
 
 // sum over the 8 lanes of a row group, in every lane of the group (two quad permutes and a
 // mirror of the half row: no LDS traffic)
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, 0xf, 0xf, false));
-}
 __device__ __forceinline__ float sum8(float v) {
     v += dpp_f<0xB1>(v);  // quad_perm [1,0,3,2]
     v += dpp_f<0x4E>(v);  // quad_perm [2,3,0,1]
@@ -512,46 +529,68 @@ __global__ __launch_bounds__(256) void attn_partial_kernel(AttnParams<T> P) {
     // runs beside the norm's
     float kr0[PREP ? E : 1], vr0[PREP ? E : 1];
     const bool first = PREP && p0 + slot < p1c;
-    if constexpr (PREP) {
-        if (first) load_row(p0 + slot, kr0, vr0);
-    }
+    const bool holds_new = PREP && pos >= p0 && pos < p1; // uniform
+    float vn[PREP ? E : 1], v_copy = 0.0f; // the new value: this lane's pieces, and the element it appends
 
     if constexpr (PREP) {
         // a wave per row (the group's q heads, then the kv head's new k), as qkv_prep_kernel does it
-        constexpr int half = HD / 2, NP = (half + 63) / 64;
-        for (int r = wave; r <= G; r += 4) {
+        // (all rows' values, the norm's weights and the rotation requested at once: one trip to memory)
+        constexpr int half = HD / 2, NP = (half + 63) / 64, RW = (G + 4) / 4; // rows a wave may hold
+        float x1[RW][NP], x2[RW][NP], w1[RW][NP], w2[RW][NP], cs[NP], sn[NP];
+#pragma unroll
+        for (int i = 0; i < NP; i++) {
+            const int p = min(lane + 64 * i, half - 1);
+            cs[i] = P.cos_sin[p], sn[i] = P.cos_sin[half + p];
+        }
+#pragma unroll
+        for (int k = 0; k < RW; k++) {
+            const int r = min(wave + 4 * k, G);
             const float* src = r < G ? reinterpret_cast<const float*>(P.q) + (int64_t)(h0 + r) * HD : P.k_new + (int64_t)kvh * HD;
             const float* w = P.qk_weight + (r < G ? 0 : HD);
-            float x1[NP], x2[NP];
-            float sum = 0.0f;
 #pragma unroll
             for (int i = 0; i < NP; i++) {
-                const int p = lane + 64 * i;
-                x1[i] = p < half ? src[p] : 0.0f;
-                x2[i] = p < half ? src[half + p] : 0.0f;
-                sum += x1[i] * x1[i] + x2[i] * x2[i];
+                const int p = min(lane + 64 * i, half - 1);
+                x1[k][i] = src[p], x2[k][i] = src[half + p];
+                w1[k][i] = w[p], w2[k][i] = w[half + p];
             }
+        }
+        if (holds_new) {
+            if (threadIdx.x < HD) v_copy = P.v_new[(int64_t)kvh * HD + threadIdx.x];
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                float t[EC];
+                ld16<float>(P.v_new + (int64_t)kvh * HD + 8 * EC * i + EC * j, t);
+#pragma unroll
+                for (int c = 0; c < EC; c++) vn[EC * i + c] = t[c];
+            }
+        }
+        if (first) load_row(p0 + slot, kr0, vr0);
+#pragma unroll
+        for (int k = 0; k < RW; k++) {
+            const int r = wave + 4 * k;
+            if (r > G) break; // uniform
+            float sum = 0.0f;
+#pragma unroll
+            for (int i = 0; i < NP; i++) sum += lane + 64 * i < half ? x1[k][i] * x1[k][i] + x2[k][i] * x2[k][i] : 0.0f;
             sum = wave_sum(sum);
             const float scale = 1.0f / sqrtf(sum / (float)HD + P.eps);
 #pragma unroll
             for (int i = 0; i < NP; i++) {
                 const int p = lane + 64 * i;
                 if (p < half) {
-                    const float n1 = x1[i] * scale * w[p], n2 = x2[i] * scale * w[half + p];
-                    const float c = P.cos_sin[p], sn = P.cos_sin[half + p];
-                    prep[r][p] = n1 * c - n2 * sn;
-                    prep[r][half + p] = n1 * sn + n2 * c;
+                    const float n1 = x1[k][i] * scale * w1[k][i], n2 = x2[k][i] * scale * w2[k][i];
+                    prep[r][p] = n1 * cs[i] - n2 * sn[i];
+                    prep[r][half + p] = n1 * sn[i] + n2 * cs[i];
                 }
             }
         }
         __syncthreads();
         // the workgroup whose positions end with the new one appends it to the caches; nobody reads
         // that cache row in this launch
-        if (pos >= p0 && pos < p1 && blockIdx.z == 0) {
-            for (int t = threadIdx.x; t < HD; t += 256) {
-                P.k_append[((int64_t)kvh * P.kv_capacity + pos) * HD + t] = prep[G][t];
-                P.v_append[((int64_t)kvh * P.kv_capacity + pos) * HD + t] = P.v_new[(int64_t)kvh * HD + t];
-            }
+        static_assert(HD <= 256);
+        if (holds_new && blockIdx.z == 0 && threadIdx.x < HD) {
+            P.k_append[((int64_t)kvh * P.kv_capacity + pos) * HD + threadIdx.x] = prep[G][threadIdx.x];
+            P.v_append[((int64_t)kvh * P.kv_capacity + pos) * HD + threadIdx.x] = v_copy;
         }
     }
 
@@ -623,16 +662,13 @@ __global__ __launch_bounds__(256) void attn_partial_kernel(AttnParams<T> P) {
     }
     if constexpr (PREP) {
         // the new position, last of its row group as it would be from the cache
-        if (pos >= p0 && pos < p1 && ((pos - p0) & 31) == slot) {
-            float kr[E], vr[E];
+        if (holds_new && ((pos - p0) & 31) == slot) {
+            float kr[E];
 #pragma unroll
             for (int i = 0; i < NI; i++)
 #pragma unroll
-                for (int c = 0; c < EC; c++) {
-                    kr[EC * i + c] = prep[G][8 * EC * i + EC * j + c];
-                    vr[EC * i + c] = P.v_new[(int64_t)kvh * HD + 8 * EC * i + EC * j + c];
-                }
-            accumulate(kr, vr);
+                for (int c = 0; c < EC; c++) kr[EC * i + c] = prep[G][8 * EC * i + EC * j + c];
+            accumulate(kr, vn);
         }
     }
     // Merge the 32 row groups of the workgroup: neighbours 8 lanes apart inside a 16-lane row by a
@@ -724,6 +760,40 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict
         for (int s = 0; s < splits; s++) a += base[(int64_t)s * (head_dim + 2) + d] * weight[s];
         st1(out + (int64_t)h * head_dim + d, a * inv);
     }
+}
+
+// The same for up to NS splits (at most 64), a thread per output element: statistics and sums of all splits requested
+// at once, the splits' weights worked out by every wave (lane s: split s) and broadcast through scalar registers.  One
+// trip to memory where the kernel above takes three one behind the other.  The same sums.
+template <typename T, int NS>
+__global__ __launch_bounds__(256) void attn_merge_few_kernel(const float* __restrict__ part, T* __restrict__ out, int splits, int head_dim) {
+    const int h = blockIdx.x, d = threadIdx.x, lane = d & 63; // (blockDim.x == head_dim)
+    const float* base = part + (int64_t)h * splits * (head_dim + 2);
+    const float2 stat = *reinterpret_cast<const float2*>(base + (int64_t)min(lane, splits - 1) * (head_dim + 2) + head_dim);
+    float v[NS];
+#pragma unroll
+    for (int s = 0; s < NS; s++) v[s] = base[(int64_t)min(s, splits - 1) * (head_dim + 2) + d];
+    const float m = lane < splits ? stat.x : -INFINITY;
+    const float mn = qmm_max_lane_rows(row16_max(m));
+    const float w = lane < splits ? merge_weight(m, mn) : 0.0f;
+    const float inv = 1.0f / wave_sum(lane < splits ? stat.y * w : 0.0f);
+    float a = 0.0f;
+#pragma unroll
+    for (int s = 0; s < NS; s++) asm volatile("" : "+v"(v[s])); // (or every load moves into its split's branch below)
+#pragma unroll
+    for (int s = 0; s < NS; s++)
+        if (s < splits) a += v[s] * __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), s)); // uniform
+    st1(out + (int64_t)h * head_dim + d, a * inv);
+}
+
+// (8, 16 and 32 are the requests in flight per thread; more splits are few-headed models on long caches)
+template <typename T>
+hipError_t launch_attn_merge(const float* part, T* out, int heads, int splits, int head_dim, hipStream_t stream) {
+    if (splits <= 8) attn_merge_few_kernel<T, 8><<<heads, head_dim, 0, stream>>>(part, out, splits, head_dim);
+    else if (splits <= 16) attn_merge_few_kernel<T, 16><<<heads, head_dim, 0, stream>>>(part, out, splits, head_dim);
+    else if (splits <= 32) attn_merge_few_kernel<T, 32><<<heads, head_dim, 0, stream>>>(part, out, splits, head_dim);
+    else attn_merge_kernel<T><<<heads, 256, 0, stream>>>(part, out, splits, head_dim);
+    return hipGetLastError();
 }
 
 template <typename T, int HD, bool PREP>
@@ -923,10 +993,7 @@ int decode_attention_impl(const T* q, const T* k, const T* v, int64_t num_heads,
                    : head_dim == 128 ? launch_attn_partial<T, 128>(P, g, grid, stream)
                                      : launch_attn_partial<T, 256>(P, g, grid, stream);
     OPS_TRY(e);
-    if (splits > 1) {
-        attn_merge_kernel<T><<<(unsigned)num_heads, 256, 0, stream>>>(P.part, P.out, (int)splits, (int)head_dim);
-        OPS_TRY(hipGetLastError());
-    }
+    if (splits > 1) OPS_TRY(launch_attn_merge<T>(P.part, P.out, (int)num_heads, (int)splits, (int)head_dim, stream));
     OPS_TRY(oo.finish(stream));
     return IZWI_QMM_OK;
 }

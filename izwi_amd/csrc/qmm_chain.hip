@@ -184,8 +184,7 @@ __global__ __launch_bounds__(64 * kChainWaves) void chain_kernel(ChainParams C) 
             float acc[1] = {0.0f};
             const int unit = min(wk * ph.s_units + (lane >> 4), k_units - 1);
             multiply_panel<QT, 1>(cur, l, unit, k_units, acc);
-            acc[0] += __shfl_xor(acc[0], 16);
-            acc[0] += __shfl_xor(acc[0], 32);
+            acc[0] = qmm_add_lane32(qmm_add_lane16(acc[0]));
             float* red = l.red + red_buf * (kChainWaves * 16);
             if (lane < 16) red[wave * 16 + lane] = acc[0];
             __syncthreads();

@@ -273,8 +273,7 @@ __device__ __forceinline__ void gemv_body(const GemvParams& P, int m_begin, int 
             // row-tile finished: combine the S units of a row, then the waves that split k
 #pragma unroll
             for (int mi = 0; mi < MT; mi++) {
-                acc[mi] += __shfl_xor(acc[mi], 16);
-                acc[mi] += __shfl_xor(acc[mi], 32);
+                acc[mi] = qmm_add_lane32(qmm_add_lane16(acc[mi]));
             }
             if (P.nwk == 1 && !GATED) {
                 const int row = rt * 16 + lane;
@@ -917,8 +916,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void moe_small_down_kernel(MoeSmall
     mask_panel<QT>(p, active);
     float acc[1] = {0.0f};
     multiply_panel<QT, 1>(p, l, min(lane >> 4, P.k_units - 1), P.k_units, acc);
-    acc[0] += __shfl_xor(acc[0], 16);
-    acc[0] += __shfl_xor(acc[0], 32);
+    acc[0] = qmm_add_lane32(qmm_add_lane16(acc[0]));
     if (lane < 16) ysum[wave * 16 + lane] = acc[0];
     __syncthreads();
     if (wave == 0 && lane < 16) {

@@ -62,6 +62,23 @@ __device__ __forceinline__ uint32_t qmm_pack_i8x4(int a, int b, int c, int d) {
     return __builtin_amdgcn_perm(cd, ab, 0x05040100u);
 }
 
+// v + v of the lane 32 (16) away, on the vector ALU (a shuffle is a trip through LDS); the same sum in both lanes
+__device__ __forceinline__ float qmm_add_lane32(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float qmm_add_lane16(float v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// the largest of the values of the lanes 16, 32 and 48 away and the lane's own (a NaN never wins)
+__device__ __forceinline__ float qmm_max_lane_rows(float v) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
 __device__ __forceinline__ float qmm_bf16_bits_to_f32(uint16_t b) {
     return __uint_as_float((uint32_t)b << 16);
 }

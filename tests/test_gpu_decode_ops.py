@@ -131,6 +131,18 @@ def test_rope_pair_shapes(qa, oracle, b, s, hq, hk, d):
     assert torch.allclose((qo ** 2).sum(-1), (dev(q) ** 2).sum(-1), rtol=1e-5)
 
 
+# 2, 8, 9, 16, 17, 32 and 33 splits of 32 positions: the edges of the merge kernels; every head width
+@pytest.mark.parametrize("kv_len", [33, 256, 257, 512, 513, 1024, 1056])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_decode_gqa_attention_splits(qa, oracle, d, kv_len):
+    heads, kv_heads = 4, 2
+    q = oracle.randn(21 + d, (1, heads, 1, d), std=3.0)
+    k, v = oracle.randn(22 + d, (1, kv_heads, kv_len, d)), oracle.randn(23 + d, (1, kv_heads, kv_len, d))
+    k[:, :, 40:] *= 0.5  # the first splits hold the maxima
+    got = qa.try_fused_decode_gqa_attention_with_kv_len(dev(q), dev(k), dev(v), heads, kv_heads, d, kv_len, d ** -0.5)
+    assert close(got, oracle.decode_gqa_attention(q, k, v, kv_len, d ** -0.5))
+
+
 @pytest.mark.parametrize("heads,kv_heads,d,kv_len,cap", [
     (32, 8, 128, 1, 1), (32, 8, 128, 17, 64), (32, 8, 128, 300, 512), (32, 8, 128, 2048, 2048),
     (32, 8, 128, 5000, 8192), (16, 8, 128, 777, 1000), (8, 8, 128, 100, 100), (24, 4, 128, 129, 200),
