@@ -722,6 +722,149 @@ __global__ __launch_bounds__(256) void attn_partial_kernel(AttnParams<T> P) {
     }
 }
 
+// The whole attention of a query head in one workgroup of W waves, 8 W cache rows at a time, NB of them per row group
+// requested ahead: one launch where the splits above take two.  Rows, lanes and arithmetic as above; the eight row
+// groups of a wave meet under the wave's maximum on the vector ALU, the waves in LDS.
+//
+// Bound by two trips to memory and, from 128 positions on, by what one compute unit reads (1 KB of f32 keys and values a
+// position at 110 GB/s).  A decode step in a graph, two launches / this (one launch and a quarter of this kernel's waves up
+// to 32 positions): 8 layers of 0.6B shapes 176 / 172 us at 11 positions, 190 / 174 at 34, 197 / 186 at 128, 200 / 198 at
+// 256, 205 / 207 at 300, 208 / 219 at 501; 4 layers of 8B shapes 216 / 206 at 26, 226 / 219 at 201, 226 / 222 at 301,
+// 229 / 230 at 501.  At 300 the launch it saves still counts where the host launches as slowly as the GPU runs (called from
+// Python 218 - 245 / 210), so the line is at 320 positions (and at a head per
+// compute unit: here every query head reads its cache rows for itself).  Two rows ahead on eight waves are the faster form up to 128
+// positions (128: 186 / 194), one on sixteen beyond (300: 210 / 207); two ahead on sixteen spill.
+constexpr int kOneLaunchPositions = 320;
+template <typename T, int HD, bool PREP, int W, int NB>
+__global__ __launch_bounds__(64 * W) void attn_one_kernel(AttnParams<T> P) {
+    static_assert(!PREP || std::is_same<T, float>::value, "the one-token step is built for f32");
+    constexpr int EC = kEC<T>, NI = HD / (8 * EC), E = EC * NI, kWaves = W, kRows = 8 * kWaves;
+    __shared__ __attribute__((aligned(16))) float red[kWaves][HD + 4]; // [.. HD): sums, [HD]: maximum, [HD + 1]: weight sum
+    __shared__ __attribute__((aligned(16))) float prep[PREP ? 3 : 1][PREP ? HD : 4]; // normed, rotated q head and k_new, v_new
+    const int h = blockIdx.x, kvh = h / P.group;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int j = lane & 7, slot = wave * 8 + (lane >> 3);
+    const int pos = P.kv_len - 1, rows = PREP ? pos : P.kv_len; // PREP: the new position is not in the cache yet
+    const T* kb = P.k + (int64_t)kvh * P.kv_capacity * HD + EC * j;
+    const T* vb = P.v + (int64_t)kvh * P.kv_capacity * HD + EC * j;
+    auto load_row = [&](int p, float (&kr)[E], float (&vr)[E]) {
+#pragma unroll
+        for (int i = 0; i < 2 * NI; i++) {
+            float t[EC];
+            ld16<T>((i < NI ? kb : vb) + (int64_t)p * HD + 8 * EC * (i % NI), t);
+#pragma unroll
+            for (int c = 0; c < EC; c++) (i < NI ? kr : vr)[EC * (i % NI) + c] = t[c];
+        }
+    };
+    float qr[E], kr[NB][E], vr[NB][E];
+    float v_copy = 0.0f;
+    auto first_rows = [&] {
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+            if (slot + b * kRows < rows) load_row(slot + b * kRows, kr[b], vr[b]);
+    };
+    if constexpr (PREP) {
+        constexpr int half = HD / 2;
+        static_assert(half <= 64, "a lane per rotated pair");
+        const int p = min(lane, half - 1);
+        const float* src = wave == 0 ? reinterpret_cast<const float*>(P.q) + (int64_t)h * HD : P.k_new + (int64_t)kvh * HD;
+        const float* w = P.qk_weight + (wave == 0 ? 0 : HD);
+        float x1 = 0.0f, x2 = 0.0f, w1 = 0.0f, w2 = 0.0f, cs = 0.0f, sn = 0.0f;
+        if (wave < 2) x1 = src[p], x2 = src[half + p], w1 = w[p], w2 = w[half + p], cs = P.cos_sin[p], sn = P.cos_sin[half + p];
+        if (threadIdx.x < HD) v_copy = P.v_new[(int64_t)kvh * HD + threadIdx.x];
+        first_rows();
+        if (wave < 2) { // as qkv_prep_kernel does it
+            const float sum = wave_sum(lane < half ? x1 * x1 + x2 * x2 : 0.0f);
+            const float scale = 1.0f / sqrtf(sum / (float)HD + P.eps);
+            const float n1 = x1 * scale * w1, n2 = x2 * scale * w2;
+            if (lane < half) prep[wave][lane] = n1 * cs - n2 * sn, prep[wave][half + lane] = n1 * sn + n2 * cs;
+        }
+        if (threadIdx.x < HD) prep[2][threadIdx.x] = v_copy;
+        __syncthreads();
+        // the first head of a kv head appends the new position; nobody reads that cache row in this launch
+        if (h == kvh * P.group && threadIdx.x < HD) {
+            P.k_append[((int64_t)kvh * P.kv_capacity + pos) * HD + threadIdx.x] = prep[1][threadIdx.x];
+            P.v_append[((int64_t)kvh * P.kv_capacity + pos) * HD + threadIdx.x] = v_copy;
+        }
+    } else {
+        first_rows();
+    }
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+        float t[EC];
+        if constexpr (PREP) {
+#pragma unroll
+            for (int c = 0; c < EC; c++) t[c] = prep[0][8 * EC * i + EC * j + c];
+        } else {
+            ld16<T>(P.q + (int64_t)h * HD + 8 * EC * i + EC * j, t);
+        }
+#pragma unroll
+        for (int c = 0; c < EC; c++) qr[EC * i + c] = t[c];
+    }
+    float m = -INFINITY, l = 0.0f, acc[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) acc[e] = 0.0f;
+    auto accumulate = [&](const float (&kr)[E], const float (&vr)[E]) {
+        float dot = 0.0f;
+#pragma unroll
+        for (int e = 0; e < E; e++) dot += qr[e] * kr[e];
+        const float s = sum8(dot) * P.scale;
+        const float mn = fmaxf(m, s), alpha = merge_weight(m, mn), pe = exp_neg(s - mn);
+        m = mn, l = l * alpha + pe;
+#pragma unroll
+        for (int e = 0; e < E; e++) acc[e] = acc[e] * alpha + pe * vr[e];
+    };
+    for (int p = slot; p < rows;) {
+#pragma unroll
+        for (int b = 0; b < NB; b++, p += kRows)
+            if (p < rows) {
+                accumulate(kr[b], vr[b]);
+                if (p + NB * kRows < rows) load_row(p + NB * kRows, kr[b], vr[b]);
+            }
+    }
+    if constexpr (PREP) {
+        if ((pos & (kRows - 1)) == slot) { // the new position, last of its row group as it would be from the cache
+#pragma unroll
+            for (int i = 0; i < NI; i++)
+#pragma unroll
+                for (int c = 0; c < EC; c++) {
+                    kr[0][EC * i + c] = prep[1][8 * EC * i + EC * j + c];
+                    vr[0][EC * i + c] = prep[2][8 * EC * i + EC * j + c];
+                }
+            accumulate(kr[0], vr[0]);
+        }
+    }
+    // (row groups 8, 16 and 32 lanes apart)
+    const float wm = qmm_max_lane_rows(fmaxf(m, dpp_f<0x128>(m))), ww = merge_weight(m, wm);
+    auto over_groups = [](float v) { return qmm_add_lane32(qmm_add_lane16(v + dpp_f<0x128>(v))); };
+    l = over_groups(l * ww);
+#pragma unroll
+    for (int e = 0; e < E; e++) acc[e] = over_groups(acc[e] * ww);
+    if (lane < 8) {
+#pragma unroll
+        for (int i = 0; i < NI; i++)
+#pragma unroll
+            for (int c = 0; c < EC; c += 4)
+                *reinterpret_cast<float4*>(&red[wave][8 * EC * i + EC * j + c]) =
+                    make_float4(acc[EC * i + c], acc[EC * i + c + 1], acc[EC * i + c + 2], acc[EC * i + c + 3]);
+        if (j == 0) red[wave][HD] = wm, red[wave][HD + 1] = l;
+    }
+    __syncthreads();
+    if (threadIdx.x < HD) {
+        const int d = threadIdx.x;
+        float mn = -INFINITY, a = 0.0f, lsum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kWaves; w++) mn = fmaxf(mn, red[w][HD]);
+#pragma unroll
+        for (int w = 0; w < kWaves; w++) {
+            const float g = merge_weight(red[w][HD], mn);
+            a += red[w][d] * g;
+            lsum += red[w][HD + 1] * g;
+        }
+        st1(P.out + (int64_t)h * HD + d, a * (1.0f / lsum));
+    }
+}
+
 // out[h] = merge of the splits' partial results.  One workgroup per head: the splits' maxima and
 // weights are worked out once, in parallel over the splits, and kept in LDS; the weighted sums
 // then run over the splits with their loads independent of each other (unrolled), not one memory
@@ -807,6 +950,19 @@ hipError_t launch_attn_partial_form(const AttnParams<T>& P, int g, dim3 grid, hi
         attn_partial_kernel<T, HD, 1, PREP><<<grid, 256, 0, stream>>>(P);
     }
     return hipGetLastError();
+}
+template <typename T, int HD, bool PREP>
+hipError_t launch_attn_one_form(const AttnParams<T>& P, hipStream_t stream) {
+    if (P.kv_len <= 128) attn_one_kernel<T, HD, PREP, 8, 2><<<P.heads, 512, 0, stream>>>(P);
+    else attn_one_kernel<T, HD, PREP, 16, 1><<<P.heads, 1024, 0, stream>>>(P);
+    return hipGetLastError();
+}
+template <typename T, int HD>
+hipError_t launch_attn_one(const AttnParams<T>& P, hipStream_t stream) {
+    if constexpr (std::is_same<T, float>::value) {
+        if (P.k_new) return launch_attn_one_form<T, HD, true>(P, stream);
+    }
+    return launch_attn_one_form<T, HD, false>(P, stream);
 }
 template <typename T, int HD>
 hipError_t launch_attn_partial(const AttnParams<T>& P, int g, dim3 grid, hipStream_t stream) {
@@ -981,6 +1137,11 @@ int decode_attention_impl(const T* q, const T* k, const T* v, int64_t num_heads,
         P.k_new = prep->k_new, P.v_new = prep->v_new, P.qk_weight = prep->qk_weight, P.cos_sin = prep->cos_sin;
         P.k_append = (float*)ki.dev, P.v_append = (float*)vi.dev;
         P.eps = prep->eps;
+    }
+    if (head_dim <= 128 && kv_len <= kOneLaunchPositions && num_heads <= n_cus) {
+        OPS_TRY((head_dim == 64 ? launch_attn_one<T, 64>(P, stream) : launch_attn_one<T, 128>(P, stream)));
+        OPS_TRY(oo.finish(stream));
+        return IZWI_QMM_OK;
     }
     QmmCallScope call; // the split partials stay this call's until the merge is queued
     if (splits > 1) {

@@ -131,8 +131,9 @@ def test_rope_pair_shapes(qa, oracle, b, s, hq, hk, d):
     assert torch.allclose((qo ** 2).sum(-1), (dev(q) ** 2).sum(-1), rtol=1e-5)
 
 
-# 2, 8, 9, 16, 17, 32 and 33 splits of 32 positions: the edges of the merge kernels; every head width
-@pytest.mark.parametrize("kv_len", [33, 256, 257, 512, 513, 1024, 1056])
+# one launch: row groups and waves without a position, one and two rounds of rows, the last length it takes; two: 11, 16,
+# 17, 32 and 33 splits of 32 positions, the edges of the merge kernels (2, 8 and 9 where head_dim is 256); f16 as well
+@pytest.mark.parametrize("kv_len", [1, 9, 64, 65, 128, 129, 256, 257, 320, 321, 512, 513, 1024, 1056])
 @pytest.mark.parametrize("d", [64, 128, 256])
 def test_decode_gqa_attention_splits(qa, oracle, d, kv_len):
     heads, kv_heads = 4, 2
@@ -141,6 +142,9 @@ def test_decode_gqa_attention_splits(qa, oracle, d, kv_len):
     k[:, :, 40:] *= 0.5  # the first splits hold the maxima
     got = qa.try_fused_decode_gqa_attention_with_kv_len(dev(q), dev(k), dev(v), heads, kv_heads, d, kv_len, d ** -0.5)
     assert close(got, oracle.decode_gqa_attention(q, k, v, kv_len, d ** -0.5))
+    q, k, v = (a.astype(np.float16).astype(np.float32) for a in (q, k, v))
+    got = qa.try_fused_decode_gqa_attention_with_kv_len(half(q), half(k), half(v), heads, kv_heads, d, kv_len, d ** -0.5)
+    assert close16(got, oracle.decode_gqa_attention(q, k, v, kv_len, d ** -0.5))
 
 
 @pytest.mark.parametrize("heads,kv_heads,d,kv_len,cap", [
@@ -233,7 +237,8 @@ def test_qk_norm_rope_append_equals_the_separate_hooks(qa, oracle, heads, kv_hea
 
 @pytest.mark.parametrize("heads,kv_heads,d,pos,cap", [
     (32, 8, 128, 0, 4), (32, 8, 128, 5, 9), (32, 8, 128, 300, 512), (32, 8, 128, 4095, 4096), (32, 8, 128, 1000, 1001),
-    (8, 8, 64, 77, 100), (6, 3, 256, 130, 200), (4, 4, 128, 64, 65),
+    (8, 8, 64, 77, 100), (6, 3, 256, 130, 200), (4, 4, 128, 64, 65), (16, 8, 128, 127, 256), (16, 8, 128, 128, 256),
+    (16, 8, 128, 319, 320), (16, 8, 128, 320, 512), (4, 2, 64, 255, 256), (320, 160, 64, 40, 41),
 ])
 def test_decode_attention_step_equals_prep_then_attention(qa, oracle, heads, kv_heads, d, pos, cap):
     """The one-call form (q/k norm, rotary and cache append inside the attention launch) against the two
