@@ -1663,7 +1663,10 @@ bool straight_line_fits(int64_t groups, int waves, int n_cus) {
 namespace {
 // The launch of a single-stage form whose workgroups quantize their own activations (P.ws: the f32 rows).
 // P is set up for the form on records; a workgroup gets more row tiles where its 16-lane groups would otherwise
-// have more than own_runs units to quantize.  hipErrorNotSupported where the quantizer launch is the cheaper
+// have more than own_runs units to quantize, or a compute unit several workgroups one after the other that each quantize
+// the same rows (gate | up of 2 x 3072 at k = 1024 and 64 rows: four row tiles of rows times 64 workgroups of six
+// waves instead of 192 of two, and the quantizer launch goes: 8 layers of 0.6B projections 348 -> 338 us in a graph, 480 -> 400
+// called from Python).  hipErrorNotSupported where the quantizer launch is the cheaper
 // one, by the activation bytes that a compute unit reads for its workgroups one after the other: a launch and the
 // gap behind it are 4 us, the loads, the quantizer's 140 instructions per (row, unit) and 16 lanes and a barrier in every workgroup
 // about 2 at 64 KB.  Layer of projections in a graph, us, with the launch / without at this limit / at 128 KB: 0.6B
@@ -1692,7 +1695,8 @@ hipError_t launch_own_quantizer(const QmmLayout& L0, MfmaParams P, int64_t x_k, 
         if (P.nwk * nwr > kMaxWaves) return hipErrorNotSupported;
         wgs = groups_of(nwr) * P.n_tiles;
         straight = full && (!q4k || straight_line_fits(wgs, P.nwk * nwr, n_cus));
-        if (items <= 4 * P.nwk * nwr * own_runs(q4k && !straight)) break;
+        if (items > 4 * P.nwk * nwr * own_runs(q4k && !straight)) continue;
+        if ((wgs + n_cus - 1) / n_cus * rows * x_k * 4 <= kOwnQuantizerBytes) break;
     }
     const int n_weights = std::max(P.n_weights, 1);
     if (P.n_weights == 0) P.rt_groups = (P.row_tiles + nwr - 1) / nwr;
@@ -1702,8 +1706,6 @@ hipError_t launch_own_quantizer(const QmmLayout& L0, MfmaParams P, int64_t x_k, 
         P.rt_groups = (int)groups;
     }
     P.nwr = nwr;
-    const int64_t rounds = (wgs + n_cus - 1) / n_cus;
-    if (rounds * rows * x_k * 4 > kOwnQuantizerBytes) return hipErrorNotSupported;
     const int waves = P.nwk * nwr;
     const size_t lds = std::max((size_t)P.window_units * unit_bytes(L0.dtype), (size_t)waves * 256 * 4);
     if (lds > 160 * 1024) return hipErrorNotSupported;

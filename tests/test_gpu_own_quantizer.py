@@ -14,6 +14,7 @@ pytestmark = pytest.mark.gpu
     (8, 16, 256, 5), (8, 3000, 1024, 16), (8, 40, 1056, 17), (8, 200, 96, 64), (8, 1024, 1024, 33), (8, 72, 2048, 8),
     (12, 24, 768, 5), (12, 500, 1024, 64), (12, 72, 1280, 33), (12, 4100, 1024, 15), (12, 40, 4096, 3), (12, 4096, 4096, 6),
     (14, 33, 512, 7), (14, 1000, 1024, 49), (14, 40, 4096, 3),
+    (8, 3072, 1024, 64), (8, 2050, 992, 49), (12, 6000, 1024, 40), (14, 3072, 768, 64),  # taller workgroups, alone and in the group
 ])
 def test_own_quantizer_equals_records(qa, oracle, dtype, n, k, m):  # noqa: F811
     import torch
