@@ -1,7 +1,7 @@
 // Prefill kernel: y[m, n] = x[m, k] * dequant(W)[n, k]^T with bf16 MFMA.
 //
 // A workgroup (8 waves, 4 x 2) owns a BM x BN output tile (256 x 256 when the
-// problem fills the chip with such tiles, 256 x 128 otherwise; few rows and small
+// problem fills the chip with such tiles, 256 x 192 or 256 x 128 otherwise; few rows and small
 // products take qmm_gemm_regb.hip); each wave a (BM/4) x (BN/2) sub-tile held in
 // v_mfma_f32_32x32x16_bf16 accumulators.
 // Per 64-wide k step the workgroup
@@ -95,9 +95,16 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
     // half the accumulators, and one issues while the other waits
     constexpr int THREADS = 64 * NW, WM = NW / 2;
     constexpr int MT = BM / WM / 32, NT = BN / 64;       // 32 x 32 accumulator tiles per wave
+    // 192 weight rows among 512 threads: at every k step one half of the waves stages rows 0 .. 127, two threads a row,
+    // and the other rows 128 .. 191, four threads a row; the halves change places with the parity of the staged step, so
+    // that each has its one and a half shares in the mean.  The two parities' rows are two sets of staging state, and
+    // the k loop exists twice, once for either half (H).
+    constexpr bool MIXED = BN == 192;
+    constexpr int NSET = MIXED ? 2 : 1;
     constexpr int XC = BM * 8 / THREADS;                 // 16-byte activation chunks per thread and k step
-    constexpr int TPR = THREADS / BN;                    // threads that share a weight row: 1, 2 or 4
+    constexpr int TPR = MIXED ? 2 : THREADS / BN;        // threads that share a weight row: 1, 2 or 4 (the fewest)
     constexpr bool Q6 = QT == QMM_Q6_K;
+    static_assert(!MIXED || (NW == 8 && BM == 256 && !Q6));
     static_assert(!Q6 || TPR == 2 || TPR == 4, "Q6_K is staged by two or four threads per weight row");
     constexpr int NCR = QT == QMM_Q4_K ? 2 : 4;          // 16-byte quant chunks per row and k step
     // Q6_K: a half unit (two k steps) shares its 64 bytes of low nibbles and 32 bytes of bit pairs.
@@ -106,10 +113,12 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
     // bit pairs, held for both steps
     constexpr int NGG = 4 / TPR, NQL = 4 * NGG, NQH = 4;
     constexpr int ND = Q6 ? NQL + NQH : 4 * NCR / TPR;   // the thread's run of quant dwords: 2 .. 16
-    constexpr int NC = Q6 ? NGG : ND >= 4 ? ND / 4 : 1; // loads per thread and k step (16 bytes; 8 if ND = 2)
-    constexpr int NP = 16 / TPR;                         // pieces of four weights per thread and k step
-    constexpr int GPK = MT * NT / 4; // groups of four MFMAs per k16 step
-    constexpr int NG = 4 * GPK;      // groups per k step: 16 (BM = 256) or 8 (BM = 128)
+    // of the thread at a step with tpr threads per row
+    auto nd_of = [](int tpr) constexpr { return Q6 ? NQL + NQH : 4 * NCR / tpr; };
+    auto nc_of = [](int tpr) constexpr { return Q6 ? NGG : 4 * NCR / tpr >= 4 ? NCR / tpr : 1; }; // loads per k step (16 bytes; 8 for two dwords)
+    constexpr int GS = NT == 3 ? 3 : 4; // MFMAs of a group
+    constexpr int GPK = MT * NT / GS;   // groups per k16 step
+    constexpr int NG = 4 * GPK;         // groups per k step: 16 (64 x 128 wave tiles) or 8
     constexpr int kStage = (BM + BN) * kRowStride;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
 
@@ -136,7 +145,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
     // before it is needed
     constexpr int XD = BN == 128 ? 2 : 1;
     u32x4 xr[XD][XC];
-    u32x4 w_hdr;      // header of the unit fetched last (Q6_K: its 16 signed scales)
+    u32x4 w_hdr[NSET]; // header of the unit fetched last (Q6_K: its 16 signed scales)
     uint32_t w_d = 0; // Q6_K: the dword with d of that unit
     // quant dwords of tile kt+1 (being dequantized) and tile kt+2 (in flight), by parity of the k step
     // (Q6_K: of the half unit; low nibbles first, bit pairs behind them)
@@ -155,28 +164,37 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
     // weights: thread t stages part t / BN of row n0 + t % BN (the lanes of a wave write 64
     // different rows of the padded LDS tile: no bank conflicts, and the part is wave-uniform);
     // rows past the matrix read the last row-tile (their output columns are never stored)
-    const int w_row = tid % BN, w_part = tid / BN;
     const int64_t rt0 = n0 >> 4;
     const int64_t rowtile_bytes = (int64_t)P.k_groups * P.panel_bytes;
     const uint8_t* w_tile = P.w + rt0 * rowtile_bytes;
     const uint32_t slot_bytes = (uint32_t)P.slots * 16u;
-    const uint32_t w_off =
-        (uint32_t)((min(rt0 + (w_row >> 4), P.row_tiles - 1) - rt0) * rowtile_bytes) + (uint32_t)(w_row & 15) * 16u;
     // part p holds dwords p ND .. p ND + ND - 1 of the row's quant dwords of a step (Q4_K: 8
     // dwords of nibbles, dword D = elements 4 D .. (low) and 32 + 4 D .. (high); Q8_0: 16 dwords of
     // int8): its first chunk (and, for half a chunk, the offset inside it) and its LDS position
-    const int w_d0 = Q6 ? 0 : w_part * ND;
-    const uint32_t w_off_q = w_off + (uint32_t)(w_d0 / 4) * slot_bytes + (uint32_t)(w_d0 % 4) * 4u;
+    const int w_part = tid / BN; // (not MIXED)
+    uint32_t w_off[NSET], w_off_q[NSET];
+    int w_lds[NSET], w_block[NSET]; // (w_block: the block of 32 elements, Q8_0)
+#pragma unroll
+    for (int p = 0; p < NSET; p++) {
+        const bool two = !MIXED || p == tid >> 8;
+        const int t = tid & 255;
+        const int row = !MIXED ? tid % BN : two ? t & 127 : 128 + (t & 63);
+        const int part = !MIXED ? w_part : two ? t >> 7 : t >> 6;
+        const int d0 = Q6 ? 0 : part * (two ? ND : ND / 2);
+        w_off[p] = (uint32_t)((min(rt0 + (row >> 4), P.row_tiles - 1) - rt0) * rowtile_bytes) + (uint32_t)(row & 15) * 16u;
+        w_off_q[p] = w_off[p] + (uint32_t)(d0 / 4) * slot_bytes + (uint32_t)(d0 % 4) * 4u;
+        w_lds[p] = (BM + row) * kRowStride + (Q6 ? 32 * part : d0 * 8);
+        w_block[p] = d0 / 8;
+    }
     // Q6_K: element 32 gg + l of the k step with nibble `nib` of half unit h is nibble `nib` of
     // ql[64 h + 32 gg + l] with bit pair 2 nib + gg of qh[32 h + l]; its 16-element group is
     // 4 (2 h + nib) + 2 gg + l / 16.  Part p: l = 16 lh .., lh = p & 1; gg = 0 and 1 (two parts)
     // or p / 2 (four parts)
     const int q6_lh = w_part & 1, q6_gg = TPR == 4 ? w_part >> 1 : 0;
-    const uint32_t w_off_ql = w_off + (uint32_t)(2 * q6_gg + q6_lh) * slot_bytes;
-    const uint32_t w_off_qh = w_off + (uint32_t)q6_lh * slot_bytes;
+    const uint32_t w_off_ql = w_off[0] + (uint32_t)(2 * q6_gg + q6_lh) * slot_bytes;
+    const uint32_t w_off_qh = w_off[0] + (uint32_t)q6_lh * slot_bytes;
     const int q6_pair_shift = 2 * q6_gg;
     const int q6_scale_shift = 8 * (2 * q6_gg + q6_lh); // of the step's four scale bytes
-    const int w_lds = (BM + w_row) * kRowStride + (Q6 ? 32 * w_part : w_d0 * 8);
     // load cursor: the unit whose chunks are fetched next (clamped to the last unit)
     int cur_us = u0 < P.k_units ? u0 % P.s : 0;
     uint32_t cur_kg_off = (uint32_t)((u0 < P.k_units ? u0 / P.s : 0) * P.panel_bytes);
@@ -207,9 +225,11 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
         }
     };
     auto w_load_hdr = [&]() {
-        w_hdr = *reinterpret_cast<const u32x4*>(w_tile + (cur_kg_off + (uint32_t)cur_us * 256u) + w_off);
+#pragma unroll
+        for (int p = 0; p < NSET; p++)
+            w_hdr[p] = *reinterpret_cast<const u32x4*>(w_tile + (cur_kg_off + (uint32_t)cur_us * 256u) + w_off[p]);
         if constexpr (Q6)
-            w_d = *reinterpret_cast<const uint32_t*>(w_tile + (cur_kg_off + (uint32_t)cur_us * 256u + 13u * slot_bytes) + w_off);
+            w_d = *reinterpret_cast<const uint32_t*>(w_tile + (cur_kg_off + (uint32_t)cur_us * 256u + 13u * slot_bytes) + w_off[0]);
     };
     // Q6_K: the low nibbles of the thread's group c (HI = 0) or its bit pairs (HI = 1, c = 0) of half
     // unit HALF of the cursor's unit
@@ -222,37 +242,45 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
         constexpr int o = hi ? NQL : 0;
         wq[half][o + 4 * c] = v.x, wq[half][o + 4 * c + 1] = v.y, wq[half][o + 4 * c + 2] = v.z, wq[half][o + 4 * c + 3] = v.w;
     };
-    auto w_load_q = [&](int sub, int c) {
+    auto w_load_q = [&](auto SUB, auto TPRS, int c) {
+        constexpr int sub = decltype(SUB)::value, par = sub & 1, set = MIXED ? par : 0;
         const uint8_t* src =
-            w_tile + (cur_kg_off + (uint32_t)cur_us * 256u + (uint32_t)(1 + sub * NCR + c) * slot_bytes) + w_off_q;
-        if constexpr (ND >= 4) {
+            w_tile + (cur_kg_off + (uint32_t)cur_us * 256u + (uint32_t)(1 + sub * NCR + c) * slot_bytes) + w_off_q[set];
+        if constexpr (nd_of(decltype(TPRS)::value) >= 4) {
             const u32x4 v = *reinterpret_cast<const u32x4*>(src);
-            wq[sub & 1][4 * c] = v.x, wq[sub & 1][4 * c + 1] = v.y, wq[sub & 1][4 * c + 2] = v.z, wq[sub & 1][4 * c + 3] = v.w;
+            wq[par][4 * c] = v.x, wq[par][4 * c + 1] = v.y, wq[par][4 * c + 2] = v.z, wq[par][4 * c + 3] = v.w;
         } else {
             const uint2 v = *reinterpret_cast<const uint2*>(src);
-            wq[sub & 1][0] = v.x, wq[sub & 1][1] = v.y;
+            wq[par][0] = v.x, wq[par][1] = v.y;
         }
     };
     // header of the unit being staged, unpacked once per unit
-    float hd = 0, hdmin = 0;                            // Q4_K: d, dmin
-    uint32_t sc_lo = 0, sc_hi = 0, mn_lo = 0, mn_hi = 0; // Q4_K: 8 scale bytes, 8 min bytes; Q8_0: 8 f16 scales
+    struct Unpacked {
+        float hd = 0, hdmin = 0;                             // Q4_K: d, dmin
+        uint32_t sc_lo = 0, sc_hi = 0, mn_lo = 0, mn_hi = 0; // Q4_K: 8 scale bytes, 8 min bytes; Q8_0: 8 f16 scales
+    } hu[NSET];
     auto w_unpack = [&]() {
-        if (QT == QMM_Q4_K) {
-            hd = qmm_f16_bits_to_f32((uint16_t)(w_hdr.x & 0xffffu));
-            hdmin = -qmm_f16_bits_to_f32((uint16_t)(w_hdr.x >> 16));
-            qmm_unpack_q4k_scales(w_hdr.y, w_hdr.z, w_hdr.w, sc_lo, sc_hi, mn_lo, mn_hi);
-        } else if (Q6) {
-            hd = qmm_f16_bits_to_f32((uint16_t)(w_d & 0xffffu));
-            sc_lo = w_hdr.x, sc_hi = w_hdr.y, mn_lo = w_hdr.z, mn_hi = w_hdr.w; // scales 4 sub .. 4 sub + 3 in dword sub
-        } else {
-            sc_lo = w_hdr.x, sc_hi = w_hdr.y, mn_lo = w_hdr.z, mn_hi = w_hdr.w;
+#pragma unroll
+        for (int p = 0; p < NSET; p++) {
+            Unpacked& u = hu[p];
+            const u32x4 h = w_hdr[p];
+            if (QT == QMM_Q4_K) {
+                u.hd = qmm_f16_bits_to_f32((uint16_t)(h.x & 0xffffu));
+                u.hdmin = -qmm_f16_bits_to_f32((uint16_t)(h.x >> 16));
+                qmm_unpack_q4k_scales(h.y, h.z, h.w, u.sc_lo, u.sc_hi, u.mn_lo, u.mn_hi);
+            } else {
+                if (Q6) u.hd = qmm_f16_bits_to_f32((uint16_t)(w_d & 0xffffu));
+                u.sc_lo = h.x, u.sc_hi = h.y, u.mn_lo = h.z, u.mn_hi = h.w; // (Q6_K: scales 4 sub .. 4 sub + 3 in dword sub)
+            }
         }
     };
     // scales of the tile being staged
     float sa = 0, ba = 0, sb = 0, bb = 0; // Q4_K: (d1, -m1, d2, -m2); Q8_0: (dA, -128 dA, dB, -128 dB)
     float sw = 0, bw = 0;                 // Q8_0, two threads per row: the scale of this thread's block
     auto w_scales = [&](auto SUB) {
-        constexpr int g = decltype(SUB)::value;
+        constexpr int g = decltype(SUB)::value, set = MIXED ? g & 1 : 0;
+        const float hd = hu[set].hd, hdmin = hu[set].hdmin;
+        const uint32_t sc_lo = hu[set].sc_lo, sc_hi = hu[set].sc_hi, mn_lo = hu[set].mn_lo, mn_hi = hu[set].mn_hi;
         if (QT == QMM_Q4_K) {
             const uint32_t sc = g < 2 ? sc_lo : sc_hi, mn = g < 2 ? mn_lo : mn_hi;
             sa = hd * ubyte_f32<(2 * g) & 3>(sc);
@@ -274,7 +302,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
             sb = qmm_f16_bits_to_f32((uint16_t)(pair >> 16));
             ba = -128.0f * sa;
             bb = -128.0f * sb;
-            sw = (w_d0 / 8) ? sb : sa; // the thread's dwords lie in one block of 8 dwords
+            sw = w_block[set] ? sb : sa; // the thread's dwords lie in one block of 8 dwords
             bw = -128.0f * sw;
         }
     };
@@ -285,7 +313,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
     // written as 16 bytes
     auto w_piece = [&](auto NSUB, auto HH, uint8_t* stage) {
         constexpr int par = decltype(NSUB)::value & 1, h = decltype(HH)::value;
-        uint8_t* row = stage + w_lds;
+        uint8_t* row = stage + w_lds[MIXED ? par : 0];
         if constexpr (Q6) {
             // dword h % 4 of the thread's 16 byte positions in its group h / 4: four elements
             constexpr int half = decltype(NSUB)::value >> 1, nib = par, gi = h / 4, dw = h % 4;
@@ -331,10 +359,10 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
     // part gi of GPK: read while group gi runs, used from group gi of the next k16 step on
     auto read_frags = [&](const uint8_t* stage, int kk, int set, auto PART) {
         constexpr int part = decltype(PART)::value;
-        constexpr int jb = GPK == 1 ? 0 : NT == 4 ? (part < GPK / 2 ? part * 2 * NT / GPK : NT) : (part == 0 ? 0 : NT);
-        constexpr int je = GPK == 1 ? NT : NT == 4 ? (part < GPK / 2 ? (part + 1) * 2 * NT / GPK : NT) : NT;
-        constexpr int ib = GPK == 1 ? 0 : NT == 4 ? (part < GPK / 2 ? 0 : (part - GPK / 2) * 2 * MT / GPK) : (part == 0 ? 0 : MT / 2);
-        constexpr int ie = GPK == 1 ? MT : NT == 4 ? (part < GPK / 2 ? 0 : (part - GPK / 2 + 1) * 2 * MT / GPK) : (part == 0 ? MT / 2 : MT);
+        constexpr int jb = GPK == 1 ? 0 : NT == 3 ? (part == 0 ? 0 : NT) : NT == 4 ? (part < GPK / 2 ? part * 2 * NT / GPK : NT) : (part == 0 ? 0 : NT);
+        constexpr int je = GPK == 1 ? NT : NT == 3 ? NT : NT == 4 ? (part < GPK / 2 ? (part + 1) * 2 * NT / GPK : NT) : NT;
+        constexpr int ib = GPK == 1 ? 0 : NT == 3 ? 0 : NT == 4 ? (part < GPK / 2 ? 0 : (part - GPK / 2) * 2 * MT / GPK) : (part == 0 ? 0 : MT / 2);
+        constexpr int ie = GPK == 1 ? MT : NT == 3 ? (part == 0 ? 0 : MT) : NT == 4 ? (part < GPK / 2 ? 0 : (part - GPK / 2 + 1) * 2 * MT / GPK) : (part == 0 ? MT / 2 : MT);
 #pragma unroll
         for (int j = jb; j < je; j++)
             fb[set][j] = *reinterpret_cast<const bf16x8*>(stage + frag_w + j * 32 * kRowStride + kk * 32);
@@ -349,8 +377,12 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
     // writes to the other one, the first fragments of step kt+1 are read while the last quarter
     // of the MFMAs runs.  Steps past the workgroup's last one stage and fetch the (clamped) last
     // tile again: nobody uses it.
-    auto k_step = [&](int unit, auto SUB) {
+    // H: the thread's half of the waves (MIXED); threads per row of the tile staged (s) and fetched (l) meanwhile
+    auto k_step = [&](int unit, auto SUB, auto H) {
         constexpr int sub = decltype(SUB)::value;
+        constexpr int tprs = !MIXED || ((sub + 1) & 1) == decltype(H)::value ? TPR : 2 * TPR;
+        constexpr int tprl = !MIXED || (sub & 1) == decltype(H)::value ? TPR : 2 * TPR;
+        constexpr int NP = 16 / tprs, NC = nc_of(tprl); // pieces of four weights and loads per thread
         constexpr int nsub = (sub + 1) & 3, lsub = (sub + 2) & 3; // sub-block staged / fetched meanwhile
         const int kt = unit * 4 + sub;
         const uint8_t* cur = smem + (sub & 1) * kStage;
@@ -363,8 +395,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
                 // the operands of the next k16 step (of the next k step in the last quarter)
                 read_frags(kk < 3 ? cur : next, (kk + 1) & 3, (kk + 1) & 1, GI);
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const int t = gi * 4 + q, i = t / NT, j = t % NT;
+                for (int q = 0; q < GS; q++) {
+                    const int t = gi * GS + q, i = t / NT, j = t % NT;
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[kk & 1][i], fb[kk & 1][j], acc[i][j], 0, 0, 0);
                 }
                 // group g's share of staging tile kt+1 (the thread's NP weight pieces and XC
@@ -393,23 +425,23 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
                 if (g == 1 && sub == (Q6 ? 1 : 2)) advance_cursor();
                 if (g == 1 && sub == 2) w_load_hdr();
                 if (g >= 2 && g < 2 + NC) {
-                    if constexpr (!Q6) w_load_q(lsub, g - 2);
+                    if constexpr (!Q6) w_load_q(std::integral_constant<int, lsub>{}, std::integral_constant<int, tprl>{}, g - 2);
                     else if constexpr (sub % 2 == 1 || g == 2)
                         w_load_q6(std::integral_constant<int, (sub == 0 || sub == 3) ? 1 : 0>{},
                                   std::integral_constant<int, (sub % 2 == 0) ? 1 : 0>{}, g - 2);
                 }
                 // inside the group: one MFMA, then its share of the other instructions, so
                 // the matrix pipe is fed while they issue
-                constexpr int valu = (Q6 ? 4 : 3) * (p1 - p0) + (g == 0 ? 4 : 1);
-                constexpr int reads = GPK == 1 ? NT + MT : NT == 4 ? (gi < GPK / 2 ? 2 * NT / GPK : 2 * MT / GPK) : (gi == 0 ? NT + MT / 2 : MT / 2);
+                constexpr int valu = (Q6 || GS == 3 ? 4 : 3) * (p1 - p0) + (g == 0 ? 4 : 1);
+                constexpr int reads = GPK == 1 ? NT + MT : NT == 3 ? (gi == 0 ? NT : MT) : NT == 4 ? (gi < GPK / 2 ? 2 * NT / GPK : 2 * MT / GPK) : (gi == 0 ? NT + MT / 2 : MT / 2);
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
+                for (int q = 0; q < GS; q++) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                     __builtin_amdgcn_sched_group_barrier(0x002, valu, 0);
                     if (q == 0) __builtin_amdgcn_sched_group_barrier(0x100, (reads + 1) / 2, 0);
                     if (q == 1) __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
                     if (q == 2) __builtin_amdgcn_sched_group_barrier(0x100, reads / 2, 0);
-                    if (q == 3) __builtin_amdgcn_sched_group_barrier(0x200, 3, 0);
+                    if (q == GS - 1) __builtin_amdgcn_sched_group_barrier(0x200, 3, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             });
@@ -423,36 +455,45 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
 
     if (u0 < u1) {
         // ---- prologue: tile (u0, 0) -> stage 0, tile (u0, 1) -> registers
+        auto run = [&](auto H) {
+            constexpr int tpr0 = !MIXED || decltype(H)::value == 0 ? TPR : 2 * TPR, tpr1 = !MIXED || decltype(H)::value == 1 ? TPR : 2 * TPR;
 #pragma unroll
-        for (int i = 0; i < XC; i++) x_load(u0 * 4, 0, i);
-        w_load_hdr();
+            for (int i = 0; i < XC; i++) x_load(u0 * 4, 0, i);
+            w_load_hdr();
 #pragma unroll
-        for (int c = 0; c < NC; c++) {
-            if constexpr (Q6) {
-                w_load_q6(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, c);
-                if (c == 0) w_load_q6(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{}, 0);
-            } else {
-                w_load_q(0, c);
+            for (int c = 0; c < nc_of(tpr0); c++) {
+                if constexpr (Q6) {
+                    w_load_q6(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, c);
+                    if (c == 0) w_load_q6(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{}, 0);
+                } else {
+                    w_load_q(std::integral_constant<int, 0>{}, std::integral_constant<int, tpr0>{}, c);
+                }
             }
-        }
 #pragma unroll
-        for (int i = 0; i < XC; i++) x_write(u0 * 4, 0, i, smem);
-        w_unpack();
-        w_scales(std::integral_constant<int, 0>{});
-        static_for<NP>([&](auto HH) { w_piece(std::integral_constant<int, 0>{}, HH, smem); });
+            for (int i = 0; i < XC; i++) x_write(u0 * 4, 0, i, smem);
+            w_unpack();
+            w_scales(std::integral_constant<int, 0>{});
+            static_for<16 / tpr0>([&](auto HH) { w_piece(std::integral_constant<int, 0>{}, HH, smem); });
 #pragma unroll
-        for (int d = 1; d <= XD; d++)
+            for (int d = 1; d <= XD; d++)
 #pragma unroll
-            for (int i = 0; i < XC; i++) x_load(u0 * 4 + d, d % XD, i);
+                for (int i = 0; i < XC; i++) x_load(u0 * 4 + d, d % XD, i);
 #pragma unroll
-        for (int c = 0; c < NC; c++) {
-            if constexpr (Q6) w_load_q6(std::integral_constant<int, 1>{}, std::integral_constant<int, 0>{}, c);
-            else w_load_q(1, c);
-        }
-        __syncthreads();
-        static_for<GPK>([&](auto PART) { read_frags(smem, 0, 0, PART); });
+            for (int c = 0; c < nc_of(tpr1); c++) {
+                if constexpr (Q6) w_load_q6(std::integral_constant<int, 1>{}, std::integral_constant<int, 0>{}, c);
+                else w_load_q(std::integral_constant<int, 1>{}, std::integral_constant<int, tpr1>{}, c);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            static_for<GPK>([&](auto PART) { read_frags(smem, 0, 0, PART); });
 
-        for (int unit = u0; unit < u1; unit++) static_for<4>([&](auto SUB) { k_step(unit, SUB); });
+            for (int unit = u0; unit < u1; unit++) static_for<4>([&](auto SUB) { k_step(unit, SUB, H); });
+        };
+        if constexpr (MIXED) {
+            if (__builtin_amdgcn_readfirstlane(wave) < NW / 2) run(std::integral_constant<int, 0>{});
+            else run(std::integral_constant<int, 1>{});
+        } else {
+            run(std::integral_constant<int, 0>{});
+        }
     }
 
     // a split-k slice stores f32 into its own [m, n] plane of the workspace
@@ -575,19 +616,19 @@ hipError_t launch_tile(GemmParams P, int slices, hipStream_t stream) {
 // second kernel adds the slices in order).  Costs are in k steps of a 256 x 256 tile
 // (relative tile efficiencies measured on the 8B shapes).
 struct GemmPlan {
-    int bm, bn;          // tile of the only / the second launch: 256 x 256 or 256 x 128
+    int bm, bn;          // tile of the only / the second launch: 256 x 256, 256 x 192 (Q4_K, Q8_0) or 256 x 128
     int slices;          // split along k
     int64_t full_cols;   // > 0: first a launch of 256 x 256 tiles over this many 256-column strips
 };
 
 // IZWI_QMM_GEMM_TILE="bm,bn,slices" (tuning aid) replaces the plan, at every number of rows, and the choice of
-// the few-row kernel: bm = 256, bn in {128, 256}.
+// the few-row kernel: bm = 256, bn in {128, 192, 256}.
 bool forced_plan(GemmPlan& plan) {
     static const GemmPlan forced = [] {
         GemmPlan p{0, 0, 1, 0};
         const char* e = getenv("IZWI_QMM_GEMM_TILE");
         if (e && sscanf(e, "%d,%d,%d", &p.bm, &p.bn, &p.slices) >= 2) {
-            const bool ok = p.bm == 256 && (p.bn == 128 || p.bn == 256) && p.slices >= 1 && p.slices <= 8;
+            const bool ok = p.bm == 256 && (p.bn == 128 || p.bn == 192 || p.bn == 256) && p.slices >= 1 && p.slices <= 8;
             if (!ok) p.bm = p.bn = 0, p.slices = 1;
         }
         return p;
@@ -597,13 +638,25 @@ bool forced_plan(GemmPlan& plan) {
     return true;
 }
 
-GemmPlan plan_gemm(int64_t m, int64_t n, int k_steps, int n_cus, bool group = false) {
+// 192-column tiles of the members; 0 for the types that have no such tile
+int64_t tiles_of_192(const QmmLayout* const* layouts, int n_weights) {
+    int64_t t = 0;
+    for (int i = 0; i < n_weights; i++) t += (layouts[i]->n + 191) / 192;
+    return n_weights > 0 && layouts[0]->dtype == QMM_Q6_K ? 0 : t;
+}
+
+GemmPlan plan_gemm(int64_t m, int64_t n, int k_steps, int n_cus, int64_t tiles_n192, bool group = false) {
     const double kQ128 = 0.76; // relative rate of a half-size tile
+    // A 256 x 192 tile takes 0.79 of the time of a whole one.  Where whole tiles would fill the last round badly, us per call (2 x
+    // 12288 x 4096, Q4_K): 112 -> 105 at 500 rows (192 whole tiles, 256 of these), 212 -> 182 at 640 (288, 384), 217 ->
+    // 197 at 1000 (384, 512), 330 -> 290 at 1400 (576, 768); 2 x 3072 x 1024 42 -> 37 at 2048 rows (192, 256).
+    const double kCost192 = 0.79;
     const int hm = 256, hn = 128;
     {
         GemmPlan forced;
         if (forced_plan(forced)) {
             while (forced.slices > 1 && k_steps / 4 < forced.slices) forced.slices /= 2;
+            if (forced.bn == 192 && tiles_n192 == 0) forced.bn = 256;
             return forced;
         }
     }
@@ -615,6 +668,7 @@ GemmPlan plan_gemm(int64_t m, int64_t n, int k_steps, int n_cus, bool group = fa
         if (cost < 0.97 * best_cost) best = p, best_cost = cost;
     };
     consider({hm, hn, 1, 0}, rounds(tiles(hm, hn, n)) * k_steps * 0.5 / kQ128);
+    if (tiles_n192 > 0) consider({256, 192, 1, 0}, rounds((m + 255) / 256 * tiles_n192) * k_steps * kCost192);
     // whole rounds of 256 x 256 tiles first, the remaining columns as half-size tiles
     const int64_t tiles_m256 = (m + 255) / 256, cols256 = (n + 255) / 256;
     const int64_t full_cols = (tiles_m256 * cols256 / n_cus) * n_cus / tiles_m256;
@@ -636,7 +690,7 @@ GemmPlan plan_gemm(int64_t m, int64_t n, int k_steps, int n_cus, bool group = fa
 
 template <int QT>
 hipError_t launch_qt(const GemmParams& P0, int n_cus, hipStream_t stream) {
-    const GemmPlan plan = plan_gemm(P0.m, P0.n, P0.k_units * 4, n_cus);
+    const GemmPlan plan = plan_gemm(P0.m, P0.n, P0.k_units * 4, n_cus, QT == QMM_Q6_K ? 0 : (P0.n + 191) / 192);
     GemmParams P = P0;
     P.n_begin = 0;
     P.n_end = P0.n;
@@ -647,6 +701,9 @@ hipError_t launch_qt(const GemmParams& P0, int n_cus, hipStream_t stream) {
         if (e != hipSuccess) return e;
         P.n_begin = P.n_end;
         P.n_end = P0.n;
+    }
+    if constexpr (QT != QMM_Q6_K) {
+        if (plan.bn == 192) return launch_tile<QT, 256, 192>(P, plan.slices, stream);
     }
     return plan.bn == 256 ? launch_tile<QT, 256, 256>(P, plan.slices, stream) : launch_tile<QT, 256, 128>(P, plan.slices, stream);
 }
@@ -660,8 +717,8 @@ int64_t group_columns(const QmmLayout* const* layouts, int n_weights) {
 }
 
 template <int QT>
-hipError_t launch_group_qt(GemmParams P, int64_t n_planned, int n_cus, hipStream_t stream) {
-    const GemmPlan plan = plan_gemm(P.m, n_planned, P.k_units * 4, n_cus, true);
+hipError_t launch_group_qt(GemmParams P, int64_t n_planned, int64_t tiles_n192, int n_cus, hipStream_t stream) {
+    const GemmPlan plan = plan_gemm(P.m, n_planned, P.k_units * 4, n_cus, tiles_n192, true);
     if (plan.slices > 1) {
         if (P.partial == nullptr) return hipErrorInvalidValue;
         float* base = P.partial;
@@ -669,6 +726,9 @@ hipError_t launch_group_qt(GemmParams P, int64_t n_planned, int n_cus, hipStream
             P.partial_v[i] = base;
             base += (size_t)plan.slices * (size_t)P.m * (size_t)P.nv[i];
         }
+    }
+    if constexpr (QT != QMM_Q6_K) {
+        if (plan.bn == 192) return launch_tile<QT, 256, 192>(P, plan.slices, stream);
     }
     return plan.bn == 256 ? launch_tile<QT, 256, 256>(P, plan.slices, stream) : launch_tile<QT, 256, 128>(P, plan.slices, stream);
 }
@@ -696,7 +756,8 @@ size_t qmm_gemm_group_workspace_bytes(const QmmLayout* const* layouts, int n_wei
         for (int i = 0; i < n_weights; i++) total += qmm_gemm_plane_bytes(*layouts[i]);
         return total;
     }
-    const GemmPlan plan = plan_gemm(m, group_columns(layouts, n_weights), (int)layouts[0]->k_units * 4, n_cus, true);
+    const GemmPlan plan = plan_gemm(m, group_columns(layouts, n_weights), (int)layouts[0]->k_units * 4, n_cus,
+                                    tiles_of_192(layouts, n_weights), true);
     if (plan.slices <= 1) return 0;
     size_t total = 0;
     for (int i = 0; i < n_weights; i++) total += (size_t)plan.slices * (size_t)m * (size_t)layouts[i]->n * sizeof(float);
@@ -747,10 +808,10 @@ hipError_t qmm_launch_gemm_bf16_multi(const QmmLayout* const* layouts, const voi
         P.partial_v[i] = nullptr;
         P.tn_end[i] = 0;
     }
-    const int64_t n_planned = group_columns(layouts, n_weights);
-    if (L0.dtype == QMM_Q6_K) return launch_group_qt<QMM_Q6_K>(P, n_planned, n_cus, stream);
-    return L0.dtype == QMM_Q4_K ? launch_group_qt<QMM_Q4_K>(P, n_planned, n_cus, stream)
-                                : launch_group_qt<QMM_Q8_0>(P, n_planned, n_cus, stream);
+    const int64_t n_planned = group_columns(layouts, n_weights), n192 = tiles_of_192(layouts, n_weights);
+    if (L0.dtype == QMM_Q6_K) return launch_group_qt<QMM_Q6_K>(P, n_planned, n192, n_cus, stream);
+    return L0.dtype == QMM_Q4_K ? launch_group_qt<QMM_Q4_K>(P, n_planned, n192, n_cus, stream)
+                                : launch_group_qt<QMM_Q8_0>(P, n_planned, n192, n_cus, stream);
 }
 
 size_t qmm_gemm_workspace_bytes(const QmmLayout& L, int64_t m, int n_cus) {
@@ -759,7 +820,7 @@ size_t qmm_gemm_workspace_bytes(const QmmLayout& L, int64_t m, int n_cus) {
     const QmmLayout* lp = &L;
     if (qmm_gemm_regb_applies(&lp, 1, m, n_cus)) return qmm_gemm_regb_workspace_bytes(&lp, 1, m, n_cus);
     if (qmm_gemm_plane_applies(L, m)) return qmm_gemm_plane_bytes(L);
-    const GemmPlan plan = plan_gemm(m, L.n, (int)L.k_units * 4, n_cus);
+    const GemmPlan plan = plan_gemm(m, L.n, (int)L.k_units * 4, n_cus, tiles_of_192(&lp, 1));
     return plan.slices > 1 ? (size_t)plan.slices * (size_t)m * (size_t)L.n * sizeof(float) : 0;
 }
 

@@ -47,6 +47,14 @@ def test_small_products(qa, oracle, tiles, dtype, m, n, k):  # noqa: F811
     check(qa, oracle, dtype, m, n, k)
 
 
+# 256 x 192 tiles (one round of these, more than one of 128 columns, too few k steps for a split): whole and ragged last
+# column tiles, rest of a tile of 16 to 191 columns, k that ends inside a unit and inside a step
+@pytest.mark.parametrize("dtype,m,n,k", [(Q4_K, 300, 16512, 512), (Q4_K, 257, 16600, 256), (Q4_K, 700, 12016, 768), (Q8_0, 500, 17000, 288),
+                                         (Q8_0, 512, 16896, 256), (Q8_0, 270, 16533, 800)])
+def test_tiles_of_192_columns(qa, oracle, tiles, dtype, m, n, k):  # noqa: F811
+    check(qa, oracle, dtype, m, n, k)
+
+
 # more 128 x 128 tiles than compute units: taken by size.  65900 columns: whole rounds of 256-column strips, then
 # half-size tiles; the others have a rest in both directions
 @pytest.mark.parametrize("dtype,m,n,k", [(Q4_K, 2100, 2100, 256), (Q8_0, 190, 17000, 320), (Q6_K, 1000, 5000, 1024), (Q4_K, 150, 65900, 256)])
@@ -54,7 +62,8 @@ def test_large_products(qa, oracle, dtype, m, n, k):  # noqa: F811
     check(qa, oracle, dtype, m, n, k)
 
 
-@pytest.mark.parametrize("dtype,m,ns,k", [(Q6_K, 300, (513, 128, 200), 4096), (Q4_K, 129, (1000, 256), 2048), (Q8_0, 400, (257, 257), 1056)])
+@pytest.mark.parametrize("dtype,m,ns,k", [(Q6_K, 300, (513, 128, 200), 4096), (Q4_K, 129, (1000, 256), 2048), (Q8_0, 400, (257, 257), 1056),
+                                          (Q4_K, 300, (9000, 8000), 256), (Q8_0, 400, (8200, 130, 8300), 544)])  # 192-column tiles
 def test_groups(qa, oracle, tiles, dtype, m, ns, k):  # noqa: F811
     parts = [weight(qa, oracle, dtype, n, k, 720 + i) for i, n in enumerate(ns)]
     x = torch.from_numpy(oracle.randn(721, (m, k))).cuda().to(torch.bfloat16)
