@@ -187,7 +187,7 @@ __device__ __forceinline__ int wave_inclusive_sum(int v, int lane) {
     return v;
 }
 
-// The whole stable counting sort in ONE workgroup (pairs up to 16384, n_experts up to 1024 as far as
+// The whole stable counting sort in ONE workgroup (pairs up to 16384 where the wide sort does not apply, n_experts up to 1024 as far as
 // LDS holds runs x experts counters): pairs are cut into runs of 64 (one wave each); a lane finds its
 // rank among the equal ids of its run through per-expert bit masks; the runs' per-expert counts are
 // scanned run by run (a wave per expert, a lane per run) and over the experts (wave scans); every
@@ -565,14 +565,20 @@ int64_t qmm_moe_sort_scratch_ints(int64_t pairs, int n_experts) {
     return chunks * n_experts;
 }
 
+// Most pairs for the one workgroup: its time grows with the pairs, that of the two launches of many workgroups does not.  us a
+// sort in a graph, one workgroup / two launches: 128 experts 5.3 / 6.3 at 1024 pairs, 6.4 / 6.5 at 2048, 8.8 / 6.6 at 4096, 13.6 /
+// 6.9 at 8192, 22.3 / 7.2 at 16384; 8 experts 6.1 / 6.2, 7.8 / 6.2 and 13.4 / 6.4 at 2048, 4096 and 16384.  Where the ranked experts
+// are wanted, which the one workgroup leaves in passing and each later launch otherwise finds by itself (3 us a layer), up to 4096.  The layer (128 experts, top-8,
+// 2048 x 768, Q4_K): 215 -> 196 at 1024 tokens, 251 -> 242 at 1500 and 316 -> 298 at 2048, with the order of the long items.
+constexpr int64_t kBlockSortPairs = 2048, kRankingSortPairs = 4096;
 hipError_t qmm_launch_moe_sort(const int32_t* ids, int64_t pairs, int n_experts, int32_t* perm,
                                int32_t* offsets, int32_t* seg_offsets, int32_t* scratch,
                                hipStream_t stream, int seg_rows, int32_t* seg_expert, int64_t max_segments,
                                int32_t* expert_order) {
     if (seg_rows < 1 || max_segments > 0x7fffffff) return hipErrorInvalidValue;
     if (n_experts < 1 || n_experts > 8192) return hipErrorInvalidValue;
-    if (expert_order && !block_sort_fits(pairs, n_experts)) return hipErrorInvalidValue; // (qmm_moe_sort_ranks_experts)
-    if (block_sort_fits(pairs, n_experts)) {
+    if (expert_order && !qmm_moe_sort_ranks_experts(pairs, n_experts)) return hipErrorInvalidValue;
+    if (block_sort_fits(pairs, n_experts) && (expert_order || pairs <= kBlockSortPairs)) {
         const size_t lds = (size_t)block_sort_lds_ints(pairs, n_experts) * sizeof(int32_t);
         if (lds > 48 * 1024) {
             hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&sort_block_kernel),
@@ -608,7 +614,7 @@ hipError_t qmm_launch_moe_sort(const int32_t* ids, int64_t pairs, int n_experts,
     return hipGetLastError();
 }
 
-bool qmm_moe_sort_ranks_experts(int64_t pairs, int n_experts) { return block_sort_fits(pairs, n_experts); }
+bool qmm_moe_sort_ranks_experts(int64_t pairs, int n_experts) { return pairs <= kRankingSortPairs && block_sort_fits(pairs, n_experts); }
 
 bool qmm_moe_segments_rank_experts(int n_experts) { return n_experts <= kSegmentsRankedExperts; }
 

@@ -112,7 +112,8 @@ def test_layer_equals_the_tile_kernels(qa, oracle, t):
 
 
 @pytest.mark.parametrize("pairs,experts", [
-    (16385, 128),   # one pair more than one workgroup's sort takes
+    (2048, 128), (2049, 128), (2049, 511), (4097, 1), (5000, 512),  # around one workgroup's sort
+    (16384, 513), (16385, 128),   # as many pairs as one workgroup can sort (where the wide sort does not apply), and one more
     (17 * 1024, 1), (40001, 3), (20000, 511), (20000, 512),
     (20000, 513),   # more experts than a workgroup of the wide sort counts
     (512 * 1024, 128), (512 * 1024 + 1, 128),  # the most workgroups, and one pair beyond them
