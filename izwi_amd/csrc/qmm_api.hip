@@ -1402,6 +1402,11 @@ int gate_up_prefill(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, cons
     uint8_t* group_ws = ws + 2 * part + (((size_t)m * L.k * sizeof(uint16_t) + 255) & ~(size_t)255);
     ProfileScope prof(gate, stream);
     HIP_TRY(qmm_launch_f32_to_bf16(x, xb, m * L.k, stream));
+    const hipError_t gated = qmm_launch_gemm_regb_gated(L, gate->tiled, up->tiled, xb, m, h, h_bf16, gate->n_cus, stream);
+    if (gated != hipErrorNotSupported) {
+        HIP_TRY(gated);
+        return IZWI_QMM_OK;
+    }
     HIP_TRY(group_bf16_launch(gu, 2, xb, m, ys, 0, group_ws, stream));
     HIP_TRY(qmm_launch_silu_mul((const float*)ys[0], (const float*)ys[1], h, h_bf16, m * L.n, stream));
     return IZWI_QMM_OK;

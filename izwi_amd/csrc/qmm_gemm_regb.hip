@@ -179,7 +179,11 @@ __device__ __forceinline__ void chain(F&& f, M&& more) {
         }
 }
 
-template <int QT, int MT>
+__device__ __forceinline__ float silu(float v) { return v / (1.0f + expf(-v)); }
+
+// GATED: members 0 and 1 are gate and up of one shape, k is not split, and y = silu(gate) * up: a workgroup owns 64 columns of
+// both (two of its four column groups each), whose sums meet in LDS; no launch behind it and no f32 products in memory.
+template <int QT, int MT, bool GATED>
 __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P) {
     constexpr int BM = 32 * MT;
     constexpr int kStage = BM * kUnitBytes;
@@ -202,17 +206,17 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
     float* partial = P.partial_v[0];
 #pragma unroll
     for (int i = 1; i < QMM_MAX_GROUP; i++)
-        if (col >= P.col_end[i - 1]) {
+        if (!GATED && col >= P.col_end[i - 1]) {
             slices = P.slices_v[i], slice_units = P.slice_units_v[i], first_col = P.col_end[i - 1];
             n = P.nv[i], row_tiles = P.row_tiles_v[i];
             weights = P.wv[i], y = P.yv[i], partial = P.partial_v[i];
         }
     const int tn = (col - first_col) / slices, slice = col - first_col - tn * slices;
-    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * kBN;
+    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * (GATED ? kBN / 2 : kBN);
     // A workgroup's units u0 .. u1 - 1 of k in turn, from `first` on: those that share an XCD begin at different
     // ones (see above).
     const int u0 = slice * slice_units, u1 = min(P.k_units, u0 + slice_units);
-    const int first = (tn >> 3) % (u1 - u0);
+    const int first = (tn >> (GATED ? 4 : 3)) % (u1 - u0); // (GATED: as the same columns' own product)
     auto unit_of = [&](int u) { return u + first < u1 ? u + first : u + first - (u1 - u0); };
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -252,10 +256,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
 
     // ---- weights: uniform unit address + 32-bit offsets
     const int64_t rt0 = n0 >> 4;
-    const uint8_t* w_tile = weights + rt0 * P.row_bytes;
+    const uint8_t* w_tile = (GATED && wc >= kCols / 2 ? P.wv[1] : weights) + rt0 * P.row_bytes;
+    const int col32 = GATED ? wc & (kCols / 2 - 1) : wc; // the wave's 32 columns of the tile
     HalfOffsets off;
     {
-        const int row = wc * 32 + (lane & 31);
+        const int row = col32 * 32 + (lane & 31);
         const int64_t rt = min(rt0 + (row >> 4), row_tiles - 1);
         const uint32_t base = (uint32_t)((rt - rt0) * P.row_bytes) + (row & 15) * 16, chunk = (uint32_t)P.slots * 16;
         off.hdr = base + (QT == QMM_Q4_K ? 0 : 8 * half);
@@ -400,8 +405,30 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
         if (half) take(std::integral_constant<int, 1>{});
         else take(std::integral_constant<int, 0>{});
     }
+    // GATED: of a wave pair (gate, up) of the same columns the one finishes block 0, the other block 1
+    const bool is_up = GATED && wc >= kCols / 2; // uniform
+    if constexpr (GATED) {
+        uint8_t* at = smem + kCols * MT * 4096 + (2 * col32 + half) * 8192 + lane * 16; // (behind the halves' sums)
+        auto put = [&](const f32x16& v, int slot) {
+            for (int r = 0; r < 4; r++)
+                *reinterpret_cast<f32x4*>(at + slot * 4096 + r * 1024) = f32x4{v[4 * r], v[4 * r + 1], v[4 * r + 2], v[4 * r + 3]};
+        };
+        if (is_up) put(sum[0], 0);
+        else if constexpr (kOwn > 1) put(sum[1], 1);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (!is_up)
+            for (int r = 0; r < 4; r++) {
+                const f32x4 v = *reinterpret_cast<const f32x4*>(at + r * 1024);
+                for (int e = 0; e < 4; e++) sum[0][4 * r + e] = silu(sum[0][4 * r + e]) * v[e];
+            }
+        else if constexpr (kOwn > 1)
+            for (int r = 0; r < 4; r++) {
+                const f32x4 v = *reinterpret_cast<const f32x4*>(at + 4096 + r * 1024);
+                for (int e = 0; e < 4; e++) sum[1][4 * r + e] = silu(v[e]) * sum[1][4 * r + e];
+            }
+    }
     const bool split = slices > 1;
-    const int64_t gn = n0 + wc * 32 + (lane & 31);
+    const int64_t gn = n0 + col32 * 32 + (lane & 31);
     const int64_t gm0 = m0 + half * 32 + 4 * h;
     const int rows = gn < n ? (int)min((int64_t)BM, P.m - gm0) : 0; // of this lane's column, from gm0 on
     auto emit = [&](auto MODE) { // 0: f32, 1: f32 + residual, 2: bf16, 3: bf16 + residual
@@ -413,7 +440,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
         static_for<kOwn>([&](auto I) {
             static_for<16>([&](auto R) {
                 constexpr int i = decltype(I)::value, r = decltype(R)::value, row = 64 * i + 8 * (r >> 2) + (r & 3);
-                if (row < rows && (2 * i + half < MT)) {
+                if (row < rows && (2 * i + half < MT) && (!GATED || i == (int)is_up)) {
                     const int64_t at = row * n;
                     float v = sum[i][r];
                     if (mode == 1) v += rf[at];
@@ -535,25 +562,45 @@ size_t partial_bytes(const RegbPlan& p, const QmmLayout& L, int i, int64_t m) {
     return p.slices[i] <= 1 ? 0 : (((size_t)p.slices[i] * (size_t)m * (size_t)L.n * sizeof(float)) + 255) & ~(size_t)255;
 }
 
-template <int QT, int MT>
+template <int QT, int MT, bool GATED>
 hipError_t launch_regb(const RegbParams& P, int64_t grid, hipStream_t stream) {
     constexpr size_t stages = (size_t)x_stages(MT) * 32 * MT * kUnitBytes; // the halves' sums reuse it
-    static_assert(stages <= 160 * 1024 && stages >= (size_t)kCols * MT * 4096, "LDS of a CU");
-    auto fn = &gemm_regb_kernel<QT, MT>;
+    static_assert(stages <= 160 * 1024 && stages >= (size_t)kCols * MT * 4096 + (GATED ? kWaves * 4096 : 0), "LDS of a CU");
+    auto fn = &gemm_regb_kernel<QT, MT, GATED>;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)stages);
     if (e != hipSuccess) return e;
     fn<<<dim3((unsigned)grid), dim3(64 * kWaves), stages, stream>>>(P);
     return hipGetLastError();
 }
 
-template <int QT>
+template <int QT, bool GATED>
 hipError_t launch_regb_qt(const RegbParams& P, const RegbPlan& p, int64_t grid, hipStream_t stream) {
     switch (p.mt) {
-        case 1: return launch_regb<QT, 1>(P, grid, stream);
-        case 2: return launch_regb<QT, 2>(P, grid, stream);
-        case 3: return launch_regb<QT, 3>(P, grid, stream);
-        default: return launch_regb<QT, 4>(P, grid, stream);
+        case 1: return launch_regb<QT, 1, GATED>(P, grid, stream);
+        case 2: return launch_regb<QT, 2, GATED>(P, grid, stream);
+        case 3: return launch_regb<QT, 3, GATED>(P, grid, stream);
+        default: return launch_regb<QT, 4, GATED>(P, grid, stream);
     }
+}
+template <bool GATED>
+hipError_t launch_regb_type(int dtype, const RegbParams& P, const RegbPlan& p, int64_t grid, hipStream_t stream) {
+    return dtype == QMM_Q6_K   ? launch_regb_qt<QMM_Q6_K, GATED>(P, p, grid, stream)
+           : dtype == QMM_Q4_K ? launch_regb_qt<QMM_Q4_K, GATED>(P, p, grid, stream)
+                               : launch_regb_qt<QMM_Q8_0, GATED>(P, p, grid, stream);
+}
+// what every member shares
+RegbParams base_params(const QmmLayout& L0, const RegbPlan& plan, const uint16_t* x_bf16, int64_t m, int out_bf16) {
+    RegbParams P;
+    P.x = x_bf16;
+    P.m = m, P.k = L0.k;
+    P.k_units = (int)L0.k_units;
+    P.s = L0.s, P.slots = L0.slots;
+    P.panel_bytes = L0.panel_bytes, P.row_bytes = L0.k_groups * L0.panel_bytes;
+    P.nibble_mask = 0x0f0f0f0fu;
+    P.out_bf16 = out_bf16;
+    P.residual = nullptr;
+    P.tiles_m = (int)((m + 32 * plan.mt - 1) / (32 * plan.mt));
+    return P;
 }
 
 } // namespace
@@ -591,16 +638,8 @@ hipError_t qmm_launch_gemm_regb(const QmmLayout* const* layouts, const void* con
     if (n_weights < 1 || n_weights > QMM_MAX_GROUP || (residual && n_weights != 1)) return hipErrorInvalidValue;
     const QmmLayout& L0 = *layouts[0];
     const RegbPlan plan = plan_regb(layouts, n_weights, m, n_cus);
-    RegbParams P;
-    P.x = x_bf16;
-    P.m = m, P.k = L0.k;
-    P.k_units = (int)L0.k_units;
-    P.s = L0.s, P.slots = L0.slots;
-    P.panel_bytes = L0.panel_bytes, P.row_bytes = L0.k_groups * L0.panel_bytes;
-    P.nibble_mask = 0x0f0f0f0fu;
-    P.out_bf16 = out_bf16;
+    RegbParams P = base_params(L0, plan, x_bf16, m, out_bf16);
     P.residual = plan.slices[0] > 1 ? nullptr : residual;
-    P.tiles_m = (int)((m + 32 * plan.mt - 1) / (32 * plan.mt));
     RegbReduceParams R;
     uint8_t* next = static_cast<uint8_t*>(workspace);
     int64_t cols = 0, blocks = 0;
@@ -629,11 +668,26 @@ hipError_t qmm_launch_gemm_regb(const QmmLayout* const* layouts, const void* con
     const int64_t grid = (cols + 7) / 8 * 8 * P.tiles_m;
     if (grid > 0x7fffffff) return hipErrorInvalidValue;
     P.cols = (int)cols;
-    hipError_t e = L0.dtype == QMM_Q6_K   ? launch_regb_qt<QMM_Q6_K>(P, plan, grid, stream)
-                   : L0.dtype == QMM_Q4_K ? launch_regb_qt<QMM_Q4_K>(P, plan, grid, stream)
-                                          : launch_regb_qt<QMM_Q8_0>(P, plan, grid, stream);
+    hipError_t e = launch_regb_type<false>(L0.dtype, P, plan, grid, stream);
     if (e != hipSuccess || blocks == 0) return e;
     R.out_bf16 = out_bf16, R.residual = residual;
     regb_reduce_kernel<<<(unsigned)blocks, 256, 0, stream>>>(R);
     return hipGetLastError();
+}
+
+hipError_t qmm_launch_gemm_regb_gated(const QmmLayout& L, const void* gate, const void* up, const uint16_t* x_bf16, int64_t m, void* h,
+                                      int h_bf16, int n_cus, hipStream_t stream) {
+    const QmmLayout* const pair[2] = {&L, &L};
+    if (!qmm_gemm_regb_applies(pair, 2, m, n_cus)) return hipErrorNotSupported;
+    const RegbPlan plan = plan_regb(pair, 2, m, n_cus);
+    if (plan.slices[0] > 1 || plan.slices[1] > 1) return hipErrorNotSupported;
+    RegbParams P = base_params(L, plan, x_bf16, m, h_bf16);
+    const int64_t cols = (L.n + kBN / 2 - 1) / (kBN / 2), grid = (cols + 7) / 8 * 8 * P.tiles_m;
+    if (grid > 0x7fffffff) return hipErrorInvalidValue;
+    P.cols = (int)cols;
+    for (int i = 0; i < QMM_MAX_GROUP; i++) {
+        P.col_end[i] = 0x7fffffff, P.slices_v[i] = 1, P.slice_units_v[i] = (int)L.k_units, P.partial_v[i] = nullptr;
+        P.wv[i] = static_cast<const uint8_t*>(i ? up : gate), P.yv[i] = h, P.nv[i] = L.n, P.row_tiles_v[i] = L.row_tiles;
+    }
+    return launch_regb_type<true>(L.dtype, P, plan, grid, stream);
 }

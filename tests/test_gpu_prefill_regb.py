@@ -146,6 +146,24 @@ def test_gate_up_sums_equal_the_projections(qa, oracle, m):
     assert bool(((h.double() - want).abs() <= 6 * 2.0 ** -24 * want.abs() + 1e-30).all())
 
 
+# silu(gate) * up in the products' own launch (k not split): one to four blocks of 32 rows per row tile, the last 64 columns
+# of gate and up whole and ragged, one column tile, k that ends inside a unit
+@pytest.mark.parametrize("dtype,m,n,k", [(Q4_K, 65, 64, 256), (Q4_K, 101, 200, 768), (Q8_0, 128, 100, 288), (Q6_K, 97, 1000, 512), (Q4_K, 70, 16400, 256),
+                                         (Q8_0, 96, 16400, 512), (Q4_K, 128, 8200, 512), (Q6_K, 129, 6000, 256), (Q8_0, 300, 3000, 768)])
+def test_gated_products(qa, oracle, dtype, m, n, k):
+    print(f"gated dtype={dtype} m={m} n={n} k={k}", flush=True)
+    gate, up, down = (weight(qa, oracle, dtype, *shape, 480 + i) for i, shape in enumerate([(n, k), (n, k), (256, n // 256 * 256 or 256)]))
+    x = torch.from_numpy(oracle.randn(481 + m, (m, k))).cuda()
+    g, u = qa.forward_group((gate, up), x)
+    gate_up = qa.Qwen3GateUpProjection.new_separate(gate, up)
+    h = gate_up.forward_silu_mul(x)
+    want = g.double() / (1.0 + torch.exp(-g.double())) * u.double()
+    # silu in f32: expf (1 ulp), one addition, one division and one product of 2^-24 each
+    assert bool(((h.double() - want).abs() <= 6 * 2.0 ** -24 * want.abs() + 1e-30).all())
+    if n % 256 == 0:
+        assert torch.equal(qa.Qwen3Mlp(gate_up, down).forward(x), down.forward(h))
+
+
 @pytest.mark.parametrize("dtype", [Q8_0, Q4_K])
 @pytest.mark.parametrize("m", [65, 129, 150, 179, 192])
 def test_mlp_of_a_small_model_at_prefill_rows(qa, oracle, dtype, m):
