@@ -397,7 +397,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
 #pragma unroll
                 for (int q = 0; q < GS; q++) {
                     const int t = gi * GS + q, i = t / NT, j = t % NT;
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[kk & 1][i], fb[kk & 1][j], acc[i][j], 0, 0, 0);
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[kk & 1][j], fa[kk & 1][i], acc[i][j], 0, 0, 0);
                 }
                 // group g's share of staging tile kt+1 (the thread's NP weight pieces and XC
                 // activation chunks over the first 3 NG / 4 groups) and of fetching tile kt+2
@@ -496,58 +496,127 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
         }
     }
 
-    // a split-k slice stores f32 into its own [m, n] plane of the workspace
-    float* out_f32 = P.partial ? P.partial + (int64_t)blockIdx.y * P.m * P.n : reinterpret_cast<float*>(P.y);
-    auto each = [&](auto B, auto&& f) { // the lane's elements of 32 x 32 block B: register, index
-        constexpr int i = decltype(B)::value / NT, j = decltype(B)::value % NT;
-        const int64_t gn = n0 + wn * (BN / 2) + j * 32 + (lane & 31);
-        if (gn >= P.n_end) return;
+    // ---- epilogue.  The weights are the matrix instruction's first operand, so a lane holds four consecutive columns at a time
+    // of one activation row: 32 rows of the wave's columns go through the wave's own LDS (f32) and leave in whole 16-byte
+    // pieces of a row, the residual comes in as such.  (Stored from the accumulators, two bytes a lane, a 2048 x 4096 product
+    // with a bf16 residual took 92 us, 75 without.)
+    constexpr int COLS = BN / 2, kOutStride = COLS * 4 + 16;
+    static_assert(NW * 32 * kOutStride <= 2 * kStage);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); // every wave has read its last fragments
+    uint8_t* out_lds = smem + wave * (32 * kOutStride);
+    const bool f32_out = P.partial || !P.out_bf16;
+    void* out = P.partial ? P.partial + (int64_t)blockIdx.y * P.m * P.n : P.y; // a split-k slice: its own f32 [m, n] plane
+    const void* residual = P.partial ? nullptr : P.residual;                   // (the second kernel finishes a slice)
+    const bool whole = P.n % 8 == 0 && ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(residual)) & 15) == 0;
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    // pieces of W columns (16 bytes of the output: 4 f32, 8 bf16) of 32 rows, consecutive lanes on consecutive pieces
+    auto rows_out = [&](auto I, auto W) {
+        constexpr int i = decltype(I)::value, w = decltype(W)::value, LPR = COLS / w, PASSES = 32 * LPR / 64, CH = PASSES > 8 ? PASSES / 2 : PASSES;
+        static_assert(32 * LPR % 64 == 0 && PASSES % CH == 0);
+        static_for<PASSES / CH>([&](auto C) {
+            int64_t at[CH];
+            int lds[CH], left[CH]; // left: columns of the piece that exist
+            u32x4 res[CH];
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int64_t gm = m0 + wm * (BM / WM) + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-            if (gm < P.m) f(r, gm * P.n + gn);
-        }
-    };
-    if (P.partial || !P.residual) { // uniform; a slice: the second kernel finishes
-        const bool f32 = P.partial || !P.out_bf16;
-        static_for<MT * NT>([&](auto B) {
-            constexpr int i = decltype(B)::value / NT, j = decltype(B)::value % NT;
-            each(B, [&](int r, int64_t at) {
-                if (f32) out_f32[at] = acc[i][j][r];
-                else qmm_store(P.y, QmmEpilogue{nullptr, 1}, at, acc[i][j][r]);
-            });
+            for (int q = 0; q < CH; q++) {
+                const int item = (decltype(C)::value * CH + q) * 64 + lane, row = item / LPR, c = item - row * LPR;
+                const int64_t gm = m0 + wm * (BM / WM) + i * 32 + row, gn = n0 + wn * COLS + c * w;
+                at[q] = gm * P.n + gn, lds[q] = row * kOutStride + c * w * 4;
+                left[q] = gm < P.m ? (int)min((int64_t)w, P.n_end - gn) : 0;
+                res[q] = u32x4{0, 0, 0, 0};
+                if (residual && whole && left[q] > 0) // (requested together: it may be the output, and the lane reads what it writes)
+                    res[q] = *reinterpret_cast<const u32x4*>(static_cast<const uint8_t*>(residual) + at[q] * (16 / w));
+            }
+#pragma unroll
+            for (int q = 0; q < CH; q++) {
+                f32x4 v[w / 4];
+#pragma unroll
+                for (int e = 0; e < w / 4; e++) v[e] = *reinterpret_cast<const f32x4*>(out_lds + lds[q] + 16 * e);
+                if (whole && left[q] > 0) { // (n is a multiple of eight: the whole piece exists)
+                    if (residual)
+#pragma unroll
+                        for (int e = 0; e < w; e++)
+                            v[e >> 2][e & 3] += __uint_as_float(w == 4 ? res[q][e] : e & 1 ? res[q][e >> 1] & 0xffff0000u : res[q][e >> 1] << 16);
+                    u32x4 o;
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        o[e] = w == 4 ? __float_as_uint(v[0][e]) : pack_bf16(v[e * w / 16][2 * e & 3], v[e * w / 16][(2 * e & 3) + 1]);
+                    *reinterpret_cast<u32x4*>(static_cast<uint8_t*>(out) + at[q] * (16 / w)) = o;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < w; e++)
+                        if (e < left[q]) qmm_store(out, QmmEpilogue{residual, w == 8}, at[q] + e, v[e >> 2][e & 3]);
+                }
+            }
         });
-        return;
-    }
-    // The residual a block ahead of the stores: it may be the output buffer, so behind a store the compiler would keep
-    // every load, a chain of 16 MT NT round trips.  (The lane reads the elements that it writes.)
-    float res[2][16];
-    auto fetch = [&](auto B) {
-        constexpr int to = decltype(B)::value & 1;
-        each(B, [&](int r, int64_t at) {
-            res[to][r] = P.out_bf16 ? qmm_bf16_bits_to_f32(static_cast<const uint16_t*>(P.residual)[at])
-                                    : static_cast<const float*>(P.residual)[at];
-        });
     };
-    fetch(std::integral_constant<int, 0>{});
-    static_for<MT * NT>([&](auto B) {
-        constexpr int b = decltype(B)::value;
-        if constexpr (b + 1 < MT * NT) fetch(std::integral_constant<int, b + 1>{});
-        each(B, [&](int r, int64_t at) { qmm_store(P.y, QmmEpilogue{nullptr, P.out_bf16}, at, acc[b / NT][b % NT][r] + res[b & 1][r]); });
+    static_for<MT>([&](auto I) {
+        constexpr int i = decltype(I)::value;
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+                *reinterpret_cast<f32x4*>(out_lds + (lane & 31) * kOutStride + (j * 32 + 8 * g + 4 * (lane >> 5)) * 4) =
+                    f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+        if (f32_out) rows_out(I, std::integral_constant<int, 4>{}); // uniform
+        else rows_out(I, std::integral_constant<int, 8>{});
     });
 }
 
 // out[i] = sum over slices (in order) of partial[s][i], as f32 or bf16; i runs over the
 // columns [n_begin, n_end) of all rows
-__global__ void splitk_reduce_kernel(const float* __restrict__ partial, int slices, int64_t m, int64_t n,
-                                     int64_t n_begin, int64_t n_end, void* y, int out_bf16, const void* residual) {
-    const int64_t width = n_end - n_begin;
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= m * width) return;
-    const int64_t row = idx / width, col = n_begin + (idx - row * width);
-    float sum = 0.0f;
-    for (int s = 0; s < slices; s++) sum += partial[((int64_t)s * m + row) * n + col];
-    qmm_store(y, QmmEpilogue{residual, out_bf16}, row * n + col, sum);
+// EIGHT: whole planes, eight values per thread in 16-byte pieces (m n a multiple of eight, everything aligned to 16 bytes).
+// Bound by memory: the product 2048 x 4096, k = 12288, in two slices with a bf16 residual (100 MB here), 205 us with the reduction
+// value by value, 194 by pieces; Q8_0 217 / 200.
+template <bool EIGHT>
+__global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ partial, int slices, int64_t m, int64_t n,
+                                                            int64_t n_begin, int64_t n_end, void* y, int out_bf16, const void* residual) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if constexpr (!EIGHT) {
+        const int64_t width = n_end - n_begin;
+        if (idx >= m * width) return;
+        const int64_t row = idx / width, col = n_begin + (idx - row * width);
+        float sum = 0.0f;
+        for (int s = 0; s < slices; s++) sum += partial[((int64_t)s * m + row) * n + col];
+        qmm_store(y, QmmEpilogue{residual, out_bf16}, row * n + col, sum);
+        return;
+    }
+    const int64_t i = idx * 8, count = m * n;
+    if (i >= count) return;
+    f32x4 res[2] = {};
+    if (residual && out_bf16) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(residual) + i);
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            res[e >> 1][2 * (e & 1)] = __uint_as_float(v[e] << 16), res[e >> 1][2 * (e & 1) + 1] = __uint_as_float(v[e] & 0xffff0000u);
+    } else if (residual) {
+        res[0] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(residual) + i);
+        res[1] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(residual) + i + 4);
+    }
+    f32x4 sum[2] = {};
+    for (int s = 0; s < slices; s++) {
+        const f32x4* p = reinterpret_cast<const f32x4*>(partial + s * count + i);
+        sum[0] += p[0], sum[1] += p[1];
+    }
+    if (residual) sum[0] += res[0], sum[1] += res[1];
+    if (out_bf16) {
+        *reinterpret_cast<u32x4*>(static_cast<uint16_t*>(y) + i) = u32x4{pack_bf16(sum[0].x, sum[0].y), pack_bf16(sum[0].z, sum[0].w),
+                                                                         pack_bf16(sum[1].x, sum[1].y), pack_bf16(sum[1].z, sum[1].w)};
+    } else {
+        *reinterpret_cast<f32x4*>(static_cast<float*>(y) + i) = sum[0];
+        *reinterpret_cast<f32x4*>(static_cast<float*>(y) + i + 4) = sum[1];
+    }
+}
+hipError_t launch_splitk_reduce(const float* partial, int slices, int64_t m, int64_t n, int64_t n_begin, int64_t n_end, void* y, int out_bf16,
+                                const void* residual, hipStream_t stream) {
+    const int64_t count = m * (n_end - n_begin);
+    const uintptr_t at = reinterpret_cast<uintptr_t>(partial) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(residual);
+    if (n_begin == 0 && n_end == n && count % 8 == 0 && at % 16 == 0)
+        splitk_reduce_kernel<true><<<(unsigned)((count / 8 + 255) / 256), 256, 0, stream>>>(partial, slices, m, n, 0, n, y, out_bf16, residual);
+    else
+        splitk_reduce_kernel<false><<<(unsigned)((count + 255) / 256), 256, 0, stream>>>(partial, slices, m, n, n_begin, n_end, y, out_bf16, residual);
+    return hipGetLastError();
 }
 
 __global__ void f32_to_bf16_kernel(const float* __restrict__ x, uint16_t* __restrict__ out,
@@ -597,15 +666,11 @@ hipError_t launch_tile(GemmParams P, int slices, hipStream_t stream) {
     else P.partial = nullptr;
     fn<<<dim3((unsigned)grid, (unsigned)slices), dim3(64 * NW), lds, stream>>>(P);
     if (slices > 1 && P.n_weights > 1) {
-        for (int i = 0; i < P.n_weights; i++) {
-            const int64_t count = P.m * P.nv[i];
-            splitk_reduce_kernel<<<(unsigned)((count + 255) / 256), 256, 0, stream>>>(
-                P.partial_v[i], slices, P.m, P.nv[i], 0, P.nv[i], P.yv[i], P.out_bf16, nullptr);
-        }
+        for (int i = 0; i < P.n_weights; i++)
+            if ((e = launch_splitk_reduce(P.partial_v[i], slices, P.m, P.nv[i], 0, P.nv[i], P.yv[i], P.out_bf16, nullptr, stream)) != hipSuccess)
+                return e;
     } else if (slices > 1) {
-        const int64_t count = P.m * (P.n_end - P.n_begin);
-        splitk_reduce_kernel<<<(unsigned)((count + 255) / 256), 256, 0, stream>>>(
-            partial, slices, P.m, P.n, P.n_begin, P.n_end, P.y, P.out_bf16, P.residual);
+        return launch_splitk_reduce(partial, slices, P.m, P.n, P.n_begin, P.n_end, P.y, P.out_bf16, P.residual, stream);
     }
     return hipGetLastError();
 }
@@ -646,7 +711,8 @@ int64_t tiles_of_192(const QmmLayout* const* layouts, int n_weights) {
 }
 
 GemmPlan plan_gemm(int64_t m, int64_t n, int k_steps, int n_cus, int64_t tiles_n192, bool group = false) {
-    const double kQ128 = 0.76; // relative rate of a half-size tile
+    // relative rate of a half-size tile: 256 of them at k = 4096 take 75 us (4096 x 4096 at 2048 rows), as many whole ones 121
+    const double kQ128 = 0.82;
     // A 256 x 192 tile takes 0.79 of the time of a whole one.  Where whole tiles would fill the last round badly, us per call (2 x
     // 12288 x 4096, Q4_K): 112 -> 105 at 500 rows (192 whole tiles, 256 of these), 212 -> 182 at 640 (288, 384), 217 ->
     // 197 at 1000 (384, 512), 330 -> 290 at 1400 (576, 768); 2 x 3072 x 1024 42 -> 37 at 2048 rows (192, 256).
@@ -676,13 +742,16 @@ GemmPlan plan_gemm(int64_t m, int64_t n, int k_steps, int n_cus, int64_t tiles_n
         consider({hm, hn, 1, full_cols},
                  (double)(tiles_m256 * full_cols / n_cus) * k_steps +
                      rounds(tiles(hm, hn, n - full_cols * 256)) * k_steps * 0.5 / kQ128);
-    // split along k: the slices' f32 tiles are written and read once more (about 4 TB/s,
-    // a 256 x 256 k step takes about 1.5 us)
+    // split along k: the slices' f32 tiles are written in the launch and read by a second one (3 us and 4.5 TB/s; a
+    // 256 x 256 k step takes 1.9 us).  4096 x 12288, us with a residual: 1100 rows 256 x 256 in two slices 182, 256 x 128 199,
+    // 256 x 192 in two slices 171; 2048 rows 198 / 211 / 260.  4096 x 4096: 1100 rows 70 / 66 / 60, 2048 rows 87 / 75 / 110.
     for (int slices = 2; slices <= 8; slices *= 2) {
         if (k_steps / slices < 8) break;
-        const double reduce_cost = 2.0 * slices * (double)m * (double)n * 4.0 / 4e12 * 1e6 / 1.5 + 2.0;
+        const double reduce_cost = (slices * (double)m * (double)n * 4.0 / 4.5e6 + 3.0) / 1.9;
         const double steps = 4.0 * (double)((k_steps / 4 + slices - 1) / slices); // slices are whole units
         consider({256, 256, slices, 0}, rounds(tiles(256, 256, n) * slices) * steps + reduce_cost);
+        if (tiles_n192 > 0)
+            consider({256, 192, slices, 0}, rounds((m + 255) / 256 * tiles_n192 * slices) * steps * kCost192 + reduce_cost);
         consider({hm, hn, slices, 0}, rounds(tiles(hm, hn, n) * slices) * steps * 0.5 / kQ128 + reduce_cost);
     }
     return best;

@@ -62,6 +62,29 @@ def test_large_products(qa, oracle, dtype, m, n, k):  # noqa: F811
     check(qa, oracle, dtype, m, n, k)
 
 
+# results and residuals that start on 2, 4 or 16 bytes, rows of a multiple of eight values and not, sums of whole pieces and of
+# single values: 256, 192 and 128-column tiles, each whole along k and in slices.  The same sums, so the same bits
+@pytest.mark.parametrize("dtype,m,n,k", [(Q4_K, 300, 520, 4096), (Q4_K, 301, 515, 4096), (Q4_K, 1100, 4096, 4096), (Q8_0, 700, 12024, 768),
+                                         (Q4_K, 2050, 2056, 512), (Q8_0, 300, 66000, 256)])
+def test_results_and_residuals_by_alignment(qa, oracle, tiles, dtype, m, n, k):  # noqa: F811
+    mm = weight(qa, oracle, dtype, n, k, 730)
+    x = torch.from_numpy(oracle.randn(731, (m, k))).cuda().to(torch.bfloat16)
+    y = mm.forward_bf16_to_f32(x)
+    assert off(y, x.double() @ dense(mm).t()) < F32_TOL
+    for out_dtype in (torch.float32, torch.bfloat16):
+        res = torch.from_numpy(oracle.randn(732, (m, n))).cuda().to(out_dtype)
+        total = (y + res.float()).to(out_dtype)
+
+        def at(skip):
+            return torch.zeros(m * n + 32, dtype=out_dtype, device="cuda")[skip:skip + m * n].view(m, n)
+
+        for to, of in ((0, 0), (1, 0), (0, 2), (8, 8), (1, 1)):
+            out, r = at(to), at(of).copy_(res)
+            assert torch.equal(mm.forward_fused(x, out=out, out_dtype=out_dtype), y.to(out_dtype))
+            assert torch.equal(mm.forward_fused(x, residual=r, out=out, out_dtype=out_dtype), total), (out_dtype, to, of)
+            assert torch.equal(r, res)
+
+
 @pytest.mark.parametrize("dtype,m,ns,k", [(Q6_K, 300, (513, 128, 200), 4096), (Q4_K, 129, (1000, 256), 2048), (Q8_0, 400, (257, 257), 1056),
                                           (Q4_K, 300, (9000, 8000), 256), (Q8_0, 400, (8200, 130, 8300), 544)])  # 192-column tiles
 def test_groups(qa, oracle, tiles, dtype, m, ns, k):  # noqa: F811
