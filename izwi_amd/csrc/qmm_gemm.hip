@@ -505,51 +505,21 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); // every wave has read its last fragments
     uint8_t* out_lds = smem + wave * (32 * kOutStride);
     const bool f32_out = P.partial || !P.out_bf16;
-    void* out = P.partial ? P.partial + (int64_t)blockIdx.y * P.m * P.n : P.y; // a split-k slice: its own f32 [m, n] plane
-    const void* residual = P.partial ? nullptr : P.residual;                   // (the second kernel finishes a slice)
-    const bool whole = P.n % 8 == 0 && ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(residual)) & 15) == 0;
+    RowsOut R; // a split-k slice: its own f32 [m, n] plane, which the second kernel finishes
+    R.out = P.partial ? P.partial + (int64_t)blockIdx.y * P.m * P.n : P.y, R.residual = P.partial ? nullptr : P.residual;
+    R.m = P.m, R.n = P.n, R.n_end = P.n_end, R.col0 = n0 + wn * COLS;
     typedef float f32x4 __attribute__((ext_vector_type(4)));
-    // pieces of W columns (16 bytes of the output: 4 f32, 8 bf16) of 32 rows, consecutive lanes on consecutive pieces
-    auto rows_out = [&](auto I, auto W) {
-        constexpr int i = decltype(I)::value, w = decltype(W)::value, LPR = COLS / w, PASSES = 32 * LPR / 64, CH = PASSES > 8 ? PASSES / 2 : PASSES;
-        static_assert(32 * LPR % 64 == 0 && PASSES % CH == 0);
+    auto four = [&](int row, int col) { return *reinterpret_cast<const f32x4*>(out_lds + row * kOutStride + col * 4); };
+    auto one = [&](int row, int col) { return *reinterpret_cast<const float*>(out_lds + row * kOutStride + col * 4); };
+    auto rows_out = [&](auto W) {
+        constexpr int w = decltype(W)::value, PASSES = COLS / w / 2, CH = PASSES > 8 ? PASSES / 2 : PASSES;
         static_for<PASSES / CH>([&](auto C) {
-            int64_t at[CH];
-            int lds[CH], left[CH]; // left: columns of the piece that exist
-            u32x4 res[CH];
-#pragma unroll
-            for (int q = 0; q < CH; q++) {
-                const int item = (decltype(C)::value * CH + q) * 64 + lane, row = item / LPR, c = item - row * LPR;
-                const int64_t gm = m0 + wm * (BM / WM) + i * 32 + row, gn = n0 + wn * COLS + c * w;
-                at[q] = gm * P.n + gn, lds[q] = row * kOutStride + c * w * 4;
-                left[q] = gm < P.m ? (int)min((int64_t)w, P.n_end - gn) : 0;
-                res[q] = u32x4{0, 0, 0, 0};
-                if (residual && whole && left[q] > 0) // (requested together: it may be the output, and the lane reads what it writes)
-                    res[q] = *reinterpret_cast<const u32x4*>(static_cast<const uint8_t*>(residual) + at[q] * (16 / w));
-            }
-#pragma unroll
-            for (int q = 0; q < CH; q++) {
-                f32x4 v[w / 4];
-#pragma unroll
-                for (int e = 0; e < w / 4; e++) v[e] = *reinterpret_cast<const f32x4*>(out_lds + lds[q] + 16 * e);
-                if (whole && left[q] > 0) { // (n is a multiple of eight: the whole piece exists)
-                    if (residual)
-#pragma unroll
-                        for (int e = 0; e < w; e++)
-                            v[e >> 2][e & 3] += __uint_as_float(w == 4 ? res[q][e] : e & 1 ? res[q][e >> 1] & 0xffff0000u : res[q][e >> 1] << 16);
-                    u32x4 o;
-#pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        o[e] = w == 4 ? __float_as_uint(v[0][e]) : pack_bf16(v[e * w / 16][2 * e & 3], v[e * w / 16][(2 * e & 3) + 1]);
-                    *reinterpret_cast<u32x4*>(static_cast<uint8_t*>(out) + at[q] * (16 / w)) = o;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < w; e++)
-                        if (e < left[q]) qmm_store(out, QmmEpilogue{residual, w == 8}, at[q] + e, v[e >> 2][e & 3]);
-                }
-            }
+            RowPieces<COLS, w, decltype(C)::value * CH, CH> pieces;
+            pieces.request(R, lane);
+            pieces.store(R, lane, four);
         });
     };
+    const bool whole = whole_pieces(R);
     static_for<MT>([&](auto I) {
         constexpr int i = decltype(I)::value;
 #pragma unroll
@@ -558,8 +528,11 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
             for (int g = 0; g < 4; g++)
                 *reinterpret_cast<f32x4*>(out_lds + (lane & 31) * kOutStride + (j * 32 + 8 * g + 4 * (lane >> 5)) * 4) =
                     f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-        if (f32_out) rows_out(I, std::integral_constant<int, 4>{}); // uniform
-        else rows_out(I, std::integral_constant<int, 8>{});
+        R.row0 = m0 + wm * (BM / WM) + i * 32;
+        if (!whole && f32_out) store_values<COLS, true>(R, lane, one); // uniform
+        else if (!whole) store_values<COLS, false>(R, lane, one);
+        else if (f32_out) rows_out(std::integral_constant<int, 4>{});
+        else rows_out(std::integral_constant<int, 8>{});
     });
 }
 

@@ -17,7 +17,7 @@
 //
 // Bound by the life of a workgroup: at 2 x 12288 x 4096 (Q4_K, cold weights; time stamps) it has its arguments after 1.0 us
 // and its first operands 4.2 later, takes 30 in sixteen units (1.95 a unit at 101 rows, 1.65 at 65; 2.1 and 1.8 with the
-// loads one unit ahead and all workgroups at the same unit) and 2.2 for the exchange of the sums and the stores.  Of a
+// loads one unit ahead and all workgroups at the same unit) and 2.2 for the exchange of the sums and stores of a value a lane.  Of a
 // unit's 1.95 us 1.57 remain without its loads and 1.3 without unpacking and activations: matrix instructions (1.0),
 // unpacking (1.0), LDS reads (0.9 to 1.2) and the loads share the compute unit, and two waves per SIMD overlap them in
 // part.  An unpacking of a fifth fewer vector instructions (mixed-precision fma on f16 denormals) gave nothing.
@@ -324,7 +324,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
     auto multiply = [&](auto SS) {
         constexpr int ss = decltype(SS)::value;
 #pragma unroll
-        for (int j = 0; j < MT; j++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[ss & 1][j], b[ss & 1], acc[j], 0, 0, 0);
+        for (int j = 0; j < MT; j++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[ss & 1], a[ss & 1][j], acc[j], 0, 0, 0);
 #pragma unroll
         for (int q = 0; q < MT; q++) { // one matrix instruction, then a share of the next one's operands
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -373,10 +373,37 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
         else turn(I, std::false_type{}, std::integral_constant<int, w_behind + (NS - 2) * XL>{}, std::integral_constant<int, w_behind>{});
     }, [&] { return u < last; });
     multiply(std::integral_constant<int, 7>{});
+
+    // ---- epilogue.  The weights are the matrix instruction's first operand: a lane holds four consecutive columns at a time of
+    // one activation row.  32 x 32 blocks of sums leave through LDS in whole 16-byte pieces; the residual is requested
+    // in front of the halves' exchange.  (Stored from the accumulators, two bytes a lane, the residual read in front of each:
+    // 4096 x 4096 with a bf16 residual, Q4_K, 32 us at 400 rows and 33 at 500 in two slices, which were the faster; so in
+    // one slice 27 and 29.)
+    constexpr int kOwn = (MT + 1) / 2; // the wave of half p finishes the blocks i with i % 2 = p
+    const bool split = slices > 1, f32_out = split || !P.out_bf16;
+    RowsOut R;
+    R.out = split ? partial + (int64_t)slice * P.m * n : y, R.residual = split ? nullptr : P.residual;
+    R.m = P.m, R.n = n, R.n_end = n, R.col0 = n0 + col32 * 32;
+    const bool is_up = GATED && wc >= kCols / 2, whole = whole_pieces(R); // uniform
+    auto rows_of = [&](auto I) {
+        RowsOut own = R;
+        own.row0 = m0 + (2 * decltype(I)::value + half) * 32;
+        return own;
+    };
+    auto own = [&](auto&& f) { // (GATED: of a wave pair (gate, up) of the same columns the one finishes block 0, the other block 1)
+        static_for<kOwn>([&](auto I) {
+            if (2 * decltype(I)::value + half < MT && (!GATED || decltype(I)::value == (int)is_up)) f(I);
+        });
+    };
+    RowPieces<32, 4, 0, 4> pieces_f32[kOwn];
+    RowPieces<32, 8, 0, 2> pieces_bf16[kOwn];
+    if (whole) own([&](auto I) {
+        if (f32_out) pieces_f32[decltype(I)::value].request(rows_of(I), lane);
+        else pieces_bf16[decltype(I)::value].request(rows_of(I), lane);
+    });
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); // (every activation request has been waited for)
 
-    // ---- the two halves' sums: the wave of half p finishes the 32-row blocks i with i % 2 = p
-    constexpr int kOwn = (MT + 1) / 2;
+    // ---- the two halves' sums
     f32x16 sum[kOwn];
     {
         uint8_t* dst = smem + wc * (MT * 4096) + lane * 16;
@@ -405,8 +432,6 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
         if (half) take(std::integral_constant<int, 1>{});
         else take(std::integral_constant<int, 0>{});
     }
-    // GATED: of a wave pair (gate, up) of the same columns the one finishes block 0, the other block 1
-    const bool is_up = GATED && wc >= kCols / 2; // uniform
     if constexpr (GATED) {
         uint8_t* at = smem + kCols * MT * 4096 + (2 * col32 + half) * 8192 + lane * 16; // (behind the halves' sums)
         auto put = [&](const f32x16& v, int slot) {
@@ -427,34 +452,37 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
                 for (int e = 0; e < 4; e++) sum[1][4 * r + e] = silu(v[e]) * sum[1][4 * r + e];
             }
     }
-    const bool split = slices > 1;
-    const int64_t gn = n0 + col32 * 32 + (lane & 31);
-    const int64_t gm0 = m0 + half * 32 + 4 * h;
-    const int rows = gn < n ? (int)min((int64_t)BM, P.m - gm0) : 0; // of this lane's column, from gm0 on
-    auto emit = [&](auto MODE) { // 0: f32, 1: f32 + residual, 2: bf16, 3: bf16 + residual
-        constexpr int mode = decltype(MODE)::value;
-        float* yf = (split ? partial + (int64_t)slice * P.m * n : static_cast<float*>(y)) + gm0 * n + gn;
-        uint16_t* yb = static_cast<uint16_t*>(y) + gm0 * n + gn;
-        const float* rf = static_cast<const float*>(P.residual) + gm0 * n + gn;
-        const uint16_t* rb = static_cast<const uint16_t*>(P.residual) + gm0 * n + gn;
-        static_for<kOwn>([&](auto I) {
-            static_for<16>([&](auto R) {
-                constexpr int i = decltype(I)::value, r = decltype(R)::value, row = 64 * i + 8 * (r >> 2) + (r & 3);
-                if (row < rows && (2 * i + half < MT) && (!GATED || i == (int)is_up)) {
-                    const int64_t at = row * n;
-                    float v = sum[i][r];
-                    if (mode == 1) v += rf[at];
-                    if (mode == 3) v += qmm_bf16_bits_to_f32(rb[at]);
-                    if (mode < 2) yf[at] = v;
-                    else yb[at] = (uint16_t)pack_bf16(v, v);
-                }
+    // A block goes where the wave has read the other half's sums of it: chunk c (four columns) of row r at chunk c ^ (r / 2 % 8)
+    auto block_at = [&](int i, int row, int col) {
+        return smem + wc * (MT * 4096) + (2 * i + half) * 4096 + row * 128 + (((col >> 2) ^ ((row >> 1) & 7)) << 4) + (col & 3) * 4;
+    };
+    auto keep = [&](auto I) {
+        constexpr int i = decltype(I)::value;
+        static_for<4>([&](auto G) {
+            constexpr int g = decltype(G)::value;
+            *reinterpret_cast<f32x4*>(block_at(i, lane & 31, 8 * g + 4 * h)) =
+                f32x4{sum[i][4 * g], sum[i][4 * g + 1], sum[i][4 * g + 2], sum[i][4 * g + 3]};
+        });
+    };
+    auto finish = [&](auto& pieces) {
+        own(keep);
+        own([&](auto I) {
+            pieces[decltype(I)::value].store(rows_of(I), lane, [&](int row, int col) {
+                return *reinterpret_cast<const f32x4*>(block_at(decltype(I)::value, row, col));
             });
         });
     };
-    if (split || !(P.out_bf16 || P.residual)) emit(std::integral_constant<int, 0>{});
-    else if (!P.out_bf16) emit(std::integral_constant<int, 1>{});
-    else if (!P.residual) emit(std::integral_constant<int, 2>{});
-    else emit(std::integral_constant<int, 3>{});
+    if (whole) {
+        if (f32_out) finish(pieces_f32);
+        else finish(pieces_bf16);
+    } else {
+        own([&](auto I) {
+            auto one = [&](int row, int col) { return *reinterpret_cast<const float*>(block_at(decltype(I)::value, row, col)); };
+            keep(I);
+            if (f32_out) store_values<32, true>(rows_of(I), lane, one);
+            else store_values<32, false>(rows_of(I), lane, one);
+        });
+    }
 }
 
 // y = sum over slices (in order) of partial[slice] (+ residual), four consecutive values per thread, all
@@ -478,24 +506,24 @@ __global__ __launch_bounds__(256) void regb_reduce_kernel(RegbReduceParams P) {
             slices = P.slices[i], first_block = P.block_end[i - 1], count = P.count[i], partial = P.partial[i], y = P.y[i];
     const int64_t i = ((int64_t)(blockIdx.x - first_block) * 256 + threadIdx.x) * 4;
     partial += i;
-    const QmmEpilogue ep{P.residual, P.out_bf16};
-    if (i + 4 <= count && (count & 3) == 0) {
+    if (i + 4 <= count && (count & 3) == 0 && ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(P.residual)) & 15) == 0) {
+        f32x4 res = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (P.residual && P.out_bf16) {
+            const u32x2 v = *reinterpret_cast<const u32x2*>(static_cast<const uint16_t*>(P.residual) + i);
+            res = f32x4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u)};
+        } else if (P.residual) {
+            res = *reinterpret_cast<const f32x4*>(static_cast<const float*>(P.residual) + i);
+        }
         f32x4 sum = *reinterpret_cast<const f32x4*>(partial);
         for (int s = 1; s < slices; s++) sum += *reinterpret_cast<const f32x4*>(partial + s * count);
-        if (ep.residual) // (all of it before the stores: it may be the output buffer)
-            sum += ep.y_bf16 ? f32x4{qmm_bf16_bits_to_f32(static_cast<const uint16_t*>(ep.residual)[i]),
-                                     qmm_bf16_bits_to_f32(static_cast<const uint16_t*>(ep.residual)[i + 1]),
-                                     qmm_bf16_bits_to_f32(static_cast<const uint16_t*>(ep.residual)[i + 2]),
-                                     qmm_bf16_bits_to_f32(static_cast<const uint16_t*>(ep.residual)[i + 3])}
-                             : f32x4{static_cast<const float*>(ep.residual)[i], static_cast<const float*>(ep.residual)[i + 1],
-                                     static_cast<const float*>(ep.residual)[i + 2], static_cast<const float*>(ep.residual)[i + 3]};
-#pragma unroll
-        for (int e = 0; e < 4; e++) qmm_store(y, QmmEpilogue{nullptr, ep.y_bf16}, i + e, sum[e]);
+        if (P.residual) sum += res;
+        if (P.out_bf16) *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(y) + i) = u32x2{pack_bf16(sum.x, sum.y), pack_bf16(sum.z, sum.w)};
+        else *reinterpret_cast<f32x4*>(static_cast<float*>(y) + i) = sum;
     } else {
         for (int e = 0; e < 4 && i + e < count; e++) {
             float sum = partial[e];
             for (int s = 1; s < slices; s++) sum += partial[s * count + e];
-            qmm_store(y, ep, i + e, sum);
+            qmm_store(y, QmmEpilogue{P.residual, P.out_bf16}, i + e, sum);
         }
     }
 }
@@ -506,8 +534,8 @@ struct RegbPlan {
 
 // Slices of k for n columns in `tiles` full-height tiles, in microseconds: a unit costs 1.2 where the row tiles are as
 // low as the compute units allow; the slices' sums a launch (4.2) and their bytes twice.
-int slices_of(int64_t tiles, int64_t n, int64_t m, int k_units, int64_t limit, int min_units, double unsplit_cost) {
-    double best = 1.2 * k_units + unsplit_cost;
+int slices_of(int64_t tiles, int64_t n, int64_t m, int k_units, int64_t limit, int min_units) {
+    double best = 1.2 * k_units;
     int slices = 1;
     for (int s = 2; s <= 8 && tiles * s <= limit; s++) {
         const int su = (k_units + s - 1) / s;
@@ -543,10 +571,8 @@ RegbPlan plan_regb(const QmmLayout* const* layouts, int n_weights, int64_t m, in
         p.slices[i] = 1, p.slice_units[i] = k_units;
         if (i >= n_weights) continue;
         const bool alone = m <= 64 || layouts[i]->k > 2 * layouts[i]->n;
-        // (one product may carry a residual, whose reads in front of the stores cost 2 to 4 us where k is not split: Q8_0
-        // 4096 x 4096 at 500 rows, bf16, 36 us in one slice, 34 in two)
-        p.slices[i] = m <= 128 ? slices_of(tiles[i], layouts[i]->n, m, k_units, alone ? n_cus : n_cus / 2, min_units, 0.0)
-                               : slices_of(all_tiles, n_total, m, k_units, n_cus, min_units, n_weights == 1 ? 3.0 : 0.0);
+        p.slices[i] = m <= 128 ? slices_of(tiles[i], layouts[i]->n, m, k_units, alone ? n_cus : n_cus / 2, min_units)
+                               : slices_of(all_tiles, n_total, m, k_units, n_cus, min_units);
         p.slice_units[i] = (k_units + p.slices[i] - 1) / p.slices[i];
         cols += tiles[i] / full_tiles * p.slices[i];
     }

@@ -197,6 +197,29 @@ def test_rows_that_do_not_start_on_sixteen_bytes(qa, oracle, dtype, m, n, k, ski
             assert torch.equal(a, b)
 
 
+# results and residuals that start on 2, 4 or 16 bytes, rows of a multiple of eight values and not, k whole and in slices: the
+# same sums, so the same bits
+@pytest.mark.parametrize("dtype,m,n,k", [(Q4_K, 97, 520, 256), (Q8_0, 70, 515, 288), (Q6_K, 129, 100, 512), (Q4_K, 300, 1032, 1024), (Q4_K, 101, 516, 4096),
+                                         (Q8_0, 65, 131, 4096)])
+def test_results_and_residuals_by_alignment(qa, oracle, dtype, m, n, k):
+    mm = weight(qa, oracle, dtype, n, k, 93)
+    x = torch.from_numpy(oracle.randn(94, (m, k))).cuda().to(torch.bfloat16)
+    y = mm.forward_bf16_to_f32(x)
+    assert off(y, x.double() @ dense(mm).t()) < F32_TOL
+    for out_dtype in (torch.float32, torch.bfloat16):
+        res = torch.from_numpy(oracle.randn(95, (m, n))).cuda().to(out_dtype)
+        total = (y + res.float()).to(out_dtype)
+
+        def at(skip):
+            return torch.zeros(m * n + 32, dtype=out_dtype, device="cuda")[skip:skip + m * n].view(m, n)
+
+        for to, of in ((0, 0), (1, 0), (0, 2), (8, 8), (1, 1)):
+            out, r = at(to), at(of).copy_(res)
+            assert torch.equal(mm.forward_fused(x, out=out, out_dtype=out_dtype), y.to(out_dtype))
+            assert torch.equal(mm.forward_fused(x, residual=r, out=out, out_dtype=out_dtype), total), (out_dtype, to, of)
+            assert torch.equal(r, res)
+
+
 def test_copied_rows_in_a_captured_graph(qa, oracle):
     """The copy of rows that do not start on 16 bytes is part of the graph: every replay reads the rows of its time."""
     m, n, k = 100, 300, 512
