@@ -1138,7 +1138,9 @@ int decode_attention_impl(const T* q, const T* k, const T* v, int64_t num_heads,
         P.k_append = (float*)ki.dev, P.v_append = (float*)vi.dev;
         P.eps = prep->eps;
     }
-    if (head_dim <= 128 && kv_len <= kOneLaunchPositions && num_heads <= n_cus) {
+    // (whoever sets a split's size asks for splits)
+    static const bool splits_asked = getenv("IZWI_ATTN_WGS_PER_CU") || getenv("IZWI_ATTN_MIN_CHUNK");
+    if (head_dim <= 128 && kv_len <= kOneLaunchPositions && num_heads <= n_cus && !splits_asked) {
         OPS_TRY((head_dim == 64 ? launch_attn_one<T, 64>(P, stream) : launch_attn_one<T, 128>(P, stream)));
         OPS_TRY(oo.finish(stream));
         return IZWI_QMM_OK;

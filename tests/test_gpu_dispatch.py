@@ -29,6 +29,10 @@ def call(kind, *sizes):
         E, hidden, inter, top_k, t = sizes
         layer, x, logits = experts(E, hidden, inter), torch.randn(t, hidden, device="cuda"), torch.randn(t, E, device="cuda")
         return lambda: layer.layer(logits, x, top_k)
+    if kind == "attention":
+        heads, kv_heads, d, positions = sizes
+        q, cache = torch.randn(1, heads, 1, d, device="cuda"), torch.randn(1, kv_heads, positions, d, device="cuda")
+        return lambda: qa.try_fused_decode_gqa_attention(q, cache, cache, heads, kv_heads, d, d ** -0.5)
     n, k, m = sizes
     mm, x = matrix(n, k), torch.randn(m, k, device="cuda")
     return lambda: mm.forward(x)
@@ -83,3 +87,15 @@ def test_prefill_kernels_by_size_and_by_the_environment():
     forced = kernels(cases, IZWI_QMM_GEMM_TILE="256,128,2")
     assert all("gemm_regb_kernel" not in names and "gemm_pipe_kernel" in names for names in forced)
     assert ["splitk_reduce_kernel" in names for names in forced] == [True, False, False]  # (k = 256 is one unit)
+
+
+def test_attention_splits_of_the_environment():
+    """IZWI_ATTN_WGS_PER_CU and IZWI_ATTN_MIN_CHUNK size the splits at every length of the cache, the short ones
+    that otherwise take one launch included."""
+    cases = [["attention", 16, 8, 128, 300], ["attention", 8, 2, 64, 40]]
+    assert all("attn_one_kernel" in names for names in kernels(cases))
+    for env in ({"IZWI_ATTN_MIN_CHUNK": "32"}, {"IZWI_ATTN_WGS_PER_CU": "1"}):
+        for names in kernels(cases, **env):
+            assert "attn_partial_kernel" in names and "attn_merge" in names and "attn_one_kernel" not in names
+    whole = kernels(cases, IZWI_ATTN_MIN_CHUNK="300")  # one split: no merge
+    assert all("attn_partial_kernel" in names and "attn_merge" not in names for names in whole)
