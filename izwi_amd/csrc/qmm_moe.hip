@@ -187,17 +187,17 @@ __device__ __forceinline__ int wave_inclusive_sum(int v, int lane) {
     return v;
 }
 
-// The whole stable counting sort in ONE workgroup (pairs up to 16384 where the wide sort does not apply, n_experts up to 1024 as far as
+// The whole stable counting sort in ONE workgroup (pairs up to 4096, n_experts below 1024 as far as
 // LDS holds runs x experts counters): pairs are cut into runs of 64 (one wave each); a lane finds its
 // rank among the equal ids of its run through per-expert bit masks; the runs' per-expert counts are
-// scanned run by run (a wave per expert, a lane per run) and over the experts (wave scans); every
+// scanned run by run (a thread per expert) and over the experts (wave scans); every
 // pair goes to offsets[e] + (pairs of e in earlier runs) + rank.  Integer arithmetic whose result does
 // not depend on the order of execution: the same perm / offsets as the three-kernel sort.
 // `ids`: the pairs' experts, in global memory or in LDS (the one-launch plan of small batches routes
 // them there first).  `sh`: block_sort_lds_ints(pairs, n_experts) ints of LDS.  Called by all
 // kBlockSortThreads threads of the workgroup.
-constexpr int kBlockSortThreads = 1024, kBlockSortMaxRuns = 16; // runs per wave
-constexpr int kBlockSortMaxLds = 152 * 1024; // (of the CU's 160 KB: 16384 pairs of 128 experts take 149 KB)
+constexpr int kBlockSortThreads = 1024, kBlockSortMaxRuns = 4; // runs per wave
+constexpr int kBlockSortMaxLds = 152 * 1024; // (of the CU's 160 KB: 2688 pairs of 513 experts take 151.5 KB)
 __host__ __device__ inline int64_t block_sort_lds_ints(int64_t pairs, int n_experts) {
     return ((pairs + 63) / 64) * (n_experts | 1) + n_experts + 1 + (int64_t)2 * n_experts * (kBlockSortThreads / 64);
 }
@@ -234,32 +234,16 @@ __device__ __forceinline__ void block_sort_body(const int32_t* ids, int pairs, i
         if (e >= 0 && e < n_experts && rank == 0) sh[run * stride + e] = total; // the first of its expert in the run
     }
     __syncthreads();
-    // per expert (a wave each, in turn): the runs' counts become the number of earlier pairs of the
-    // expert; lane = run, 64 runs per step
-    // (few runs: a thread per expert walks them - consecutive experts, consecutive LDS words - instead
-    // of eight wave scans in a row per wave with two lanes in use)
-    if (runs <= 64) {
-        for (int e = threadIdx.x; e < n_experts; e += kBlockSortThreads) {
-            int carry = 0;
-            for (int r = 0; r < runs; r++) {
-                const int h = sh[r * stride + e];
-                sh[r * stride + e] = carry;
-                carry += h;
-            }
-            start[e] = carry;
+    // per expert (a thread each: consecutive experts, consecutive LDS words): the runs' counts become the number
+    // of earlier pairs of the expert
+    for (int e = threadIdx.x; e < n_experts; e += kBlockSortThreads) {
+        int carry = 0;
+        for (int r = 0; r < runs; r++) {
+            const int h = sh[r * stride + e];
+            sh[r * stride + e] = carry;
+            carry += h;
         }
-    } else {
-        for (int e = wave; e < n_experts; e += waves) {
-            int carry = 0;
-            for (int r0 = 0; r0 < runs; r0 += 64) {
-                const int r = r0 + lane;
-                const int h = r < runs ? sh[r * stride + e] : 0;
-                const int inc = wave_inclusive_sum(h, lane);
-                if (r < runs) sh[r * stride + e] = carry + inc - h;
-                carry += __shfl(inc, 63);
-            }
-            if (lane == 0) start[e] = carry; // the expert's total, for now
-        }
+        start[e] = carry;
     }
     __syncthreads();
     // exclusive scan over the experts: thread e holds expert e (n_experts <= 1024), wave scans, then the
@@ -568,9 +552,10 @@ int64_t qmm_moe_sort_scratch_ints(int64_t pairs, int n_experts) {
 // Most pairs for the one workgroup: its time grows with the pairs, that of the two launches of many workgroups does not.  us a
 // sort in a graph, one workgroup / two launches: 128 experts 5.3 / 6.3 at 1024 pairs, 6.4 / 6.5 at 2048, 8.8 / 6.6 at 4096, 13.6 /
 // 6.9 at 8192, 22.3 / 7.2 at 16384; 8 experts 6.1 / 6.2, 7.8 / 6.2 and 13.4 / 6.4 at 2048, 4096 and 16384.  Where the ranked experts
-// are wanted, which the one workgroup leaves in passing and each later launch otherwise finds by itself (3 us a layer), up to 4096.  The layer (128 experts, top-8,
-// 2048 x 768, Q4_K): 215 -> 196 at 1024 tokens, 251 -> 242 at 1500 and 316 -> 298 at 2048, with the order of the long items.
-constexpr int64_t kBlockSortPairs = 2048, kRankingSortPairs = 4096;
+// are wanted, which the one workgroup leaves in passing and each later launch otherwise finds by itself (3 us a layer), as many as it holds (4096).
+// With more experts than the two launches count what is left are three launches with a serial scan (513 experts: 7.8 / 136 at 2049
+// pairs, 8.7 / 138 at 2688): there the one workgroup as far as its LDS reaches.
+constexpr int64_t kBlockSortPairs = 2048;
 hipError_t qmm_launch_moe_sort(const int32_t* ids, int64_t pairs, int n_experts, int32_t* perm,
                                int32_t* offsets, int32_t* seg_offsets, int32_t* scratch,
                                hipStream_t stream, int seg_rows, int32_t* seg_expert, int64_t max_segments,
@@ -578,7 +563,7 @@ hipError_t qmm_launch_moe_sort(const int32_t* ids, int64_t pairs, int n_experts,
     if (seg_rows < 1 || max_segments > 0x7fffffff) return hipErrorInvalidValue;
     if (n_experts < 1 || n_experts > 8192) return hipErrorInvalidValue;
     if (expert_order && !qmm_moe_sort_ranks_experts(pairs, n_experts)) return hipErrorInvalidValue;
-    if (block_sort_fits(pairs, n_experts) && (expert_order || pairs <= kBlockSortPairs)) {
+    if (block_sort_fits(pairs, n_experts) && (expert_order || pairs <= kBlockSortPairs || n_experts > kWideSortMaxExperts)) {
         const size_t lds = (size_t)block_sort_lds_ints(pairs, n_experts) * sizeof(int32_t);
         if (lds > 48 * 1024) {
             hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&sort_block_kernel),
@@ -614,7 +599,7 @@ hipError_t qmm_launch_moe_sort(const int32_t* ids, int64_t pairs, int n_experts,
     return hipGetLastError();
 }
 
-bool qmm_moe_sort_ranks_experts(int64_t pairs, int n_experts) { return pairs <= kRankingSortPairs && block_sort_fits(pairs, n_experts); }
+bool qmm_moe_sort_ranks_experts(int64_t pairs, int n_experts) { return block_sort_fits(pairs, n_experts); }
 
 bool qmm_moe_segments_rank_experts(int n_experts) { return n_experts <= kSegmentsRankedExperts; }
 

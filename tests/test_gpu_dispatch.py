@@ -33,6 +33,10 @@ def call(kind, *sizes):
         heads, kv_heads, d, positions = sizes
         q, cache = torch.randn(1, heads, 1, d, device="cuda"), torch.randn(1, kv_heads, positions, d, device="cuda")
         return lambda: qa.try_fused_decode_gqa_attention(q, cache, cache, heads, kv_heads, d, d ** -0.5)
+    if kind == "sort":
+        E, pairs = sizes
+        ids = torch.randint(0, E, (pairs, 1), device="cuda", dtype=torch.int32)
+        return lambda: qa.moe_sort(ids, E)
     n, k, m = sizes
     mm, x = matrix(n, k), torch.randn(m, k, device="cuda")
     return lambda: mm.forward(x)
@@ -99,3 +103,13 @@ def test_attention_splits_of_the_environment():
             assert "attn_partial_kernel" in names and "attn_merge" in names and "attn_one_kernel" not in names
     whole = kernels(cases, IZWI_ATTN_MIN_CHUNK="300")  # one split: no merge
     assert all("attn_partial_kernel" in names and "attn_merge" not in names for names in whole)
+
+
+def test_sort_launches():
+    """One workgroup up to 2048 pairs, two launches of many beyond; with more experts than those count (512) one
+    workgroup as far as its LDS reaches, and only then the three launches with a serial scan."""
+    cases = [["sort", 128, 2048], ["sort", 128, 2049], ["sort", 512, 2049], ["sort", 513, 2049], ["sort", 513, 2688], ["sort", 589, 2049],
+             ["sort", 513, 2689]]
+    forms = [tuple(f in names for f in ("sort_block_kernel", "sort_wide_kernel", "sort_scan_kernel")) for names in kernels(cases)]
+    block, wide, scan = (True, False, False), (False, True, False), (False, False, True)
+    assert forms == [block, wide, wide, block, block, block, scan]

@@ -113,7 +113,8 @@ def test_layer_equals_the_tile_kernels(qa, oracle, t):
 
 @pytest.mark.parametrize("pairs,experts", [
     (2048, 128), (2049, 128), (2049, 511), (4097, 1), (5000, 512),  # around one workgroup's sort
-    (16384, 513), (16385, 128),   # as many pairs as one workgroup can sort (where the wide sort does not apply), and one more
+    (2688, 513), (2689, 513), (2049, 589), (16384, 513),  # more experts than the wide sort counts: as many pairs as one workgroup's LDS holds, more
+    (64, 1023), (16385, 128),
     (17 * 1024, 1), (40001, 3), (20000, 511), (20000, 512),
     (20000, 513),   # more experts than a workgroup of the wide sort counts
     (512 * 1024, 128), (512 * 1024 + 1, 128),  # the most workgroups, and one pair beyond them
