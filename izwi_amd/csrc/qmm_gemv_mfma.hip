@@ -1663,15 +1663,18 @@ bool straight_line_fits(int64_t groups, int waves, int n_cus) {
 namespace {
 // The launch of a single-stage form whose workgroups quantize their own activations (P.ws: the f32 rows).
 // P is set up for the form on records; a workgroup gets more row tiles where its 16-lane groups would otherwise
-// have more than own_runs units to quantize, or a compute unit several workgroups one after the other that each quantize
-// the same rows (gate | up of 2 x 3072 at k = 1024 and 64 rows: four row tiles of rows times 64 workgroups of six
-// waves instead of 192 of two, and the quantizer launch goes: 8 layers of 0.6B projections 348 -> 338 us in a graph, 480 -> 400
-// called from Python).  hipErrorNotSupported where the quantizer launch is the cheaper
+// have more than own_runs units to quantize.  hipErrorNotSupported where the quantizer launch is the cheaper
 // one, by the activation bytes that a compute unit reads for its workgroups one after the other: a launch and the
 // gap behind it are 4 us, the loads, the quantizer's 140 instructions per (row, unit) and 16 lanes and a barrier in every workgroup
 // about 2 at 64 KB.  Layer of projections in a graph, us, with the launch / without at this limit / at 128 KB: 0.6B
 // Q8_0 5 rows 38.7 / 32.9 / 33.3, 8 rows 38.8 / 35.1 / 35.5, 16 rows 39.4 / 38.5 / 41.0, 64 rows 45.3 / 43.4 / 46.5; 8B Q4_K
 // 3 rows 55.6 / 53.3 / 53.6, 8 rows 57.1 / 57.2 / 59.9; 8B Q8_0 4 rows 80.5 / 78.4 / 77.6, 8 rows 81.1 / 81.1 / 82.7.
+// Beyond the limit workgroups may also get as tall as it takes for every compute unit to have one, which then quantizes its
+// rows once, or else for fewer rounds within the limit (groups at k = 1024, us with the launch / so: Q4_K 2 x 3072 at 64 rows 8.5 / 7.6, 2 x 4096 at 64 8.8 / 7.9, Q8_0 2 x 3072
+// at 40 9.3 / 8.5, 2 x 9728 at 20 14.2 / 11.1; k = 768: Q8_0 2 x 6144 at 48 13.6 / 12.6, 2 x 8960 at 56, two rounds for four, 21.0 / 17.6; k = 1536: Q8_0 2 x 2048 at 50 10.8 / 10.1, Q4_K 2 x 6144 at 17 10.5 / 9.2).  One
+// too many on some compute unit and the launch takes a round more: workgroups of five waves and more do not share one (Q4_K 9728 + 1024 + 1024
+// at k = 1024, 33 workgroups of nine waves for the 32 compute units of an XCD, 9.7 / 15.4; Q8_0 2 x 6144 at k = 768 and 48 rows, workgroups of five, 13.6 / 17.2).  Not for
+// Q6_K, whose unpacking next to the quantizer is the longer part: 9728 at 32 rows 10.6 / 11.3, 2 x 3072 at k = 1280 and 64 rows 13.5 / 14.7.
 constexpr int64_t kOwnQuantizerBytes = 96 * 1024;
 hipError_t launch_own_quantizer(const QmmLayout& L0, MfmaParams P, int64_t x_k, int n_cus, bool epilogue, hipStream_t stream) {
     // (an output that overlaps the activations: they have to be read whole before a sum is stored)
@@ -1691,12 +1694,33 @@ hipError_t launch_own_quantizer(const QmmLayout& L0, MfmaParams P, int64_t x_k, 
         for (int i = 0; i < P.n_weights; i++) groups += (P.row_tiles_v[i] + per - 1) / per;
         return groups;
     };
+    // workgroups one after the other on a compute unit; of up to four waves three run side by side (tiles of rows: the workgroups of
+    // an XCD are whole row groups, all tiles of each)
+    auto rounds_of = [&](int per) {
+        const int64_t groups = groups_of(per), side_by_side = P.nwk * per <= 4 ? 3 : 1;
+        const int64_t wgs_xcd = P.n_tiles > 1 ? (groups + 7) / 8 * P.n_tiles : (groups + 7) / 8;
+        return std::max<int64_t>(1, (wgs_xcd + n_cus / 8 * side_by_side - 1) / std::max<int64_t>(1, n_cus / 8 * side_by_side));
+    };
+    auto one_per_cu = [&](int per) { return P.n_tiles > 1 ? (groups_of(per) + 7) / 8 * P.n_tiles <= n_cus / 8 : groups_of(per) <= n_cus; };
+    int64_t limit = 0; // what the fewest row tiles that leave a group own_runs units come to
+    int taller = 0;
     for (;; nwr++) {
-        if (P.nwk * nwr > kMaxWaves) return hipErrorNotSupported;
+        if (P.nwk * nwr > kMaxWaves) {
+            if (!taller) return hipErrorNotSupported;
+            nwr = taller;
+        }
         wgs = groups_of(nwr) * P.n_tiles;
         straight = full && (!q4k || straight_line_fits(wgs, P.nwk * nwr, n_cus));
+        if (nwr == taller) break;
         if (items > 4 * P.nwk * nwr * own_runs(q4k && !straight)) continue;
-        if ((wgs + n_cus - 1) / n_cus * rows * x_k * 4 <= kOwnQuantizerBytes) break;
+        const bool reads_fit = (wgs + n_cus - 1) / n_cus * rows * x_k * 4 <= kOwnQuantizerBytes;
+        if (reads_fit && (!limit || (q4k && !straight))) break; // (the compact form's registers leave room for several anyway)
+        if (!limit) {
+            if (L0.dtype == QMM_Q6_K || rows * x_k * 4 > kOwnQuantizerBytes) return hipErrorNotSupported;
+            limit = rounds_of(nwr);
+        }
+        if (one_per_cu(nwr)) break;
+        if (!taller && rounds_of(nwr) < limit && rounds_of(nwr) * rows * x_k * 4 <= kOwnQuantizerBytes) taller = nwr;
     }
     const int n_weights = std::max(P.n_weights, 1);
     if (P.n_weights == 0) P.rt_groups = (P.row_tiles + nwr - 1) / nwr;

@@ -16,8 +16,8 @@ import numpy as np, torch
 import izwi_amd as qa
 from oracle import oracle
 
-def matrix(n, k):
-    return qa.QMatMul.from_qtensor(qa.QTensor.from_blocks(qa.GgmlDType.Q4K, oracle.quantize(12, oracle.randn(n, (n, k), std=0.02)), (n, k)))
+def matrix(n, k, dtype=12):
+    return qa.QMatMul.from_qtensor(qa.QTensor.from_blocks(qa.GgmlDType(dtype), oracle.quantize(dtype, oracle.randn(n, (n, k), std=0.02)), (n, k)))
 
 def experts(E, hidden, inter):
     one = {n * k: oracle.quantize(12, oracle.randn(n, (n, k), std=0.02)).reshape(-1) for n, k in ((inter, hidden), (hidden, inter))}
@@ -33,6 +33,10 @@ def call(kind, *sizes):
         heads, kv_heads, d, positions = sizes
         q, cache = torch.randn(1, heads, 1, d, device="cuda"), torch.randn(1, kv_heads, positions, d, device="cuda")
         return lambda: qa.try_fused_decode_gqa_attention(q, cache, cache, heads, kv_heads, d, d ** -0.5)
+    if kind == "group":
+        dtype, ns, k, m = sizes
+        parts, x = [matrix(n, k, dtype) for n in ns], torch.randn(m, k, device="cuda")
+        return lambda: qa.forward_group(parts, x)
     if kind == "sort":
         E, pairs = sizes
         ids = torch.randint(0, E, (pairs, 1), device="cuda", dtype=torch.int32)
@@ -113,3 +117,11 @@ def test_sort_launches():
     forms = [tuple(f in names for f in ("sort_block_kernel", "sort_wide_kernel", "sort_scan_kernel")) for names in kernels(cases)]
     block, wide, scan = (True, False, False), (False, True, False), (False, False, True)
     assert forms == [block, wide, wide, block, block, block, scan]
+
+
+def test_taller_workgroups_of_the_batched_decode():
+    """Workgroups grow until they may quantize their rows themselves only where every compute unit then has one, or
+    they take fewer rounds; elsewhere the quantizer is a launch of its own."""
+    cases = [["group", 8, [3072, 3072], 1024, 64], ["group", 12, [9728, 1024, 1024], 1024, 48], ["group", 8, [8960, 8960], 768, 56],
+             ["group", 8, [8960, 8960], 256, 56], ["group", 8, [12288, 1024, 1024], 1024, 64], ["group", 8, [12288, 1024, 1024], 768, 64]]
+    assert ["quantize_ws_kernel" in names for names in kernels(cases)] == [False, False, False, False, True, True]

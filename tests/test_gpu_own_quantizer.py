@@ -15,6 +15,7 @@ pytestmark = pytest.mark.gpu
     (12, 24, 768, 5), (12, 500, 1024, 64), (12, 72, 1280, 33), (12, 4100, 1024, 15), (12, 40, 4096, 3), (12, 4096, 4096, 6),
     (14, 33, 512, 7), (14, 1000, 1024, 49), (14, 40, 4096, 3),
     (8, 3072, 1024, 64), (8, 2050, 992, 49), (12, 6000, 1024, 40), (14, 3072, 768, 64),  # taller workgroups, alone and in the group
+    (12, 3244, 1024, 48), (8, 6144, 768, 60),  # as tall as it takes for one per compute unit (of each XCD, too); more than that
 ])
 def test_own_quantizer_equals_records(qa, oracle, dtype, n, k, m):  # noqa: F811
     import torch
