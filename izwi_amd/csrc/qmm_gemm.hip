@@ -522,12 +522,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_pipe_kernel(GemmParams P_in) {
     const bool whole = whole_pieces(R);
     static_for<MT>([&](auto I) {
         constexpr int i = decltype(I)::value;
+        lanes_exchange(); // (the rows before these have been read)
 #pragma unroll
         for (int j = 0; j < NT; j++)
 #pragma unroll
             for (int g = 0; g < 4; g++)
                 *reinterpret_cast<f32x4*>(out_lds + (lane & 31) * kOutStride + (j * 32 + 8 * g + 4 * (lane >> 5)) * 4) =
                     f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+        lanes_exchange();
         R.row0 = m0 + wm * (BM / WM) + i * 32;
         if (!whole && f32_out) store_values<COLS, true>(R, lane, one); // uniform
         else if (!whole) store_values<COLS, false>(R, lane, one);

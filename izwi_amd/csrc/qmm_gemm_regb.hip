@@ -464,8 +464,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
                 f32x4{sum[i][4 * g], sum[i][4 * g + 1], sum[i][4 * g + 2], sum[i][4 * g + 3]};
         });
     };
+    lanes_exchange(); // (the other half's sums have been read)
     auto finish = [&](auto& pieces) {
         own(keep);
+        lanes_exchange();
         own([&](auto I) {
             pieces[decltype(I)::value].store(rows_of(I), lane, [&](int row, int col) {
                 return *reinterpret_cast<const f32x4*>(block_at(decltype(I)::value, row, col));
@@ -479,6 +481,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
         own([&](auto I) {
             auto one = [&](int row, int col) { return *reinterpret_cast<const float*>(block_at(decltype(I)::value, row, col)); };
             keep(I);
+            lanes_exchange();
             if (f32_out) store_values<32, true>(rows_of(I), lane, one);
             else store_values<32, false>(rows_of(I), lane, one);
         });

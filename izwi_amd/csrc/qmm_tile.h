@@ -39,6 +39,13 @@ __device__ __forceinline__ void load_to_lds4(const uint8_t* base, uint32_t lane_
     asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(lane_off), "s"(base) : "memory", "m0");
 }
 
+// Between a wave's writes to LDS and its reads of what other lanes wrote, or the other way round: its LDS instructions run in
+// their order, this keeps the compiler from changing it (it sees one lane's addresses).  No instruction.
+__device__ __forceinline__ void lanes_exchange() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // A wave's 32 rows of results from (row0, col0) on, which stand as f32 in its own LDS, on their way to memory.
 struct RowsOut {
     void* out;            // the matrix of m x n values; columns from n_end on are not written
