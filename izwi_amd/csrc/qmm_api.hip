@@ -1384,12 +1384,13 @@ int gate_up_silu_impl(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, co
                       int mem_space, void* stream_, const float* norm_weight, float norm_eps);
 
 // gate | up at prefill sizes (m > 64, bf16 arithmetic) and silu(gate) * up as f32 or bf16, in
-// gate_up_prefill_bytes of scratch at `ws`: the two products | bf16 x | the group's workspace.
+// gate_up_prefill_bytes of scratch at `ws`: bf16 x and, where one launch does not do it all, the two products | the
+// group's workspace.
 size_t gate_up_prefill_bytes(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, int64_t m) {
     const QmmLayout& L = gate->layout;
     const izwi_qmm_weight* ws[2] = {gate, up};
-    const size_t part = ((size_t)m * L.n * sizeof(float) + 255) & ~(size_t)255;
-    return 2 * part + (((size_t)m * L.k * sizeof(uint16_t) + 255) & ~(size_t)255) + group_bf16_workspace(ws, 2, m);
+    const size_t part = ((size_t)m * L.n * sizeof(float) + 255) & ~(size_t)255, x = ((size_t)m * L.k * sizeof(uint16_t) + 255) & ~(size_t)255;
+    return qmm_gemm_regb_gated_applies(L, m, gate->n_cus) ? x : x + 2 * part + group_bf16_workspace(ws, 2, m);
 }
 
 int gate_up_prefill(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, const float* x, int64_t m, void* h, int h_bf16, uint8_t* ws,
@@ -1397,9 +1398,10 @@ int gate_up_prefill(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, cons
     const QmmLayout& L = gate->layout;
     const izwi_qmm_weight* gu[2] = {gate, up};
     const size_t part = ((size_t)m * L.n * sizeof(float) + 255) & ~(size_t)255;
-    void* ys[2] = {ws, ws + part};
-    uint16_t* xb = reinterpret_cast<uint16_t*>(ws + 2 * part);
-    uint8_t* group_ws = ws + 2 * part + (((size_t)m * L.k * sizeof(uint16_t) + 255) & ~(size_t)255);
+    uint16_t* xb = reinterpret_cast<uint16_t*>(ws);
+    uint8_t* products = ws + (((size_t)m * L.k * sizeof(uint16_t) + 255) & ~(size_t)255);
+    void* ys[2] = {products, products + part};
+    uint8_t* group_ws = products + 2 * part;
     ProfileScope prof(gate, stream);
     HIP_TRY(qmm_launch_f32_to_bf16(x, xb, m * L.k, stream));
     const hipError_t gated = qmm_launch_gemm_regb_gated(L, gate->tiled, up->tiled, xb, m, h, h_bf16, gate->n_cus, stream);

@@ -704,12 +704,18 @@ hipError_t qmm_launch_gemm_regb(const QmmLayout* const* layouts, const void* con
     return hipGetLastError();
 }
 
+bool qmm_gemm_regb_gated_applies(const QmmLayout& L, int64_t m, int n_cus) {
+    const QmmLayout* const pair[2] = {&L, &L};
+    if (!qmm_gemm_regb_applies(pair, 2, m, n_cus)) return false;
+    const RegbPlan plan = plan_regb(pair, 2, m, n_cus);
+    return plan.slices[0] == 1 && plan.slices[1] == 1;
+}
+
 hipError_t qmm_launch_gemm_regb_gated(const QmmLayout& L, const void* gate, const void* up, const uint16_t* x_bf16, int64_t m, void* h,
                                       int h_bf16, int n_cus, hipStream_t stream) {
+    if (!qmm_gemm_regb_gated_applies(L, m, n_cus)) return hipErrorNotSupported;
     const QmmLayout* const pair[2] = {&L, &L};
-    if (!qmm_gemm_regb_applies(pair, 2, m, n_cus)) return hipErrorNotSupported;
     const RegbPlan plan = plan_regb(pair, 2, m, n_cus);
-    if (plan.slices[0] > 1 || plan.slices[1] > 1) return hipErrorNotSupported;
     RegbParams P = base_params(L, plan, x_bf16, m, h_bf16);
     const int64_t cols = (L.n + kBN / 2 - 1) / (kBN / 2), grid = (cols + 7) / 8 * 8 * P.tiles_m;
     if (grid > 0x7fffffff) return hipErrorInvalidValue;

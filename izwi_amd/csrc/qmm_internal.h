@@ -267,7 +267,8 @@ hipError_t qmm_launch_gemm_regb(const QmmLayout* const* layouts, const void* con
                                 const uint16_t* x_bf16, int64_t m, void* const* ys, int out_bf16, void* workspace,
                                 int n_cus, hipStream_t stream, const void* residual = nullptr);
 // h = silu(gate x) * (up x), f32 or bf16, as one launch of that form (gate and up of one shape and type); the sums are those of
-// the group's launch.  hipErrorNotSupported, nothing launched, where the group takes another form or splits k.
+// the group's launch.  Where it does not apply (the group takes another form or splits k): hipErrorNotSupported, nothing launched.
+bool qmm_gemm_regb_gated_applies(const QmmLayout& L, int64_t m, int n_cus);
 hipError_t qmm_launch_gemm_regb_gated(const QmmLayout& L, const void* gate, const void* up, const uint16_t* x_bf16, int64_t m, void* h,
                                       int h_bf16, int n_cus, hipStream_t stream);
 // y[i] = t[i] (+ residual[i]) as f32 or bf16: the epilogue as a kernel of its own, for the forms

@@ -149,7 +149,8 @@ def test_gate_up_sums_equal_the_projections(qa, oracle, m):
 # silu(gate) * up in the products' own launch (k not split): one to four blocks of 32 rows per row tile, the last 64 columns
 # of gate and up whole and ragged, one column tile, k that ends inside a unit
 @pytest.mark.parametrize("dtype,m,n,k", [(Q4_K, 65, 64, 256), (Q4_K, 101, 200, 768), (Q8_0, 128, 100, 288), (Q6_K, 97, 1000, 512), (Q4_K, 70, 16400, 256),
-                                         (Q8_0, 96, 16400, 512), (Q4_K, 128, 8200, 512), (Q6_K, 129, 6000, 256), (Q8_0, 300, 3000, 768)])
+                                         (Q8_0, 96, 16400, 512), (Q4_K, 128, 8200, 512), (Q6_K, 129, 6000, 256), (Q8_0, 300, 3000, 768),
+                                         (Q6_K, 97, 1024, 512), (Q4_K, 101, 8192, 256), (Q8_0, 300, 3072, 768), (Q8_0, 65, 256, 288)])
 def test_gated_products(qa, oracle, dtype, m, n, k):
     print(f"gated dtype={dtype} m={m} n={n} k={k}", flush=True)
     gate, up, down = (weight(qa, oracle, dtype, *shape, 480 + i) for i, shape in enumerate([(n, k), (n, k), (256, n // 256 * 256 or 256)]))
@@ -162,6 +163,27 @@ def test_gated_products(qa, oracle, dtype, m, n, k):
     assert bool(((h.double() - want).abs() <= 6 * 2.0 ** -24 * want.abs() + 1e-30).all())
     if n % 256 == 0:
         assert torch.equal(qa.Qwen3Mlp(gate_up, down).forward(x), down.forward(h))
+
+
+def test_gated_products_reserve_no_room_for_the_separate_ones(qa, oracle):
+    """The scratch memory of a stream's first call: bf16 x (64 KB, and at least 1 MiB) and not two f32 products (2 x 32 MiB,
+    and half as much again) that the one launch does not write."""
+    from izwi_amd import capi
+    m, n, k = 128, 65536, 256
+    gate, up = (weight(qa, oracle, Q4_K, n, k, 490 + i) for i in range(2))
+    x, h = torch.randn(m, k, device="cuda"), torch.empty(m, n, device="cuda")
+
+    def call(stream):
+        capi.check(capi.lib().izwi_qmm_forward_gate_up_silu_f32(gate.qtensor._h, up.qtensor._h, x.data_ptr(), m, h.data_ptr(), capi.DEVICE,
+                                                                stream.cuda_stream))
+        torch.cuda.synchronize()
+
+    call(torch.cuda.current_stream())
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    call(stream)
+    assert free - torch.cuda.mem_get_info()[0] <= 32 << 20
 
 
 @pytest.mark.parametrize("dtype", [Q8_0, Q4_K])
