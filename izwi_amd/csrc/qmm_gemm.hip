@@ -685,13 +685,13 @@ int64_t tiles_of_192(const QmmLayout* const* layouts, int n_weights) {
     return n_weights > 0 && layouts[0]->dtype == QMM_Q6_K ? 0 : t;
 }
 
-GemmPlan plan_gemm(int64_t m, int64_t n, int k_steps, int n_cus, int64_t tiles_n192, bool group = false) {
-    // relative rate of a half-size tile: 256 of them at k = 4096 take 75 us (4096 x 4096 at 2048 rows), as many whole ones 121
-    const double kQ128 = 0.82;
-    // A 256 x 192 tile takes 0.79 of the time of a whole one.  Where whole tiles would fill the last round badly, us per call (2 x
+// `n_weights` members planned as one matrix of n columns (a group: more than one, or a split's sums per member)
+GemmPlan plan_gemm(int64_t m, int64_t n, int k_steps, int n_cus, int64_t tiles_n192, int n_weights = 1) {
+    const double kQ128 = 0.76; // relative rate of a half-size tile
+    // A 256 x 192 tile takes 0.82 of the time of a whole one.  Where whole tiles would fill the last round badly, us per call (2 x
     // 12288 x 4096, Q4_K): 112 -> 105 at 500 rows (192 whole tiles, 256 of these), 212 -> 182 at 640 (288, 384), 217 ->
     // 197 at 1000 (384, 512), 330 -> 290 at 1400 (576, 768); 2 x 3072 x 1024 42 -> 37 at 2048 rows (192, 256).
-    const double kCost192 = 0.79;
+    const double kCost192 = 0.82;
     const int hm = 256, hn = 128;
     {
         GemmPlan forced;
@@ -706,23 +706,26 @@ GemmPlan plan_gemm(int64_t m, int64_t n, int k_steps, int n_cus, int64_t tiles_n
     GemmPlan best{256, 256, 1, 0};
     double best_cost = rounds(tiles(256, 256, n)) * k_steps;
     auto consider = [&](GemmPlan p, double cost) {
-        if (cost < 0.97 * best_cost) best = p, best_cost = cost;
+        if (cost < 0.98 * best_cost) best = p, best_cost = cost;
     };
     consider({hm, hn, 1, 0}, rounds(tiles(hm, hn, n)) * k_steps * 0.5 / kQ128);
     if (tiles_n192 > 0) consider({256, 192, 1, 0}, rounds((m + 255) / 256 * tiles_n192) * k_steps * kCost192);
     // whole rounds of 256 x 256 tiles first, the remaining columns as half-size tiles
     const int64_t tiles_m256 = (m + 255) / 256, cols256 = (n + 255) / 256;
     const int64_t full_cols = (tiles_m256 * cols256 / n_cus) * n_cus / tiles_m256;
-    if (!group && full_cols > 0 && full_cols < cols256)
+    if (n_weights == 1 && full_cols > 0 && full_cols < cols256)
         consider({hm, hn, 1, full_cols},
                  (double)(tiles_m256 * full_cols / n_cus) * k_steps +
                      rounds(tiles(hm, hn, n - full_cols * 256)) * k_steps * 0.5 / kQ128);
-    // split along k: the slices' f32 tiles are written in the launch and read by a second one (3 us and 4.5 TB/s; a
-    // 256 x 256 k step takes 1.9 us).  4096 x 12288, us with a residual: 1100 rows 256 x 256 in two slices 182, 256 x 128 199,
-    // 256 x 192 in two slices 171; 2048 rows 198 / 211 / 260.  4096 x 4096: 1100 rows 70 / 66 / 60, 2048 rows 87 / 75 / 110.
+    // split along k: the slices' f32 tiles are written in the launch and read by a second one per member (4.5 us, and 2 TB/s for
+    // both ways; a 256 x 256 k step takes 1.9 us).  Constants from every form of 249 products (15 shapes, three types, 129 to 3000
+    // rows): the plan's form takes 1.001 of the best one's time in the mean, 1.045 at worst.  Priced at one launch and the
+    // reads alone (3 us, 4.5 TB/s), splits were taken where they cost 5 to 20 %: 2 x 6144 x 2048 at 400 rows 37.9 / 44.9 in two slices of
+    // 192 columns, 4096 x 12288 at 1400 rows 163 in two slices / 196 in eight, 8192 x 8192 at 1400 rows 203 / 237 in four.
+    // Where a split pays (bf16 residual): 4096 x 12288 at 1400 rows, 256 x 256 whole 252, in two slices 163.
     for (int slices = 2; slices <= 8; slices *= 2) {
         if (k_steps / slices < 8) break;
-        const double reduce_cost = (slices * (double)m * (double)n * 4.0 / 4.5e6 + 3.0) / 1.9;
+        const double reduce_cost = (slices * (double)m * (double)n * 4.0 / 2e6 + 4.5 * n_weights) / 1.9;
         const double steps = 4.0 * (double)((k_steps / 4 + slices - 1) / slices); // slices are whole units
         consider({256, 256, slices, 0}, rounds(tiles(256, 256, n) * slices) * steps + reduce_cost);
         if (tiles_n192 > 0)
@@ -762,7 +765,7 @@ int64_t group_columns(const QmmLayout* const* layouts, int n_weights) {
 
 template <int QT>
 hipError_t launch_group_qt(GemmParams P, int64_t n_planned, int64_t tiles_n192, int n_cus, hipStream_t stream) {
-    const GemmPlan plan = plan_gemm(P.m, n_planned, P.k_units * 4, n_cus, tiles_n192, true);
+    const GemmPlan plan = plan_gemm(P.m, n_planned, P.k_units * 4, n_cus, tiles_n192, P.n_weights);
     if (plan.slices > 1) {
         if (P.partial == nullptr) return hipErrorInvalidValue;
         float* base = P.partial;
@@ -801,7 +804,7 @@ size_t qmm_gemm_group_workspace_bytes(const QmmLayout* const* layouts, int n_wei
         return total;
     }
     const GemmPlan plan = plan_gemm(m, group_columns(layouts, n_weights), (int)layouts[0]->k_units * 4, n_cus,
-                                    tiles_of_192(layouts, n_weights), true);
+                                    tiles_of_192(layouts, n_weights), n_weights);
     if (plan.slices <= 1) return 0;
     size_t total = 0;
     for (int i = 0; i < n_weights; i++) total += (size_t)plan.slices * (size_t)m * (size_t)layouts[i]->n * sizeof(float);

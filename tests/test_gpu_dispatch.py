@@ -97,6 +97,14 @@ def test_prefill_kernels_by_size_and_by_the_environment():
     assert ["splitk_reduce_kernel" in names for names in forced] == [True, False, False]  # (k = 256 is one unit)
 
 
+def test_prefill_splits_where_they_pay():
+    """A split along k costs a launch per member and its sums both ways: one where few tiles meet a long k, none for a
+    product that 128-column tiles cover in one round."""
+    split = ["splitk_reduce_kernel" in names for names in kernels([["product", 11000, 1536, 300], ["group", 12, [6144, 6144], 2048, 400],
+                                                                   ["product", 2200, 6144, 2000]])]
+    assert split == [False, False, True]
+
+
 def test_attention_splits_of_the_environment():
     """IZWI_ATTN_WGS_PER_CU and IZWI_ATTN_MIN_CHUNK size the splits at every length of the cache, the short ones
     that otherwise take one launch included."""
