@@ -2002,8 +2002,7 @@ int moe_gemm(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, const izwi_
         e = qmm_launch_moe_gemm_gate_up(G, gate->tiled, up->tiled, ws + x_at, top_k, perm, offsets, chunks, owner, n_experts,
                                         pairs, max_chunks, ws + h_at, stream);
     if (e == hipSuccess)
-        e = qmm_launch_moe_gemm_down(D, down->tiled, ws + h_at, perm, offsets, chunks, owner, n_experts, pairs, max_chunks, y,
-                                     stream);
+        e = qmm_launch_moe_gemm_down(D, down->tiled, ws + h_at, perm, offsets, chunks, owner, n_experts, max_chunks, y, stream);
     if (e == hipSuccess) e = qmm_launch_moe_combine(y, weights, t, top_k, hidden, out, stream);
     if (e != hipSuccess) return fail_hip(e, "expert products");
     if (profiling()) g_silu_fused.fetch_add(1, std::memory_order_relaxed);

@@ -398,7 +398,7 @@ hipError_t qmm_launch_moe_gemm_gate_up(const QmmLayout& G, const void* gate, con
                                        hipStream_t stream);
 hipError_t qmm_launch_moe_gemm_down(const QmmLayout& D, const void* down, const void* records, const int32_t* perm,
                                     const int32_t* offsets, const int32_t* chunks, const int32_t* chunk_expert, int n_experts,
-                                    int64_t pairs, int64_t max_chunks, float* y, hipStream_t stream);
+                                    int64_t max_chunks, float* y, hipStream_t stream);
 // qmm_launch_moe_route that also writes the row records of the tokens' activation rows x [t, k]
 hipError_t qmm_launch_moe_route_rows(const float* logits, int64_t t, int n_experts, int top_k, int32_t* ids,
                                      float* weights, hipStream_t stream, const float* x, int64_t k, int dtype,

@@ -27,7 +27,7 @@
 // instructions (544 cycles), which two waves per SIMD overlap in part: at 4096 tokens the vector ALU is busy
 // 56 % of the cycles of gate | up and the matrix pipe 36 %.
 // 128 experts, top-8, 2048 x 768: gate | up 282 us and down 164 at 4096 tokens (730 and 630 TOP/s), where the
-// 16-row-tile kernels took 480 and 260 and the quantizer between them 40; 80 and 41 at 512 tokens (75 and 38 with the long
+// 16-row-tile kernels took 480 and 260 and the quantizer between them 40; 80 and 41 at 512 tokens (70 with the long
 // items first), before 92, 48 and 8 (a workgroup's life is 40 us there, 1.5 per compute unit).  The layer 823 -> 497 us and 156 -> 136.  Of that,
 // starting on the first unit's records while the others land, stores at 32-bit offsets and the two waves
 // of a SIMD half a phase apart with the one in its matrix instructions preferred: 556 -> 497 and 150 -> 136.
@@ -72,6 +72,7 @@ struct MoeGemmParams {
     int row_div;
     int n_experts, parts, n, row_tiles, k_units, k_groups, s, slots, panel_bytes;
     int out_units;
+    int fill2; // long items first: twice the short items asked for per place of the last round
 };
 
 __device__ __forceinline__ void barrier_lds() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
@@ -318,10 +319,10 @@ __global__ __launch_bounds__(64 * kWaves) void moe_gemm_q4k_kernel(MoeGemmParams
     const int slot = (int)(blockIdx.x >> 3), first = (int)(blockIdx.x & 7) * per_xcd;
     const int run = min(per_xcd, items - first); // items of this XCD
     if (slot >= run) return; // uniform
-    // Where a run is a few items per compute unit, those of more than 32 pairs go first (every wave looks at the
-    // whole run, a lane per item) and the short ones fill in behind them.
-    WorkItem it;
-    if (ORDERED && run <= kOrderedItems) {
+    // Where the last of an XCD's rounds can hold short items alone, those of more than 32 pairs go first (every wave looks at
+    // the whole run, a lane per item) and the short ones fill in behind them.
+    WorkItem it = work_item(P, first + slot);
+    if (ORDERED && run > kCusPerXcd && run <= kOrderedItems) {
         WorkItem mine[kOrderedPerLane];
         uint64_t heavy[kOrderedPerLane], light[kOrderedPerLane];
         int heavies = 0;
@@ -335,23 +336,24 @@ __global__ __launch_bounds__(64 * kWaves) void moe_gemm_q4k_kernel(MoeGemmParams
             light[j] = __ballot(exists && mine[j].pos_end - mine[j].pos_begin <= 32);
             heavies += __popcll(heavy[j]);
         }
-        int rank = slot < heavies ? slot : slot - heavies;
-        bool found = false;
+        const int lights = run - heavies, last_round = (run - 1) % kCusPerXcd + 1;
+        if (heavies > 0 && 2 * lights >= P.fill2 * last_round) { // uniform, the same in all workgroups of the run
+            int rank = slot < heavies ? slot : slot - heavies;
+            bool found = false;
 #pragma unroll
-        for (int j = 0; j < kOrderedPerLane; j++) {
-            const uint64_t set = slot < heavies ? heavy[j] : light[j];
-            const int in_set = __popcll(set);
-            if (!found && rank < in_set) { // uniform
-                const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(set >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)set, 0));
-                const int at = __ffsll((unsigned long long)__ballot((set >> lane & 1) && below == rank)) - 1;
-                it.e = __builtin_amdgcn_readlane(mine[j].e, at), it.part = __builtin_amdgcn_readlane(mine[j].part, at);
-                it.pos_begin = __builtin_amdgcn_readlane(mine[j].pos_begin, at), it.pos_end = __builtin_amdgcn_readlane(mine[j].pos_end, at);
-                found = true;
+            for (int j = 0; j < kOrderedPerLane; j++) {
+                const uint64_t set = slot < heavies ? heavy[j] : light[j];
+                const int in_set = __popcll(set);
+                if (!found && rank < in_set) { // uniform
+                    const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(set >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)set, 0));
+                    const int at = __ffsll((unsigned long long)__ballot((set >> lane & 1) && below == rank)) - 1;
+                    it.e = __builtin_amdgcn_readlane(mine[j].e, at), it.part = __builtin_amdgcn_readlane(mine[j].part, at);
+                    it.pos_begin = __builtin_amdgcn_readlane(mine[j].pos_begin, at), it.pos_end = __builtin_amdgcn_readlane(mine[j].pos_end, at);
+                    found = true;
+                }
+                rank -= in_set;
             }
-            rank -= in_set;
         }
-    } else {
-        it = work_item(P, first + slot);
     }
     const int e = it.e, part = it.part, pos_begin = it.pos_begin, pos_end = it.pos_end;
     const int nrb = pos_end - pos_begin > 32 ? 2 : 1;
@@ -445,7 +447,7 @@ __global__ void route_wide_rows_kernel(const float* __restrict__ logits, int64_t
 }
 
 template <bool GATE_UP, bool ORDERED>
-hipError_t launch_form(const MoeGemmParams& P, int64_t max_chunks, hipStream_t stream) {
+hipError_t launch(const MoeGemmParams& P, int64_t max_chunks, hipStream_t stream) {
     const size_t window = (size_t)P.k_units * kUnitLds, hbuf = GATE_UP ? (size_t)kRows * kHStride * 4 : 0;
     const size_t lds = window > hbuf ? window : hbuf;
     auto fn = &moe_gemm_q4k_kernel<GATE_UP, ORDERED>;
@@ -456,19 +458,19 @@ hipError_t launch_form(const MoeGemmParams& P, int64_t max_chunks, hipStream_t s
     return hipGetLastError();
 }
 
-// An item of up to 32 pairs is done in two thirds of the time of a longer one, and at one to three items per compute
-// unit a launch ends with whoever started a long one last.  The order pays where long items are about one per compute unit
-// and short ones follow: around the 22 to 32 pairs per expert at which a third to half of the experts have more than 32,
-// and around one chunk, where many experts spill a short second one.  us per layer (128 experts, top-8, 2048 x 768) in the
-// order of the experts / long ones first: 128.5 / 121 at 370 to 420 tokens, 145 / 137 at 512, 206 / 202 at 1000, 215 / 205 at
-// 1024.  Elsewhere finding the order costs up to two microseconds (200 tokens 113.5 / 114.5, 560 to 950 2 % more), and
-// from 80 pairs on an expert's chunks, set apart, read its weights again (1500 tokens 250 / 263, 4096 521 / 542).
-template <bool GATE_UP>
-hipError_t launch(const MoeGemmParams& P, int64_t pairs, int64_t max_chunks, hipStream_t stream) {
+// An item of up to 32 pairs is done in two thirds of the time of a longer one, and at one to four items per compute
+// unit a launch ends with whoever started a long one last.  Long ones first pays where short items fill the last round: the kernel
+// sees the counts and decides per XCD.  Here only where such counts are likely, because looking costs half a microsecond: around the 22 to
+// 32 pairs per expert at which a few to half of the experts have more than 32, and at 61 to 72, where many spill a short second chunk.
+// Set apart from the first that chunk reads its weights again, so there half as many short items again as the last round has places are
+// asked for (29 for 29 cost 3 %); from 80 pairs on it never pays (1500 tokens 250 / 263, 4096 521 / 542).  us of gate | up (top-8, k =
+// 2048) over the order of the experts, by pairs per expert: 128 experts x 768 -10 at 24 to 30, -21 at 64, -7 at 72; 192 x 512 -10 and
+// -20; 256 x 512 -9 at 24 to 28, +5 to +7 at 61 and 64, -13 at 72; 160 x 768 -9 at 28, +4 at 64, -16 at 72.  Not for down, whose items
+// are short already: 3 less to 3 us more, 5 at 256 experts.
+// Returns twice the short items per place that the last round asks for, 0: the order of the experts.
+int long_items_first(const MoeGemmParams& P, int64_t pairs) {
     const int64_t per_expert = pairs / P.n_experts;
-    const bool ordered = ((per_expert >= 22 && per_expert <= 32) || (per_expert >= 61 && per_expert <= 68)) &&
-                         P.n_experts * P.parts > 8 * kCusPerXcd;
-    return ordered ? launch_form<GATE_UP, true>(P, max_chunks, stream) : launch_form<GATE_UP, false>(P, max_chunks, stream);
+    return per_expert >= 22 && per_expert <= 32 ? 2 : per_expert >= 61 && per_expert <= 72 ? 3 : 0;
 }
 
 MoeGemmParams base_params(const QmmLayout& L, const int32_t* perm, const int32_t* offsets, const int32_t* chunks,
@@ -525,16 +527,17 @@ hipError_t qmm_launch_moe_gemm_gate_up(const QmmLayout& G, const void* gate, con
     P.row_div = top_k;
     P.row_magic = top_k > 1 ? (uint32_t)((((uint64_t)1 << 32) / (uint32_t)top_k) + 1) : 0;
     P.parts = (int)(G.n / 256), P.out_units = P.parts;
-    return launch<true>(P, pairs, max_chunks, stream);
+    P.fill2 = long_items_first(P, pairs);
+    return P.fill2 ? launch<true, true>(P, max_chunks, stream) : launch<true, false>(P, max_chunks, stream);
 }
 
 hipError_t qmm_launch_moe_gemm_down(const QmmLayout& D, const void* down, const void* records, const int32_t* perm,
                                     const int32_t* offsets, const int32_t* chunks, const int32_t* chunk_expert, int n_experts,
-                                    int64_t pairs, int64_t max_chunks, float* y, hipStream_t stream) {
+                                    int64_t max_chunks, float* y, hipStream_t stream) {
     MoeGemmParams P = base_params(D, perm, offsets, chunks, chunk_expert, n_experts);
     P.w0 = P.w1 = (const uint8_t*)down;
     P.records = (const uint8_t*)records, P.out = y;
     P.row_div = 0;
     P.parts = (int)((D.n + 511) / 512);
-    return launch<false>(P, pairs, max_chunks, stream);
+    return launch<false, false>(P, max_chunks, stream);
 }

@@ -86,6 +86,14 @@ def test_expert_threshold_of_the_environment():
     assert "moe_gemm_q4k_kernel" in kernels([case], IZWI_QMM_MOE_MFMA_MIN_ROWS="20")[0]
 
 
+def test_expert_products_with_long_items_first():
+    """Gate | up alone, around 22 to 32 and 61 to 72 pairs per expert."""
+    cases = [["moe", 16, 512, 512, 4, 4 * per] for per in (21, 22, 32, 33, 60, 61, 72, 73)]
+    names = kernels(cases)
+    assert ["moe_gemm_q4k_kernel<true, true>" in n for n in names] == [False, True, True, False, False, True, True, False]
+    assert all("moe_gemm_q4k_kernel<false, false>" in n and "moe_gemm_q4k_kernel<false, true>" not in n for n in names)
+
+
 def test_prefill_kernels_by_size_and_by_the_environment():
     """The few-row kernel up to 128 rows and one tile per compute unit, the 256-row tiles beyond and wherever
     IZWI_QMM_GEMM_TILE asks for them."""

@@ -57,13 +57,17 @@ def test_chunks_equal_the_tile_kernels(qa, oracle, E, hidden, inter, counts):
     assert np.linalg.norm(g - want) <= 1e-3 * np.linalg.norm(want)
 
 
-# long work items before short ones (22 to 32 and 61 to 68 pairs per expert, several items per compute unit): even and
-# skewed counts, experts with none, a run of an XCD's items longer than what is put in order
-@pytest.mark.parametrize("per_expert,skew", [(21, 0), (22, 0), (27, 9), (32, 20), (33, 5), (61, 0), (64, 30), (68, 60), (69, 3)])
-def test_long_items_first(qa, per_expert, skew):
+# long work items before short ones (22 to 32 and 61 to 72 pairs per expert, several items per compute unit): even and
+# skewed counts, experts with none, too few short ones for the last round, a run of an XCD's items (items of gate | up) longer than
+# what is put in order
+@pytest.mark.parametrize("per_expert,skew,inter,items", [
+    (21, 0, 768, 384), (22, 0, 768, 384), (27, 9, 768, None), (32, 20, 768, None), (30, 60, 768, None), (33, 5, 768, None), (61, 0, 768, 384),
+    (64, 30, 768, None), (68, 60, 768, None), (69, 3, 768, None), (72, 0, 768, 768), (73, 3, 768, None),
+    (68, 0, 1280, 8 * 160), (28, 9, 2304, 125 * 9)])
+def test_long_items_first(qa, per_expert, skew, inter, items):
     import torch
     from izwi_amd import capi
-    E, hidden, inter = 128, 1280, 768  # 384 items in both products where no expert has more than 64 pairs
+    E, hidden = 128, 1280
     rng = np.random.default_rng(4700 + per_expert)
 
     def stack(n, k):
@@ -77,6 +81,7 @@ def test_long_items_first(qa, per_expert, skew):
         take = min(int(counts[2 * i]), int(rng.integers(1, per_expert + 1)) if i % 3 else per_expert)
         counts[2 * i] -= take
         counts[2 * i + 1] += take
+    assert items is None or items == ((counts + 63) // 64).sum() * (inter // 256)
     t = int(counts.sum())
     ids = torch.from_numpy(rng.permutation(np.repeat(np.arange(E, dtype=np.int32), counts)).reshape(t, 1)).cuda()
     gen = torch.Generator(device="cuda").manual_seed(4701)
