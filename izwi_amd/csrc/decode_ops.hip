@@ -727,14 +727,16 @@ __global__ __launch_bounds__(256) void attn_partial_kernel(AttnParams<T> P) {
 // groups of a wave meet under the wave's maximum on the vector ALU, the waves in LDS.
 //
 // Bound by two trips to memory and, from 128 positions on, by what one compute unit reads (1 KB of f32 keys and values a
-// position at 110 GB/s).  A decode step in a graph, two launches / this (one launch and a quarter of this kernel's waves up
-// to 32 positions): 8 layers of 0.6B shapes 176 / 172 us at 11 positions, 190 / 174 at 34, 197 / 186 at 128, 200 / 198 at
-// 256, 205 / 207 at 300, 208 / 219 at 501; 4 layers of 8B shapes 216 / 206 at 26, 226 / 219 at 201, 226 / 222 at 301,
-// 229 / 230 at 501.  At 300 the launch it saves still counts where the host launches as slowly as the GPU runs (called from
-// Python 218 - 245 / 210), so the line is at 320 positions (and at a head per
-// compute unit: here every query head reads its cache rows for itself).  Two rows ahead on eight waves are the faster form up to 128
-// positions (128: 186 / 194), one on sixteen beyond (300: 210 / 207); two ahead on sixteen spill.
-constexpr int kOneLaunchPositions = 320;
+// position at 110 GB/s).  Decode layers in a graph, us each, splits and their merge (one launch up to 32 positions) / this, at
+// 33, 128, 256, 300 and 320 positions: 16 query heads on 8 20.8 / 18.1, 21.0 / 19.1, 20.8 / 20.6, 20.9 / 21.1, 20.9 / 21.0; 32 on 8
+// 51.7 / 46.8, 51.7 / 48.4, 51.7 / 50.3, 51.8 / 50.9, 51.8 / 51.2; 40 on 8 52.3 / 50.4, 52.4 / 52.0, 53.3 / 53.5, 53.3 / 54.2,
+// 53.3 / 54.3; 8 on 8 of 64 elements 18.7 / 16.7, 18.8 / 17.2, 18.7 / 18.2, 18.8 / 18.1, 18.8 / 18.2; 4 on 1 21.5 / 17.2 to 21.7 / 19.9.
+// The line is where the splits catch up: they read a cache row once for `g` query heads (g below: 4, 2 or 1), here every head reads its
+// rows for itself, but with few heads per row they leave more of the chip busy.  Two heads: at 300 positions still this, whose
+// launch saved counts where the host launches as slowly as the GPU runs (16 on 8 called from Python 218 - 245 / 210).  And a head per
+// compute unit at the most.  Two rows ahead on eight waves are the faster form up to 128
+// positions (128: 186 / 194 for 8 layers), one on sixteen beyond (300: 210 / 207); two ahead on sixteen spill.
+inline int one_launch_positions(int64_t head_dim, int g) { return head_dim > 128 ? 0 : head_dim == 128 && g == 1 ? 256 : 320; }
 template <typename T, int HD, bool PREP, int W, int NB>
 __global__ __launch_bounds__(64 * W) void attn_one_kernel(AttnParams<T> P) {
     static_assert(!PREP || std::is_same<T, float>::value, "the one-token step is built for f32");
@@ -1140,7 +1142,7 @@ int decode_attention_impl(const T* q, const T* k, const T* v, int64_t num_heads,
     }
     // (whoever sets a split's size asks for splits)
     static const bool splits_asked = getenv("IZWI_ATTN_WGS_PER_CU") || getenv("IZWI_ATTN_MIN_CHUNK");
-    if (head_dim <= 128 && kv_len <= kOneLaunchPositions && num_heads <= n_cus && !splits_asked) {
+    if (kv_len <= one_launch_positions(head_dim, g) && num_heads <= n_cus && !splits_asked) {
         OPS_TRY((head_dim == 64 ? launch_attn_one<T, 64>(P, stream) : launch_attn_one<T, 128>(P, stream)));
         OPS_TRY(oo.finish(stream));
         return IZWI_QMM_OK;

@@ -113,6 +113,13 @@ def test_prefill_splits_where_they_pay():
     assert split == [False, False, True]
 
 
+def test_attention_launches_by_length_and_heads():
+    """One launch up to 320 positions (256 where a workgroup of the splits would hold one query head of 128 elements)."""
+    cases = [["attention", 16, 8, 128, 320], ["attention", 16, 8, 128, 321], ["attention", 32, 8, 128, 320], ["attention", 8, 8, 64, 320],
+             ["attention", 40, 8, 128, 256], ["attention", 40, 8, 128, 257], ["attention", 4, 2, 256, 33]]
+    assert ["attn_one_kernel" in names for names in kernels(cases)] == [True, False, True, True, True, False, False]
+
+
 def test_attention_splits_of_the_environment():
     """IZWI_ATTN_WGS_PER_CU and IZWI_ATTN_MIN_CHUNK size the splits at every length of the cache, the short ones
     that otherwise take one launch included."""
