@@ -5,19 +5,23 @@
 // dequantized once and needs no trip through LDS.  A workgroup of eight waves owns 32 * MT
 // activation rows x 128 weight rows; wave (c, p) owns 32 of the weight rows and, of every unit of
 // 256 k-elements, half p.  A lane's 16-byte quant chunk holds k-elements of one weight row only,
-// which is what a lane supplies to v_mfma_f32_32x32x16_bf16: the chunk is unpacked into B operands
-// in registers, in the k order the chunk has, and the A operand (activations, staged in LDS by
+// which is what a lane supplies to v_mfma_f32_32x32x16_bf16: the chunk is unpacked into weight operands (the
+// instruction's first) in registers, in the k order the chunk has, and the activation operand (staged in LDS by
 // LDS-direct loads) is picked in the same order.  No weight tile in LDS, no LDS writes, one barrier per
 // unit.  The two halves' sums meet in LDS at the end.  Where the tiles alone leave compute units idle, k is
 // split over workgroups and the row tiles get lower.
 //
-// The loads run ahead of the units: weights four to six units in registers, activations two or three in LDS, and the
+// The loads run ahead of the units: weights four units in registers, activations two in LDS, and the
 // first unit waits for its own loads alone.  The workgroups of an XCD begin at different units of k: beginning
 // together they read the same 512 bytes of every activation row at once, and rows lie a power of two apart.
+// One unit ahead and all at the same unit / four ahead / six and three (bf16 rows, us in a graph, cold weights): 2048 + 1024 + 1024
+// at k = 2048, Q6_K, 80 rows 13.7 / 13.4 / 14.2, Q8_0 97 rows 14.5 / 14.1 / 14.8; 4096 x 4096 Q6_K 97 rows 17.9 / 16.9 / 17.5; 4096 + 1024 +
+// 1024 Q8_0 66 rows 20.9 / 19.6 / 20.8, 128 rows 24.2 / 23.0 / 22.5; 3 x 1024 at k = 1024, Q8_0, 10.2 / 8.6 / 9.4: slices of four to
+// eight units request deeper than they are long, in front of the second unit's activations.
 //
 // Bound by the life of a workgroup: at 2 x 12288 x 4096 (Q4_K, cold weights; time stamps) it has its arguments after 1.0 us
 // and its first operands 4.2 later, takes 30 in sixteen units (1.95 a unit at 101 rows, 1.65 at 65; 2.1 and 1.8 with the
-// loads one unit ahead and all workgroups at the same unit) and 2.2 for the exchange of the sums and stores of a value a lane.  Of a
+// loads one unit ahead and all workgroups at the same unit) and 2.2 for the exchange of the sums and stores (of a value a lane; since in 16-byte pieces).  Of a
 // unit's 1.95 us 1.57 remain without its loads and 1.3 without unpacking and activations: matrix instructions (1.0),
 // unpacking (1.0), LDS reads (0.9 to 1.2) and the loads share the compute unit, and two waves per SIMD overlap them in
 // part.  An unpacking of a fifth fewer vector instructions (mixed-precision fma on f16 denormals) gave nothing.
@@ -25,8 +29,7 @@
 // 14 us per workgroup instead: the exchange of the sums is 512 KB of LDS traffic there, 128 KB here.  us per
 // call on f32 rows in a graph, one call per weight on 128 x 256 / 64 x 128 tiles with the weights through
 // LDS / here with the loads one unit ahead.  Q4_K, 101 rows: q|k|v 81 / 27, 4096 x 4096 28 / 19, gate|up 82 / 47, down 47 / 32; Q6_K down
-// 201 / 35; 512 rows: q|k|v 54 / 45; 0.6B shapes at 512: q|k|v 27 / 15.  The calls of one layer on bf16 rows, loads one unit
-// ahead / now: 8B Q4_K 111 / 107 us at 128 rows, Q8_0 116 / 112, 0.6B Q4_K 39.1 / 38.2 at 65, 55.8 / 53.7 at 400.
+// 201 / 35; 512 rows: q|k|v 54 / 45; 0.6B shapes at 512: q|k|v 27 / 15.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -107,8 +110,9 @@ __device__ __forceinline__ void load_half(HalfRegs<QT>& r, const uint8_t* unit, 
     }
 }
 
-// A use of the loaded registers: the compiler's own wait for them stands here, where the counter is zero
-// anyway, and not behind the next unit's requests (of which it counts only the register loads).
+// A use of the loaded registers: the compiler's own wait for them stands here and not behind the next unit's requests.  The
+// counted wait in front covers the activations alone; up to two units' weights are in flight behind these, and the compiler,
+// which counts the register loads only, waits until no more than those of the units behind are.
 template <int QT>
 __device__ __forceinline__ void arrived(HalfRegs<QT>& r) {
     asm volatile("" : "+v"(r.hdr));
@@ -144,7 +148,7 @@ __device__ __forceinline__ StepScales step_scales(const HalfRegs<QT>& r, int hal
     return s;
 }
 
-// B operand of matrix instruction SS (of eight): k-elements 64 (SS / 4) + 32 (SS / 2 % 2) + 16 h + 8 (SS % 2) .. + 7
+// Weight operand of matrix instruction SS (of eight): k-elements 64 (SS / 4) + 32 (SS / 2 % 2) + 16 h + 8 (SS % 2) .. + 7
 // of the half unit.
 template <int QT, int SS>
 __device__ __forceinline__ bf16x8 half_operand(const HalfRegs<QT>& r, const StepScales& s, uint32_t nibble_mask) {
@@ -163,9 +167,8 @@ __device__ __forceinline__ bf16x8 half_operand(const HalfRegs<QT>& r, const Step
     return scaled_bytes(lo, hi, s.scale[q], s.bias[q]);
 }
 
-// Stages of activations in LDS (as many units as fit, up to three) and units of weights in registers, for row tiles of 32 * mt
-constexpr int x_stages(int mt) { return mt <= 3 ? 3 : 2; }
-constexpr int weight_buffers(int mt) { return mt <= 3 ? 6 : 4; }
+// Stages of activations in LDS and units of weights in registers
+constexpr int kStages = 2, kBuffers = 4;
 
 // f(I, false); if there is more, f(I, true) and the same from I + 1 on (nested, not a loop with exits: every
 // step is reached from one place, so the compiler's waits there are for what was requested on that path)
@@ -188,8 +191,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
     constexpr int BM = 32 * MT;
     constexpr int kStage = BM * kUnitBytes;
     constexpr int XL = BM / 2 / kWaves; // LDS-direct loads per wave and unit (1 KiB = two rows each)
-    constexpr int NS = x_stages(MT), DW = weight_buffers(MT), WL = HalfRegs<QT>::kLoads;
-    static_assert(DW % NS == 0 && (DW - 2) * WL >= WL + (NS - 2) * (XL + WL));
+    constexpr int NS = kStages, DW = kBuffers, WL = HalfRegs<QT>::kLoads;
+    static_assert(NS == 2 && DW % NS == 0 && DW >= 3); // (the waits below)
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
 
     // Workgroups go to the eight XCDs round-robin by their index; the row tiles of one (column tile,
@@ -281,7 +284,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[i][r] = 0.0f;
 
-    // A operand of matrix instruction ss: row l & 31 of each 32-row block, chunk 16 half + 8 (ss / 4) + 4 (ss / 2 % 2)
+    // Activation operand of matrix instruction ss: row l & 31 of each 32-row block, chunk 16 half + 8 (ss / 4) + 4 (ss / 2 % 2)
     // + 2 h + ss % 2 of the unit
     const int frag_x = (lane & 31) * kUnitBytes + (((16 * half + 2 * h) ^ (lane & 15)) << 4);
 
@@ -289,8 +292,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
     // the unit's only barrier sits in front of its last one, where every activation of the unit is in
     // registers and the next unit has landed; behind it the activations NS units on and the weights DW units
     // on are requested, in this order.  Loads land in order: what may still be in flight at a barrier is
-    // what was requested behind the next unit's activations.  (The compiler's own waits count the weights
-    // alone; DW is as large as it takes for them to ask for no more.)
+    // what was requested behind the next unit's activations, one unit's weights.  (The compiler's own waits count the weights
+    // alone; with three units of them or more they ask for no more.)
     HalfRegs<QT> w[DW];
     StepScales sc[2];
     bf16x8 a[2][MT], b[2];
@@ -307,16 +310,13 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
         asm volatile("" ::: "memory"); // the requests stay here, in this order
     };
     issue_x(u0, 0);
-    static_for<DW - NS + 1>(request_w);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((DW - NS) * WL) : "memory");
+    static_for<DW - 1>(request_w);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((DW - 2) * WL) : "memory");
     zero_tail(u0, 0);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     arrived<QT>(w[0]);
-    static_for<NS - 1>([&](auto I) { // only now: the first unit does not wait for them
-        constexpr int i = decltype(I)::value + 1;
-        if (u0 + i <= last) issue_x(u0 + i, i);
-        request_w(std::integral_constant<int, DW - NS + i>{});
-    });
+    if (u0 + 1 <= last) issue_x(u0 + 1, 1); // only now: the first unit does not wait for them
+    request_w(std::integral_constant<int, DW - 1>{});
     read_a(0, std::integral_constant<int, 0>{});
     sc[0] = step_scales<QT, 0>(w[0], half, h);
     b[0] = half_operand<QT, 0>(w[0], sc[0], P.nibble_mask);
@@ -343,11 +343,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
         });
     };
     // The turn to the next unit around the last matrix instruction.  Behind the next unit's activations may still
-    // fly: the weights requested with them and, per turn since, activations (where there were any left) and weights.
-    auto turn = [&](auto I, auto REQUESTS, auto BEHIND, auto BEHIND_LAST) {
+    // fly: the weights requested with them (BEHIND).
+    auto turn = [&](auto I, auto REQUESTS, auto BEHIND) {
         constexpr int i = decltype(I)::value, next = (i + 1) % DW;
-        if (NS > 2 && u + 2 <= last) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(BEHIND)::value) : "memory");
-        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(BEHIND_LAST)::value) : "memory");
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(BEHIND)::value) : "memory");
         zero_tail(u + 1, (i + 1) % NS);
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         arrived<QT>(w[next]);
@@ -364,13 +363,12 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
     while (u + DW <= last)
         static_for<DW>([&](auto I) {
             front(I);
-            turn(I, std::true_type{}, std::integral_constant<int, WL + (NS - 2) * (XL + WL)>{}, std::integral_constant<int, (NS - 1) * WL>{});
+            turn(I, std::true_type{}, std::integral_constant<int, WL>{});
         });
     // the last 1 .. DW units, whose weights have all been requested
     chain<0, DW>([&](auto I, auto MORE) {
-        constexpr int i = decltype(I)::value, w_behind = i < NS - 1 ? (NS - 1 - i) * WL : 0;
         if constexpr (!decltype(MORE)::value) front(I);
-        else turn(I, std::false_type{}, std::integral_constant<int, w_behind + (NS - 2) * XL>{}, std::integral_constant<int, w_behind>{});
+        else turn(I, std::false_type{}, std::integral_constant<int, decltype(I)::value == 0 ? WL : 0>{});
     }, [&] { return u < last; });
     multiply(std::integral_constant<int, 7>{});
 
@@ -593,8 +591,8 @@ size_t partial_bytes(const RegbPlan& p, const QmmLayout& L, int i, int64_t m) {
 
 template <int QT, int MT, bool GATED>
 hipError_t launch_regb(const RegbParams& P, int64_t grid, hipStream_t stream) {
-    constexpr size_t stages = (size_t)x_stages(MT) * 32 * MT * kUnitBytes; // the halves' sums reuse it
-    static_assert(stages <= 160 * 1024 && stages >= (size_t)kCols * MT * 4096 + (GATED ? kWaves * 4096 : 0), "LDS of a CU");
+    constexpr size_t stages = std::max((size_t)kStages * 32 * MT * kUnitBytes, (size_t)kCols * MT * 4096 + (GATED ? kWaves * 4096 : 0)); // (the sums' exchange)
+    static_assert(stages <= 160 * 1024, "LDS of a CU");
     auto fn = &gemm_regb_kernel<QT, MT, GATED>;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)stages);
     if (e != hipSuccess) return e;
