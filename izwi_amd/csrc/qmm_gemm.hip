@@ -661,15 +661,17 @@ struct GemmPlan {
     int64_t full_cols;   // > 0: first a launch of 256 x 256 tiles over this many 256-column strips
 };
 
-// IZWI_QMM_GEMM_TILE="bm,bn,slices" (tuning aid) replaces the plan, at every number of rows, and the choice of
-// the few-row kernel: bm = 256, bn in {128, 192, 256}.
+// IZWI_QMM_GEMM_TILE="bm,bn,slices,strips" (tuning aid; the last two 1 and 0 if left out) replaces the plan, at every number of
+// rows, and the choice of the few-row kernel: bm = 256, bn in {128, 192, 256}.
 bool forced_plan(GemmPlan& plan) {
     static const GemmPlan forced = [] {
         GemmPlan p{0, 0, 1, 0};
         const char* e = getenv("IZWI_QMM_GEMM_TILE");
-        if (e && sscanf(e, "%d,%d,%d", &p.bm, &p.bn, &p.slices) >= 2) {
-            const bool ok = p.bm == 256 && (p.bn == 128 || p.bn == 192 || p.bn == 256) && p.slices >= 1 && p.slices <= 8;
+        int strips = 0;
+        if (e && sscanf(e, "%d,%d,%d,%d", &p.bm, &p.bn, &p.slices, &strips) >= 2) {
+            const bool ok = p.bm == 256 && (p.bn == 128 || p.bn == 192 || p.bn == 256) && p.slices >= 1 && p.slices <= 8 && strips >= 0;
             if (!ok) p.bm = p.bn = 0, p.slices = 1;
+            else p.full_cols = strips;
         }
         return p;
     }();
@@ -698,6 +700,7 @@ GemmPlan plan_gemm(int64_t m, int64_t n, int k_steps, int n_cus, int64_t tiles_n
         if (forced_plan(forced)) {
             while (forced.slices > 1 && k_steps / 4 < forced.slices) forced.slices /= 2;
             if (forced.bn == 192 && tiles_n192 == 0) forced.bn = 256;
+            if (n_weights > 1 || forced.full_cols * 256 >= n) forced.full_cols = 0;
             return forced;
         }
     }

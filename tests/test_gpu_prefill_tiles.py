@@ -5,6 +5,11 @@ stores, in place as well.  Products that would take the few-row kernel come here
 Reference: float64 products of the bf16 activations with the dequantized weights rounded to bf16; bounds as in
 test_gpu_prefill_regb.py.  With a residual the result is the plain call's f32 sum plus the residual, rounded once:
 the same bits."""
+import json
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -55,18 +60,24 @@ def test_tiles_of_192_columns(qa, oracle, tiles, dtype, m, n, k):  # noqa: F811
     check(qa, oracle, dtype, m, n, k)
 
 
-# more 128 x 128 tiles than compute units: taken by size.  65900 columns: whole rounds of 256-column strips, then
+# more 128 x 128 tiles than compute units: taken by size.  Q6_K at 65900 columns: whole rounds of 256-column strips, then
 # half-size tiles; the others have a rest in both directions
-@pytest.mark.parametrize("dtype,m,n,k", [(Q4_K, 2100, 2100, 256), (Q8_0, 190, 17000, 320), (Q6_K, 1000, 5000, 1024), (Q4_K, 150, 65900, 256)])
+@pytest.mark.parametrize("dtype,m,n,k", [(Q4_K, 2100, 2100, 256), (Q8_0, 190, 17000, 320), (Q6_K, 1000, 5000, 1024), (Q4_K, 150, 65900, 256),
+                                         (Q6_K, 150, 65900, 256)])
 def test_large_products(qa, oracle, dtype, m, n, k):  # noqa: F811
     check(qa, oracle, dtype, m, n, k)
 
 
 # results and residuals that start on 2, 4 or 16 bytes, rows of a multiple of eight values and not, sums of whole pieces and of
-# single values: 256, 192 and 128-column tiles, each whole along k and in slices.  The same sums, so the same bits
+# single values, as the plan has them (below: every form).  The same sums, so the same bits
 @pytest.mark.parametrize("dtype,m,n,k", [(Q4_K, 300, 520, 4096), (Q4_K, 301, 515, 4096), (Q4_K, 1100, 4096, 4096), (Q8_0, 700, 12024, 768),
                                          (Q4_K, 2050, 2056, 512), (Q8_0, 300, 66000, 256)])
 def test_results_and_residuals_by_alignment(qa, oracle, tiles, dtype, m, n, k):  # noqa: F811
+    alignments(qa, oracle, dtype, m, n, k)
+
+
+def alignments(qa, oracle, dtype, m, n, k):  # noqa: F811
+    print(f"alignments dtype={dtype} m={m} n={n} k={k}", flush=True)
     mm = weight(qa, oracle, dtype, n, k, 730)
     x = torch.from_numpy(oracle.randn(731, (m, k))).cuda().to(torch.bfloat16)
     y = mm.forward_bf16_to_f32(x)
@@ -94,3 +105,30 @@ def test_groups(qa, oracle, tiles, dtype, m, ns, k):  # noqa: F811
         want = x.double() @ dense(mm).t()
         assert off(got_f, want) < F32_TOL
         assert off(got_b, want) < BF16_TOL
+
+
+FORCED = """
+import json, sys
+sys.path[:0] = sys.argv[1:3]
+import izwi_amd as qa
+from oracle import oracle
+import test_gpu_prefill_tiles as t
+for case in json.loads(sys.argv[3]):
+    t.check(qa, oracle, *case)
+    t.alignments(qa, oracle, *case)
+print("PASSED")
+"""
+
+
+# Every form of tile, whole along k and in slices (up to one per unit of k, the last ones shorter), and strips of whole tiles in
+# front of narrower ones, asked for by name: whole and ragged last tiles in both directions, n a multiple of eight and not.  In a
+# process of its own, because the switch is read once
+@pytest.mark.parametrize("form", ["256,256,1", "256,256,2", "256,256,4", "256,192,1", "256,192,2", "256,192,3", "256,128,1", "256,128,2",
+                                  "256,128,1,2", "256,192,1,1", "256,128,2,1"])
+def test_forms_by_name(qa, form):  # noqa: F811
+    cases = [(Q4_K, 129, 520, 1024), (Q4_K, 300, 777, 1280), (Q8_0, 257, 1000, 1120), (Q8_0, 256, 515, 1024), (Q6_K, 300, 1040, 1024),
+             (Q6_K, 515, 769, 2048)]
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    run = subprocess.run([sys.executable, "-c", FORCED, root, os.path.join(root, "tests"), json.dumps(cases)], cwd=root,
+                         env={**os.environ, "IZWI_QMM_GEMM_TILE": form}, capture_output=True, text=True, timeout=100)
+    assert run.returncode == 0 and "PASSED" in run.stdout, run.stdout[-1000:] + run.stderr[-2000:]
