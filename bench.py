@@ -901,7 +901,9 @@ def layer_stack_extra(torch, qa, dtype, steps=10, warmup=3):
         out[f"kv{kv_len}"] = {"ms_per_token": round(ms, 4), "tokens_per_s": round(1e3 / ms, 1)}
         del caches, g
         torch.cuda.empty_cache()
-    out["launches_per_token"] = N_LAYERS_8B * 6 + 5  # embedding row, LM head with the norm, two for the argmax, the token copy
+    # (attention: one launch up to 320 positions, splits and their merge beyond; and the embedding row, LM head with the norm, two
+    # for the argmax, the token copy)
+    out["launches_per_token"] = {"kv256": N_LAYERS_8B * 5 + 5, "kv4096": N_LAYERS_8B * 6 + 5}
     del layers, weights
     torch.cuda.empty_cache()
     return out

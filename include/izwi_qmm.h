@@ -404,7 +404,8 @@ int izwi_qmm_mlp_forward_f32(const izwi_qmm_weight* gate, const izwi_qmm_weight*
                              const float* x, int64_t m, float* y, int mem_space, void* stream);
 
 /* One decoder layer at one token, `Qwen3Layer::forward` (qwen3/core.rs:1863-1881), as one call for the
- * host: the six launches of izwi_qmm_forward_group_normed_f32 (q | k | v behind the input norm),
+ * host: the five launches (six where the attention is split over the cache) of izwi_qmm_forward_group_normed_f32
+ * (q | k | v behind the input norm),
  * izwi_decode_attention_step_f32 (scale head_dim^-1/2), izwi_qmm_forward_fused (o, + x),
  * izwi_qmm_forward_gate_up_silu_normed_f32 and izwi_qmm_forward_fused (down, + residual), whose
  * arguments and results these are, value for value.  q is `[num_heads * head_dim, hidden]`, k and v

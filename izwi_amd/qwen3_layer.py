@@ -4,9 +4,9 @@ Mirror of `Qwen3Layer::forward` (qwen3/core.rs:1863-1881) with `Qwen3Attention::
 single-token path (core.rs:1446-1575: q/k/v projections, per-head q/k norm, rotary embedding, cache
 append, grouped-query attention, output projection) and `Qwen3Mlp::forward` (core.rs:1786-1798),
 f32 activations.  Every arithmetic step is one library call; torch only appends the new key /
-value rows to the caches in the unfused form and owns the tensors.  Per layer: 6 kernel launches
-(the two RMSNorms ride in the projection launches behind them; q/k norm, rotary and the cache
-append ride in the attention launch) behind one library call, or 12 with the reference's separate hooks and two copies,
+value rows to the caches in the unfused form and owns the tensors.  Per layer: 5 kernel launches, 6 where
+the attention is split over the cache (the two RMSNorms ride in the projection launches behind them; q/k norm, rotary and the cache
+append ride in the attention launch) behind one library call, or 11 to 12 with the reference's separate hooks and two copies,
 where the reference's eager path issues one per operator.
 """
 from __future__ import annotations

@@ -97,7 +97,7 @@ def test_long_items_first(qa, per_expert, skew, inter, items):
     assert torch.equal(got.view(torch.int32), tiles.view(torch.int32))
 
 
-@pytest.mark.parametrize("t", [144, 500, 2100])  # 2100 * 8 pairs: beyond the one-workgroup sort
+@pytest.mark.parametrize("t", [144, 500, 2100])  # 144 * 8 pairs: the one-workgroup sort; beyond 2048 pairs two launches
 def test_layer_equals_the_tile_kernels(qa, oracle, t):
     import torch
     from izwi_amd import capi

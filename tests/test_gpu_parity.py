@@ -503,12 +503,12 @@ def test_moe_route_and_sort_bit_exact(qa, oracle, t):
 
 
 @pytest.mark.parametrize("rows,experts", [
-    (5000, 128),   # 40000 pairs: the three-launch sort
-    (1024, 128),   # 8192 pairs: one workgroup, 83 KB of LDS
-    (2048, 128),   # 16384 pairs: the most one workgroup takes (149 KB)
-    (2049, 128),   # one row more: three launches
-    (1500, 200),   # 12000 pairs of 200 experts: 152 KB would not do, three launches
-    (700, 512),    # many experts, few runs
+    (5000, 128),   # 40000 pairs: two launches, 40 workgroups
+    (1024, 128),   # 8192 pairs: whole workgroups of 1024
+    (2048, 128),
+    (2049, 128),   # a last workgroup of eight pairs
+    (1500, 200),   # an expert count that is no power of two
+    (700, 512),    # the most experts of the two launches
 ])
 def test_moe_sort_many_pairs(qa, oracle, rows, experts):
     rng = np.random.default_rng(3 + rows)
