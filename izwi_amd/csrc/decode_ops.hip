@@ -736,7 +736,8 @@ __global__ __launch_bounds__(256) void attn_partial_kernel(AttnParams<T> P) {
 // launch saved counts where the host launches as slowly as the GPU runs (16 on 8 called from Python 218 - 245 / 210).  And a head per
 // compute unit at the most.  Two rows ahead on eight waves are the faster form up to 128
 // positions (128: 186 / 194 for 8 layers), one on sixteen beyond (300: 210 / 207); two ahead on sixteen spill.
-inline int one_launch_positions(int64_t head_dim, int g) { return head_dim > 128 ? 0 : head_dim == 128 && g == 1 ? 256 : 320; }
+constexpr int kOneLaunchPositions = 320;
+inline int one_launch_positions(int64_t head_dim, int g) { return head_dim == 128 && g == 1 ? 256 : kOneLaunchPositions; }
 template <typename T, int HD, bool PREP, int W, int NB>
 __global__ __launch_bounds__(64 * W) void attn_one_kernel(AttnParams<T> P) {
     static_assert(!PREP || std::is_same<T, float>::value, "the one-token step is built for f32");
@@ -1142,16 +1143,20 @@ int decode_attention_impl(const T* q, const T* k, const T* v, int64_t num_heads,
     }
     // (whoever sets a split's size asks for splits)
     static const bool splits_asked = getenv("IZWI_ATTN_WGS_PER_CU") || getenv("IZWI_ATTN_MIN_CHUNK");
-    if (kv_len <= one_launch_positions(head_dim, g) && num_heads <= n_cus && !splits_asked) {
+    const bool one_launch = kv_len <= kOneLaunchPositions && head_dim <= 128 && num_heads <= n_cus && !splits_asked;
+    bool one_launch_pays = one_launch && kv_len <= one_launch_positions(head_dim, g);
+    QmmCallScope call; // the split partials stay this call's until the merge is queued
+    if (splits > 1) { // (asked for with one launch too: the first token of a stream makes room for later, captured ones)
+        void* scratch = nullptr;
+        const hipError_t e = qmm_get_scratch(device, stream, (size_t)num_heads * splits * (head_dim + 2) * sizeof(float), &scratch);
+        if (e != hipSuccess && one_launch) (void)hipGetLastError(), one_launch_pays = true;
+        else OPS_TRY(e);
+        P.part = (float*)scratch;
+    }
+    if (one_launch_pays) {
         OPS_TRY((head_dim == 64 ? launch_attn_one<T, 64>(P, stream) : launch_attn_one<T, 128>(P, stream)));
         OPS_TRY(oo.finish(stream));
         return IZWI_QMM_OK;
-    }
-    QmmCallScope call; // the split partials stay this call's until the merge is queued
-    if (splits > 1) {
-        void* scratch = nullptr;
-        OPS_TRY(qmm_get_scratch(device, stream, (size_t)num_heads * splits * (head_dim + 2) * sizeof(float), &scratch));
-        P.part = (float*)scratch;
     }
     const dim3 grid((unsigned)num_kv_heads, (unsigned)splits, (unsigned)z);
     hipError_t e = head_dim == 64    ? launch_attn_partial<T, 64>(P, g, grid, stream)

@@ -73,3 +73,44 @@ def test_decode_layer_step_replays_equal_eager(qa, oracle):
         assert torch.equal(got_y, want_y), i
         assert torch.equal(got_tok, want_tok), i
         assert torch.equal(got_k, kc_e[0, :, pos]), i
+
+
+def new_stream():
+    """A stream of its own (torch's come from a pool, and may have scratch memory from an earlier use)."""
+    import ctypes
+    handle = ctypes.c_void_p()
+    assert ctypes.CDLL("libamdhip64.so").hipStreamCreate(ctypes.byref(handle)) == 0
+    return torch.cuda.ExternalStream(handle.value)
+
+
+@pytest.mark.parametrize("heads,kv_heads,d,eager,captured", [
+    (16, 8, 128, 100, 400),   # an eager token in one launch makes room for a captured one that is split
+    (8, 2, 64, 40, 1500),
+    (5, 1, 128, None, 300),   # no eager token, no room: one launch although splits would be the faster form
+    (16, 8, 128, None, 300),
+])
+def test_attention_captured_at_another_length_than_the_eager_token(qa, oracle, heads, kv_heads, d, eager, captured):
+    dev = lambda a: torch.from_numpy(a).cuda()  # noqa: E731
+    cap = captured + 7
+    q, k, v = dev(oracle.randn(90, (1, heads, 1, d))), dev(oracle.randn(91, (1, kv_heads, cap, d))), dev(oracle.randn(92, (1, kv_heads, cap, d)))
+
+    def attention(kv_len):
+        return qa.try_fused_decode_gqa_attention_with_kv_len(q, k, v, heads, kv_heads, d, kv_len, d ** -0.5)
+
+    attention(captured)  # kernels are loaded, on another stream
+    torch.cuda.synchronize()
+    stream = new_stream()
+    with torch.cuda.stream(stream):
+        if eager:
+            attention(eager)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        out = attention(captured)
+    for i in range(3):
+        q.copy_(dev(oracle.randn(93 + i, (1, heads, 1, d))))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        want = oracle.decode_gqa_attention(q.cpu().numpy(), k.cpu().numpy(), v.cpu().numpy(), captured, d ** -0.5)
+        assert np.abs(out.cpu().numpy() - want).max() <= 1e-5
