@@ -78,8 +78,9 @@ def test_decode_layer_step_replays_equal_eager(qa, oracle):
 def new_stream():
     """A stream of its own (torch's come from a pool, and may have scratch memory from an earlier use)."""
     import ctypes
+    from izwi_amd import capi
     handle = ctypes.c_void_p()
-    assert ctypes.CDLL("libamdhip64.so").hipStreamCreate(ctypes.byref(handle)) == 0
+    assert capi.lib().hipStreamCreate(ctypes.byref(handle)) == 0  # (of the runtime that the library is linked to)
     return torch.cuda.ExternalStream(handle.value)
 
 
