@@ -13,25 +13,29 @@
 // below 2^24 in its f32 sum.  The same integers and the same f32 operations in the same order as
 // q4k_panel_dot: the same bits.
 //
-// A workgroup of eight waves owns up to 64 sorted pairs (two blocks of 32) of one expert and, of every
-// wave, two blocks of 32 weight rows: gate and up of the same 32 columns, or two blocks of down.  The
-// pairs' activation records stay in LDS over all of k (up to eight units), so that after one barrier the
-// waves walk k on their own; a lane's weight chunks are requested one unit ahead.
+// A work item is up to 64 sorted pairs (two blocks of 32) of one expert and, of every one of eight waves, two blocks of 32
+// weight rows: gate and up of the same 32 columns, or two blocks of down.  A workgroup per compute unit takes its items in turn.
+// The pairs' activation records pass through a ring of four units in LDS, requested two steps (units) ahead and on into the next
+// item, the weights of a wave one unit ahead in its registers, so that between items only the finish of the sums stands still.  No
+// barrier in between: the waves of a SIMD run half a phase apart, and a barrier would bring them together; counters in LDS say which
+// steps have landed and which slots are free.  One wave of eight requests all of a step's records in its turn.
 //
 // gate | up: the 256 columns of a workgroup are one unit of the down projection's input, so
 // silu(gate) * up is quantized here, in LDS, and leaves as records: 9.5 bytes instead of 64 per eight
 // values, no launch in between.
 //
-// Bound by vector instructions (about 160 per block of 32 x 32 outputs and unit in the loop, half of them the
-// unpacking that two blocks of pairs share, 640 cycles; 209 and 191 with everything around it) beside 17 matrix
-// instructions (544 cycles), which two waves per SIMD overlap in part: at 4096 tokens the vector ALU is busy
-// 56 % of the cycles of gate | up and the matrix pipe 36 %.
-// 128 experts, top-8, 2048 x 768: gate | up 282 us and down 164 at 4096 tokens (730 and 630 TOP/s), where the
-// 16-row-tile kernels took 480 and 260 and the quantizer between them 40; 80 and 41 at 512 tokens (70 with the long
-// items first), before 92, 48 and 8 (a workgroup's life is 40 us there, 1.5 per compute unit).  The layer 823 -> 497 us and 156 -> 136.  Of that,
-// starting on the first unit's records while the others land, stores at 32-bit offsets and the two waves
-// of a SIMD half a phase apart with the one in its matrix instructions preferred: 556 -> 497 and 150 -> 136.
+// Bound by the issue of vector instructions, 640 per unit and wave (320 of them the finish of the sums, 300 the unpacking, which two
+// blocks of pairs share) beside 68 matrix instructions: a SIMD with two waves issues one in 4.4 to 4.9 cycles, which makes 6900 of the
+// 7250 cycles that a unit takes; and by the clock, which falls to 1.45 to 1.75 GHz under it.  (A start of the items with the long ones
+// first at every size, 3 % fewer cycles at the end of a launch, was therefore no faster.)
+// 128 experts, top-8, 2048 x 768, layer: items as workgroups of their own, each with its records over all of k, 7 to 8 of 42 us of
+// a gate | up item and 7 of 18 of a down item before the first unit was done / now: 106 / 101 us at 150 tokens, 127 / 120 at 512,
+// 180 / 168 at 1024, 282 / 266 at 2048, 505 / 471 at 4096.  Each wave requesting its share of every step's records instead:
+// 8200 cycles a unit, 486 us at 4096.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstddef>
 
 #include "qmm_internal.h"
 #include "qmm_moe_route.h"
@@ -56,7 +60,12 @@ constexpr int kMaxUnits = 8;
 // Chunk c of a row's 128 bytes sits at position c ^ ((row >> 1) & 7), half h of its sums at
 // h ^ ((row >> 3) & 1): sixteen lanes that read one chunk of sixteen rows touch every bank once.
 constexpr int kSumsAt = 2 * kRows * 128, kScalesAt = kSumsAt + kRows * 32, kUnitLds = kScalesAt + kRows * 4;
+static_assert(kUnitLds % 128 == 0);
 constexpr int kHStride = 264; // floats per row of silu(gate) * up in LDS
+constexpr int kRing = 4, kAhead = 2; // units of records in LDS, and how many steps ahead of its use one is requested
+constexpr int kTables = 8, kTablesAhead = 4; // items whose rows are known, and how many items ahead
+// s_waitcnt vmcnt(n), n < 16, the other counters left alone
+constexpr int wait_vector(int n) { return 0x0f70 | n; }
 
 struct MoeGemmParams {
     const uint8_t *w0, *w1;   // gate, up; down: the stack twice
@@ -76,7 +85,29 @@ struct MoeGemmParams {
 };
 
 __device__ __forceinline__ void barrier_lds() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+// Counters in LDS between the waves of a workgroup.  A wave's LDS instructions run in their order, so what it read or wrote
+// before it counts is read or written; the asm keeps the compiler to that order.
+// (One lane adds, without a branch: a block that ends between a unit's products and its sums costs registers.)
+__device__ __forceinline__ void count_up(uint32_t* counter) {
+    uint64_t all;
+    asm volatile("s_mov_b64 %0, exec\n\ts_mov_b64 exec, 1\n\tds_add_u32 %1, %2\n\ts_mov_b64 exec, %0"
+                 : "=&s"(all)
+                 : "v"((uint32_t)(uintptr_t)counter), "v"(1u)
+                 : "memory");
+}
+__device__ __forceinline__ void wait_for(const uint32_t* counter, uint32_t at_least) {
+    while (__builtin_amdgcn_readfirstlane(__hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) < at_least)
+        __builtin_amdgcn_s_sleep(1);
+    asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ i32x4 lds_i32x4(uint32_t at) { return *reinterpret_cast<const __attribute__((address_space(3))) i32x4*>(at); }
 __device__ __forceinline__ float silu(float v) { return v / (1.0f + expf(-v)); }
+
+// The lane's number, worked out anew: what depends on it is not kept in registers over the loops.
+__device__ __forceinline__ int lane_here(int lane) {
+    asm volatile("" : "+v"(lane));
+    return lane;
+}
 
 // What a lane holds of its weight row's unit: the header and, of every chunk pair b, chunk 2b + h.
 struct UnitRegs {
@@ -99,23 +130,103 @@ __device__ __forceinline__ f16x2 mins_pair(uint32_t m, f16x2 c, f16x2 minus_1024
     return __builtin_elementwise_fma(v, c, minus_1024_c);
 }
 
+constexpr int kCusPerXcd = 32;
+constexpr int kOrderedItems = 4 * kCusPerXcd; // the longest run of an XCD's items that is put in order
+
+struct WorkItem {
+    int e, part, pos_begin, pos_end;
+};
+
+// What the waves of a workgroup share beside the records: counters that only grow, and the tables of the items.
+struct Shared {
+    uint32_t ready[kRing];  // steps whose records have landed in a slot
+    uint32_t done[kRing];   // waves that have read them
+    uint32_t h_written, h_read; // gate | up: waves that have written (read) silu(gate) * up of an item
+    uint32_t pad[2];
+    uint32_t known[kTables]; // 1 + the item whose table stands there
+    WorkItem items[kTables];
+    uint32_t src_off[kTables][kRows]; // byte offsets of the rows' records
+    uint32_t out_off[kTables][kRows]; // down: of the output rows
+    uint8_t order[kOrderedItems];     // ORDERED: this run's items, long ones first
+};
+
+// A wave's place in the stream of (item, unit) steps
+struct Stream {
+    int n_items;              // of this workgroup
+    int step;                 // being multiplied
+    int l_step, l_item, l_unit; // whose records are requested next
+    const uint8_t* wp[2];     // the panels of the wave's first row tile: gate and up, or two blocks of down
+    uint32_t unit_off;        // of the unit to request: panel, then unit in the panel
+    int in_panel;
+};
+
+__device__ __forceinline__ WorkItem uniform_item(const Shared& S, int j) {
+    const WorkItem& it = S.items[j & (kTables - 1)];
+    return {__builtin_amdgcn_readfirstlane(it.e), __builtin_amdgcn_readfirstlane(it.part), __builtin_amdgcn_readfirstlane(it.pos_begin),
+            __builtin_amdgcn_readfirstlane(it.pos_end)};
+}
+
+template <bool GATE_UP>
+__device__ __forceinline__ void first_panels(const MoeGemmParams& P, const WorkItem& it, int wave, const uint8_t* (&wp)[2]) {
+    const int64_t matrix = (int64_t)it.e * P.matrix_bytes;
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        const int rt = (GATE_UP ? it.part * 16 : it.part * 32 + c * 16) + wave * 2; // (a block past the end: multiplied, not stored)
+        wp[c] = (c ? P.w1 : P.w0) + matrix + (uint32_t)(min(rt, P.row_tiles - 2) * P.k_groups) * (uint32_t)P.panel_bytes;
+    }
+}
+
+__device__ __forceinline__ void request_unit(UnitRegs& w, const uint8_t* unit, uint32_t lane_off, uint32_t half_off, uint32_t slots16) {
+    w.hdr = *reinterpret_cast<const u32x4*>(unit + lane_off);
+#pragma unroll
+    for (int b = 0; b < 4; b++) w.q[b] = *reinterpret_cast<const u32x4*>(unit + (uint32_t)(1 + 2 * b) * slots16 + half_off);
+}
+
+// The next step's records into their LDS image, all of them by the wave whose turn it is (shared out, the instructions around the
+// loads are issued eight times).
+__device__ __forceinline__ void request_records(const MoeGemmParams& P, Stream& t, Shared& S, uint8_t* smem, int wave, int lane) {
+    if (t.l_item >= t.n_items) return; // uniform
+    if ((t.l_step & (kWaves - 1)) == wave) {
+        lane = lane_here(lane);
+        const int slot = t.l_step & (kRing - 1), table = t.l_item & (kTables - 1);
+        wait_for(&S.known[table], (uint32_t)t.l_item + 1);
+        wait_for(&S.done[slot], (uint32_t)(t.l_step / kRing) * kWaves);
+        const int groups = __builtin_amdgcn_readfirstlane(S.items[table].pos_end - S.items[table].pos_begin) > 32 ? 8 : 4;
+        const uint32_t unit_lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem + (uint32_t)slot * kUnitLds);
+        const uint8_t* base = P.records + t.l_unit * kWideRowUnitBytes;
+        const uint32_t* src = S.src_off[table];
+#pragma unroll 1
+        for (int g = 0; g < groups; g++) { // eight rows: both halves of the quants
+            const int r = g * 8 + (lane >> 3);
+            const uint32_t from = src[r] + (uint32_t)((lane & 7) ^ ((r >> 1) & 7)) * 16u;
+            load_to_lds(base, from, unit_lds + g * 1024);
+            load_to_lds(base, from + 128u, unit_lds + kRows * 128 + g * 1024);
+        }
+#pragma unroll 1
+        for (int q = 0; q < groups / 4; q++) { // 32 rows: their sums
+            const int r = q * 32 + (lane >> 1);
+            load_to_lds(base, src[r] + 256u + (uint32_t)((lane & 1) ^ ((r >> 3) & 1)) * 16u, unit_lds + kSumsAt + q * 1024);
+        }
+        load_to_lds4(base, src[lane] + 288u, unit_lds + kScalesAt);
+    }
+    t.l_step++;
+    if (++t.l_unit == P.k_units) t.l_unit = 0, t.l_item++;
+}
+
 template <bool GATE_UP, int NRB>
-__device__ __forceinline__ void chunk_body(const MoeGemmParams& P, const uint8_t* wbase0, const uint8_t* wbase1, uint8_t* smem,
-                                           UnitRegs (&raw)[2], const uint32_t (&lane_off)[2], const uint32_t* out_off, int part,
-                                           int pos_begin, int pos_end, int wave, int lane) {
+__device__ __forceinline__ void chunk_body(const MoeGemmParams& P, Shared& S, Stream& t, uint8_t* smem, UnitRegs (&raw)[2], int item,
+                                           const WorkItem& it, int wave, int lane) {
     const int row = lane & 31, h = lane >> 5;
-    // byte offsets of the lane's A chunks: [b & 1][i], of its sums, and of its four runs of scales
-    const uint32_t sw = (uint32_t)(row >> 1) & 7u;
-    uint32_t a_off[2][2];
-#pragma unroll
-    for (int bb = 0; bb < 2; bb++)
-#pragma unroll
-        for (int i = 0; i < 2; i++) a_off[bb][i] = (uint32_t)row * 128u + (((uint32_t)(4 * bb + 2 * h + i)) ^ sw) * 16u;
+    // byte offsets of the lane's A chunks, of its sums, and of its four runs of scales
+    // (the four chunks' differ in bits that the swizzle leaves apart, and images start on 128 bytes)
+    const uint32_t a_off = (uint32_t)row * 128u + (((uint32_t)(2 * h)) ^ ((uint32_t)(row >> 1) & 7u)) * 16u;
     const uint32_t sum_off = (uint32_t)kSumsAt + (uint32_t)row * 32u + (((uint32_t)h ^ ((uint32_t)(row >> 3) & 1u)) * 16u);
     const uint32_t scale_off = (uint32_t)kScalesAt + (uint32_t)h * 16u;
     const _Float16 cf = h ? (_Float16)32.0f : (_Float16)1.0f, kf = h ? (_Float16)-32768.0f : (_Float16)-1024.0f;
     const f16x2 c2 = {cf, cf}, k2 = {kf, kf};
     const uint32_t slots16 = (uint32_t)P.slots * 16u;
+    const uint32_t lane_off = (uint32_t)((lane >> 4) & 1) * (uint32_t)P.k_groups * (uint32_t)P.panel_bytes + (uint32_t)(lane & 15) * 16u;
+    const uint32_t half_off = lane_off + (uint32_t)h * slots16;
 
     f32x16 acc[2][NRB];
 #pragma unroll
@@ -125,20 +236,30 @@ __device__ __forceinline__ void chunk_body(const MoeGemmParams& P, const uint8_t
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[c][rb][r] = 0.0f;
 
-    uint32_t unit_off = 0;                    // of the next unit to request: panel, then unit in the panel
-    int in_panel = 0;
-    const uint8_t* lds = smem;
-    if (wave >= kWaves / 2) __builtin_amdgcn_s_sleep(10); // the two waves of a SIMD half a phase apart
-    for (int u = 0; u < P.k_units; u++, lds += kUnitLds) {
-        if (u == 1) { // the other units' records have landed
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            barrier_lds();
-        }
-        // (past the last unit the same one is requested again: no branch around the loads)
+    for (int u = 0; u < P.k_units; u++) {
+        // (known to be the same in all lanes)
+        t.step = __builtin_amdgcn_readfirstlane(t.step);
+        t.l_step = __builtin_amdgcn_readfirstlane(t.l_step), t.l_item = __builtin_amdgcn_readfirstlane(t.l_item);
+        t.l_unit = __builtin_amdgcn_readfirstlane(t.l_unit);
+        t.unit_off = __builtin_amdgcn_readfirstlane(t.unit_off), t.in_panel = __builtin_amdgcn_readfirstlane(t.in_panel);
+        // Behind the records that this wave requested at the last step came ten loads of weights, so with five left open they have
+        // landed.  (The builtin also tells the compiler, which otherwise waited for all of the weights here.)
+        __builtin_amdgcn_s_waitcnt(wait_vector(5));
+        if (((t.step + kAhead - 1) & (kWaves - 1)) == wave) count_up(&S.ready[(t.step + kAhead - 1) & (kRing - 1)]);
+        // the weights to request next: the following unit's, or the first of the next item (of the last: the same again)
         if (u + 1 < P.k_units) {
-            if (++in_panel == P.s) in_panel = 0, unit_off += (uint32_t)P.panel_bytes - (uint32_t)(P.s - 1) * 256u;
-            else unit_off += 256u;
+            if (++t.in_panel == P.s) t.in_panel = 0, t.unit_off += (uint32_t)P.panel_bytes - (uint32_t)(P.s - 1) * 256u;
+            else t.unit_off += 256u;
+        } else if (item + 1 < t.n_items) {
+            wait_for(&S.known[(item + 1) & (kTables - 1)], (uint32_t)item + 2);
+            first_panels<GATE_UP>(P, uniform_item(S, item + 1), wave, t.wp);
+            t.unit_off = 0, t.in_panel = 0;
         }
+        request_records(P, t, S, smem, wave, lane);
+        const int slot = t.step & (kRing - 1);
+        const uint8_t* lds = smem + slot * kUnitLds;
+        const uint32_t a_at = (uint32_t)(uintptr_t)lds + a_off;
+        wait_for(&S.ready[slot], (uint32_t)(t.step / kRing + 1));
 #pragma unroll
         for (int c = 0; c < 2; c++) {
             // (a wave in its matrix instructions goes before the other one of its SIMD in its finish)
@@ -171,7 +292,7 @@ __device__ __forceinline__ void chunk_body(const MoeGemmParams& P, const uint8_t
                     }
 #pragma unroll
                     for (int rb = 0; rb < NRB; rb++) {
-                        const i32x4 a = *reinterpret_cast<const i32x4*>(lds + (b >> 1) * (kRows * 128) + rb * 4096 + a_off[b & 1][i]);
+                        const i32x4 a = lds_i32x4((a_at ^ (uint32_t)(64 * (b & 1) + 16 * i)) + (b >> 1) * (kRows * 128) + rb * 4096);
                         if (b == 0 && i == 0) {
                             lo[rb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, __builtin_bit_cast(i32x4, wl), i32x16{}, 0, 0, 0);
                             hi[rb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, __builtin_bit_cast(i32x4, wh), i32x16{}, 0, 0, 0);
@@ -188,113 +309,94 @@ __device__ __forceinline__ void chunk_body(const MoeGemmParams& P, const uint8_t
             const uint32_t mn_hi = ((hdr.w >> 4) & 0x0f0f0f0fu) | (((hdr.z >> 6) & 0x03030303u) << 4);
             const f16x2 mm[4] = {mins_pair<0>(mn_lo, c2, k2), mins_pair<1>(mn_lo, c2, k2), mins_pair<0>(mn_hi, c2, k2), mins_pair<1>(mn_hi, c2, k2)};
             const f16x8 mins = {mm[0][0], mm[0][1], mm[1][0], mm[1][1], mm[2][0], mm[2][1], mm[3][0], mm[3][1]};
-            // the unit is consumed: the next one into its registers (the fences keep the scheduler from
-            // gathering the loads of both columns at the loop's end, where nothing is left to cover them)
-            asm volatile("" : "+v"(d), "+v"(dmin)); // (computed here, so that the header's registers are free)
-            __builtin_amdgcn_s_setprio(0);
-            if (NRB > 1) __builtin_amdgcn_sched_barrier(0);
-            const uint8_t* wu = (c ? wbase1 : wbase0) + unit_off;
-            w.hdr = *reinterpret_cast<const u32x4*>(wu + lane_off[c]);
-#pragma unroll
-            for (int b = 0; b < 4; b++)
-                w.q[b] = *reinterpret_cast<const u32x4*>(wu + (uint32_t)(1 + 2 * b) * slots16 + (lane_off[c] + (uint32_t)h * slots16));
-            if (NRB > 1) __builtin_amdgcn_sched_barrier(0);
+            // What the finish reads from LDS, and the min term, behind the last products: their latencies run under those.
+            f32x16 msum[NRB];
+            f32x4 dx[4];
 #pragma unroll
             for (int rb = 0; rb < NRB; rb++) {
                 const f16x8 sums = *reinterpret_cast<const f16x8*>(lds + sum_off + rb * 1024);
-                const f32x16 msum = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, mins, f32x16{}, 0, 0, 0);
+                msum[rb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, mins, f32x16{}, 0, 0, 0);
+            }
 #pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    const f32x4 dx = *reinterpret_cast<const f32x4*>(lds + scale_off + rb * 128 + g * 32);
+            for (int g = 0; g < 4; g++) dx[g] = *reinterpret_cast<const f32x4*>(lds + scale_off + g * 32);
+            asm volatile("" : "+v"(d), "+v"(dmin)); // (computed here, so that the header's registers are free)
+            __builtin_amdgcn_s_setprio(0);
+            // the unit is consumed: the next one into its registers (the fences keep the scheduler from
+            // gathering the loads of both columns at the loop's end, where nothing is left to cover them)
+            __builtin_amdgcn_sched_barrier(0);
+            request_unit(w, t.wp[c] + t.unit_off, lane_off, half_off, slots16);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const int isum = (hi[rb][4 * g + r] << 3) + lo[rb][4 * g + r];
-                        acc[c][rb][4 * g + r] =
-                            fmaf(fmaf(-dmin, msum[4 * g + r], d * (float)isum), dx[r], acc[c][rb][4 * g + r]);
-                    }
+            for (int rb = 0; rb < NRB; rb++) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int isum = (hi[rb][r] << 3) + lo[rb][r];
+                    acc[c][rb][r] = fmaf(fmaf(-dmin, msum[rb][r], d * (float)isum), dx[r >> 2][r & 3], acc[c][rb][r]);
+                    if (rb + 1 < NRB && (r & 3) == 3) dx[r >> 2] = *reinterpret_cast<const f32x4*>(lds + scale_off + (rb + 1) * 128 + (r >> 2) * 32);
                 }
-                if (NRB > 1) __builtin_amdgcn_sched_barrier(0);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
+        count_up(&S.done[slot]);
+        t.step++;
     }
 
-    const int col = wave * 32 + row;
+    lane = lane_here(lane);
+    const int h_ = lane >> 5, col = wave * 32 + (lane & 31);
     if constexpr (GATE_UP) {
-        barrier_lds(); // every wave has read its last activations
-        float* hbuf = reinterpret_cast<float*>(smem);
+        float* hbuf = reinterpret_cast<float*>(smem + kRing * kUnitLds);
+#pragma unroll
+        for (int rb = 0; rb < NRB; rb++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[0][rb][r] = silu(acc[0][rb][r]) * acc[1][rb][r];
+        // (the next item's weights have landed; the compiler, told so, does not wait for the stores behind at the top of the loop)
+        __builtin_amdgcn_s_waitcnt(wait_vector(0));
+        wait_for(&S.h_read, (uint32_t)item * kWaves); // the last item's
 #pragma unroll
         for (int rb = 0; rb < NRB; rb++)
 #pragma unroll
             for (int r = 0; r < 16; r++)
-                hbuf[(rb * 32 + (r & 3) + 8 * (r >> 2) + 4 * h) * kHStride + col] = silu(acc[0][rb][r]) * acc[1][rb][r];
-        barrier_lds();
+                hbuf[(rb * 32 + (r & 3) + 8 * (r >> 2) + 4 * h_) * kHStride + col] = acc[0][rb][r];
+        count_up(&S.h_written);
+        wait_for(&S.h_written, (uint32_t)(item + 1) * kWaves);
         const int j = lane & 15;
 #pragma unroll
         for (int pass = 0; pass < NRB; pass++) {
-            const int m = pass * 32 + (int)(threadIdx.x >> 4);
+            const int m = pass * 32 + wave * 4 + (lane >> 4);
             float v[16];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const f32x4 f = *reinterpret_cast<const f32x4*>(hbuf + m * kHStride + 16 * j + 4 * i);
                 v[4 * i] = f.x, v[4 * i + 1] = f.y, v[4 * i + 2] = f.z, v[4 * i + 3] = f.w;
             }
-            if (pos_begin + m < pos_end) // (whole 16-lane groups)
+            if (pass == NRB - 1) count_up(&S.h_read);
+            if (it.pos_begin + m < it.pos_end) // (whole 16-lane groups)
                 quantize_into_record<QMM_Q4_K, kWideRowRecord>(
-                    v, j, 0, static_cast<uint8_t*>(P.out) + ((int64_t)(pos_begin + m) * P.out_units + part) * kWideRowUnitBytes);
+                    v, j, 0, static_cast<uint8_t*>(P.out) + ((int64_t)(it.pos_begin + m) * P.out_units + it.part) * kWideRowUnitBytes);
         }
     } else {
+        __builtin_amdgcn_s_waitcnt(wait_vector(0)); // (as above)
         // 32-bit byte offsets from one uniform base; only an expert's last chunk has rows that do not exist
         uint8_t* y = static_cast<uint8_t*>(P.out);
-        const bool whole = pos_end - pos_begin == NRB * 32;
+        const uint32_t* out_off = S.out_off[item & (kTables - 1)];
+        const bool whole = it.pos_end - it.pos_begin == NRB * 32;
 #pragma unroll
         for (int c = 0; c < 2; c++) {
-            const int n = part * 512 + c * 256 + col;
+            const int n = it.part * 512 + c * 256 + col;
             if (n >= P.n) continue; // (uniform: n is a multiple of 256)
 #pragma unroll
             for (int rb = 0; rb < NRB; rb++)
 #pragma unroll
                 for (int g = 0; g < 4; g++) {
-                    const u32x4 rows = *reinterpret_cast<const u32x4*>(out_off + rb * 32 + 8 * g + 4 * h);
+                    const u32x4 rows = *reinterpret_cast<const u32x4*>(out_off + rb * 32 + 8 * g + 4 * h_);
 #pragma unroll
                     for (int r = 0; r < 4; r++)
-                        if (whole || rb * 32 + 8 * g + 4 * h + r < pos_end - pos_begin)
+                        if (whole || rb * 32 + 8 * g + 4 * h_ + r < it.pos_end - it.pos_begin)
                             *reinterpret_cast<float*>(y + (rows[r] + (uint32_t)n * 4u)) = acc[c][rb][4 * g + r];
                 }
         }
     }
 }
-
-// The records of units [u0, u1) of the chunk's rows into their LDS images
-__device__ __forceinline__ void issue_records(const MoeGemmParams& P, const uint32_t* src_off, uint8_t* smem, int nrb, int u0, int u1,
-                                              int wave, int lane) {
-    const uint32_t lds_base = (uint32_t)(uintptr_t)smem;
-    const int groups = nrb * 4, per_unit = 2 * groups + nrb + 1; // pieces of quants (two halves), sums, scales
-    for (int piece = u0 * per_unit + wave; piece < u1 * per_unit; piece += kWaves) {
-        const int u = piece / per_unit, sub = piece - u * per_unit;
-        const uint32_t unit_lds = lds_base + (uint32_t)u * kUnitLds;
-        const uint8_t* base = P.records + u * kWideRowUnitBytes;
-        if (sub < 2 * groups) {
-            const int p = sub / groups, g = sub - p * groups;
-            const int r = g * 8 + (lane >> 3);
-            const uint32_t to = __builtin_amdgcn_readfirstlane(unit_lds + p * (kRows * 128) + g * 1024);
-            load_to_lds(base, src_off[r] + (uint32_t)p * 128u + (uint32_t)((lane & 7) ^ ((r >> 1) & 7)) * 16u, to);
-        } else if (sub < 2 * groups + nrb) {
-            const int q = sub - 2 * groups, r = q * 32 + (lane >> 1);
-            const uint32_t to = __builtin_amdgcn_readfirstlane(unit_lds + kSumsAt + q * 1024);
-            load_to_lds(base, src_off[r] + 256u + (uint32_t)((lane & 1) ^ ((r >> 3) & 1)) * 16u, to);
-        } else {
-            const uint32_t to = __builtin_amdgcn_readfirstlane(unit_lds + kScalesAt);
-            load_to_lds4(base, src_off[lane] + 288u, to);
-        }
-    }
-}
-
-struct WorkItem {
-    int e, part, pos_begin, pos_end;
-};
-constexpr int kCusPerXcd = 32;
-constexpr int kOrderedItems = 4 * kCusPerXcd; // the longest run of an XCD's items that is put in order
-constexpr int kOrderedPerLane = (kOrderedItems + 63) / 64;
 
 __device__ __forceinline__ WorkItem work_item(const MoeGemmParams& P, int item) {
     const int e = P.chunk_expert[item / P.parts]; // (an expert's items begin at parts * its first chunk)
@@ -304,102 +406,94 @@ __device__ __forceinline__ WorkItem work_item(const MoeGemmParams& P, int item) 
     return {e, part, begin, min(P.offsets[e + 1], begin + kRows)};
 }
 
+// A wave leaves the table of this workgroup's item j.
+__device__ __forceinline__ void prepare_item(const MoeGemmParams& P, Shared& S, const WorkItem& it, int j, int lane) {
+    const int at = j & (kTables - 1);
+    lane = lane_here(lane);
+    // (a row past the end reads the chunk's first row; its sums are never stored)
+    const int pos = it.pos_begin + lane < it.pos_end ? it.pos_begin + lane : it.pos_begin;
+    const uint32_t pair = (uint32_t)P.perm[pos];
+    const uint32_t src = P.row_div == 0 ? (uint32_t)pos : P.row_div == 1 ? pair : __umulhi(pair, P.row_magic);
+    S.src_off[at][lane] = src * P.row_bytes;
+    S.out_off[at][lane] = pair * (uint32_t)P.n * 4u;
+    if (lane == 0) S.items[at] = it;
+    asm volatile("" ::: "memory");
+    if (lane == 0) __hip_atomic_store(&S.known[at], (uint32_t)j + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Where the last of an XCD's rounds can hold short items alone, those of more than 32 pairs go first (a lane per item)
+// and the short ones fill in behind them.  Leaves the run's order in S.order; one wave.
+__device__ __forceinline__ void order_items(const MoeGemmParams& P, Shared& S, int first, int run, int lane) {
+    constexpr int kPerLane = (kOrderedItems + 63) / 64;
+    uint64_t heavy[kPerLane], exist[kPerLane];
+    int heavies = 0;
+#pragma unroll
+    for (int j = 0; j < kPerLane; j++) {
+        const bool exists = 64 * j + lane < run;
+        const WorkItem mine = work_item(P, first + (exists ? 64 * j + lane : 0));
+        heavy[j] = __ballot(exists && mine.pos_end - mine.pos_begin > 32), exist[j] = __ballot(exists);
+        heavies += __popcll(heavy[j]);
+    }
+    const int lights = run - heavies, last_round = (run - 1) % kCusPerXcd + 1;
+    const bool sorted = heavies > 0 && 2 * lights >= P.fill2 * last_round; // uniform, the same in all workgroups of the run
+    int at_heavy = 0, at_light = heavies;
+#pragma unroll
+    for (int j = 0; j < kPerLane; j++) {
+        const bool is_heavy = heavy[j] >> lane & 1;
+        const uint64_t light = exist[j] & ~heavy[j], set = is_heavy ? heavy[j] : light;
+        const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(set >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)set, 0));
+        const int rank = sorted ? (is_heavy ? at_heavy : at_light) + below : 64 * j + lane;
+        if (exist[j] >> lane & 1) S.order[rank] = (uint8_t)(64 * j + lane);
+        at_heavy += __popcll(heavy[j]), at_light += __popcll(light);
+    }
+}
+
 template <bool GATE_UP, bool ORDERED>
 __global__ __launch_bounds__(64 * kWaves) void moe_gemm_q4k_kernel(MoeGemmParams P) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    __shared__ __attribute__((aligned(16))) uint32_t out_off[kRows]; // down: byte offsets of the output rows
-    __shared__ uint32_t src_off[kRows];
+    extern __shared__ __attribute__((aligned(128))) uint8_t smem[];
+    __shared__ __attribute__((aligned(16))) Shared S;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
     // Work items in the order (expert, part of the weight rows, chunk of the pairs), cut into eight equal
     // runs: workgroups go to the XCDs round-robin, so a run is one XCD's, and the chunks that read the same weights
-    // follow one another there and find them in its L2.
+    // follow one another there and find them in its L2.  A workgroup takes its items from every round of the run, in turn from
+    // its front and its back.
     const int items = P.chunks[P.n_experts] * P.parts, per_xcd = (items + 7) >> 3;
-    const int slot = (int)(blockIdx.x >> 3), first = (int)(blockIdx.x & 7) * per_xcd;
+    const int slot = (int)(blockIdx.x >> 3), slots = (int)(gridDim.x >> 3), first = (int)(blockIdx.x & 7) * per_xcd;
     const int run = min(per_xcd, items - first); // items of this XCD
     if (slot >= run) return; // uniform
-    // Where the last of an XCD's rounds can hold short items alone, those of more than 32 pairs go first (every wave looks at
-    // the whole run, a lane per item) and the short ones fill in behind them.
-    WorkItem it = work_item(P, first + slot);
-    if (ORDERED && run > kCusPerXcd && run <= kOrderedItems) {
-        WorkItem mine[kOrderedPerLane];
-        uint64_t heavy[kOrderedPerLane], light[kOrderedPerLane];
-        int heavies = 0;
-#pragma unroll
-        for (int j = 0; j < kOrderedPerLane; j++) {
-            heavy[j] = light[j] = 0;
-            if (64 * j >= run) continue; // uniform
-            const bool exists = 64 * j + lane < run;
-            mine[j] = work_item(P, first + (exists ? 64 * j + lane : 0));
-            heavy[j] = __ballot(exists && mine[j].pos_end - mine[j].pos_begin > 32);
-            light[j] = __ballot(exists && mine[j].pos_end - mine[j].pos_begin <= 32);
-            heavies += __popcll(heavy[j]);
-        }
-        const int lights = run - heavies, last_round = (run - 1) % kCusPerXcd + 1;
-        if (heavies > 0 && 2 * lights >= P.fill2 * last_round) { // uniform, the same in all workgroups of the run
-            int rank = slot < heavies ? slot : slot - heavies;
-            bool found = false;
-#pragma unroll
-            for (int j = 0; j < kOrderedPerLane; j++) {
-                const uint64_t set = slot < heavies ? heavy[j] : light[j];
-                const int in_set = __popcll(set);
-                if (!found && rank < in_set) { // uniform
-                    const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(set >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)set, 0));
-                    const int at = __ffsll((unsigned long long)__ballot((set >> lane & 1) && below == rank)) - 1;
-                    it.e = __builtin_amdgcn_readlane(mine[j].e, at), it.part = __builtin_amdgcn_readlane(mine[j].part, at);
-                    it.pos_begin = __builtin_amdgcn_readlane(mine[j].pos_begin, at), it.pos_end = __builtin_amdgcn_readlane(mine[j].pos_end, at);
-                    found = true;
-                }
-                rank -= in_set;
-            }
-        }
-    }
-    const int e = it.e, part = it.part, pos_begin = it.pos_begin, pos_end = it.pos_end;
-    const int nrb = pos_end - pos_begin > 32 ? 2 : 1;
+    const auto place = [&](int j) { return j * slots + (j & 1 ? slots - 1 - slot : slot); };
+    const bool ordered = ORDERED && run > kCusPerXcd && run <= kOrderedItems; // uniform
+    const auto local_item = [&](int j) { return ordered ? (int)__builtin_amdgcn_readfirstlane(S.order[place(j)]) : place(j); };
+    Stream t{};
+    t.n_items = __builtin_amdgcn_readfirstlane(run / slots + (place(run / slots) < run));
+    if (threadIdx.x < (int)(offsetof(Shared, items) / 4)) reinterpret_cast<uint32_t*>(&S)[threadIdx.x] = 0;
+    if (ordered && wave == 0) order_items(P, S, first, run, lane);
+    barrier_lds();
 
-    const uint8_t* wbase0 = P.w0 + (int64_t)e * P.matrix_bytes;
-    const uint8_t* wbase1 = P.w1 + (int64_t)e * P.matrix_bytes;
-    const int h = lane >> 5;
-    uint32_t lane_off[2];
+    // The first item's weights, the first items' tables, the first steps' records
+    const uint32_t slots16 = (uint32_t)P.slots * 16u;
+    const uint32_t lane_off = (uint32_t)((lane >> 4) & 1) * (uint32_t)P.k_groups * (uint32_t)P.panel_bytes + (uint32_t)(lane & 15) * 16u;
+    first_panels<GATE_UP>(P, work_item(P, first + local_item(0)), wave, t.wp);
     UnitRegs raw[2];
 #pragma unroll
-    for (int c = 0; c < 2; c++) {
-        const int rt = (GATE_UP ? part * 16 : part * 32 + c * 16) + wave * 2 + ((lane >> 4) & 1);
-        lane_off[c] = (uint32_t)(min(rt, P.row_tiles - 1) * P.k_groups) * (uint32_t)P.panel_bytes + (uint32_t)(lane & 15) * 16u;
-        const uint8_t* wu = c ? wbase1 : wbase0;
-        const uint32_t slots16 = (uint32_t)P.slots * 16u;
-        raw[c].hdr = *reinterpret_cast<const u32x4*>(wu + lane_off[c]);
-#pragma unroll
-        for (int b = 0; b < 4; b++)
-            raw[c].q[b] = *reinterpret_cast<const u32x4*>(wu + (uint32_t)(1 + 2 * b) * slots16 + (lane_off[c] + (uint32_t)h * slots16));
+    for (int c = 0; c < 2; c++) request_unit(raw[c], t.wp[c], lane_off, lane_off + (uint32_t)(lane >> 5) * slots16, slots16);
+    if (wave < kTablesAhead && wave < t.n_items) prepare_item(P, S, work_item(P, first + local_item(wave)), wave, lane);
+    static_assert(kAhead == 2);
+    request_records(P, t, S, smem, wave, lane);
+    request_records(P, t, S, smem, wave, lane);
+    __builtin_amdgcn_s_waitcnt(wait_vector(0));
+    if (wave == 0) count_up(&S.ready[0]); // (the second step's: at the top of the loop)
+    if (wave >= kWaves / 2) __builtin_amdgcn_s_sleep(10); // the two waves of a SIMD half a phase apart
+    for (int i = 0; i < t.n_items; i++) {
+        if ((i & (kWaves - 1)) == wave && i + kTablesAhead < t.n_items)
+            prepare_item(P, S, work_item(P, first + local_item(i + kTablesAhead)), i + kTablesAhead, lane);
+        wait_for(&S.known[i & (kTables - 1)], (uint32_t)i + 1);
+        const WorkItem it = uniform_item(S, i);
+        if (it.pos_end - it.pos_begin > 32) chunk_body<GATE_UP, 2>(P, S, t, smem, raw, i, it, wave, lane);
+        else chunk_body<GATE_UP, 1>(P, S, t, smem, raw, i, it, wave, lane);
     }
-    if (threadIdx.x < kRows) {
-        // (a row past the end reads the chunk's first row; its sums are never stored)
-        const int pos = pos_begin + (int)threadIdx.x;
-        const int at = pos < pos_end ? pos : pos_begin;
-        const uint32_t pair = (uint32_t)P.perm[at];
-        const uint32_t src = P.row_div == 0 ? (uint32_t)at : P.row_div == 1 ? pair : __umulhi(pair, P.row_magic);
-        src_off[threadIdx.x] = src * P.row_bytes;
-        out_off[threadIdx.x] = pair * (uint32_t)P.n * 4u;
-    }
-    barrier_lds();
-    // The first unit's records, then, under the arithmetic of the first unit, the others'
-    issue_records(P, src_off, smem, nrb, 0, 1, wave, lane);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    // (a use of the loaded registers: the compiler's own wait for them stands here, not in the loop)
-#pragma unroll
-    for (int c = 0; c < 2; c++) {
-        asm volatile("" : "+v"(raw[c].hdr));
-#pragma unroll
-        for (int b = 0; b < 4; b++) asm volatile("" : "+v"(raw[c].q[b]));
-    }
-    barrier_lds();
-    issue_records(P, src_off, smem, nrb, 1, P.k_units, wave, lane);
-    if (nrb == 2)
-        chunk_body<GATE_UP, 2>(P, wbase0, wbase1, smem, raw, lane_off, out_off, part, pos_begin, pos_end, wave, lane);
-    else
-        chunk_body<GATE_UP, 1>(P, wbase0, wbase1, smem, raw, lane_off, out_off, part, pos_begin, pos_end, wave, lane);
 }
 
 // ---- the activation rows' records, 16 lanes per (row, unit) ----------------------------------
@@ -448,12 +542,11 @@ __global__ void route_wide_rows_kernel(const float* __restrict__ logits, int64_t
 
 template <bool GATE_UP, bool ORDERED>
 hipError_t launch(const MoeGemmParams& P, int64_t max_chunks, hipStream_t stream) {
-    const size_t window = (size_t)P.k_units * kUnitLds, hbuf = GATE_UP ? (size_t)kRows * kHStride * 4 : 0;
-    const size_t lds = window > hbuf ? window : hbuf;
+    constexpr size_t lds = kRing * kUnitLds + (GATE_UP ? (size_t)kRows * kHStride * 4 : 0);
     auto fn = &moe_gemm_q4k_kernel<GATE_UP, ORDERED>;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kMaxUnits * kUnitLds);
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    const unsigned grid = (unsigned)((max_chunks * P.parts + 7) / 8 * 8);
+    const unsigned grid = (unsigned)std::min<int64_t>((max_chunks * P.parts + 7) / 8 * 8, 8 * kCusPerXcd);
     fn<<<grid, 64 * kWaves, lds, stream>>>(P);
     return hipGetLastError();
 }

@@ -97,6 +97,38 @@ def test_long_items_first(qa, per_expert, skew, inter, items):
     assert torch.equal(got.view(torch.int32), tiles.view(torch.int32))
 
 
+# a workgroup's items in turn, up to ten of gate | up and past the tables' eight: one, two, three and eight units of k (fewer steps
+# per item than the records are requested ahead, and more), items of 32 pairs and fewer between longer ones
+@pytest.mark.parametrize("E,hidden,inter", [(30, 256, 2048), (30, 2048, 256), (36, 512, 1536), (60, 768, 1024)])
+def test_many_items_per_workgroup(qa, E, hidden, inter):
+    import torch
+    from izwi_amd import capi
+    rng = np.random.default_rng(4800 + hidden)
+
+    def stack(n, k):
+        blocks = rng.integers(0, 256, size=(E * n * k // 256, 144), dtype=np.uint8)
+        blocks[:, :4] = (1e-3 * rng.uniform(0.5, 2.0, size=(blocks.shape[0], 2))).astype(np.float16).view(np.uint8)
+        return qa.QTensor.from_blocks(qa.GgmlDType.Q4K, blocks.reshape(-1), (E, n, k))
+
+    experts = qa.MoeExperts(stack(inter, hidden), stack(inter, hidden), stack(hidden, inter))
+    counts = rng.integers(300, 900, size=E)
+    counts[:4] = [0, 1, 640, 609]
+    t = int(counts.sum())
+    ids = torch.from_numpy(rng.permutation(np.repeat(np.arange(E, dtype=np.int32), counts)).reshape(t, 1)).cuda()
+    gen = torch.Generator(device="cuda").manual_seed(4801)
+    x = torch.randn(t, hidden, device="cuda", generator=gen)
+    wts = torch.rand(t, 1, device="cuda", generator=gen)
+    perm, offsets = qa.moe_sort(ids, E)
+    got = [experts.forward(x, ids, wts, perm, offsets) for _ in range(3)]
+    try:
+        capi.check(capi.lib().izwi_qmm_set_moe_expert_form(1))
+        tiles = experts.forward(x, ids, wts, perm, offsets)
+    finally:
+        capi.check(capi.lib().izwi_qmm_set_moe_expert_form(-1))
+    for g in got:
+        assert torch.equal(g.view(torch.int32), tiles.view(torch.int32))
+
+
 @pytest.mark.parametrize("t", [144, 500, 2100])  # 144 * 8 pairs: the one-workgroup sort; beyond 2048 pairs two launches
 def test_layer_equals_the_tile_kernels(qa, oracle, t):
     import torch
