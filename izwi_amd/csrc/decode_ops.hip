@@ -722,44 +722,51 @@ __global__ __launch_bounds__(256) void attn_partial_kernel(AttnParams<T> P) {
     }
 }
 
-// The whole attention of a query head in one workgroup of W waves, 8 W cache rows at a time, NB of them per row group
-// requested ahead: one launch where the splits above take two.  Rows, lanes and arithmetic as above; the eight row
-// groups of a wave meet under the wave's maximum on the vector ALU, the waves in LDS.
+// The whole attention of a query head in VS workgroups of W waves, 8 W cache rows at a time, NB of them per row group
+// requested ahead: one launch where the splits above take two.  Each of the VS works out all scores and sums its share of the
+// values' elements.  Rows, lanes and arithmetic as above; the eight row groups of a wave meet under the wave's maximum on the vector
+// ALU, the waves in LDS.
 //
-// Bound by two trips to memory and, from 128 positions on, by what one compute unit reads (1 KB of f32 keys and values a
-// position at 110 GB/s).  Decode layers in a graph, us each, splits and their merge (one launch up to 32 positions) / this, at
-// 33, 128, 256, 300 and 320 positions: 16 query heads on 8 20.8 / 18.1, 21.0 / 19.1, 20.8 / 20.6, 20.9 / 21.1, 20.9 / 21.0; 32 on 8
+// Bound by two trips to memory and by what one compute unit reads at 110 GB/s: of f32, 512 bytes of keys a position and, with VS = 4, 128
+// of values (512 with one workgroup per head).  us a call in a graph (without PREP), one workgroup per head, sixteen waves and a row ahead
+// beyond 128 positions, eight and two below / VS = 4, eight waves, two rows, at 33, 128, 200, 256 and 320 positions: 16 heads of 128 on 8
+// 3.3 4.8 5.9 6.2 6.9 / 2.7 3.7 4.2 4.5 4.9; 64 on 8 3.9 5.1 6.2 6.6 7.3 / 3.3 4.1 4.6 5.2 5.7; VS = 2: 100 on 10 3.9 5.1 6.3 6.7 7.5 /
+// 3.5 4.6 5.4 6.1 6.7, 128 on 16 4.1 5.8 7.3 7.9 9.1 / 3.6 5.3 6.5 7.7 8.7, 16 on 8 of 64 elements 2.7 3.7 4.5 4.7 5.0 / 2.5 3.4 3.7
+// 3.9 4.2, f16 16 on 8 3.4 4.6 6.0 6.6 7.4 / 2.9 4.0 4.9 5.3 6.1.  The 28 layers of the 0.6B shapes and the head at 300 positions 633 / 578 us
+// (VS = 4; sixteen waves, one row 576, two rows 583, three 590; eight waves, four rows 582; VS = 2: 593 to 602), at 121 positions 568 / 537
+// (546, 548, 548; 539; 550 to 558), at 21 508 / 490 (505, 505, 505; 494; 497 to 514).  As many workgroups per head as the compute units
+// have room for: beyond that (more than half as many heads as compute units, or f16 heads of 64 elements, whose rows are one
+// 128-byte piece a row group) a head stays in one.
+//
+// Where it is taken (us a decode layer in a graph when the line was drawn, splits and their merge / one workgroup per head, at 33,
+// 128, 256, 300 and 320 positions): 16 query heads on 8 20.8 / 18.1, 21.0 / 19.1, 20.8 / 20.6, 20.9 / 21.1, 20.9 / 21.0; 32 on 8
 // 51.7 / 46.8, 51.7 / 48.4, 51.7 / 50.3, 51.8 / 50.9, 51.8 / 51.2; 40 on 8 52.3 / 50.4, 52.4 / 52.0, 53.3 / 53.5, 53.3 / 54.2,
-// 53.3 / 54.3; 8 on 8 of 64 elements 18.7 / 16.7, 18.8 / 17.2, 18.7 / 18.2, 18.8 / 18.1, 18.8 / 18.2; 4 on 1 21.5 / 17.2 to 21.7 / 19.9.
-// The line is where the splits catch up: they read a cache row once for `g` query heads (g below: 4, 2 or 1), here every head reads its
-// rows for itself, but with few heads per row they leave more of the chip busy.  Two heads: at 300 positions still this, whose
-// launch saved counts where the host launches as slowly as the GPU runs (16 on 8 called from Python 218 - 245 / 210).  And a head per
-// compute unit at the most.  Two rows ahead on eight waves are the faster form up to 128
-// positions (128: 186 / 194 for 8 layers), one on sixteen beyond (300: 210 / 207); two ahead on sixteen spill.
+// 53.3 / 54.3.  And a head per compute unit at the most.
 constexpr int kOneLaunchPositions = 320;
 inline int one_launch_positions(int64_t head_dim, int g) { return head_dim == 128 && g == 1 ? 256 : kOneLaunchPositions; }
-template <typename T, int HD, bool PREP, int W, int NB>
+template <typename T, int HD, bool PREP, int W, int NB, int VS>
 __global__ __launch_bounds__(64 * W) void attn_one_kernel(AttnParams<T> P) {
     static_assert(!PREP || std::is_same<T, float>::value, "the one-token step is built for f32");
-    constexpr int EC = kEC<T>, NI = HD / (8 * EC), E = EC * NI, kWaves = W, kRows = 8 * kWaves;
-    __shared__ __attribute__((aligned(16))) float red[kWaves][HD + 4]; // [.. HD): sums, [HD]: maximum, [HD + 1]: weight sum
+    constexpr int EC = kEC<T>, NI = HD / (8 * EC), E = EC * NI, NV = NI / VS, EV = EC * NV, DV = HD / VS, kWaves = W, kRows = 8 * kWaves;
+    static_assert(NI % VS == 0);
+    __shared__ __attribute__((aligned(16))) float red[kWaves][DV + 4]; // [.. DV): sums, [DV]: maximum, [DV + 1]: weight sum
     __shared__ __attribute__((aligned(16))) float prep[PREP ? 3 : 1][PREP ? HD : 4]; // normed, rotated q head and k_new, v_new
-    const int h = blockIdx.x, kvh = h / P.group;
+    const int h = blockIdx.x, kvh = h / P.group, d0 = VS > 1 ? blockIdx.y * DV : 0; // values d0 .. d0 + DV - 1 of the head
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j = lane & 7, slot = wave * 8 + (lane >> 3);
     const int pos = P.kv_len - 1, rows = PREP ? pos : P.kv_len; // PREP: the new position is not in the cache yet
     const T* kb = P.k + (int64_t)kvh * P.kv_capacity * HD + EC * j;
-    const T* vb = P.v + (int64_t)kvh * P.kv_capacity * HD + EC * j;
-    auto load_row = [&](int p, float (&kr)[E], float (&vr)[E]) {
+    const T* vb = P.v + (int64_t)kvh * P.kv_capacity * HD + d0 + EC * j;
+    auto load_row = [&](int p, float (&kr)[E], float (&vr)[EV]) {
 #pragma unroll
-        for (int i = 0; i < 2 * NI; i++) {
+        for (int i = 0; i < NI + NV; i++) {
             float t[EC];
             ld16<T>((i < NI ? kb : vb) + (int64_t)p * HD + 8 * EC * (i % NI), t);
 #pragma unroll
             for (int c = 0; c < EC; c++) (i < NI ? kr : vr)[EC * (i % NI) + c] = t[c];
         }
     };
-    float qr[E], kr[NB][E], vr[NB][E];
+    float qr[E], kr[NB][E], vr[NB][EV];
     float v_copy = 0.0f;
     auto first_rows = [&] {
 #pragma unroll
@@ -785,7 +792,7 @@ __global__ __launch_bounds__(64 * W) void attn_one_kernel(AttnParams<T> P) {
         if (threadIdx.x < HD) prep[2][threadIdx.x] = v_copy;
         __syncthreads();
         // the first head of a kv head appends the new position; nobody reads that cache row in this launch
-        if (h == kvh * P.group && threadIdx.x < HD) {
+        if (h == kvh * P.group && d0 == 0 && threadIdx.x < HD) {
             P.k_append[((int64_t)kvh * P.kv_capacity + pos) * HD + threadIdx.x] = prep[1][threadIdx.x];
             P.v_append[((int64_t)kvh * P.kv_capacity + pos) * HD + threadIdx.x] = v_copy;
         }
@@ -804,10 +811,10 @@ __global__ __launch_bounds__(64 * W) void attn_one_kernel(AttnParams<T> P) {
 #pragma unroll
         for (int c = 0; c < EC; c++) qr[EC * i + c] = t[c];
     }
-    float m = -INFINITY, l = 0.0f, acc[E];
+    float m = -INFINITY, l = 0.0f, acc[EV];
 #pragma unroll
-    for (int e = 0; e < E; e++) acc[e] = 0.0f;
-    auto accumulate = [&](const float (&kr)[E], const float (&vr)[E]) {
+    for (int e = 0; e < EV; e++) acc[e] = 0.0f;
+    auto accumulate = [&](const float (&kr)[E], const float (&vr)[EV]) {
         float dot = 0.0f;
 #pragma unroll
         for (int e = 0; e < E; e++) dot += qr[e] * kr[e];
@@ -815,7 +822,7 @@ __global__ __launch_bounds__(64 * W) void attn_one_kernel(AttnParams<T> P) {
         const float mn = fmaxf(m, s), alpha = merge_weight(m, mn), pe = exp_neg(s - mn);
         m = mn, l = l * alpha + pe;
 #pragma unroll
-        for (int e = 0; e < E; e++) acc[e] = acc[e] * alpha + pe * vr[e];
+        for (int e = 0; e < EV; e++) acc[e] = acc[e] * alpha + pe * vr[e];
     };
     for (int p = slot; p < rows;) {
 #pragma unroll
@@ -832,7 +839,7 @@ __global__ __launch_bounds__(64 * W) void attn_one_kernel(AttnParams<T> P) {
 #pragma unroll
                 for (int c = 0; c < EC; c++) {
                     kr[0][EC * i + c] = prep[1][8 * EC * i + EC * j + c];
-                    vr[0][EC * i + c] = prep[2][8 * EC * i + EC * j + c];
+                    if (i < NV) vr[0][EC * i + c] = prep[2][d0 + 8 * EC * i + EC * j + c];
                 }
             accumulate(kr[0], vr[0]);
         }
@@ -842,29 +849,29 @@ __global__ __launch_bounds__(64 * W) void attn_one_kernel(AttnParams<T> P) {
     auto over_groups = [](float v) { return qmm_add_lane32(qmm_add_lane16(v + dpp_f<0x128>(v))); };
     l = over_groups(l * ww);
 #pragma unroll
-    for (int e = 0; e < E; e++) acc[e] = over_groups(acc[e] * ww);
+    for (int e = 0; e < EV; e++) acc[e] = over_groups(acc[e] * ww);
     if (lane < 8) {
 #pragma unroll
-        for (int i = 0; i < NI; i++)
+        for (int i = 0; i < NV; i++)
 #pragma unroll
             for (int c = 0; c < EC; c += 4)
                 *reinterpret_cast<float4*>(&red[wave][8 * EC * i + EC * j + c]) =
                     make_float4(acc[EC * i + c], acc[EC * i + c + 1], acc[EC * i + c + 2], acc[EC * i + c + 3]);
-        if (j == 0) red[wave][HD] = wm, red[wave][HD + 1] = l;
+        if (j == 0) red[wave][DV] = wm, red[wave][DV + 1] = l;
     }
     __syncthreads();
-    if (threadIdx.x < HD) {
+    if (threadIdx.x < DV) {
         const int d = threadIdx.x;
         float mn = -INFINITY, a = 0.0f, lsum = 0.0f;
 #pragma unroll
-        for (int w = 0; w < kWaves; w++) mn = fmaxf(mn, red[w][HD]);
+        for (int w = 0; w < kWaves; w++) mn = fmaxf(mn, red[w][DV]);
 #pragma unroll
         for (int w = 0; w < kWaves; w++) {
-            const float g = merge_weight(red[w][HD], mn);
+            const float g = merge_weight(red[w][DV], mn);
             a += red[w][d] * g;
-            lsum += red[w][HD + 1] * g;
+            lsum += red[w][DV + 1] * g;
         }
-        st1(P.out + (int64_t)h * HD + d, a * (1.0f / lsum));
+        st1(P.out + (int64_t)h * HD + d0 + d, a * (1.0f / lsum));
     }
 }
 
@@ -955,17 +962,21 @@ hipError_t launch_attn_partial_form(const AttnParams<T>& P, int g, dim3 grid, hi
     return hipGetLastError();
 }
 template <typename T, int HD, bool PREP>
-hipError_t launch_attn_one_form(const AttnParams<T>& P, hipStream_t stream) {
-    if (P.kv_len <= 128) attn_one_kernel<T, HD, PREP, 8, 2><<<P.heads, 512, 0, stream>>>(P);
-    else attn_one_kernel<T, HD, PREP, 16, 1><<<P.heads, 1024, 0, stream>>>(P);
+hipError_t launch_attn_one_form(const AttnParams<T>& P, int n_cus, hipStream_t stream) {
+    constexpr int NI = HD / (8 * kEC<T>);
+    constexpr auto most = [](int vs) { return NI % vs ? 1 : vs; };
+    if (NI % 4 == 0 && 4 * P.heads <= n_cus) attn_one_kernel<T, HD, PREP, 8, 2, most(4)><<<dim3(P.heads, 4), 512, 0, stream>>>(P);
+    else if (NI % 2 == 0 && 2 * P.heads <= n_cus) attn_one_kernel<T, HD, PREP, 8, 2, most(2)><<<dim3(P.heads, 2), 512, 0, stream>>>(P);
+    else if (P.kv_len <= 128) attn_one_kernel<T, HD, PREP, 8, 2, 1><<<P.heads, 512, 0, stream>>>(P);
+    else attn_one_kernel<T, HD, PREP, 16, 1, 1><<<P.heads, 1024, 0, stream>>>(P);
     return hipGetLastError();
 }
 template <typename T, int HD>
-hipError_t launch_attn_one(const AttnParams<T>& P, hipStream_t stream) {
+hipError_t launch_attn_one(const AttnParams<T>& P, int n_cus, hipStream_t stream) {
     if constexpr (std::is_same<T, float>::value) {
-        if (P.k_new) return launch_attn_one_form<T, HD, true>(P, stream);
+        if (P.k_new) return launch_attn_one_form<T, HD, true>(P, n_cus, stream);
     }
-    return launch_attn_one_form<T, HD, false>(P, stream);
+    return launch_attn_one_form<T, HD, false>(P, n_cus, stream);
 }
 template <typename T, int HD>
 hipError_t launch_attn_partial(const AttnParams<T>& P, int g, dim3 grid, hipStream_t stream) {
@@ -1154,7 +1165,7 @@ int decode_attention_impl(const T* q, const T* k, const T* v, int64_t num_heads,
         P.part = (float*)scratch;
     }
     if (one_launch_pays) {
-        OPS_TRY((head_dim == 64 ? launch_attn_one<T, 64>(P, stream) : launch_attn_one<T, 128>(P, stream)));
+        OPS_TRY((head_dim == 64 ? launch_attn_one<T, 64>(P, n_cus, stream) : launch_attn_one<T, 128>(P, n_cus, stream)));
         OPS_TRY(oo.finish(stream));
         return IZWI_QMM_OK;
     }

@@ -147,6 +147,21 @@ def test_decode_gqa_attention_splits(qa, oracle, d, kv_len):
     assert close16(got, oracle.decode_gqa_attention(q, k, v, kv_len, d ** -0.5))
 
 
+# a head in four, two and one workgroups, each with its share of the value elements: rows of a wave, of all waves, of two rounds
+# and one more
+@pytest.mark.parametrize("heads,kv_heads,d", [(64, 8, 128), (65, 13, 128), (128, 16, 64), (136, 8, 128)])
+@pytest.mark.parametrize("kv_len", [1, 8, 63, 65, 128, 129, 256])
+def test_decode_gqa_attention_shares_of_the_values(qa, oracle, heads, kv_heads, d, kv_len):
+    _say(f"attention heads={heads} kv_heads={kv_heads} d={d} kv_len={kv_len}")
+    q = oracle.randn(31 + kv_len, (1, heads, 1, d))
+    k, v = oracle.randn(32 + d, (1, kv_heads, kv_len, d)), oracle.randn(33 + d, (1, kv_heads, kv_len, d))
+    got = qa.try_fused_decode_gqa_attention_with_kv_len(dev(q), dev(k), dev(v), heads, kv_heads, d, kv_len, d ** -0.5)
+    assert close(got, oracle.decode_gqa_attention(q, k, v, kv_len, d ** -0.5))
+    q, k, v = (t.astype(np.float16).astype(np.float32) for t in (q, k, v))
+    got = qa.try_fused_decode_gqa_attention_with_kv_len(half(q), half(k), half(v), heads, kv_heads, d, kv_len, d ** -0.5)
+    assert close16(got, oracle.decode_gqa_attention(q, k, v, kv_len, d ** -0.5))
+
+
 @pytest.mark.parametrize("heads,kv_heads,d,kv_len,cap", [
     (32, 8, 128, 1, 1), (32, 8, 128, 17, 64), (32, 8, 128, 300, 512), (32, 8, 128, 2048, 2048),
     (32, 8, 128, 5000, 8192), (16, 8, 128, 777, 1000), (8, 8, 128, 100, 100), (24, 4, 128, 129, 200),
