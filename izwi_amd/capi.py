@@ -7,6 +7,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 
 OK = 0
+ERR_INVALID = -1
 DEVICE, HOST = 0, 1
 OUT_F32, OUT_BF16 = 0, 1
 LARGE_M_BF16, LARGE_M_INT8 = 0, 1  # izwi_qmm_large_m

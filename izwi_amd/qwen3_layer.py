@@ -13,8 +13,8 @@ from __future__ import annotations
 
 import torch
 
-from .capi import check, lib
-from .decode_ops import (_ok, decode_attention_step, qk_norm_rope_append, try_fused_decode_gqa_attention_with_kv_len, try_fused_qk_rms_norm,
+from .capi import ERR_INVALID, check, lib
+from .decode_ops import (decode_attention_step, qk_norm_rope_append, try_fused_decode_gqa_attention_with_kv_len, try_fused_qk_rms_norm,
                          try_fused_rms_norm, try_fused_rope_pair_bshd)
 from .qmatmul import QMatMul, Qwen3GateUpProjection, _stream_ptr, forward_group
 
@@ -72,24 +72,29 @@ class Qwen3DecodeLayer:
         launches of a 0.6B layer run for (28 layers and the head: 1850 us a token as calls, 855 this way).
         None for arguments it does not cover: those go call by call."""
         gate_up = self.gate_up._parts
-        if gate_up is None or not _ok(x, self.w_in, self.w_post, self.qk_w, cos_sin, k_cache, v_cache):
+        if gate_up is None:
             return None
-        q, k, v, o, down = (p.qtensor for p in (*self.qkv, self.o_proj, self.down_proj))
-        gate, up = gate_up[0].qtensor, gate_up[1].qtensor
-        h, kv, d, hidden, inter = self.heads, self.kv_heads, self.d, q._k, gate._n
-        cache = k_cache.shape
-        if (x.dtype is not torch.float32 or x.shape != (1, hidden) or self.w_in.numel() != hidden or self.w_post.numel() != hidden
-                or self.qk_w.numel() != 2 * d or cos_sin.numel() != d or len(cache) != 4 or cache[0] != 1 or cache[1] != kv
-                or cache[3] != d or v_cache.shape != cache):
-            return None
-        for w, n, cols in ((q, h * d, hidden), (k, kv * d, hidden), (v, kv * d, hidden), (o, hidden, h * d), (gate, inter, hidden),
-                           (up, inter, hidden), (down, hidden, inter)):
-            if w._n != n or w._k != cols or w._e != 1:
+        # (written out: every attribute and call here is paid once per layer and token; weights that do not fit together are refused by
+        # the library before it launches anything, and then go call by call like everything else)
+        w_in, w_post, qk_w = self.w_in, self.w_post, self.qk_w
+        device = x.get_device()
+        for t in (x, w_in, w_post, qk_w, cos_sin, k_cache, v_cache):
+            if t.dtype is not torch.float32 or t.get_device() != device or not t.is_contiguous():
                 return None
-        floats = sum(-(-n // 128) * 128 for n in (h * d, kv * d, kv * d, h * d, hidden, inter))
+        qkv, h, kv, d = self.qkv, self.heads, self.kv_heads, self.d
+        q, gate = qkv[0].qtensor, gate_up[0].qtensor
+        hidden, cache = q._k, k_cache.shape
+        if (device < 0 or x.shape != (1, hidden) or w_in.numel() != hidden or w_post.numel() != hidden or qk_w.numel() != 2 * d
+                or cos_sin.numel() != d or len(cache) != 4 or cache[0] != 1 or cache[1] != kv or cache[3] != d or v_cache.shape != cache):
+            return None
+        floats = 2 * (h * d + 127 & -128) + 2 * (kv * d + 127 & -128) + (hidden + 127 & -128) + (gate._n + 127 & -128)
         workspace, y = x.new_empty(floats), x.new_empty((1, hidden))
-        check(lib().izwi_qmm_decode_layer_f32(q._h, k._h, v._h, o._h, gate._h, up._h, down._h, x.data_ptr(), self.w_in.data_ptr(),
-                                              self.w_post.data_ptr(), self.qk_w.data_ptr(), cos_sin.data_ptr(), h, kv, d, self.eps,
-                                              k_cache.data_ptr(), v_cache.data_ptr(), cache[2], pos, workspace.data_ptr(),
-                                              4 * floats, y.data_ptr(), _stream_ptr(x)))
+        rc = lib().izwi_qmm_decode_layer_f32(q._h, qkv[1].qtensor._h, qkv[2].qtensor._h, self.o_proj.qtensor._h, gate._h,
+                                             gate_up[1].qtensor._h, self.down_proj.qtensor._h, x.data_ptr(), w_in.data_ptr(),
+                                             w_post.data_ptr(), qk_w.data_ptr(), cos_sin.data_ptr(), h, kv, d, self.eps,
+                                             k_cache.data_ptr(), v_cache.data_ptr(), cache[2], pos, workspace.data_ptr(),
+                                             4 * floats, y.data_ptr(), _stream_ptr(x))
+        if rc == ERR_INVALID:
+            return None
+        check(rc)
         return y
