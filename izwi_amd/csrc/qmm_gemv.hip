@@ -207,8 +207,26 @@ __device__ __forceinline__ void gemv_body(const GemvParams& P, int m_begin, int 
                     const XSource xs{P.x, GROUPED ? P.perm : nullptr, P.x_div, m0, m_end, P.k, k_units};
                     float4 f[4];
                     float v[16];
-                    const bool in0 = x_item_issue<MT, XB>(xs, group, group < items, f);
                     float4 fnw[4];
+                    // one row of whole 256-value units: an item that exists is in range, and only those are quantized
+                    constexpr bool kWhole = MT == 1 && QT != QMM_Q8_0 && !GATED; // (the gated form measured no faster with it)
+                    // One row in straight-line form: a wave has four 16-lane groups and its one panel at most four units, so no group
+                    // takes a second item.  Left out, the loop's registers beside the panel bring the NORM form of Q4_K from 90 to 77
+                    // (six waves per SIMD instead of five: all 768 workgroups of an 8B gate | up at once) and Q6_K's from 116 to 92; a
+                    // decode step of 8 layers of the 8B shapes 409 -> 402.5 us, with Q4_K_M's types 417 -> 410.  Not Q8_0 (28 layers of
+                    // the 0.6B shapes 581.7 -> 584.5) and not the gated form without a norm (the expert layer of one to three tokens
+                    // 11.9 -> 12.5, 13.9 -> 14.7, 18.3 -> 18.9; of four 22.2 -> 21.0).
+                    constexpr bool kOnePass = ONESHOT && MT == 1 && QT != QMM_Q8_0 && (NORM || !GATED);
+                    // NORM: sum of the raw squares of the item (all 16 lanes of the group), then x * norm_w
+                    auto norm_item = [&](int item, bool in_range, const float4 (&fw)[4]) {
+                        float wv[16], ss = 0.0f;
+                        x16_finish<false>(fw, in_range, wv);
+#pragma unroll
+                        for (int i = 0; i < 16; i++) ss += v[i] * v[i], v[i] *= wv[i];
+                        ss = row16_sum(ss);
+                        if ((threadIdx.x & 15) == 0) xss[(item % MT) * k_units + item / MT] = ss;
+                    };
+                    const bool in0 = x_item_issue<MT, XB>(xs, group, group < items, f);
                     if (NORM) x16_issue<false>(P.norm_w + (group / MT) * 256 + 16 * (threadIdx.x & 15), P.norm_w, in0, fnw);
                     if (IO != 0 || NORM) __builtin_amdgcn_sched_barrier(0); // the activation loads stay in front
                     if constexpr (Pick::kActive) {
@@ -232,21 +250,10 @@ __device__ __forceinline__ void gemv_body(const GemvParams& P, int m_begin, int 
                         res_raw = *reinterpret_cast<const uint32_t*>(rp);
                     }
                     if (m0 != m_begin) lds_barrier(); // the previous rows' readers are done
-                    // one row of whole 256-value units: an item that exists is in range, and only those are quantized
-                    constexpr bool kWhole = MT == 1 && QT != QMM_Q8_0 && !GATED; // (the gated form measured no faster with it)
                     x16_finish<XB, kWhole>(f, in0, v);
-                    // NORM: sum of the raw squares of the item (all 16 lanes of the group), then x * norm_w
-                    auto norm_item = [&](int item, bool in_range, const float4 (&fw)[4]) {
-                        float wv[16], ss = 0.0f;
-                        x16_finish<false>(fw, in_range, wv);
-#pragma unroll
-                        for (int i = 0; i < 16; i++) ss += v[i] * v[i], v[i] *= wv[i];
-                        ss = row16_sum(ss);
-                        if ((threadIdx.x & 15) == 0) xss[(item % MT) * k_units + item / MT] = ss;
-                    };
                     if (NORM && group < items) norm_item(group, in0, fnw);
                     if (group < items) x_item_quantize<QT, MT>(l, k_units, group, v);
-                    for (int item = group + n_groups; item < items; item += n_groups) {
+                    for (int item = group + n_groups; !kOnePass && item < items; item += n_groups) {
                         const bool in1 = x_item_issue<MT, XB>(xs, item, true, f);
                         if (NORM) x16_issue<false>(P.norm_w + (item / MT) * 256 + 16 * (threadIdx.x & 15), P.norm_w, in1, fnw);
                         x16_finish<XB, kWhole>(f, in1, v);
@@ -338,7 +345,7 @@ __device__ __forceinline__ void gemv_body(const GemvParams& P, int m_begin, int 
 // small batch hold one or two pairs, and a row costs its share of the arithmetic
 // whether it exists or not.
 // The dense straight-line single-row Q4_K form is held to 80 registers: six waves per SIMD,
-// i.e. two 12-wave workgroups per CU.
+// i.e. two 12-wave workgroups per CU, three of eight waves.
 template <int QT, int MT, bool GATED, bool GROUPED, bool ONESHOT, int IO, bool NORM, bool TILEMAP, bool XBLK = false>
 __device__ __forceinline__ void gemv_entry(const GemvParams& P, const GemvParams& P0, int n_weights) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -379,7 +386,7 @@ __device__ __forceinline__ void gemv_entry(const GemvParams& P, const GemvParams
 // of a group of weights are indexed in the block itself, P0).
 template <int QT, int MT, bool GATED, bool GROUPED, bool ONESHOT = false, int IO = 0, bool NORM = false, bool TILEMAP = false>
 __global__ __launch_bounds__(64 * kMaxWaves)
-__attribute__((amdgpu_waves_per_eu(NORM ? 3 : (ONESHOT && MT == 1 && QT == QMM_Q4_K) ? 6 : 3)))
+__attribute__((amdgpu_waves_per_eu(ONESHOT && MT == 1 && QT == QMM_Q4_K ? 6 : 3)))
 void gemv_kernel(const uint8_t* w_arg, const float* x_arg, float* y_arg, int m_arg, int n_arg, int k_arg, int k_groups_arg,
                  int panel_bytes_arg, int row_tiles_arg, int split_arg, int wave_magic_arg, GemvParams P0) {
     static_assert(!GROUPED, "the expert-grouped launches go through gemv_grouped_kernel");
