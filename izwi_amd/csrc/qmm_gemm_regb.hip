@@ -182,8 +182,6 @@ __device__ __forceinline__ void chain(F&& f, M&& more) {
         }
 }
 
-__device__ __forceinline__ float silu(float v) { return v / (1.0f + expf(-v)); }
-
 // GATED: members 0 and 1 are gate and up of one shape, k is not split, and y = silu(gate) * up: a workgroup owns 64 columns of
 // both (two of its four column groups each), whose sums meet in LDS; no launch behind it and no f32 products in memory.
 template <int QT, int MT, bool GATED>
@@ -442,12 +440,12 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_regb_kernel(RegbParams P)
         if (!is_up)
             for (int r = 0; r < 4; r++) {
                 const f32x4 v = *reinterpret_cast<const f32x4*>(at + r * 1024);
-                for (int e = 0; e < 4; e++) sum[0][4 * r + e] = silu(sum[0][4 * r + e]) * v[e];
+                for (int e = 0; e < 4; e++) sum[0][4 * r + e] = qmm_silu(sum[0][4 * r + e]) * v[e];
             }
         else if constexpr (kOwn > 1)
             for (int r = 0; r < 4; r++) {
                 const f32x4 v = *reinterpret_cast<const f32x4*>(at + 4096 + r * 1024);
-                for (int e = 0; e < 4; e++) sum[1][4 * r + e] = silu(v[e]) * sum[1][4 * r + e];
+                for (int e = 0; e < 4; e++) sum[1][4 * r + e] = qmm_silu(v[e]) * sum[1][4 * r + e];
             }
     }
     // A block goes where the wave has read the other half's sums of it: chunk c (four columns) of row r at chunk c ^ (r / 2 % 8)

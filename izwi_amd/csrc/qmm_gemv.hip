@@ -81,8 +81,6 @@ struct GemvParams {
 };
 static_assert(offsetof(GemvParams, k_units) == 64, "first-load fields must fill one 64-byte line");
 
-__device__ __forceinline__ float silu(float v) { return v / (1.0f + expf(-v)); }
-
 // MT rows per pass.  GATED: two weight stacks share x and the result is
 // silu(w x) * (w2 x) (the expert MLP's gate/up pair); the second half of the
 // workgroup's waves works on the second stack, so that the panels of both are
@@ -330,7 +328,7 @@ __device__ __forceinline__ void gemv_body(const GemvParams& P, int m_begin, int 
                                                             : __uint_as_float(res_raw);
                             qmm_store(y_out, QmmEpilogue{nullptr, P.ep.y_bf16}, idx, sum + res);
                         } else {
-                            y_out[yr * n_rows + row] = GATED ? silu(sum) * sum2 : sum;
+                            y_out[yr * n_rows + row] = GATED ? qmm_silu(sum) * sum2 : sum;
                         }
                     }
                 }
@@ -719,9 +717,9 @@ __global__ void silu_mul_kernel(const float* __restrict__ gate, const float* __r
     const bool whole = aligned && i + 4 <= count;
     if (whole) {
         const float4 g = *reinterpret_cast<const float4*>(gate + i), u = *reinterpret_cast<const float4*>(up + i);
-        v[0] = silu(g.x) * u.x, v[1] = silu(g.y) * u.y, v[2] = silu(g.z) * u.z, v[3] = silu(g.w) * u.w;
+        v[0] = qmm_silu(g.x) * u.x, v[1] = qmm_silu(g.y) * u.y, v[2] = qmm_silu(g.z) * u.z, v[3] = qmm_silu(g.w) * u.w;
     } else {
-        for (int e = 0; e < 4; e++) v[e] = i + e < count ? silu(gate[i + e]) * up[i + e] : 0.0f;
+        for (int e = 0; e < 4; e++) v[e] = i + e < count ? qmm_silu(gate[i + e]) * up[i + e] : 0.0f;
     }
     if (BF16) {
         uint16_t* o = static_cast<uint16_t*>(out) + i;

@@ -126,8 +126,6 @@ __global__ void quantize_ws_kernel(const void* __restrict__ x, int m, int k, int
     quantize_into_record<QT>(v, j, mr, ws + ((int64_t)tile * k_units + unit) * Unit<QT>::kBytes);
 }
 
-__device__ __forceinline__ float silu_f(float v) { return v / (1.0f + expf(-v)); }
-
 // The same quantizer on silu(gate) * up (the MLP's activation, worked out on the way in).
 template <int QT>
 __global__ void quantize_silu_mul_ws_kernel(const float* __restrict__ gate, const float* __restrict__ up, int m, int k,
@@ -145,7 +143,7 @@ __global__ void quantize_silu_mul_ws_kernel(const float* __restrict__ gate, cons
     load_run16<false>(gate + (int64_t)row * k + k0, gate, ok, g);
     load_run16<false>(up + (int64_t)row * k + k0, up, ok, u);
 #pragma unroll
-    for (int i = 0; i < 16; i++) g[i] = silu_f(g[i]) * u[i];
+    for (int i = 0; i < 16; i++) g[i] = qmm_silu(g[i]) * u[i];
     quantize_into_record<QT>(g, j, mr, ws + ((int64_t)tile * k_units + unit) * Unit<QT>::kBytes);
 }
 
@@ -191,7 +189,7 @@ __global__ void quantize_grouped_kernel(const float* __restrict__ x, const float
         float u[16];
         load_run16(x2 + src_row * k + k0, x2, in_range, u);
 #pragma unroll
-        for (int i = 0; i < 16; i++) v[i] = silu_f(v[i]) * u[i];
+        for (int i = 0; i < 16; i++) v[i] = qmm_silu(v[i]) * u[i];
     }
     quantize_into_record<QT>(v, j, mr, ws + ((int64_t)tile * k_units + unit) * Unit<QT>::kBytes);
 }
@@ -214,7 +212,7 @@ __global__ void quantize_rows_kernel(const float* __restrict__ x, const float* _
         float u[16];
         load_run16(x2 + row * k + k0, x2, in_range, u);
 #pragma unroll
-        for (int i = 0; i < 16; i++) v[i] = silu_f(v[i]) * u[i];
+        for (int i = 0; i < 16; i++) v[i] = qmm_silu(v[i]) * u[i];
     }
     quantize_into_record<QT, kRowRecord>(v, j, 0, out + group * kRowUnitBytes);
 }

@@ -101,8 +101,6 @@ __device__ __forceinline__ void wait_for(const uint32_t* counter, uint32_t at_le
     asm volatile("" ::: "memory");
 }
 __device__ __forceinline__ i32x4 lds_i32x4(uint32_t at) { return *reinterpret_cast<const __attribute__((address_space(3))) i32x4*>(at); }
-__device__ __forceinline__ float silu(float v) { return v / (1.0f + expf(-v)); }
-
 // The lane's number, worked out anew: what depends on it is not kept in registers over the loops.
 __device__ __forceinline__ int lane_here(int lane) {
     asm volatile("" : "+v"(lane));
@@ -348,7 +346,7 @@ __device__ __forceinline__ void chunk_body(const MoeGemmParams& P, Shared& S, St
 #pragma unroll
         for (int rb = 0; rb < NRB; rb++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[0][rb][r] = silu(acc[0][rb][r]) * acc[1][rb][r];
+            for (int r = 0; r < 16; r++) acc[0][rb][r] = qmm_silu(acc[0][rb][r]) * acc[1][rb][r];
         // (the next item's weights have landed; the compiler, told so, does not wait for the stores behind at the top of the loop)
         __builtin_amdgcn_s_waitcnt(wait_vector(0));
         wait_for(&S.h_read, (uint32_t)item * kWaves); // the last item's
