@@ -1987,7 +1987,7 @@ int moe_gemm(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, const izwi_
         const RoutingOut routing(ids_out, weights_out, ws + ids_at, ws + w_at, logits, x, out, t, top_k, n_experts, hidden);
         int32_t *r_ids = routing.ids, *r_perm = (int32_t*)(ws + perm_at), *r_off = (int32_t*)(ws + off_at);
         float* r_w = routing.weights;
-        e = qmm_launch_moe_route_wide_rows(logits, t, n_experts, top_k, r_ids, r_w, x, hidden, ws + x_at, stream);
+        e = qmm_launch_moe_route_wide_rows(logits, t, n_experts, top_k, r_ids, r_w, x, hidden, ws + x_at, ws + h_at, pairs, inter, stream);
         if (e == hipSuccess)
             e = qmm_launch_moe_sort(r_ids, pairs, n_experts, r_perm, r_off, chunks, (int32_t*)(ws + sort_at), stream,
                                     QMM_MOE_CHUNK_ROWS, owner, max_chunks, nullptr);
@@ -1996,13 +1996,13 @@ int moe_gemm(const izwi_qmm_weight* gate, const izwi_qmm_weight* up, const izwi_
         weights = r_w, perm = r_perm, offsets = r_off;
     } else {
         e = qmm_launch_moe_segments(offsets, n_experts, QMM_MOE_CHUNK_ROWS, chunks, owner, max_chunks, stream, nullptr);
-        if (e == hipSuccess) e = qmm_launch_wide_rows(x, t, hidden, ws + x_at, stream);
+        if (e == hipSuccess) e = qmm_launch_wide_rows(x, t, hidden, ws + x_at, ws + h_at, pairs, inter, stream);
     }
     if (e == hipSuccess)
         e = qmm_launch_moe_gemm_gate_up(G, gate->tiled, up->tiled, ws + x_at, top_k, perm, offsets, chunks, owner, n_experts,
                                         pairs, max_chunks, ws + h_at, stream);
     if (e == hipSuccess)
-        e = qmm_launch_moe_gemm_down(D, down->tiled, ws + h_at, perm, offsets, chunks, owner, n_experts, max_chunks, y, stream);
+        e = qmm_launch_moe_gemm_down(D, down->tiled, ws + h_at, perm, offsets, chunks, owner, n_experts, pairs, max_chunks, y, stream);
     if (e == hipSuccess) e = qmm_launch_moe_combine(y, weights, t, top_k, hidden, out, stream);
     if (e != hipSuccess) return fail_hip(e, "expert products");
     if (profiling()) g_silu_fused.fetch_add(1, std::memory_order_relaxed);

@@ -400,20 +400,23 @@ hipError_t qmm_launch_quantize_rows(int dtype, const float* x, const float* x2, 
 // Expert MLP of Q4_K stacks in chunks of QMM_MOE_CHUNK_ROWS sorted pairs of one expert (qmm_moe_gemm.hip):
 // the source rows as wide row records (a launch of its own, or inside the routing), gate | up with
 // silu(gate) * up leaving as wide row records by sorted position, down with f32 rows by pair.  `chunks` and
-// `chunk_expert`: the sort's tables for QMM_MOE_CHUNK_ROWS, max_chunks entries.
+// `chunk_expert`: the sort's tables for QMM_MOE_CHUNK_ROWS, max_chunks entries.  Behind both record buffers (`records` of the rows of x,
+// `h_records` of h_rows pairs, h_k values each) stands a row of zeros for the rows that a chunk lacks, left by the first launch.
 #define QMM_MOE_CHUNK_ROWS 64
 bool qmm_moe_gemm_supported(const QmmLayout& G, const QmmLayout& D, int64_t t, int top_k);
 size_t qmm_wide_records_bytes(int64_t rows, int64_t k);
-hipError_t qmm_launch_wide_rows(const float* x, int64_t rows, int64_t k, void* records, hipStream_t stream);
+hipError_t qmm_launch_wide_rows(const float* x, int64_t rows, int64_t k, void* records, void* h_records, int64_t h_rows, int64_t h_k,
+                                hipStream_t stream);
 hipError_t qmm_launch_moe_route_wide_rows(const float* logits, int64_t t, int n_experts, int top_k, int32_t* ids, float* weights,
-                                          const float* x, int64_t k, void* records, hipStream_t stream);
+                                          const float* x, int64_t k, void* records, void* h_records, int64_t h_rows, int64_t h_k,
+                                          hipStream_t stream);
 hipError_t qmm_launch_moe_gemm_gate_up(const QmmLayout& G, const void* gate, const void* up, const void* records, int top_k,
                                        const int32_t* perm, const int32_t* offsets, const int32_t* chunks,
                                        const int32_t* chunk_expert, int n_experts, int64_t pairs, int64_t max_chunks, void* out_records,
                                        hipStream_t stream);
 hipError_t qmm_launch_moe_gemm_down(const QmmLayout& D, const void* down, const void* records, const int32_t* perm,
                                     const int32_t* offsets, const int32_t* chunks, const int32_t* chunk_expert, int n_experts,
-                                    int64_t max_chunks, float* y, hipStream_t stream);
+                                    int64_t pairs, int64_t max_chunks, float* y, hipStream_t stream);
 // qmm_launch_moe_route that also writes the row records of the tokens' activation rows x [t, k]
 hipError_t qmm_launch_moe_route_rows(const float* logits, int64_t t, int n_experts, int top_k, int32_t* ids,
                                      float* weights, hipStream_t stream, const float* x, int64_t k, int dtype,
