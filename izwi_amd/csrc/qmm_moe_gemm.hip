@@ -63,7 +63,11 @@ constexpr int kSumsAt = 2 * kRows * 128, kScalesAt = kSumsAt + kRows * 32, kUnit
 static_assert(kUnitLds % 128 == 0);
 constexpr int kHStride = 264; // floats per row of silu(gate) * up in LDS
 constexpr int kRing = 4, kAhead = 2; // units of records in LDS, and how many steps ahead of its use one is requested
-constexpr int kTables = 8, kTablesAhead = 4; // items whose rows are known, and how many items ahead
+// Items whose rows are known, and how many items ahead.  A wave that enters item i writes the table of item i + kTablesAhead; with one
+// unit per item the slowest wave may then still store item i - kRing - 1 (it has counted that step as done), so the tables reach
+// further than from there to here: eight of them did not (an item's rows could go where a later item's belong).
+constexpr int kTables = 16, kTablesAhead = 4;
+static_assert(kTables >= kTablesAhead + kRing + 2 && (kTables & (kTables - 1)) == 0);
 // s_waitcnt vmcnt(n), n < 16, the other counters left alone
 constexpr int wait_vector(int n) { return 0x0f70 | n; }
 

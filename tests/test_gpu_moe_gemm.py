@@ -97,9 +97,11 @@ def test_long_items_first(qa, per_expert, skew, inter, items):
     assert torch.equal(got.view(torch.int32), tiles.view(torch.int32))
 
 
-# a workgroup's items in turn, up to ten of gate | up and past the tables' eight: one, two, three and eight units of k (fewer steps
-# per item than the records are requested ahead, and more), items of 32 pairs and fewer between longer ones
-@pytest.mark.parametrize("E,hidden,inter", [(30, 256, 2048), (30, 2048, 256), (36, 512, 1536), (60, 768, 1024)])
+# a workgroup's items in turn, eight of them and, of gate | up and of down with one unit of k, past the tables' sixteen: one, two, three
+# and eight units of k (fewer steps per item than the records are requested ahead, and more), items of 32 pairs and fewer between
+# longer ones
+@pytest.mark.parametrize("E,hidden,inter", [(30, 256, 2048), (30, 2048, 256), (36, 512, 1536), (60, 768, 1024), (64, 256, 2048),
+                                            (120, 2048, 256)])
 def test_many_items_per_workgroup(qa, E, hidden, inter):
     import torch
     from izwi_amd import capi
