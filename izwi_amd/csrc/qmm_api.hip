@@ -1941,7 +1941,7 @@ struct RoutingOut {
 };
 
 // Whether the Q4_K expert MLP runs as matrix products over 64-pair chunks: from nine sorted pairs per expert
-// on average.  Measured at 128 experts, top-8, hidden 2048, inter 768, per layer, chunks / expert form on
+// on average, or above eight (below).  As first built, at 128 experts, top-8, hidden 2048, inter 768, per layer, chunks / expert form on
 // 16-row tiles: 106 / 91 us at 56 tokens, 104 / 103 at 128, 108 / 111 at 144 (9 pairs), 108 / 118 at 256,
 // 136 / 156 at 512, 206 / 253 at 1024, 294 / 426 at 2048, 497 / 823 at 4096: below, the prefix of a workgroup (its
 // 32 rows at least, over all of k) is not paid back.
@@ -1952,11 +1952,17 @@ struct RoutingOut {
 // and 58 / 60 at 14.  With up to twelve units (inter 1024: 48 / 47, 48 / 48 and 52 / 53 at 9; inter 768: 46 / 46, 46 / 47
 // and 48 / 52) or workgroups for half of the compute units (32 experts, inter 1536: 66 / 66 at 9, 66 / 72 at 10; 64 experts,
 // inter 2048: 127 / 137) nine are enough.
+// From 16 experts on, more than eight: some expert has its second tile of 16 rows there, and here a workgroup takes its items in turn.
+// Tiles / this at 8.1 to 8.95 pairs, means of four routings: 128 experts top-8 of 2048 x 768 99 / 97 us (up to 1.4 % slower where no
+// expert has a second tile, 6 % faster where one has), 256 of 2048 x 512 138 / 125, 64 of 2048 x 1024 73 / 65, 64 of 2048 x 2048 112 / 112, 32 of
+// 2048 x 1536 62 / 58, 16 of 1024 x 1024 41 / 37, 16 of 2048 x 768 45 / 44, 128 of 512 x 256 40 / 30.  At eight and fewer the tiles:
+// 128 of 2048 x 768 90 / 96, 32 of 2048 x 1536 55 / 57, 16 of 1024 x 1024 30 / 37.
 bool moe_on_gemm(const QmmLayout& G, const QmmLayout& D, int64_t t, int top_k, int n_cus) {
-    const bool few_long = G.k_units + D.k_units > 12 && G.n_stacked * (G.n / 256) * 2 <= n_cus;
+    const int64_t E = G.n_stacked;
+    const bool few_long = G.k_units + D.k_units > 12 && E * (G.n / 256) * 2 <= n_cus;
     // (moe_on_tiles: a threshold raised through the environment holds for these kernels too)
     return qmm_moe_expert_form() < 0 && moe_on_tiles(t * top_k, (int)G.n_stacked) &&
-           t * top_k >= (few_long ? 14 : 9) * G.n_stacked && qmm_moe_gemm_supported(G, D, t, top_k);
+           t * top_k >= (few_long ? 14 * E : E >= 16 ? 8 * E + 1 : 9 * E) && qmm_moe_gemm_supported(G, D, t, top_k);
 }
 
 // moe_core on the kernels of qmm_moe_gemm.hip; workspace: y [pairs, hidden] | the token rows' records | the

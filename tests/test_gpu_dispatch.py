@@ -77,6 +77,14 @@ def test_expert_layers_of_few_experts():
     assert taken == [False, True, False, True, True, False, True]
 
 
+def test_expert_layers_of_sixteen_experts_and_more():
+    """Above eight pairs per expert the expert products."""
+    cases = [["moe", 64, 512, 512, 8, 64], ["moe", 64, 512, 512, 8, 65], ["moe", 16, 512, 512, 2, 64], ["moe", 16, 512, 512, 1, 129],
+             ["moe", 15, 512, 512, 1, 128]]
+    taken = ["moe_gemm_q4k_kernel" in names for names in kernels(cases)]
+    assert taken == [False, True, False, True, False]
+
+
 def test_expert_threshold_of_the_environment():
     """IZWI_QMM_MOE_MFMA_MIN_ROWS: below that many pairs per expert no matrix-core kernel, the products included."""
     case = ["moe", 8, 512, 512, 2, 80]  # 20 pairs per expert

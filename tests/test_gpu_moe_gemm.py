@@ -131,7 +131,7 @@ def test_many_items_per_workgroup(qa, E, hidden, inter):
         assert torch.equal(g.view(torch.int32), tiles.view(torch.int32))
 
 
-@pytest.mark.parametrize("t", [144, 500, 2100])  # 144 * 8 pairs: the one-workgroup sort; beyond 2048 pairs two launches
+@pytest.mark.parametrize("t", [129, 144, 500, 2100])  # 129: just over eight pairs per expert; 144 * 8 pairs: the one-workgroup sort; beyond 2048 pairs two launches
 def test_layer_equals_the_tile_kernels(qa, oracle, t):
     import torch
     from izwi_amd import capi
