@@ -736,7 +736,8 @@ __global__ __launch_bounds__(256) void attn_partial_kernel(AttnParams<T> P) {
 // (VS = 4; sixteen waves, one row 576, two rows 583, three 590; eight waves, four rows 582; VS = 2: 593 to 602), at 121 positions 568 / 537
 // (546, 548, 548; 539; 550 to 558), at 21 508 / 490 (505, 505, 505; 494; 497 to 514).  As many workgroups per head as the compute units
 // have room for: beyond that (more than half as many heads as compute units, or f16 heads of 64 elements, whose rows are one
-// 128-byte piece a row group) a head stays in one.
+// 128-byte piece a row group) a head stays in one.  So it does where `out` shares memory with what is read (out may be q): only
+// within a workgroup is everything read before the first store.
 //
 // Where it is taken (us a decode layer in a graph when the line was drawn, splits and their merge / one workgroup per head, at 33,
 // 128, 256, 300 and 320 positions): 16 query heads on 8 20.8 / 18.1, 21.0 / 19.1, 20.8 / 20.6, 20.9 / 21.1, 20.9 / 21.0; 32 on 8
@@ -962,21 +963,22 @@ hipError_t launch_attn_partial_form(const AttnParams<T>& P, int g, dim3 grid, hi
     return hipGetLastError();
 }
 template <typename T, int HD, bool PREP>
-hipError_t launch_attn_one_form(const AttnParams<T>& P, int n_cus, hipStream_t stream) {
+hipError_t launch_attn_one_form(const AttnParams<T>& P, int n_cus, bool in_place, hipStream_t stream) {
     constexpr int NI = HD / (8 * kEC<T>);
     constexpr auto most = [](int vs) { return NI % vs ? 1 : vs; };
-    if (NI % 4 == 0 && 4 * P.heads <= n_cus) attn_one_kernel<T, HD, PREP, 8, 2, most(4)><<<dim3(P.heads, 4), 512, 0, stream>>>(P);
-    else if (NI % 2 == 0 && 2 * P.heads <= n_cus) attn_one_kernel<T, HD, PREP, 8, 2, most(2)><<<dim3(P.heads, 2), 512, 0, stream>>>(P);
+    const int wgs = in_place ? 1 : n_cus / P.heads; // workgroups that a head may have
+    if (NI % 4 == 0 && wgs >= 4) attn_one_kernel<T, HD, PREP, 8, 2, most(4)><<<dim3(P.heads, 4), 512, 0, stream>>>(P);
+    else if (NI % 2 == 0 && wgs >= 2) attn_one_kernel<T, HD, PREP, 8, 2, most(2)><<<dim3(P.heads, 2), 512, 0, stream>>>(P);
     else if (P.kv_len <= 128) attn_one_kernel<T, HD, PREP, 8, 2, 1><<<P.heads, 512, 0, stream>>>(P);
     else attn_one_kernel<T, HD, PREP, 16, 1, 1><<<P.heads, 1024, 0, stream>>>(P);
     return hipGetLastError();
 }
 template <typename T, int HD>
-hipError_t launch_attn_one(const AttnParams<T>& P, int n_cus, hipStream_t stream) {
+hipError_t launch_attn_one(const AttnParams<T>& P, int n_cus, bool in_place, hipStream_t stream) {
     if constexpr (std::is_same<T, float>::value) {
-        if (P.k_new) return launch_attn_one_form<T, HD, true>(P, n_cus, stream);
+        if (P.k_new) return launch_attn_one_form<T, HD, true>(P, n_cus, in_place, stream);
     }
-    return launch_attn_one_form<T, HD, false>(P, n_cus, stream);
+    return launch_attn_one_form<T, HD, false>(P, n_cus, in_place, stream);
 }
 template <typename T, int HD>
 hipError_t launch_attn_partial(const AttnParams<T>& P, int g, dim3 grid, hipStream_t stream) {
@@ -1165,7 +1167,14 @@ int decode_attention_impl(const T* q, const T* k, const T* v, int64_t num_heads,
         P.part = (float*)scratch;
     }
     if (one_launch_pays) {
-        OPS_TRY((head_dim == 64 ? launch_attn_one<T, 64>(P, n_cus, stream) : launch_attn_one<T, 128>(P, n_cus, stream)));
+        const auto written = [&](const void* p, size_t bytes) {
+            const uintptr_t a = (uintptr_t)P.out, b = (uintptr_t)p;
+            return p != nullptr && a < b + bytes && b < a + qbytes;
+        };
+        const size_t new_bytes = (size_t)num_kv_heads * head_dim * sizeof(T), row_bytes = (size_t)head_dim * sizeof(T);
+        const bool in_place = written(P.q, qbytes) || written(P.k, cbytes) || written(P.v, cbytes) || written(P.k_new, new_bytes) ||
+                              written(P.v_new, new_bytes) || written(P.qk_weight, 2 * row_bytes) || written(P.cos_sin, row_bytes);
+        OPS_TRY((head_dim == 64 ? launch_attn_one<T, 64>(P, n_cus, in_place, stream) : launch_attn_one<T, 128>(P, n_cus, in_place, stream)));
         OPS_TRY(oo.finish(stream));
         return IZWI_QMM_OK;
     }

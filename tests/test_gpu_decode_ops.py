@@ -162,6 +162,36 @@ def test_decode_gqa_attention_shares_of_the_values(qa, oracle, heads, kv_heads, 
     assert close16(got, oracle.decode_gqa_attention(q, k, v, kv_len, d ** -0.5))
 
 
+# counts at which a head otherwise has four and two workgroups, and one position more than the one launch takes
+@pytest.mark.parametrize("heads,kv_heads,d,kv_len", [(16, 8, 128, 40), (64, 8, 128, 320), (100, 10, 128, 200), (128, 16, 64, 129), (1, 1, 128, 9),
+                                                     (16, 8, 128, 321)])
+def test_decode_gqa_attention_in_place(qa, oracle, heads, kv_heads, d, kv_len):
+    """out is q: both forms of the call and the one-token step."""
+    from izwi_amd import capi
+    _say(f"attention in place heads={heads} kv_heads={kv_heads} d={d} kv_len={kv_len}")
+    L, scale = capi.lib(), d ** -0.5
+    q, k, v = oracle.randn(41, (1, heads, 1, d)), oracle.randn(42, (1, kv_heads, kv_len, d)), oracle.randn(43, (1, kv_heads, kv_len, d))
+    got, kd, vd = dev(q), dev(k), dev(v)
+    capi.check(L.izwi_decode_gqa_attention_f32(got.data_ptr(), kd.data_ptr(), vd.data_ptr(), heads, kv_heads, d, kv_len, kv_len, scale,
+                                               got.data_ptr(), capi.DEVICE, None))
+    assert close(got, oracle.decode_gqa_attention(q, k, v, kv_len, scale))
+    q16, k16, v16 = (t.astype(np.float16).astype(np.float32) for t in (q, k, v))
+    got, kd, vd = half(q16), half(k16), half(v16)
+    capi.check(L.izwi_decode_gqa_attention_f16(got.data_ptr(), kd.data_ptr(), vd.data_ptr(), heads, kv_heads, d, kv_len, kv_len, scale,
+                                               got.data_ptr(), capi.DEVICE, None))
+    assert close16(got, oracle.decode_gqa_attention(q16, k16, v16, kv_len, scale))
+    w, ang = oracle.randn(44, (2 * d,), mean=1.0, std=0.2), oracle.randn(45, (d // 2,)) * 3.0
+    cs = np.concatenate([np.cos(ang), np.sin(ang)]).astype(np.float32)
+    k_new, v_new = oracle.randn(46, (kv_heads * d,)), oracle.randn(47, (kv_heads * d,))
+    got, kd, vd, kn, vn, wd, cd = dev(q), dev(k), dev(v), dev(k_new), dev(v_new), dev(w), dev(cs)
+    capi.check(L.izwi_decode_attention_step_f32(got.data_ptr(), kn.data_ptr(), vn.data_ptr(), wd.data_ptr(), cd.data_ptr(), heads, kv_heads,
+                                                d, 1e-6, kd.data_ptr(), vd.data_ptr(), kv_len, kv_len - 1, scale, got.data_ptr(), None))
+    qn, kn = oracle.qk_rms_norm(q.reshape(1, 1, heads, d), k_new.reshape(1, 1, kv_heads, d), w, 1e-6)
+    qr, kr = oracle.rope_pair_bshd(qn, kn, cs.reshape(1, d))
+    k[0, :, kv_len - 1], v[0, :, kv_len - 1] = kr.reshape(kv_heads, d), v_new.reshape(kv_heads, d)
+    assert close(got, oracle.decode_gqa_attention(qr.reshape(1, heads, 1, d), k, v, kv_len, scale)) and close(kd, k)
+
+
 @pytest.mark.parametrize("heads,kv_heads,d,kv_len,cap", [
     (32, 8, 128, 1, 1), (32, 8, 128, 17, 64), (32, 8, 128, 300, 512), (32, 8, 128, 2048, 2048),
     (32, 8, 128, 5000, 8192), (16, 8, 128, 777, 1000), (8, 8, 128, 100, 100), (24, 4, 128, 129, 200),

@@ -14,6 +14,7 @@ CHILD = """
 import json, sys
 import numpy as np, torch
 import izwi_amd as qa
+from izwi_amd import capi
 from oracle import oracle
 
 def matrix(n, k, dtype=12):
@@ -33,6 +34,12 @@ def call(kind, *sizes):
         heads, kv_heads, d, positions = sizes
         q, cache = torch.randn(1, heads, 1, d, device="cuda"), torch.randn(1, kv_heads, positions, d, device="cuda")
         return lambda: qa.try_fused_decode_gqa_attention(q, cache, cache, heads, kv_heads, d, d ** -0.5)
+    if kind == "attention in place":
+        heads, kv_heads, d, positions, at = sizes  # out begins `at` values into q
+        q, cache = torch.randn((heads + 1) * d, device="cuda"), torch.randn(1, kv_heads, positions, d, device="cuda")
+        return lambda: capi.check(capi.lib().izwi_decode_gqa_attention_f32(
+            q.data_ptr(), cache.data_ptr(), cache.data_ptr(), heads, kv_heads, d, positions, positions, d ** -0.5,
+            q.data_ptr() + 4 * at, capi.DEVICE, None))
     if kind == "group":
         dtype, ns, k, m = sizes
         parts, x = [matrix(n, k, dtype) for n in ns], torch.randn(m, k, device="cuda")
@@ -126,6 +133,17 @@ def test_attention_launches_by_length_and_heads():
     cases = [["attention", 16, 8, 128, 320], ["attention", 16, 8, 128, 321], ["attention", 32, 8, 128, 320], ["attention", 8, 8, 64, 320],
              ["attention", 40, 8, 128, 256], ["attention", 40, 8, 128, 257], ["attention", 4, 2, 256, 33]]
     assert ["attn_one_kernel" in names for names in kernels(cases)] == [True, False, True, True, True, False, False]
+
+
+def test_attention_in_place_keeps_a_head_in_one_workgroup():
+    """Several workgroups per head (the last template argument) only where none reads what another writes."""
+    cases = [["attention", 16, 8, 128, 40], ["attention", 100, 10, 128, 300], ["attention", 16, 8, 64, 300]]
+    assert [any(f", 2, {wgs}>" in names for wgs in (4, 2)) for names in kernels(cases)] == [True] * 3
+    for at in (0, 4, 64):
+        placed = kernels([["attention in place", *sizes, at] for _, *sizes in cases])
+        assert ["8, 2, 1>" in names or "16, 1, 1>" in names for names in placed] == [True] * 3
+    beside, = kernels([["attention in place", 1, 1, 128, 40, 128]])  # right behind q
+    assert "8, 2, 4>" in beside
 
 
 def test_attention_splits_of_the_environment():
