@@ -71,21 +71,9 @@ __device__ __forceinline__ float qmm_add_lane16(float v) {
     const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
-// v / (1 + e^-v), with the results of expf and an IEEE division (16 million values between -90 and 90, infinities and NaN: all the
-// same bits but below 2^-126) in 17 vector instructions instead of 25: 8 layers of the 0.6B shapes at 64 rows, where a lane of the
-// quantizer behind gate | up takes sixteen, 342.6 -> 339.8 us, at 20 rows 323.4 -> 320.2 (the expert layers the same within a
-// percent).  e^x = 2^n 2^f of the product x log2(e) and what its rounding lost; the argument is held where
-// 1 + e^-v is exactly 1 (from 17 on) and infinite, so neither needs a case of its own; both sides of the division a
-// quarter, so that the reciprocal is no subnormal, one Newton step, and the hardware's fix-up for zeros, infinities and NaN.
-__device__ __forceinline__ float qmm_silu(float v) {
-    const float x = __builtin_amdgcn_fmed3f(-v, -64.0f, 104.0f);
-    const float p = x * 0x1.715476p+0f; // log2(e) = this + 0x1.4ae0bep-26
-    const float lost = __builtin_fmaf(x, 0x1.4ae0bep-26f, __builtin_fmaf(x, 0x1.715476p+0f, -p));
-    const float n = __builtin_rintf(p);
-    const float e = __builtin_ldexpf(__builtin_amdgcn_exp2f((p - n) + lost), (int)n);
-    const float a = 0.25f * v, b = __builtin_fmaf(e, 0.25f, 0.25f), r = __builtin_amdgcn_rcpf(b), q = a * r;
-    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-b, q, a), r, q), b, a);
-}
+// In f32 with one rounding a step, for subnormal and huge v as well.  (Exp2 and a corrected reciprocal took 17 vector instructions
+// instead of 25 and 1 % off 8 layers of the 0.6B shapes at 64 rows, nothing off the expert layers, but lost bits of small v.)
+__device__ __forceinline__ float qmm_silu(float v) { return v / (1.0f + expf(-v)); }
 // the largest of the values of the lanes 16, 32 and 48 away and the lane's own (a NaN never wins)
 __device__ __forceinline__ float qmm_max_lane_rows(float v) {
     const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
