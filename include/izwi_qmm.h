@@ -412,7 +412,8 @@ int izwi_qmm_mlp_forward_f32(const izwi_qmm_weight* gate, const izwi_qmm_weight*
  * `[num_kv_heads * head_dim, hidden]`, o `[hidden, num_heads * head_dim]`, gate and up `[inter, hidden]`,
  * down `[hidden, inter]`; x and y are `[hidden]` (y may be x).  The intermediate results lie in `workspace`,
  * device memory of at least workspace_bytes: q, k, v, attention output (num_heads * head_dim), layer input
- * of the MLP (hidden) and its product (inter), each rounded up to 128 floats.  Device pointers only. */
+ * of the MLP (hidden) and its product (inter), each rounded up to 128 floats.  Device pointers only.
+ * IZWI_QMM_ERR_INVALID (shapes, a position outside the caches, gate and up of two types) is found before anything is launched. */
 int izwi_qmm_decode_layer_f32(const izwi_qmm_weight* q, const izwi_qmm_weight* k, const izwi_qmm_weight* v,
                               const izwi_qmm_weight* o, const izwi_qmm_weight* gate, const izwi_qmm_weight* up,
                               const izwi_qmm_weight* down, const float* x, const float* input_norm,

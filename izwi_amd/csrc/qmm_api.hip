@@ -1538,6 +1538,13 @@ int izwi_qmm_decode_layer_f32(const izwi_qmm_weight* q, const izwi_qmm_weight* k
     if (!is(q, n_q, hidden) || !is(k, n_kv, hidden) || !is(v, n_kv, hidden) || !is(o, hidden, n_q) || !is(gate, inter, hidden) ||
         !is(up, inter, hidden) || !is(down, hidden, inter))
         return fail(IZWI_QMM_ERR_INVALID, "decode_layer: the weights' shapes do not fit together");
+    // (what a later step would refuse as well: nothing is launched then)
+    if (gate->layout.dtype != up->layout.dtype || gate->device != up->device)
+        return fail(IZWI_QMM_ERR_INVALID, "decode_layer: gate and up are of different ggml dtypes (%d, %d) or live on different devices",
+                    gate->layout.dtype, up->layout.dtype);
+    if (num_heads % num_kv_heads || num_heads > 65535 || kv_capacity > 0x3fffffff || pos < 0 || pos >= kv_capacity)
+        return fail(IZWI_QMM_ERR_INVALID, "decode_layer: %lld heads, %lld kv heads, position %lld of %lld", (long long)num_heads,
+                    (long long)num_kv_heads, (long long)pos, (long long)kv_capacity);
     auto padded = [](int64_t count) { return (count + 127) & ~(int64_t)127; };
     const int64_t pieces[6] = {n_q, n_kv, n_kv, n_q, hidden, inter};
     float* at[6];

@@ -74,8 +74,8 @@ class Qwen3DecodeLayer:
         gate_up = self.gate_up._parts
         if gate_up is None:
             return None
-        # (written out: every attribute and call here is paid once per layer and token; weights that do not fit together are refused by
-        # the library before it launches anything, and then go call by call like everything else)
+        # (written out: every attribute and call here is paid once per layer and token; weights that do not fit together and a position
+        # outside the caches are refused by the library before it launches anything, and then go call by call like everything else)
         w_in, w_post, qk_w = self.w_in, self.w_post, self.qk_w
         device = x.get_device()
         for t in (x, w_in, w_post, qk_w, cos_sin, k_cache, v_cache):

@@ -103,3 +103,37 @@ def test_one_call_layer_equals_its_calls(qa, oracle, hidden, heads, kv_heads, d,
         assert torch.equal(got, want) and torch.equal(caches[0], ref[0]) and torch.equal(caches[1], ref[1])
     with pytest.raises(qa.QmmError):
         layer.forward(x, cos_sin, caches[0], caches[1], cap)
+
+
+def test_one_call_layer_refuses_before_it_launches(qa, oracle):
+    """Gate and up of two block types, heads that do not divide and a position outside the caches: refused with the caches and
+    the workspace as they were; the layer raises."""
+    from izwi_amd import capi
+    from izwi_amd.qwen3_layer import Qwen3DecodeLayer
+    hidden, heads, kv_heads, d, inter, cap = 512, 4, 2, 64, 512, 8
+    shapes = {"q": (heads * d, hidden), "k": (kv_heads * d, hidden), "v": (kv_heads * d, hidden), "o": (hidden, heads * d),
+              "gate": (inter, hidden), "up": (inter, hidden), "up8": (inter, hidden), "down": (hidden, inter)}
+    mm = {}
+    for i, (n, s) in enumerate(shapes.items()):
+        t = 8 if n == "up8" else 12
+        mm[n] = qa.QMatMul.from_qtensor(qa.QTensor.from_blocks(qa.GgmlDType(t), oracle.quantize(t, oracle.randn(80 + i, s, std=0.03)).reshape(-1), s))
+    dev = lambda seed, shape: torch.from_numpy(oracle.randn(seed, shape)).cuda()  # noqa: E731
+    x, w_in, w_post, qk_w, cos_sin = dev(90, (1, hidden)), dev(91, (hidden,)), dev(92, (hidden,)), dev(93, (2 * d,)), dev(94, (1, d))
+    caches = [dev(95 + i, (1, kv_heads, cap, d)) for i in range(2)]
+    workspace, y = torch.full((4096,), 7.0, device="cuda"), torch.full((1, hidden), 7.0, device="cuda")
+
+    def call(up, kv, pos):
+        h = [mm[n].qtensor._h for n in ("q", "k", "v", "o", "gate", up, "down")]
+        return capi.lib().izwi_qmm_decode_layer_f32(
+            *h, *(t.data_ptr() for t in (x, w_in, w_post, qk_w, cos_sin)), heads, kv, d, 1e-6, caches[0].data_ptr(), caches[1].data_ptr(),
+            cap, pos, workspace.data_ptr(), 4 * workspace.numel(), y.data_ptr(), torch.cuda.current_stream().cuda_stream)
+
+    before = [c.clone() for c in caches]
+    for args in (("up8", kv_heads, 0), ("up", kv_heads, cap), ("up", kv_heads, -1), ("up", 3, 0)):
+        assert call(*args) == capi.ERR_INVALID, args
+        torch.cuda.synchronize()
+        assert bool((workspace == 7.0).all()) and bool((y == 7.0).all()) and all(torch.equal(a, b) for a, b in zip(caches, before)), args
+    assert call("up", kv_heads, 0) == 0
+    layer = Qwen3DecodeLayer(w_in, w_post, mm["q"], mm["k"], mm["v"], qk_w, mm["o"], mm["gate"], mm["up8"], mm["down"], heads, kv_heads, d)
+    with pytest.raises(qa.QmmError):
+        layer.forward(x, cos_sin, caches[0], caches[1], 0)
