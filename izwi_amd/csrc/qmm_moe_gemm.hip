@@ -453,6 +453,25 @@ __device__ __forceinline__ void order_items(const MoeGemmParams& P, Shared& S, i
     }
 }
 
+// A run of two rounds: the second item of a workgroup, -1 if it has none.  Those whose first item is short are done first and are
+// first to take one, long ones first.  Places that heed no lengths gave some a long item behind a long one while their neighbours
+// were done: layer of 64 experts of 2048 x 1024 at 384 tokens with uneven counts (logits and N(0, 0.4) per expert) 125 us, and 119 with a
+// workgroup of its own for every item, which the hardware starts as others end; this way 112.  Even counts 82 / 83 / 82.  With more
+// rounds the differences even out.  A lane per item; the look brings the first item with it.
+__device__ __forceinline__ int second_item(const MoeGemmParams& P, int first, int run, int slot, int lane, WorkItem& it) {
+    const WorkItem mine = work_item(P, first + min(lane, run - 1));
+    const uint64_t heavy = __ballot(lane < run && mine.pos_end - mine.pos_begin > 32);
+    it = {__builtin_amdgcn_readlane(mine.e, slot), __builtin_amdgcn_readlane(mine.part, slot),
+          __builtin_amdgcn_readlane(mine.pos_begin, slot), __builtin_amdgcn_readlane(mine.pos_end, slot)};
+    const uint32_t before = (1u << slot) - 1, long0 = (uint32_t)heavy, long1 = (uint32_t)(heavy >> kCusPerXcd);
+    const uint32_t short1 = ~(uint32_t)0 >> (2 * kCusPerXcd - run) & ~long1; // (run > kCusPerXcd)
+    const int rank = long0 >> slot & 1 ? __popc(~long0) + __popc(long0 & before) : __popc(~long0 & before), longs = __popc(long1);
+    const uint32_t set = rank < longs ? long1 : short1;
+    const int nth = rank < longs ? rank : rank - longs;
+    const uint64_t at = __ballot(lane < kCusPerXcd && (set >> (lane & 31) & 1) && (int)__builtin_amdgcn_mbcnt_lo(set, 0) == nth);
+    return at ? kCusPerXcd + __ffsll((unsigned long long)at) - 1 : -1;
+}
+
 template <bool GATE_UP, bool ORDERED>
 __global__ __launch_bounds__(64 * kWaves) void moe_gemm_q4k_kernel(MoeGemmParams P) {
     extern __shared__ __attribute__((aligned(128))) uint8_t smem[];
@@ -463,14 +482,18 @@ __global__ __launch_bounds__(64 * kWaves) void moe_gemm_q4k_kernel(MoeGemmParams
     // Work items in the order (expert, part of the weight rows, chunk of the pairs), cut into eight equal
     // runs: workgroups go to the XCDs round-robin, so a run is one XCD's, and the chunks that read the same weights
     // follow one another there and find them in its L2.  A workgroup takes its items from every round of the run, in turn from
-    // its front and its back.
+    // its front and its back, of two rounds by their lengths.
     const int items = P.chunks[P.n_experts] * P.parts, per_xcd = (items + 7) >> 3;
     const int slot = (int)(blockIdx.x >> 3), slots = (int)(gridDim.x >> 3), first = (int)(blockIdx.x & 7) * per_xcd;
     const int run = min(per_xcd, items - first); // items of this XCD
     if (slot >= run) return; // uniform
     const auto place = [&](int j) { return j * slots + (j & 1 ? slots - 1 - slot : slot); };
     const bool ordered = ORDERED && run > kCusPerXcd && run <= kOrderedItems; // uniform
-    const auto local_item = [&](int j) { return ordered ? (int)__builtin_amdgcn_readfirstlane(S.order[place(j)]) : place(j); };
+    const bool two_rounds = !ORDERED && run > kCusPerXcd && run <= 2 * kCusPerXcd; // uniform
+    int second = -1;
+    const auto local_item = [&](int j) {
+        return ordered ? (int)__builtin_amdgcn_readfirstlane(S.order[place(j)]) : two_rounds && j == 1 ? second : place(j);
+    };
     Stream t{};
     t.n_items = __builtin_amdgcn_readfirstlane(run / slots + (place(run / slots) < run));
     if (threadIdx.x < (int)(offsetof(Shared, items) / 4)) reinterpret_cast<uint32_t*>(&S)[threadIdx.x] = 0;
@@ -480,7 +503,10 @@ __global__ __launch_bounds__(64 * kWaves) void moe_gemm_q4k_kernel(MoeGemmParams
     // The first item's weights, the first items' tables, the first steps' records
     const uint32_t slots16 = (uint32_t)P.slots * 16u;
     const uint32_t lane_off = (uint32_t)((lane >> 4) & 1) * (uint32_t)P.k_groups * (uint32_t)P.panel_bytes + (uint32_t)(lane & 15) * 16u;
-    first_panels<GATE_UP>(P, work_item(P, first + local_item(0)), wave, t.wp);
+    WorkItem it0;
+    if (two_rounds) second = second_item(P, first, run, slot, lane, it0), t.n_items = second < 0 ? 1 : 2;
+    else it0 = work_item(P, first + local_item(0));
+    first_panels<GATE_UP>(P, it0, wave, t.wp);
     UnitRegs raw[2];
 #pragma unroll
     for (int c = 0; c < 2; c++) request_unit(raw[c], t.wp[c], lane_off, lane_off + (uint32_t)(lane >> 5) * slots16, slots16);

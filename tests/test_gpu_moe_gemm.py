@@ -97,6 +97,36 @@ def test_long_items_first(qa, per_expert, skew, inter, items):
     assert torch.equal(got.view(torch.int32), tiles.view(torch.int32))
 
 
+# runs of an XCD's items around one, two and three rounds of 32 workgroups, of two the second items given out by length: all short, all
+# long, and both in every order; one, two and five units of k, of which a second item's are requested from the start
+@pytest.mark.parametrize("hidden", [256, 512, 1280])
+@pytest.mark.parametrize("per_xcd", [32, 33, 47, 63, 64, 65, 97])
+def test_second_items_by_length(qa, per_xcd, hidden):
+    import torch
+    from izwi_amd import capi
+    E, inter, rng = 8 * per_xcd // 2, 512, np.random.default_rng(4900 + per_xcd)  # two items per expert and chunk
+
+    def stack(n, k):
+        blocks = rng.integers(0, 256, size=(E * n * k // 256, 144), dtype=np.uint8)
+        blocks[:, :4] = (1e-3 * rng.uniform(0.5, 2.0, size=(blocks.shape[0], 2))).astype(np.float16).view(np.uint8)
+        return qa.QTensor.from_blocks(qa.GgmlDType.Q4K, blocks.reshape(-1), (E, n, k))
+
+    experts = qa.MoeExperts(stack(inter, hidden), stack(inter, hidden), stack(hidden, inter))
+    for counts in (np.full(E, 11), np.full(E, 34), np.where(rng.random(E) < 0.4, 40, 12), np.where(np.arange(E) < E // 3, 12, 50)):
+        t = int(counts.sum())
+        ids = torch.from_numpy(rng.permutation(np.repeat(np.arange(E, dtype=np.int32), counts)).reshape(t, 1)).cuda()
+        gen = torch.Generator(device="cuda").manual_seed(4901)
+        x, wts = torch.randn(t, hidden, device="cuda", generator=gen), torch.rand(t, 1, device="cuda", generator=gen)
+        perm, offsets = qa.moe_sort(ids, E)
+        got = experts.forward(x, ids, wts, perm, offsets)
+        try:
+            capi.check(capi.lib().izwi_qmm_set_moe_expert_form(1))
+            tiles = experts.forward(x, ids, wts, perm, offsets)
+        finally:
+            capi.check(capi.lib().izwi_qmm_set_moe_expert_form(-1))
+        assert torch.equal(got.view(torch.int32), tiles.view(torch.int32))
+
+
 # a workgroup's items in turn, eight of them and, of gate | up and of down with one unit of k, past the tables' sixteen: one, two, three
 # and eight units of k (fewer steps per item than the records are requested ahead, and more), items of 32 pairs and fewer between
 # longer ones
