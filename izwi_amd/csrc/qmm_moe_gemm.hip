@@ -457,12 +457,10 @@ __device__ __forceinline__ void order_items(const MoeGemmParams& P, Shared& S, i
 // first to take one, long ones first.  Places that heed no lengths gave some a long item behind a long one while their neighbours
 // were done: layer of 64 experts of 2048 x 1024 at 384 tokens with uneven counts (logits and N(0, 0.4) per expert) 125 us, and 119 with a
 // workgroup of its own for every item, which the hardware starts as others end; this way 112.  Even counts 82 / 83 / 82.  With more
-// rounds the differences even out.  A lane per item; the look brings the first item with it.
-__device__ __forceinline__ int second_item(const MoeGemmParams& P, int first, int run, int slot, int lane, WorkItem& it) {
+// rounds the differences even out.  A lane per item, while the first records are on their way (ahead of them a launch took 1 us more).
+__device__ __forceinline__ int second_item(const MoeGemmParams& P, int first, int run, int slot, int lane) {
     const WorkItem mine = work_item(P, first + min(lane, run - 1));
     const uint64_t heavy = __ballot(lane < run && mine.pos_end - mine.pos_begin > 32);
-    it = {__builtin_amdgcn_readlane(mine.e, slot), __builtin_amdgcn_readlane(mine.part, slot),
-          __builtin_amdgcn_readlane(mine.pos_begin, slot), __builtin_amdgcn_readlane(mine.pos_end, slot)};
     const uint32_t before = (1u << slot) - 1, long0 = (uint32_t)heavy, long1 = (uint32_t)(heavy >> kCusPerXcd);
     const uint32_t short1 = ~(uint32_t)0 >> (2 * kCusPerXcd - run) & ~long1; // (run > kCusPerXcd)
     const int rank = long0 >> slot & 1 ? __popc(~long0) + __popc(long0 & before) : __popc(~long0 & before), longs = __popc(long1);
@@ -503,16 +501,15 @@ __global__ __launch_bounds__(64 * kWaves) void moe_gemm_q4k_kernel(MoeGemmParams
     // The first item's weights, the first items' tables, the first steps' records
     const uint32_t slots16 = (uint32_t)P.slots * 16u;
     const uint32_t lane_off = (uint32_t)((lane >> 4) & 1) * (uint32_t)P.k_groups * (uint32_t)P.panel_bytes + (uint32_t)(lane & 15) * 16u;
-    WorkItem it0;
-    if (two_rounds) second = second_item(P, first, run, slot, lane, it0), t.n_items = second < 0 ? 1 : 2;
-    else it0 = work_item(P, first + local_item(0));
-    first_panels<GATE_UP>(P, it0, wave, t.wp);
+    first_panels<GATE_UP>(P, work_item(P, first + local_item(0)), wave, t.wp);
     UnitRegs raw[2];
 #pragma unroll
     for (int c = 0; c < 2; c++) request_unit(raw[c], t.wp[c], lane_off, lane_off + (uint32_t)(lane >> 5) * slots16, slots16);
-    if (wave < kTablesAhead && wave < t.n_items) prepare_item(P, S, work_item(P, first + local_item(wave)), wave, lane);
+    if (wave == 0) prepare_item(P, S, work_item(P, first + local_item(0)), 0, lane);
     static_assert(kAhead == 2);
     request_records(P, t, S, smem, wave, lane);
+    if (two_rounds) second = second_item(P, first, run, slot, lane), t.n_items = second < 0 ? 1 : 2;
+    if (wave > 0 && wave < kTablesAhead && wave < t.n_items) prepare_item(P, S, work_item(P, first + local_item(wave)), wave, lane);
     request_records(P, t, S, smem, wave, lane);
     __builtin_amdgcn_s_waitcnt(wait_vector(0));
     if (wave == 0) count_up(&S.ready[0]); // (the second step's: at the top of the loop)
