@@ -1959,17 +1959,21 @@ struct RoutingOut {
 // and 58 / 60 at 14.  With up to twelve units (inter 1024: 48 / 47, 48 / 48 and 52 / 53 at 9; inter 768: 46 / 46, 46 / 47
 // and 48 / 52) or workgroups for half of the compute units (32 experts, inter 1536: 66 / 66 at 9, 66 / 72 at 10; 64 experts,
 // inter 2048: 127 / 137) nine are enough.
-// From 16 experts on, more than eight: some expert has its second tile of 16 rows there, and here a workgroup takes its items in turn.
-// Tiles / this at 8.1 to 8.95 pairs, means of four routings: 128 experts top-8 of 2048 x 768 99 / 97 us (up to 1.4 % slower where no
-// expert has a second tile, 6 % faster where one has), 256 of 2048 x 512 138 / 125, 64 of 2048 x 1024 73 / 65, 64 of 2048 x 2048 112 / 112, 32 of
-// 2048 x 1536 62 / 58, 16 of 1024 x 1024 41 / 37, 16 of 2048 x 768 45 / 44, 128 of 512 x 256 40 / 30.  At eight and fewer the tiles:
-// 128 of 2048 x 768 90 / 96, 32 of 2048 x 1536 55 / 57, 16 of 1024 x 1024 30 / 37.
+// From 48 experts on, and from 16 with up to four units: above eight, where some expert has its second tile of 16 rows.  Tiles /
+// this at 8.1 to 8.95 pairs: 128 experts top-8 of 2048 x 768 100 / 99 to 106 / 98 us, 256 of 2048 x 512 132 / 125 to 140 / 125, 64 of 2048 x 1024
+// 76 / 66, 64 of 2048 x 2048 115 / 112 to 118 / 112, 48 of 1024 x 1024 52 / 41, 16 of 512 x 512 36 / 28; with uneven counts (logits and N(0, 1) per
+// expert) 135 / 100, 286 / 113, 82 / 68, 120 / 110, 58 / 51 and 40 / 34.  At eight and fewer the tiles: 128 of 2048 x 768 90 / 96, 16 of
+// 1024 x 1024 30 / 37.  Fewer experts wait for nine: 16 of 2048 x 768 with even counts 45.5 / 44.5, 32 50 / 47 and of 1024 x 1024 45 / 39, but
+// with uneven ones 48 / 56, 49 / 59 and 44 / 49, because an item of more than 32 pairs takes half as long again over all of k.  (Of 48 and
+// more, those whose items leave much of the compute units' last round empty lose as well where counts are even, 72 of 2048 x 1024 86 / 94, 96
+// of 2048 x 768 87 / 90, 60 of 2048 x 1536 94 / 99, but less than the tiles do where they are not: 127 / 68, 135 / 73, 124 / 96.)
 bool moe_on_gemm(const QmmLayout& G, const QmmLayout& D, int64_t t, int top_k, int n_cus) {
-    const int64_t E = G.n_stacked;
-    const bool few_long = G.k_units + D.k_units > 12 && E * (G.n / 256) * 2 <= n_cus;
+    const int64_t E = G.n_stacked, units = G.k_units + D.k_units;
+    const bool few_long = units > 12 && E * (G.n / 256) * 2 <= n_cus;
+    const bool above_eight = E >= 48 || (E >= 16 && units <= 4);
     // (moe_on_tiles: a threshold raised through the environment holds for these kernels too)
     return qmm_moe_expert_form() < 0 && moe_on_tiles(t * top_k, (int)G.n_stacked) &&
-           t * top_k >= (few_long ? 14 * E : E >= 16 ? 8 * E + 1 : 9 * E) && qmm_moe_gemm_supported(G, D, t, top_k);
+           t * top_k >= (few_long ? 14 * E : above_eight ? 8 * E + 1 : 9 * E) && qmm_moe_gemm_supported(G, D, t, top_k);
 }
 
 // moe_core on the kernels of qmm_moe_gemm.hip; workspace: y [pairs, hidden] | the token rows' records | the

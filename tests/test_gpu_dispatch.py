@@ -92,6 +92,14 @@ def test_expert_layers_of_sixteen_experts_and_more():
     assert taken == [False, True, False, True, False]
 
 
+def test_expert_layers_above_eight_pairs_where_uneven_counts_cost():
+    """Fewer than 48 experts with more than four units of k wait for nine pairs per expert."""
+    cases = [["moe", 32, 1024, 1024, 4, 69], ["moe", 32, 1024, 1024, 4, 72], ["moe", 16, 2048, 768, 2, 70], ["moe", 47, 512, 768, 1, 420],
+             ["moe", 48, 512, 768, 1, 420], ["moe", 64, 2048, 2048, 8, 69]]
+    taken = ["moe_gemm_q4k_kernel" in names for names in kernels(cases)]
+    assert taken == [False, True, False, False, True, True]
+
+
 def test_expert_threshold_of_the_environment():
     """IZWI_QMM_MOE_MFMA_MIN_ROWS: below that many pairs per expert no matrix-core kernel, the products included."""
     case = ["moe", 8, 512, 512, 2, 80]  # 20 pairs per expert
