@@ -284,6 +284,9 @@ def test_qk_norm_rope_append_equals_the_separate_hooks(qa, oracle, heads, kv_hea
     (32, 8, 128, 0, 4), (32, 8, 128, 5, 9), (32, 8, 128, 300, 512), (32, 8, 128, 4095, 4096), (32, 8, 128, 1000, 1001),
     (8, 8, 64, 77, 100), (6, 3, 256, 130, 200), (4, 4, 128, 64, 65), (16, 8, 128, 127, 256), (16, 8, 128, 128, 256),
     (16, 8, 128, 319, 320), (16, 8, 128, 320, 512), (4, 2, 64, 255, 256), (320, 160, 64, 40, 41),
+    # four, two and one workgroups per head, on both sides of 128 positions
+    (64, 8, 128, 63, 64), (64, 8, 128, 200, 256), (65, 13, 128, 127, 128), (100, 10, 128, 40, 41), (100, 10, 128, 255, 256), (128, 16, 64, 130, 256),
+    (136, 8, 128, 40, 41), (136, 8, 128, 127, 128), (136, 8, 128, 199, 256), (256, 16, 128, 128, 129),
 ])
 def test_decode_attention_step_equals_prep_then_attention(qa, oracle, heads, kv_heads, d, pos, cap):
     """The one-call form (q/k norm, rotary and cache append inside the attention launch) against the two
