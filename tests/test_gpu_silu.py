@@ -1,4 +1,5 @@
-"""silu(gate) * up over the whole range of f32 arguments, where the kernels share one definition: v / (1 + expf(-v)) in f32."""
+"""silu(gate) * up over the whole range of f32 arguments; the kernels share one definition, which is to be no further off than
+v / (1 + expf(-v)) in f32."""
 import numpy as np
 import pytest
 
