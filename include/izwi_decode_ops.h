@@ -97,7 +97,7 @@ int izwi_qk_norm_rope_append_f32(const float* q, const float* k, const float* v,
  * (key, value) as position `pos` and appends them to the caches on its way.  Arguments as
  * izwi_qk_norm_rope_append_f32 (without q_out) and izwi_decode_gqa_attention_f32 with
  * kv_len = pos + 1; out is `[num_heads, head_dim]`.  Results are those of the two calls bit for bit
- * (the same arithmetic in the same order).  Device pointers only; head_dim 64, 128 or 256. */
+ * (the same arithmetic in the same order) where out shares no memory with the inputs.  Device pointers only; head_dim 64, 128 or 256. */
 int izwi_decode_attention_step_f32(const float* q, const float* k, const float* v, const float* qk_weight,
                                    const float* cos_sin, int64_t num_heads, int64_t num_kv_heads,
                                    int64_t head_dim, float eps, float* k_cache, float* v_cache,
@@ -111,7 +111,7 @@ int izwi_decode_attention_step_f32(const float* q, const float* k, const float* 
  * softmax_p((q . k_p) * scale) . v.  The reference's shader refuses kv_len > 2048; here the
  * positions are split over workgroups and merged (any kv_len).  head_dim must be 64, 128 or 256
  * (IZWI_QMM_ERR_UNSUPPORTED otherwise).  Uses the library's per-stream scratch when the positions
- * are split. */
+ * are split.  With out == q a short cache takes another form of the kernel, whose f32 sums are in another order. */
 int izwi_decode_gqa_attention_f32(const float* q, const float* k, const float* v, int64_t num_heads,
                                   int64_t num_kv_heads, int64_t head_dim, int64_t kv_len,
                                   int64_t kv_capacity, float scale, float* out, int mem_space,

@@ -742,7 +742,10 @@ __global__ __launch_bounds__(256) void attn_partial_kernel(AttnParams<T> P) {
 // Where it is taken (us a decode layer in a graph when the line was drawn, splits and their merge / one workgroup per head, at 33,
 // 128, 256, 300 and 320 positions): 16 query heads on 8 20.8 / 18.1, 21.0 / 19.1, 20.8 / 20.6, 20.9 / 21.1, 20.9 / 21.0; 32 on 8
 // 51.7 / 46.8, 51.7 / 48.4, 51.7 / 50.3, 51.8 / 50.9, 51.8 / 51.2; 40 on 8 52.3 / 50.4, 52.4 / 52.0, 53.3 / 53.5, 53.3 / 54.2,
-// 53.3 / 54.3.  And a head per compute unit at the most.
+// 53.3 / 54.3.  And a head per compute unit at the most.  (With the values shared out the two meet further on: us a call in a graph,
+// splits and merge / this, at 320, 448, 512 and 768 positions, 16 on 8 5.7 / 4.2, 5.8 / 4.9, 5.8 / 5.9, 6.3 / 7.6; 32 on 8 7.5 / 5.1, 7.6 / 5.9, 7.7 / 6.4,
+// 8.0 / 8.1; 40 on 8 6.0 / 5.0, 6.2 / 6.0, 6.6 / 6.5, 7.1 / 8.2; 100 on 10 7.8 / 6.6, 8.6 / 8.1, 9.0 / 9.0, 9.8 / 11.7; 8 on 8 of 64 elements 4.5 / 3.6,
+// 4.6 / 3.9, 4.6 / 4.2, 4.9 / 5.1.  The line has not been moved.)
 constexpr int kOneLaunchPositions = 320;
 inline int one_launch_positions(int64_t head_dim, int g) { return head_dim == 128 && g == 1 ? 256 : kOneLaunchPositions; }
 template <typename T, int HD, bool PREP, int W, int NB, int VS>

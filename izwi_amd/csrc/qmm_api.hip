@@ -1954,9 +1954,11 @@ struct RoutingOut {
 // 32 rows at least, over all of k) is not paid back.
 // A workgroup walks all of k alone, about 2.3 us per unit of both products together, whether its neighbours are idle
 // or not, where the tile form cuts an expert's rows into more parts when experts are few.  So few experts with a
-// long k wait for fourteen: hidden 2048, inter 2048, 4, 8 and 16 experts 57 / 53, 60 / 55 and 64 / 59 us at 9 pairs, 57 / 54,
-// 59 / 62 and 64 / 61 at 12, 57 / 61, 60 / 63 and 63 / 67 at 14; inter 1536 52 / 50, 54 / 51 and 58 / 54 at 9, 52 / 57, 54 / 58
-// and 58 / 60 at 14.  With up to twelve units (inter 1024: 48 / 47, 48 / 48 and 52 / 53 at 9; inter 768: 46 / 46, 46 / 47
+// long k wait for fourteen, where the products are ahead at all of them: tiles / products, hidden 2048, inter 2048, 4, 8 and 16 experts
+// 51 / 55, 52 / 56 and 57 / 59 us at 9 pairs, 51 / 55, 52 / 55 and 61 / 59 at 11, 56 / 55, 60 / 56 and 63 / 59 at 13, 59 / 55, 60 / 56 and
+// 64 / 59 at 14; inter 1536 48 / 50, 49 / 51 and 52 / 53 at 9, 48 / 50, 49 / 51 and 55 / 53 at 11, 52 / 51, 55 / 51 and 57 / 53 at 13, 55 / 51, 55 / 51
+// and 58 / 53 at 14.  (The line was drawn for items as workgroups of their own; for these it would lie between 10 and 13.)  With up to
+// twelve units (as first built, inter 1024: 48 / 47, 48 / 48 and 52 / 53 at 9; inter 768: 46 / 46, 46 / 47
 // and 48 / 52) or workgroups for half of the compute units (32 experts, inter 1536: 66 / 66 at 9, 66 / 72 at 10; 64 experts,
 // inter 2048: 127 / 137) nine are enough.
 // From 48 experts on, and from 16 with up to four units: above eight, where some expert has its second tile of 16 rows.  Tiles /

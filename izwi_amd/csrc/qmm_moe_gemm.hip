@@ -29,9 +29,10 @@
 // 7250 cycles that a unit takes; and by the clock, which falls to 1.45 to 1.75 GHz under it.  (A start of the items with the long ones
 // first at every size, 3 % fewer cycles at the end of a launch, was therefore no faster.)
 // 128 experts, top-8, 2048 x 768, layer: items as workgroups of their own, each with its records over all of k, 7 to 8 of 42 us of
-// a gate | up item and 7 of 18 of a down item before the first unit was done / now: 106 / 101 us at 150 tokens, 127 / 120 at 512,
-// 180 / 168 at 1024, 282 / 266 at 2048, 505 / 471 at 4096.  Each wave requesting its share of every step's records instead:
-// 8200 cycles a unit, 486 us at 4096.
+// a gate | up item and 7 of 18 of a down item before the first unit was done / now: 108 / 102 us at 256 tokens, 133 / 124 at 512,
+// 185 / 169 at 1024, 281 / 265 at 2048, 498 / 471 at 4096, where 32 % of gate | up's cycles and 39 % of down's still pass outside the units
+// (finish, exchange of silu(gate) * up, stores, the last round).  Each wave requesting its share of every step's records instead of
+// one in turn: 8200 cycles a unit, 486 us at 4096 when the one in turn took 471.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -592,14 +593,16 @@ hipError_t launch(const MoeGemmParams& P, int64_t max_chunks, hipStream_t stream
 }
 
 // An item of up to 32 pairs is done in two thirds of the time of a longer one, and at one to four items per compute
-// unit a launch ends with whoever started a long one last.  Long ones first pays where short items fill the last round: the kernel
+// unit a launch ends with whoever has the most of them.  Long ones first pays where short items fill the last round: the kernel
 // sees the counts and decides per XCD.  Here only where such counts are likely, because looking costs half a microsecond: around the 22 to
 // 32 pairs per expert at which a few to half of the experts have more than 32, and at 61 to 72, where many spill a short second chunk.
 // Set apart from the first that chunk reads its weights again, so there half as many short items again as the last round has places are
-// asked for (29 for 29 cost 3 %); from 80 pairs on it never pays (1500 tokens 250 / 263, 4096 521 / 542).  us of gate | up (top-8, k =
-// 2048) over the order of the experts, by pairs per expert: 128 experts x 768 -10 at 24 to 30, -21 at 64, -7 at 72; 192 x 512 -10 and
-// -20; 256 x 512 -9 at 24 to 28, +5 to +7 at 61 and 64, -13 at 72; 160 x 768 -9 at 28, +4 at 64, -16 at 72.  Not for down, whose items
-// are short already: 3 less to 3 us more, 5 at 256 experts.
+// asked for (29 for 29 cost 3 % when items were workgroups of their own; from 80 pairs on it never paid there).  us a layer (k = 2048), places that
+// heed lengths in two rounds alone / this, even counts: 128 experts x 768 at 24, 28, 61, 64, 68 and 72 pairs 126 / 119, 127 / 119, 188 / 179,
+// 198 / 191, 208 / 215, 211 / 215; 192 x 512 131 / 127, 135 / 133, 184 / 184, 215 / 207, 217 / 219, 224 / 229; 256 x 512 161 / 155, 163 / 158, then the
+// same within 1 %; 160 x 768 148 / 145, then the same; 32 x 1536 78 / 78, 79 / 79, 102 / 99, 116 / 116, 115 / 118, 115 / 121.  Uneven counts (logits
+// and N(0, 0.5) per expert) 0.92 to 1.02, where the last two columns of 32 x 1536 are 118 / 119 and 123 / 122.  Over 144 such layers 0.987.  Not for down,
+// whose items are short already: 3 less to 3 us more when it was drawn, 5 at 256 experts.
 // Returns twice the short items per place that the last round asks for, 0: the order of the experts.
 int long_items_first(const MoeGemmParams& P, int64_t pairs) {
     const int64_t per_expert = pairs / P.n_experts;
